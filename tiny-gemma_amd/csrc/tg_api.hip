@@ -235,38 +235,53 @@ struct tg_model {
 
 namespace {
 // Device copy of the balanced work list of the causal (window < 0) or the local prefill layers of S tokens, with
-// its scratch.
+// its scratch.  The buffers grow on demand and are kept: the portions of a conversation all have lists of their own, and
+// hipMalloc / hipFree of five buffers would cost more than the portion's attention.
 struct AttnPlanDev {
 	TgAttnPrefillPlan p;
 	bool use = false;
-	int S = -1, tq = 0, window = -1;  // what the lists were built for
+	int S = -1, tq = 0, window = -1, past = 0;  // what the lists were built for
 	void *bufs[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
+	size_t caps[5] = {0, 0, 0, 0, 0};
 	std::vector<int4> items, split;  // host copies stay alive until the uploads have completed
 	std::vector<int2> tiles;
-	int build(int n_tokens, int win) {
+	int build(int n_tokens, int win, int n_past = 0) {
 		const int tile = tg_attn_prefill_query_tile(n_tokens, g_n_cu);
-		if (n_tokens == S && tile == tq && win == window) return TG_OK;
-		release();
-		const int rc = build_uncached(n_tokens, tile, win);
-		if (rc != TG_OK) release();  // nothing half-built stays behind as a cache hit
-		return rc;
-	}
-	int build_uncached(int n_tokens, int tile, int win) {
-		int nslots = 0;
-		use = tg_attn_prefill_plan(n_tokens, g_n_cu, tile, win, items, split, nslots);
+		if (n_tokens == S && tile == tq && win == window && n_past == past) return TG_OK;
+		S = -1;  // nothing half-built stays behind as a cache hit
+		use = false;
+		if (int rc = build_uncached(n_tokens, tile, win, n_past)) {
+			release();
+			return rc;
+		}
 		S = n_tokens;
 		tq = tile;
 		window = win;
+		past = n_past;
+		return TG_OK;
+	}
+	int need(int i, size_t bytes) {
+		if (bytes <= caps[i]) return TG_OK;
+		if (bufs[i]) (void)hipFree(bufs[i]);  // waits for the launches that use it
+		bufs[i] = nullptr;
+		caps[i] = 0;
+		TG_HIP(hipMalloc(&bufs[i], bytes));
+		caps[i] = bytes;
+		return TG_OK;
+	}
+	int build_uncached(int n_tokens, int tile, int win, int n_past) {
+		int nslots = 0;
+		use = tg_attn_prefill_plan(n_tokens, g_n_cu, tile, win, items, split, nslots, n_past);
 		if (!use) return TG_OK;
-		TG_HIP(hipMalloc(&bufs[0], items.size() * sizeof(int4)));
-		TG_HIP(hipMalloc(&bufs[1], split.size() * sizeof(int4)));
-		TG_HIP(hipMalloc(&bufs[2], tg_attn_prefill_part_floats(nslots, tile) * sizeof(float)));
-		TG_HIP(hipMalloc(&bufs[3], tg_attn_prefill_ml_floats(nslots, tile) * sizeof(float)));
-		TG_HIP(hipMemcpyAsync(bufs[0], items.data(), items.size() * sizeof(int4), hipMemcpyHostToDevice, g_stream));
-		TG_HIP(hipMemcpyAsync(bufs[1], split.data(), split.size() * sizeof(int4), hipMemcpyHostToDevice, g_stream));
 		tiles.assign((size_t)((n_tokens + tile - 1) / tile), int2{-1, 1});
 		for (const int4 &sp : split) tiles[(size_t)sp.x] = int2{sp.y, sp.z};
-		TG_HIP(hipMalloc(&bufs[4], tiles.size() * sizeof(int2)));
+		if (int rc = need(0, items.size() * sizeof(int4))) return rc;
+		if (int rc = need(1, split.size() * sizeof(int4))) return rc;
+		if (int rc = need(2, tg_attn_prefill_part_floats(nslots, tile) * sizeof(float))) return rc;
+		if (int rc = need(3, tg_attn_prefill_ml_floats(nslots, tile) * sizeof(float))) return rc;
+		if (int rc = need(4, tiles.size() * sizeof(int2))) return rc;
+		TG_HIP(hipMemcpyAsync(bufs[0], items.data(), items.size() * sizeof(int4), hipMemcpyHostToDevice, g_stream));
+		TG_HIP(hipMemcpyAsync(bufs[1], split.data(), split.size() * sizeof(int4), hipMemcpyHostToDevice, g_stream));
 		TG_HIP(hipMemcpyAsync(bufs[4], tiles.data(), tiles.size() * sizeof(int2), hipMemcpyHostToDevice, g_stream));
 		p.items = (const int4 *)bufs[0];
 		p.split = (const int4 *)bufs[1];
@@ -279,14 +294,16 @@ struct AttnPlanDev {
 	}
 	const TgAttnPrefillPlan *get() const { return use ? &p : nullptr; }
 	void release() {
-		for (void *&b : bufs) {
-			if (b) (void)hipFree(b);
-			b = nullptr;
+		for (int i = 0; i < 5; i++) {
+			if (bufs[i]) (void)hipFree(bufs[i]);
+			bufs[i] = nullptr;
+			caps[i] = 0;
 		}
 		use = false;
 		S = -1;
 		tq = 0;
 		window = -1;
+		past = 0;
 	}
 };
 }  // namespace
@@ -343,6 +360,7 @@ struct tg_session {
 	void *pf_ws = nullptr;
 	size_t pf_ws_bytes = 0;
 	AttnPlanDev pf_plan, pf_plan_local;
+	AttnPlanDev ext_plan, ext_plan_local;  // the same for the last later portion (tg_forward_tokens)
 	// one-kernel decode step (tg_decode_fused.hip): built on first use; fused_state 0 = not built yet, 1 = usable,
 	// -1 = not usable for this model or device, or a wait timed out (the session then stays on the launch path)
 	int fused_state = 0, fused_variant = -1;
@@ -358,6 +376,8 @@ struct tg_session {
 namespace {
 constexpr int ATTN_MAX_BLOCKS = TG_ATTN_MAX_BLOCKS;
 constexpr int PREFILL_TAP_MAX_ROWS = 1024;
+// A later portion of a Gemma model goes through the kernels of a prompt from this many tokens on, below it token by token.
+constexpr int TG_EXTEND_MIN = 4;
 
 bool layer_is_local(const tg_config &c, int l) { return (l % c.window_pattern) != (c.window_pattern - 1); }  // transformer.hpp:43
 
@@ -922,6 +942,8 @@ void tg_session_destroy(tg_session *s) {
 		if (p) (void)hipFree(p);
 	s->pf_plan.release();
 	s->pf_plan_local.release();
+	s->ext_plan.release();
+	s->ext_plan_local.release();
 	tg_net_seq_free(s->seq);
 	for (float *p : s->kc)
 		if (p) (void)hipFree(p);
@@ -1943,6 +1965,8 @@ int tg_session_release_workspace(tg_session *s) {
 	s->tap_rows = 0;
 	s->pf_plan.release();
 	s->pf_plan_local.release();
+	s->ext_plan.release();
+	s->ext_plan_local.release();
 	return TG_OK;
 }
 
@@ -2166,9 +2190,10 @@ struct PrefillCtx {
 	const TgAttnPrefillPlan *plan_global = nullptr, *plan_local = nullptr;
 	int o_parts = 1, d_parts = 1;
 	size_t tpart = 0;
+	int at = -1;             // position of the first row of a later portion (-1: a whole prompt from an empty session)
 };
 
-int prefill_setup(tg_session *s, int n, PrefillCtx *ctx, bool with_taps) {
+int prefill_setup(tg_session *s, int n, PrefillCtx *ctx, bool with_taps, int at = -1) {
 	tg_model *m = s->m;
 	const tg_config &c = m->cfg;
 	const int L = c.n_layers, h = c.hidden_size, f = c.intermediate_size, hd = c.head_dim;
@@ -2218,14 +2243,22 @@ int prefill_setup(tg_session *s, int n, PrefillCtx *ctx, bool with_taps) {
 	ctx->amax = g_gemm_mfma ? (float *)(ws + o_amax) : nullptr;  // max|hb| per row, folded by the up|gate product
 	s->taps = tap_rows ? (float *)(ws + o_taps) : nullptr;
 	s->tap_rows = tap_rows;
-	// Work lists of the attention launches.  A local layer whose window covers the whole prompt is a causal layer.
-	const bool local_is_causal = n <= c.n_pos_local + 1;
-	if (int rc = s->pf_plan.build(n, -1)) return rc;
-	if (!local_is_causal) {
-		if (int rc = s->pf_plan_local.build(n, c.n_pos_local)) return rc;
+	ctx->at = at;
+	if (at < 0) {
+		// Work lists of the attention launches.  A local layer whose window covers the whole prompt is a causal layer.
+		const bool local_is_causal = n <= c.n_pos_local + 1;
+		if (int rc = s->pf_plan.build(n, -1)) return rc;
+		if (!local_is_causal) {
+			if (int rc = s->pf_plan_local.build(n, c.n_pos_local)) return rc;
+		}
+		ctx->plan_global = s->pf_plan.get();
+		ctx->plan_local = local_is_causal ? ctx->plan_global : s->pf_plan_local.get();
+	} else {
+		if (int rc = s->ext_plan.build(n, -1, at)) return rc;
+		if (int rc = s->ext_plan_local.build(n, c.n_pos_local - 1, std::min(at, c.n_pos_local - 1))) return rc;
+		ctx->plan_global = s->ext_plan.get();
+		ctx->plan_local = s->ext_plan_local.get();
 	}
-	ctx->plan_global = s->pf_plan.get();
-	ctx->plan_local = local_is_causal ? ctx->plan_global : s->pf_plan_local.get();
 	// products that would otherwise leave most compute units idle (a badly filled last round of workgroups; a short
 	// prompt's long-K products) run in 2 or 4 parts of K with separate partial results; the norm that consumes them adds
 	// the parts
@@ -2260,6 +2293,35 @@ void prefill_attention_launches(const PrefillCtx &p, int l) {
 	const int mp = s->max_pos[(size_t)l];
 	// Q|K|V (modules.hpp:106-108)
 	launch_gemm(p.qkv, p.xn, h, Ld.qkv, n, TG_EPI_STORE, nullptr, 0, 0, 0, p.apack, p.rowscale, p.pk);
+	if (p.at >= 0) {
+		// A later portion sees what its tokens would see one by one: the keys of the cache, in a local layer at most
+		// n_pos_local with the token's own, and enters the cache in the slots it would take then (KVCache::update_single,
+		// decode.hpp:49-70), behind the attention.
+		const float *cs = Ld.is_sw ? s->cos_l : s->cos_g, *sn = Ld.is_sw ? s->sin_l : s->sin_g;
+		const size_t row0 = (size_t)p.at * (hd / 2);
+		tg_launch_qk_norm_rope_rows(p.qkv, p.qkv + qo, p.qkv + qo + hd, Ld.rms_q, Ld.rms_k, cs + row0, sn + row0, nullptr, nullptr, mp, n, c.n_head, hd, nq,
+		                            nq, g_stream);
+		const int bp = Ld.is_sw ? s->bp_local : s->bp_global, slot = bp % mp;
+		TgAttnPast past;
+		past.kc = s->kc[(size_t)l];
+		past.vc = s->vc[(size_t)l];
+		past.n = Ld.is_sw ? std::min(p.at, mp - 1) : p.at;
+		past.ring = mp;
+		past.slot0 = ((bp - past.n) % mp + mp) % mp;
+		const TgAttnPrefillPlan *plan = Ld.is_sw ? p.plan_local : p.plan_global;
+		tg_launch_attn_extend(p.ao, p.qkv, p.qkv + qo, p.qkv + qo + hd, n, nq, nq, qo, Ld.is_sw ? 1 : 0, mp - 1, plan, past, g_n_cu, g_stream);
+		TgCacheRows rows;
+		rows.k = p.qkv + qo;
+		rows.v = p.qkv + qo + hd;
+		rows.kc = s->kc[(size_t)l];
+		rows.vc = s->vc[(size_t)l];
+		rows.ld = nq;
+		rows.slot = slot;
+		rows.ring = mp;
+		tg_launch_attn_prefill_finish(p.ao, n, qo, plan, g_n_cu, p.apack, p.rowscale, g_stream, rows);
+		launch_gemm(p.t, p.ao, qo, Ld.o, n, TG_EPI_STORE, nullptr, 0, 0, 0, p.apack, p.rowscale, p.pk, nullptr, nullptr, p.o_parts, p.tpart);
+		return;
+	}
 	// q/k norm + RoPE from position 0, KV write (modules.hpp:115-121)
 	tg_launch_qk_norm_rope_rows(p.qkv, p.qkv + qo, p.qkv + qo + hd, Ld.rms_q, Ld.rms_k, Ld.is_sw ? s->cos_l : s->cos_g,
 	                            Ld.is_sw ? s->sin_l : s->sin_g, s->kc[(size_t)l], s->vc[(size_t)l], mp, n, c.n_head, hd, nq, nq, g_stream);
@@ -2291,6 +2353,42 @@ void prefill_block_end(const PrefillCtx &p, int nparts, const float *w_post, con
 	const bool planes = p.pk && !want_fp32;
 	tg_launch_norm_rows(planes ? nullptr : p.xn, p.t, nparts, p.tpart, next_pre, w_post, p.x, p.x, p.n, h, planes ? p.apack : nullptr, p.rowscale,
 	                    g_stream, clear_amax ? p.amax : nullptr);
+}
+
+// Embedding and all layers of the context's rows: p.xn = rmsnorm(x, RMSw), the rows that the LM head takes
+int prefill_rows(const PrefillCtx &p, const int32_t *ids) {
+	tg_session *s = p.s;
+	tg_model *m = s->m;
+	const tg_config &c = m->cfg;
+	const int L = c.n_layers, n = p.n;
+	TG_HIP(hipMemcpyAsync(p.d_ids, ids, sizeof(int) * (size_t)n, hipMemcpyHostToDevice, g_stream));
+	tg_launch_embed_rows(p.x, p.d_ids, n, m->wte, m->wte_scales, c.hidden_size, c.n_vocab, g_stream);
+	TG_HIP(prefill_tap(p, 0));
+	// With the int8 MFMA GEMM a norm writes the next GEMM's digit planes itself and the fp32 row is not stored.
+	prefill_first_norm(p, m->L[0].apre, false);
+	for (int l = 0; l < L; l++) {
+		const LayerDev &Ld = m->L[(size_t)l];
+		prefill_attention_launches(p, l);
+		prefill_block_end(p, p.o_parts, Ld.apost, Ld.mpre, false, true);  // also clears the row maxima the up|gate product folds into
+		TG_HIP(prefill_tap(p, 2 * l + 1));
+		prefill_mlp_launches(p, l);
+		// the last layer's final norm feeds the LM head GEMV, which reads the fp32 row
+		const bool last = l + 1 == L;
+		prefill_block_end(p, p.d_parts, Ld.mpost, last ? m->rmsw : m->L[(size_t)l + 1].apre, last, false);
+		TG_HIP(prefill_tap(p, 2 * l + 2));
+	}
+	return TG_OK;
+}
+
+// logits and per-workgroup maxima of one row of p.xn
+void prefill_head(const PrefillCtx &p, int row) {
+	tg_session *s = p.s;
+	TgGemv g = gemv_base(s->m->lm);
+	g.x = p.xn + (size_t)row * s->m->cfg.hidden_size;
+	g.y = s->logits;
+	g.blk_val = s->blk_val;
+	g.blk_idx = s->blk_idx;
+	tg_launch_gemv(g, TG_ROLE_LMHEAD_PLAIN, g_stream);
 }
 
 // KVCache::update_prefill's counters (decode.hpp:99-104) after n tokens
@@ -2325,6 +2423,33 @@ static int net_extend(tg_session *s, const int32_t *ids, int n, const int32_t *w
 	return TG_OK;
 }
 
+// A portion of several tokens of a Gemma model behind whatever the session holds, through the kernels of a prompt.  The token
+// log starts anew with the portion's pick, as behind a prefill.
+static int gemma_extend(tg_session *s, const int32_t *ids, int n, const int32_t *want, int n_want, float *logits, int32_t *argmax) {
+	const size_t V = (size_t)s->m->cfg.n_vocab;
+	PrefillCtx p;
+	if (int rc = prefill_setup(s, n, &p, true, s->pos)) return rc;
+	if (int rc = prefill_rows(p, ids)) return rc;
+	for (int w = 0; w < n_want; w++) {
+		prefill_head(p, want[w]);
+		TG_HIP(hipMemcpyAsync(logits + (size_t)w * V, s->logits, sizeof(float) * V, hipMemcpyDeviceToHost, g_stream));
+	}
+	if (n_want == 0 || want[n_want - 1] != n - 1) prefill_head(p, n - 1);
+	s->pos += n;
+	s->bp_local += n;
+	s->bp_global += n;
+	s->steps = 1;
+	const int ctr[4] = {s->pos, s->bp_local, s->bp_global, 0};
+	TG_HIP(hipMemcpyAsync(s->ctr, ctr, sizeof(ctr), hipMemcpyHostToDevice, g_stream));
+	tg_launch_argmax_finish(s->blk_val, s->blk_idx, s->m->lm.ntiles, s->ctr, s->tok_log, 0, g_stream);
+	TG_HIP(hipGetLastError());
+	int32_t tok = -1;
+	TG_HIP(hipMemcpyAsync(&tok, s->ctr + 4, sizeof(int), hipMemcpyDeviceToHost, g_stream));
+	TG_HIP(hipStreamSynchronize(g_stream));
+	if (argmax) *argmax = tok;
+	return TG_OK;
+}
+
 int tg_forward_tokens(tg_session *s, const int32_t *ids, int n, const int32_t *want, int n_want, float *logits, int32_t *argmax) {
 	if (!s || !ids || n_want < 0 || (n_want > 0 && (!want || !logits))) return tg_fail(TG_ERR_BAD_ARG, "bad argument");
 	if (int rc = session_usable(s)) return rc;
@@ -2337,9 +2462,10 @@ int tg_forward_tokens(tg_session *s, const int32_t *ids, int n, const int32_t *w
 	if (s->pos + n > s->capacity) return tg_fail(TG_ERR_STATE, "context is full (n_pos)");
 	flush_pick(s);
 	if (s->m->net && n > 1) return net_extend(s, ids, n, want, n_want, logits, nullptr, argmax);
-	// a whole prompt of which only the end is wanted is a prefill; anything else of a Gemma model goes token by token
+	// a whole prompt of which only the end is wanted is a prefill
 	if (!s->m->net && s->pos == 0 && n > 1 && (n_want == 0 || (n_want == 1 && want[0] == n - 1)))
 		return tg_forward_prefill(s, ids, n, n_want ? logits : nullptr, argmax);
+	if (!s->m->net && n >= TG_EXTEND_MIN && g_gemm_mfma && g_attn_prefill_split) return gemma_extend(s, ids, n, want, n_want, logits, argmax);
 	for (int i = 0, w = 0; i < n; i++) {
 		const bool is = w < n_want && want[w] == i;
 		if (int rc = tg_forward_decode(s, ids[i], is ? logits + (size_t)w * c.n_vocab : nullptr, argmax)) return rc;
@@ -2357,36 +2483,11 @@ int tg_forward_prefill(tg_session *s, const int32_t *ids, int n, float *logits, 
 	if (s->pos != 0) return tg_fail(TG_ERR_STATE, "prefill needs an empty session (decode.hpp:78-79)");
 	if (n > s->capacity) return tg_fail(TG_ERR_STATE, "prompt longer than n_pos");
 	if (m->net) return net_extend(s, ids, n, nullptr, 0, nullptr, logits, argmax);
-	const int L = c.n_layers, h = c.hidden_size;
-	const size_t S = (size_t)n;
 	PrefillCtx p;
 	if (int rc = prefill_setup(s, n, &p, true)) return rc;
-	TG_HIP(hipMemcpyAsync(p.d_ids, ids, sizeof(int) * S, hipMemcpyHostToDevice, g_stream));
-	tg_launch_embed_rows(p.x, p.d_ids, n, m->wte, m->wte_scales, h, c.n_vocab, g_stream);
-	TG_HIP(prefill_tap(p, 0));
-	// With the int8 MFMA GEMM a norm writes the next GEMM's digit planes itself and the fp32 row is not stored.
-	prefill_first_norm(p, m->L[0].apre, false);
-	for (int l = 0; l < L; l++) {
-		const LayerDev &Ld = m->L[(size_t)l];
-		prefill_attention_launches(p, l);
-		prefill_block_end(p, p.o_parts, Ld.apost, Ld.mpre, false, true);  // also clears the row maxima the up|gate product folds into
-		TG_HIP(prefill_tap(p, 2 * l + 1));
-		prefill_mlp_launches(p, l);
-		// the last layer's final norm feeds the LM head GEMV, which reads the fp32 row
-		const bool last = l + 1 == L;
-		prefill_block_end(p, p.d_parts, Ld.mpost, last ? m->rmsw : m->L[(size_t)l + 1].apre, last, false);
-		TG_HIP(prefill_tap(p, 2 * l + 2));
-	}
-	// LM head on the last position only (modules.hpp:232-240): xn already holds rmsnorm(x, RMSw)
-	{
-		TgGemv g = gemv_base(m->lm);
-		g.x = p.xn + (S - 1) * h;
-		g.y = s->logits;
-		g.blk_val = s->blk_val;
-		g.blk_idx = s->blk_idx;
-		tg_launch_gemv(g, TG_ROLE_LMHEAD_PLAIN, g_stream);
-		tg_launch_argmax_finish(s->blk_val, s->blk_idx, m->lm.ntiles, s->ctr, s->tok_log, 0, g_stream);
-	}
+	if (int rc = prefill_rows(p, ids)) return rc;
+	prefill_head(p, n - 1);  // on the last position only (modules.hpp:232-240)
+	tg_launch_argmax_finish(s->blk_val, s->blk_idx, m->lm.ntiles, s->ctr, s->tok_log, 0, g_stream);
 	TG_HIP(hipGetLastError());
 	s->steps = 1;
 	if (int rc = set_counters_after_prefill(s, n)) return rc;

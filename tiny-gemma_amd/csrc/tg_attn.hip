@@ -97,7 +97,7 @@ __global__ __launch_bounds__(ANT) void attn_merge_kernel(const TgAttnDecode a, f
 
 // One workgroup per prompt position: q heads and k normalised + rotated in place
 // (modules.hpp:115-119), k/v rows of the last min(S, max_pos) positions copied to cache slots
-// 0.. (KVCache::update_prefill, decode.hpp:72-105).
+// 0.. (KVCache::update_prefill, decode.hpp:72-105); a later portion (kc null) enters the cache behind its attention.
 __global__ __launch_bounds__(ANT) void qk_norm_rope_rows_kernel(float *q, float *k, const float *v, const float *rms_q,
                                                                 const float *rms_k, const float *cos_t, const float *sin_t,
                                                                 float *kc, float *vc, int max_pos, int S, int ldq, int ldkv) {
@@ -108,7 +108,7 @@ __global__ __launch_bounds__(ANT) void qk_norm_rope_rows_kernel(float *q, float 
 	norm_rope_head(qrow, rms_q, cs, sn, 1.0f, o, lane);
 #pragma unroll
 	for (int i = 0; i < 4; i++) qrow[lane + 64 * i] = o[i];
-	const int start = (S >= max_pos) ? S - max_pos : 0;
+	const int start = kc == nullptr ? S : (S >= max_pos) ? S - max_pos : 0;
 	float *krow = k + (size_t)s * ldkv;
 	if (w == 0) {
 		norm_rope_head(krow, rms_k, cs, sn, 1.0f, o, lane);

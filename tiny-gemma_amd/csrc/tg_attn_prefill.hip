@@ -334,10 +334,15 @@ constexpr int NT32 = HD / 32;  // k steps of a score product
 // with its own four waves (heads).  QG = 2: a K/V tile is fetched, split and staged once for 32 queries x 4 heads,
 // and the two waves a SIMD then holds overlap each other's LDS reads, matrix and vector work; the launcher takes it
 // for prompts long enough to keep the compute units busy with such workgroups, else QG = 1.
-template <int QG, typename F>
+//
+// PAST: the S queries stand behind `past.n` keys that the session's cache holds already (a later portion of a sequence).
+// Key j of the launch is then cache row (past.slot0 + j) mod past.ring for j < past.n and row j - past.n of k / v (the
+// portion's own keys, not yet in the cache: a local layer's ring still holds the keys they will overwrite, which the first
+// queries need) from there on; the key ranges of the work list count from the first cached key.
+template <int QG, typename F, bool PAST>
 __global__ __launch_bounds__(256 * QG) void attn_prefill_split_kernel(float *o, const float *q, const float *k, const float *v, int S, int ldq,
                                                                 int ldkv, int ldo, int is_sw, int window, const int4 *items,
-                                                                float *part_o, float *part_ml, int *range_flag) {
+                                                                float *part_o, float *part_ml, int *range_flag, TgAttnPast past) {
 	typedef typename F::vec vec;
 	typedef PlanesT<F> Planes;
 	extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -356,11 +361,12 @@ __global__ __launch_bounds__(256 * QG) void attn_prefill_split_kernel(float *o, 
 		q0 = item.x * BQ;
 		slot = item.w;
 	}
-	const int q0w = q0 + 16 * qh;  // first query of this wave's group
-	const int qpos = q0w + c;
-	const int qrow = qpos < S ? qpos : S - 1;
-	int kb = (is_sw && q0 > window) ? q0 - window : 0;
-	int ke = (q0 + BQ < S) ? q0 + BQ : S;  // exclusive
+	const int np = PAST ? past.n : 0;  // keys in front of query 0
+	const int q0w = q0 + 16 * qh;      // first query of this wave's group
+	const int qrow = q0w + c < S ? q0w + c : S - 1;
+	const int qpos = np + q0w + c;     // the query's own key
+	int kb = (is_sw && np + q0 > window) ? np + q0 - window : 0;
+	int ke = np + ((q0 + BQ < S) ? q0 + BQ : S);  // exclusive
 	if (items != nullptr) {
 		kb = item.y * TK;
 		ke = min(ke, item.z * TK);
@@ -375,12 +381,18 @@ __global__ __launch_bounds__(256 * QG) void attn_prefill_split_kernel(float *o, 
 	const int sv_g = w & 3, sv_d = 64 * (w >> 2) + lane;
 	f32x4 kpre[SU][2];
 	float vpre[SU][8];
-	auto key_row = [&](int tile, int key) {
+	auto key_row = [&](int tile, int key, const float *own, const float *cache) -> const float * {
 		int j = kb + tile * TK + key;
-		return (size_t)(j < ke ? j : ke - 1) * ldkv;
+		j = j < ke ? j : ke - 1;
+		if (PAST && j < np) {
+			int r = past.slot0 + j;
+			r = r < past.ring ? r : r - past.ring;
+			return cache + (size_t)r * HD;
+		}
+		return own + (size_t)(j - np) * ldkv;
 	};
 	auto fetch = [&](int tile) {
-		const float *kp = k + key_row(tile, sk_key) + 8 * sk_g;
+		const float *kp = key_row(tile, sk_key, k, past.kc) + 8 * sk_g;
 #pragma unroll
 		for (int u = 0; u < SU; u++) {
 			kpre[u][0] = *reinterpret_cast<const f32x4 *>(kp + 32 * (sk_t0 + 2 * QG * u));
@@ -388,7 +400,7 @@ __global__ __launch_bounds__(256 * QG) void attn_prefill_split_kernel(float *o, 
 		}
 #pragma unroll
 		for (int sl = 0; sl < 8; sl++) {
-			const float *vp = v + key_row(tile, (sl < 4 ? 4 * sv_g + sl : 12 + 4 * sv_g + sl)) + sv_d;
+			const float *vp = key_row(tile, (sl < 4 ? 4 * sv_g + sl : 12 + 4 * sv_g + sl), v, past.vc) + sv_d;
 #pragma unroll
 			for (int u = 0; u < SU; u++) vpre[u][sl] = vp[64 * QG * u];
 		}
@@ -444,7 +456,7 @@ __global__ __launch_bounds__(256 * QG) void attn_prefill_split_kernel(float *o, 
 		tg_lds_barrier();
 		if (tile + 1 < ntiles) fetch(tile + 1);  // in flight during the products
 		// a tile that starts behind this group's last query holds none of its keys (the other group still needs it)
-		if (kb + tile * TK > q0w + 15) continue;
+		if (kb + tile * TK > np + q0w + 15) continue;
 
 		// ---- scores of the tile's two groups of 16 keys; even and odd k steps in separate accumulators ----
 		f32x4 sa[2][2];
@@ -1275,12 +1287,22 @@ __global__ __launch_bounds__(PNT) void attn_prefill_merge_kernel(float *o, int S
 // merged (as attn_prefill_merge_kernel does), the row maximum over all four heads gives the power-of-two row factor,
 // and the row is written as digit planes.  Two rows per workgroup, a thread = 8 consecutive dims of a row (two waves
 // per row: heads 0-1 and 2-3).  Rows of whole query tiles are read from o, where their workgroup wrote them.
+// cr (a later portion of a sequence, else cr.k is null): the rows' keys and values go into the cache here, the last
+// cr.ring of them, row i into slot (cr.slot + i) mod cr.ring.
 __global__ __launch_bounds__(PNT) void attn_prefill_finish_kernel(const float *o, int S, int ldo, const int2 *tiles, const float *part_o,
-                                                                 const float *part_ml, int tq, int8_t *apack, float *rowfac, int Mpad) {
+                                                                 const float *part_ml, int tq, int8_t *apack, float *rowfac, int Mpad,
+                                                                 TgCacheRows cr) {
 	__shared__ float wmax[PNT / 64];
 	const int tid = threadIdx.x, t = tid & 127, half = tid >> 7;
 	const int row = 2 * (int)blockIdx.x + half, qrow = row < S ? row : S - 1;  // the odd last row is computed twice, written once
 	const int head = t >> 5, d0 = 8 * (t & 31);
+	if (cr.k != nullptr && row < S && row >= S - cr.ring) {  // a portion's keys and values enter the cache behind its attention
+		int r = cr.slot + row % cr.ring;
+		r = r < cr.ring ? r : r - cr.ring;
+		const int at = 4 * (t & 63);
+		const float *src = (t < 64 ? cr.k : cr.v) + (size_t)row * cr.ld + at;
+		*reinterpret_cast<f32x4 *>((t < 64 ? cr.kc : cr.vc) + (size_t)r * HD + at) = *reinterpret_cast<const f32x4 *>(src);
+	}
 	int2 ti = int2{-1, 1};
 	if (tiles != nullptr) ti = tiles[qrow / tq];
 	float v[8];
@@ -1362,10 +1384,10 @@ int tg_attn_prefill_query_tile(int S, int n_cu) {
 	return (g_attn_prefill_split == 2 || (g_attn_prefill_split == 1 && (S + 31) / 32 >= n_cu / 8)) ? 32 : TQ;
 }
 
-bool tg_attn_prefill_plan(int S, int n_cu, int tq, int window, std::vector<int4> &items, std::vector<int4> &split, int &nslots) {
+bool tg_attn_prefill_plan(int S, int n_cu, int tq, int window, std::vector<int4> &items, std::vector<int4> &split, int &nslots, int past) {
 	const int nq = (S + tq - 1) / tq;
-	auto first_tile = [&](int qt) { return (window >= 0 && qt * tq > window) ? (qt * tq - window) / TK : 0; };
-	auto end_tile = [&](int qt) { return (std::min(qt * tq + tq, S) + TK - 1) / TK; };
+	auto first_tile = [&](int qt) { return (window >= 0 && past + qt * tq > window) ? (past + qt * tq - window) / TK : 0; };
+	auto end_tile = [&](int qt) { return (past + std::min(qt * tq + tq, S) + TK - 1) / TK; };
 	long total = 0;
 	int longest = 1;
 	for (int qt = 0; qt < nq; qt++) {
@@ -1398,9 +1420,9 @@ bool tg_attn_prefill_plan(int S, int n_cu, int tq, int window, std::vector<int4>
 	// inside the kernel), the units take the items in list order.  0.05-0.6 ms on the host for 4096-32768 tokens, once
 	// per prompt length and process.
 	if (window < 0 && !one_round) {
-		static std::map<std::tuple<int, int, int>, int> chosen;
+		static std::map<std::tuple<int, int, int>, int> chosen;  // whole prompts only: portions behind a past hardly ever repeat
 		const auto key = std::make_tuple(S, n_cu, tq);
-		const auto hit = chosen.find(key);
+		const auto hit = past == 0 ? chosen.find(key) : chosen.end();
 		if (hit != chosen.end()) {
 			chunk = hit->second;
 		} else {
@@ -1452,7 +1474,7 @@ bool tg_attn_prefill_plan(int S, int n_cu, int tq, int window, std::vector<int4>
 				}
 			}
 			chunk = best_c;
-			chosen[key] = chunk;
+			if (past == 0) chosen[key] = chunk;
 		}
 	}
 	items.clear();
@@ -1506,8 +1528,8 @@ void launch_split(dim3 grid, int tq, bool planes, float *o, const float *q, cons
 	if (!lds_set) {  // more than 64 KB of dynamic LDS needs the opt-in
 		(void)hipFuncSetAttribute(reinterpret_cast<const void *>(attn_prefill_planes_kernel<1, F>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)ring);
 		(void)hipFuncSetAttribute(reinterpret_cast<const void *>(attn_prefill_planes_kernel<2, F>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)ring);
-		(void)hipFuncSetAttribute(reinterpret_cast<const void *>(attn_prefill_split_kernel<1, F>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)staged);
-		(void)hipFuncSetAttribute(reinterpret_cast<const void *>(attn_prefill_split_kernel<2, F>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)staged);
+		(void)hipFuncSetAttribute(reinterpret_cast<const void *>(attn_prefill_split_kernel<1, F, false>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)staged);
+		(void)hipFuncSetAttribute(reinterpret_cast<const void *>(attn_prefill_split_kernel<2, F, false>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)staged);
 		lds_set = true;
 	}
 	if constexpr (std::is_same<F, FmtF16x2>::value) {
@@ -1533,11 +1555,11 @@ void launch_split(dim3 grid, int tq, bool planes, float *o, const float *q, cons
 			hipLaunchKernelGGL((attn_prefill_planes_kernel<1, F>), grid, dim3(256), ring, s, o, q, pw, S, ldq, ldo, is_sw, window, items, po, pml,
 			                   range_flag);
 	} else if (tq == 32) {
-		hipLaunchKernelGGL((attn_prefill_split_kernel<2, F>), grid, dim3(512), staged, s, o, q, k, v, S, ldq, ldkv, ldo, is_sw, window, items, po,
-		                   pml, range_flag);
+		hipLaunchKernelGGL((attn_prefill_split_kernel<2, F, false>), grid, dim3(512), staged, s, o, q, k, v, S, ldq, ldkv, ldo, is_sw, window, items, po,
+		                   pml, range_flag, TgAttnPast{});
 	} else {
-		hipLaunchKernelGGL((attn_prefill_split_kernel<1, F>), grid, dim3(256), staged, s, o, q, k, v, S, ldq, ldkv, ldo, is_sw, window, items, po,
-		                   pml, range_flag);
+		hipLaunchKernelGGL((attn_prefill_split_kernel<1, F, false>), grid, dim3(256), staged, s, o, q, k, v, S, ldq, ldkv, ldo, is_sw, window, items, po,
+		                   pml, range_flag, TgAttnPast{});
 	}
 }
 }  // namespace
@@ -1567,10 +1589,34 @@ void tg_launch_attn_prefill(float *o, const float *q, const float *k, const floa
 	                   plan->part_o, plan->part_ml, tq);
 }
 
+// A later portion of a sequence: S queries behind past.n cached keys.  The planes are the three bf16 ones, whose exponent range
+// is fp32's: a portion has no operand that it could not take, as the decode steps that would otherwise take it have none.
+// Split query tiles are merged by tg_launch_attn_prefill_finish.
+void tg_launch_attn_extend(float *o, const float *q, const float *k, const float *v, int S, int ldq, int ldkv, int ldo, int is_sw, int window,
+                           const TgAttnPrefillPlan *plan, const TgAttnPast &past, int n_cu, hipStream_t s) {
+	static bool lds_set = false;
+	constexpr size_t staged = split_lds_bytes<FmtBf16x3>();
+	if (!lds_set) {
+		(void)hipFuncSetAttribute(reinterpret_cast<const void *>(attn_prefill_split_kernel<1, FmtBf16x3, true>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)staged);
+		(void)hipFuncSetAttribute(reinterpret_cast<const void *>(attn_prefill_split_kernel<2, FmtBf16x3, true>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)staged);
+		lds_set = true;
+	}
+	const int tq = tg_attn_prefill_query_tile(S, n_cu);
+	const dim3 grid(plan ? (unsigned)plan->nitems : (unsigned)((S + tq - 1) / tq));
+	const int4 *items = plan ? plan->items : nullptr;
+	float *po = plan ? plan->part_o : nullptr, *pml = plan ? plan->part_ml : nullptr;
+	if (tq == 32)
+		hipLaunchKernelGGL((attn_prefill_split_kernel<2, FmtBf16x3, true>), grid, dim3(512), staged, s, o, q, k, v, S, ldq, ldkv, ldo, is_sw, window, items,
+		                   po, pml, nullptr, past);
+	else
+		hipLaunchKernelGGL((attn_prefill_split_kernel<1, FmtBf16x3, true>), grid, dim3(256), staged, s, o, q, k, v, S, ldq, ldkv, ldo, is_sw, window, items,
+		                   po, pml, nullptr, past);
+}
+
 void tg_launch_attn_prefill_finish(const float *o, int S, int ldo, const TgAttnPrefillPlan *plan, int n_cu, int8_t *apack, float *rowfac,
-                                   hipStream_t s) {
+                                   hipStream_t s, const TgCacheRows &rows) {
 	const int tq = tg_attn_prefill_query_tile(S, n_cu);
 	hipLaunchKernelGGL(attn_prefill_finish_kernel, dim3((unsigned)((S + 1) / 2)), dim3(PNT), 0, s, o, S, ldo,
 	                   plan ? plan->tiles : nullptr, plan ? plan->part_o : nullptr, plan ? plan->part_ml : nullptr, tq, apack, rowfac,
-	                   (int)tg_gemm_mfma_rows(S));
+	                   (int)tg_gemm_mfma_rows(S), rows);
 }

@@ -254,7 +254,7 @@ void tg_launch_norm_rows(float *out, const float *in, int nparts, size_t part_st
                          float *clear_rows = nullptr);  // clear_rows: S floats set to 0 (row maxima the next product folds into)
 void tg_launch_qk_norm_rope_rows(float *q, float *k, const float *v, const float *rms_q, const float *rms_k, const float *cos_t,
                                  const float *sin_t, float *kc, float *vc, int max_pos, int S, int n_head, int hd, int ldq, int ldkv,
-                                 hipStream_t s);
+                                 hipStream_t s);  // cos_t / sin_t: the tables' row of the first token; kc null: nothing goes into a cache
 // Balanced work list of a prefill layer (device copies of what tg_attn_prefill_plan returns) + scratch.
 struct TgAttnPrefillPlan {
 	const int4 *items;  // [nitems] {query tile, first key tile, end key tile, slot or -1}
@@ -266,7 +266,8 @@ struct TgAttnPrefillPlan {
 extern int g_attn_prefill_split;  // prefill attention: 0 = fp32 matrix path, 1 = split-precision matrix path (two fp16 or three bf16 planes), 2 = the same with 32-query workgroups at any length, 3 = the same with 16-query workgroups at any length
 int tg_attn_prefill_query_tile(int S, int n_cu);  // query positions per workgroup of the kernel a launch will take
 // window < 0: causal layer; else a local layer whose queries see `window` keys before them and themselves
-bool tg_attn_prefill_plan(int S, int n_cu, int tq, int window, std::vector<int4> &items, std::vector<int4> &split, int &nslots);
+// past: keys in front of the S queries (their ranges are then counted from the first of those)
+bool tg_attn_prefill_plan(int S, int n_cu, int tq, int window, std::vector<int4> &items, std::vector<int4> &split, int &nslots, int past = 0);
 size_t tg_attn_prefill_part_floats(int nslots, int tq);
 size_t tg_attn_prefill_ml_floats(int nslots, int tq);
 void tg_launch_attn_prefill(float *o, const float *q, const float *k, const float *v, int S, int n_head, int hd, int ldq, int ldkv,
@@ -281,8 +282,20 @@ size_t tg_attn_prefill_planes_bytes(int S);
 // The rows of o (S x 1024, 4 heads x 256) -> digit planes + row factors of the int8 MFMA GEMM, merging the partial
 // results of split query tiles on the way (instead of attn_prefill_merge_kernel + the two quantising launches);
 // tg_launch_attn_prefill must then have been called with finish_later = true
+struct TgCacheRows {  // rows that the finishing launch copies into a layer's cache (k null: none)
+	const float *k = nullptr, *v = nullptr;
+	float *kc = nullptr, *vc = nullptr;
+	int ld = 0, slot = 0, ring = 1;  // row stride of k and v, slot of row 0, rows of the cache
+};
 void tg_launch_attn_prefill_finish(const float *o, int S, int ldo, const TgAttnPrefillPlan *plan, int n_cu, int8_t *apack, float *rowfac,
-                                   hipStream_t s);
+                                   hipStream_t s, const TgCacheRows &rows = TgCacheRows());
+// Attention of a later portion of a sequence: the n keys in front of it are rows (slot0 + j) mod ring of the cache
+struct TgAttnPast {
+	const float *kc = nullptr, *vc = nullptr;
+	int n = 0, slot0 = 0, ring = 1;
+};
+void tg_launch_attn_extend(float *o, const float *q, const float *k, const float *v, int S, int ldq, int ldkv, int ldo, int is_sw, int window,
+                           const TgAttnPrefillPlan *plan, const TgAttnPast &past, int n_cu, hipStream_t s);
 // exact-order GEMM on the GEMV tiling (ntiles tiles of Ct columns): C[m][N] = (A[m][K] . W) * scales; epi GEGLU writes C[m][N/2]
 void tg_launch_gemm(float *C, const float *A, const int8_t *Wp, const float *scales, int m, int K, int ntiles, int Ct, int epi,
                     const float *lut, float gmin, float geps, int lut_size, hipStream_t s);
