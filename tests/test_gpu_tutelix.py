@@ -125,6 +125,15 @@ def test_dense_feed_forward_and_norms_alone(tg, folder, width, ff, dtype):
     rows_close(np.concatenate([s.forward([t])[1] for t in ids]), want, TOL[dtype], "logits, token by token")
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("ff,n", [(1000, 33), (2100, 5), (3100, 70), (6500, 40)])
+def test_products_in_parts_of_k(tg, folder, ff, n, dtype):
+    """Down projections of few rows, whose K is cut in 1, 2, 4 and 8 parts (the last one shorter) that the norm behind them adds."""
+    cfg = one_layer(nm.delta(1, 1, 8, 8, 2), nm.dense(ff), width=300)
+    path, om = folder(("t_parts", ff), cfg, seed=16, edit=zero_mixer)
+    check_layer(tg, cfg, path, om, dtype, n, block=2)
+
+
 # ---- whole models ------------------------------------------------------------------------------------------------------------
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("name", nm.TUTELIX)

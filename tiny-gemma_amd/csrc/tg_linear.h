@@ -171,6 +171,8 @@ struct TgGemm {
 	int ldc2, n_split;
 	float mult;
 	const float *bias;     // STORE: added to the columns below n_split (null: none)
+	int kparts;            // F32: parts of K (0: one); part p writes its sums to C2 + p * part_stride, the consumer adds them
+	size_t part_stride;
 	int rows_out;          // TRANS: output columns written (>= M: the last row repeats)
 	// grouped: tile t of the list covers rows [tiles[t].y, tiles[t].z) with the matrix of group tiles[t].x
 	const int4 *tiles;     // null: one matrix
@@ -181,3 +183,5 @@ struct TgGemm {
 	long long group_frags; // fragments between the matrices of consecutive groups
 };
 void tg_launch_linear(const TgGemm &g, int dt, int epi, hipStream_t s);
+// parts of K (1, 2, 4, 8) that a product with TG_GE_F32 should run in when its consumer can add them
+int tg_linear_kparts(int rows, int N, int K, int dt);

@@ -577,6 +577,7 @@ __global__ __launch_bounds__(256, 2) void linear_kernel(TgGemm g) {
 	__shared__ __align__(16) Frag lds[2][NF * 64];
 	const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 	const int ntn = (g.N + BN - 1) / BN;
+	constexpr bool PARTS = EPI == TG_GE_F32 && !GROUPED && BM == 32;
 
 	// Workgroups go to the 8 XCDs in turn: give each XCD a contiguous run of the tile order, so that the workgroups it
 	// runs side by side share weight tiles and activation rows in its L2.  (A list of groups launches as many workgroups
@@ -585,12 +586,16 @@ __global__ __launch_bounds__(256, 2) void linear_kernel(TgGemm g) {
 	const int ntm = GROUPED ? *g.ntiles : (mrows + BM - 1) / BM;
 	int b;
 	{
-		const int total = ntm * ntn, q = total >> 3, r = total & 7, x = (int)blockIdx.x & 7, i = (int)blockIdx.x >> 3;
+		const int total = ntm * ntn * (PARTS ? g.kparts : 1), q = total >> 3, r = total & 7, x = (int)blockIdx.x & 7, i = (int)blockIdx.x >> 3;
 		if (i >= q + (x < r ? 1 : 0)) return;
 		b = x * q + min(x, r) + i;
 	}
-	int m0, m1, tn;
+	int m0, m1, tn, part = 0;
 	const Frag *W = reinterpret_cast<const Frag *>(g.W);
+	if constexpr (PARTS) {
+		part = b / (ntm * ntn);
+		b -= part * ntm * ntn;
+	}
 	if constexpr (GROUPED) {
 		const int t = b / ntn;
 		tn = b - t * ntn;
@@ -603,7 +608,13 @@ __global__ __launch_bounds__(256, 2) void linear_kernel(TgGemm g) {
 		m0 = (b - tn * ntm) * BM;
 		m1 = g.M;
 	}
-	const int kfr = g.K / TR::KF, nst = kfr / 2, nfr = g.N / 16;
+	const int kfr = g.K / TR::KF, nfr = g.N / 16;
+	int nst = kfr / 2, s0 = 0;  // stages of this workgroup, the first of them
+	if constexpr (PARTS) {
+		const int per = (nst + g.kparts - 1) / g.kparts;
+		s0 = part * per;
+		nst = min(per, nst - s0);  // (tg_linear_kparts leaves no part empty)
+	}
 
 	// this wave's fragments of a stage: f = w * PW + i; the first 2 AF are A (row tile f / 2, k half f % 2), then B
 	// (addresses: a base that the wave shares, 32-bit offsets per lane; operands are below 4 GiB)
@@ -625,6 +636,7 @@ __global__ __launch_bounds__(256, 2) void linear_kernel(TgGemm g) {
 			off[i] = (unsigned)lane * 16u;
 			adv[i] = 2048;
 		}
+		if constexpr (PARTS) base[i] += (size_t)s0 * adv[i];
 	}
 	Frag st[2][PW];
 	auto fetch = [&](int set, int s) {
@@ -753,7 +765,7 @@ __global__ __launch_bounds__(256, 2) void linear_kernel(TgGemm g) {
 						for (int e = 0; e < 4; e++) r[e] = tg_gelu(acc[i][j][e]);
 						tg_store4((T *)g.C + (size_t)m * g.ldc + n, r);
 					} else if constexpr (EPI == TG_GE_F32) {
-						tg_store4(g.C2 + (size_t)m * g.ldc2 + n, acc[i][j]);
+						tg_store4(g.C2 + (PARTS ? (size_t)part * g.part_stride : 0) + (size_t)m * g.ldc2 + n, acc[i][j]);
 					} else {
 						float *c = g.C2 + (size_t)m * g.ldc2 + n;
 						f32x4_t x = tg_load4(c);
@@ -808,6 +820,9 @@ __global__ __launch_bounds__(256) void linear_thin_kernel(TgGemm g) {
 	if (m0 + lr < g.M && n0 + w < nfr) tg_store4(g.C2 + (size_t)(m0 + lr) * g.ldc2 + (n0 + w) * 16 + 4 * lg, r);
 }
 
+// 128-row tiles where they fill the device's 512 places (two workgroups per compute unit), then 64 rows, then 32
+bool linear_rows32(int rows, int ntn) { return (rows + 127) / 128 * ntn < 448 && (rows + 63) / 64 * ntn < 256; }
+
 template <class TR, int EPI>
 void launch_linear_t(const TgGemm &g, hipStream_t s) {
 	if constexpr (EPI == TG_GE_F32) {
@@ -829,11 +844,18 @@ void launch_linear_t(const TgGemm &g, hipStream_t s) {
 		return;
 	}
 	const int ntn = (g.N + 127) / 128, rows = EPI == TG_GE_TRANS ? g.rows_out : g.M;
-	// 128-row tiles where they fill the device's 512 places (two workgroups per compute unit), then 64 rows, then 32
+	if constexpr (EPI == TG_GE_F32) {
+		TgGemm p = g;
+		p.kparts = g.kparts > 1 ? g.kparts : 1;
+		if (linear_rows32(rows, ntn)) {
+			hipLaunchKernelGGL((linear_kernel<TR, EPI, 1, 4, 2, 2, false>), dim3((unsigned)((rows + 31) / 32 * ntn * p.kparts)), dim3(256), 0, s, p);
+			return;
+		}
+	}
 	const int t128 = (rows + 127) / 128 * ntn, t64 = (rows + 63) / 64 * ntn;
 	if (t128 >= 448)
 		hipLaunchKernelGGL((linear_kernel<TR, EPI, 2, 2, 4, 4, false>), dim3((unsigned)((rows + 127) / 128 * ntn)), dim3(256), 0, s, g);
-	else if (t64 >= 256)
+	else if (!linear_rows32(rows, ntn))
 		hipLaunchKernelGGL((linear_kernel<TR, EPI, 2, 2, 2, 4, false>), dim3((unsigned)t64), dim3(256), 0, s, g);
 	else
 		hipLaunchKernelGGL((linear_kernel<TR, EPI, 1, 4, 2, 2, false>), dim3((unsigned)((rows + 31) / 32 * ntn)), dim3(256), 0, s, g);
@@ -882,6 +904,20 @@ int tg_vec_ksplit(int ntiles, int nz, int kfrags, int n_cu) {
 void tg_launch_vec(const TgVec &v, int dt, int pro, int epi, hipStream_t s) {
 	if (dt == TG_DT_BF16) launch_vec_dt<TgB16>(v, pro, epi, s);
 	else launch_vec_dt<TgF32>(v, pro, epi, s);
+}
+
+// A product of few rows has few tiles, and each walks all of K at the pace of one workgroup on an otherwise idle compute unit
+// (0.33 us a stage of 128 bytes of K: 53 us for 130 rows x 1152 columns x K 10368 in 45 workgroups).  Its K is cut until the parts
+// fill the 512 places or are down to TG_LINEAR_PART_STAGES stages, whose start-up and sums would cost more than they save.  A
+// Tutelix prompt of 600 tokens in portions of 130 (width 1152, 26 layer runs) with 24 steps behind it: 51.0 -> 45.8 ms.
+constexpr int TG_LINEAR_PART_STAGES = 12;
+int tg_linear_kparts(int rows, int N, int K, int dt) {
+	const int ntn = (N + 127) / 128, stages = K * (int)tg_dt_bytes(dt) / 128;
+	if (N <= 256 || !linear_rows32(rows, ntn)) return 1;
+	const int tiles = (rows + 31) / 32 * ntn;
+	int p = 1;
+	while (p < 8 && 2 * p * tiles <= 512 && stages / (2 * p) >= TG_LINEAR_PART_STAGES) p *= 2;
+	return p;
 }
 
 void tg_launch_linear(const TgGemm &g, int dt, int epi, hipStream_t s) {

@@ -1230,12 +1230,15 @@ void rows_layout(const TgNet *n, int rows, int past, int n_want, int tap_rows, A
 	const TgNetCfg &c = n->cfg;
 	const size_t N = (size_t)rows, Dp = (size_t)c.wp(), eb = tg_dt_bytes(n->dt);
 	size_t in = 0, low = 0, mix = 0, gla = 0, k = 0, vt = 0, rl = 0, top = 0, u = 0, cnt = 0, tiles = 0, qn = 0, ql = 0, gate = 0;
+	int parts = 1;
 	for (size_t l = 0; l < c.layers.size(); l++) {
 		const TgNetLayerCfg &lc = c.layers[l];
 		const LayerW &w = n->lw((int)l);
 		in = std::max(in, (size_t)w.n_split);
 		low = std::max(low, (size_t)(w.in.n - w.n_split));
 		mix = std::max(mix, (size_t)w.out.k);
+		parts = std::max(parts, tg_linear_kparts(rows, w.out.n, w.out.k, n->dt));
+		if (lc.mlp == TG_FF_DENSE) parts = std::max(parts, tg_linear_kparts(rows, w.down.n, w.down.k, n->dt));
 		const size_t ctxp = (size_t)tg_up(past + rows - window_start(lc.mix, past), 64);
 		if (lc.mix.kind == TG_MIX_GLA) {
 			gla = std::max(gla, tg_gla_scratch(gla_of(n, (int)l, nullptr, 0), rows, nullptr, nullptr));
@@ -1271,7 +1274,7 @@ void rows_layout(const TgNet *n, int rows, int past, int n_want, int tap_rows, A
 	a->take(&r->qn, N * qn * eb);
 	a->take(&r->q, N * ql * eb);
 	a->take(&r->gate, N * gate * eb);
-	a->take(&r->sub, c.norm == TG_NORM_RMS ? N * Dp * 4 : 0);
+	a->take(&r->sub, c.norm == TG_NORM_RMS ? N * Dp * 4 * (size_t)parts : 0);
 	a->take(&r->gla, gla);
 	a->take(&r->k, k);
 	a->take(&r->vt, vt);
@@ -1316,6 +1319,7 @@ struct Pass {
 	hipStream_t s = n->stream;
 	TgRowsDyt d = {};           // state of the residual stream: what the next row step still adds
 	const float *post = nullptr;  // (root mean square norms) weight of the norm behind the sublayer in r.sub; null: nothing waits
+	int sub_parts = 1;            // addends of a row of r.sub
 	bool embed = true;
 	int due[2] = {-1, -1};      // blocks whose residual is complete behind the next row step
 
@@ -1356,6 +1360,8 @@ struct Pass {
 			if (post) {
 				k.y = r.sub;
 				k.ldy = Dp;
+				k.yparts = sub_parts;
+				k.ystride = (size_t)rows * Dp;
 				k.post = post;
 			}
 			k.out = nm ? r.h : nullptr;
@@ -1588,6 +1594,10 @@ struct Pass {
 		o.C2 = rms ? r.sub : r.x;
 		o.ldc2 = Dp;
 		o.mult = c.residual_mult;
+		if (rms) {
+			o.kparts = sub_parts = tg_linear_kparts(rows, w.n, w.k, dt);
+			o.part_stride = (size_t)rows * Dp;
+		}
 		tg_launch_linear(o, dt, rms ? TG_GE_F32 : TG_GE_RESID, s);
 		post = after.w;
 	}

@@ -19,7 +19,8 @@ struct TgRowsRms {
 	int vocab;
 	float embed_scale;
 	const float *y;
-	int ldy;
+	int ldy, yparts;       // y is the sum of yparts (0: one) of them,
+	size_t ystride;        // ystride apart
 	const float *post;
 	const float *nw;
 	float eps;

@@ -44,6 +44,20 @@ __global__ __launch_bounds__(256) void rows_rms_kernel(TgRowsRms r) {
 		}
 	}
 	if (r.y) {
+		for (int p0 = 1; p0 < r.yparts; p0 += 4) {  // four parts requested before one is added
+			f32x4_t more[4][NP];
+#pragma unroll
+			for (int p = 0; p < 4; p++)
+#pragma unroll
+				for (int i = 0; i < NP; i++)
+					more[p][i] = tg_load4(r.y + (size_t)min(p0 + p, r.yparts - 1) * r.ystride + (size_t)t * r.ldy + min(4 * (lane + i * 64 * WPR), r.cols - 4));
+#pragma unroll
+			for (int p = 0; p < 4; p++)
+				if (p0 + p < r.yparts)
+#pragma unroll
+					for (int i = 0; i < NP; i++)
+						if (4 * (lane + i * 64 * WPR) < r.cols) y[i] += more[p][i];
+		}
 		float ss = 0.0f;
 #pragma unroll
 		for (int i = 0; i < NP; i++)
