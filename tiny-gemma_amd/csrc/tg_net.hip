@@ -1697,6 +1697,10 @@ static int net_pass(TgNetSeq *q, const int32_t *ids, int rows, int pos, const in
 	TG_HIP(hipMemcpyAsync(r.ids, ids, sizeof(int) * (size_t)rows, hipMemcpyHostToDevice, s));
 	Pass p{q, r, rows, pos, tap_rows};
 	p.run();
+	// The pick behind the portion takes the last row through the head alone, as a decode step does; where that row is wanted
+	// its logits are those.
+	const bool last = hd && n_want > 0 && want[n_want - 1] == rows - 1;
+	if (last) n_want--;
 	for (int w0 = 0; w0 < n_want; w0 += WANT_ROWS) {
 		const int nw = std::min(WANT_ROWS, n_want - w0);
 		TG_HIP(hipMemcpyAsync(r.want, want + w0, sizeof(int) * (size_t)nw, hipMemcpyHostToDevice, s));
@@ -1713,6 +1717,7 @@ static int net_pass(TgNetSeq *q, const int32_t *ids, int rows, int pos, const in
 		v.blk_val = hd->blk_val;
 		v.blk_idx = hd->blk_idx;
 		tg_launch_vec(v, dt, norm_kind(n), TG_VE_LOGITS, s);
+		if (last) TG_HIP(hipMemcpyAsync(logits + (size_t)n_want * c.vocab, hd->logits, sizeof(float) * (size_t)c.vocab, hipMemcpyDeviceToHost, s));
 	}
 	q->taps = tap_rows ? r.taps : nullptr;
 	q->tap_rows = tap_rows;
