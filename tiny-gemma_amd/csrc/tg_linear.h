@@ -96,7 +96,8 @@ enum {
 	TG_VP_HEADNORM,    // heads normalised by their root mean square, times silu(gate) or sigmoid(gate)
 	TG_VP_MERGE,       // merged attention partials of head z
 	TG_VP_MERGE_HEADS, // the same of all heads, side by side (vdimp elements each): groups of `group` heads, each padded to 16
-	TG_VP_EXPERT       // x, for the z-th of the experts that the router's logits select
+	TG_VP_EXPERT,      // x, for the z-th of the experts that the router's logits select
+	TG_VP_ROUTE        // DYT, then the router's product on its result, then EXPERT: routers of one tile (at most 16 experts)
 };
 enum {
 	TG_VE_STORE = 0,
@@ -133,7 +134,8 @@ struct TgVec {
 	float eps;
 	const float *part_acc, *part_ml;  // MERGE: [nmerge][heads padded to 16][x_zstride], [nmerge][heads padded to 16][2]
 	int nmerge, heads16, group, heads;  // MERGE_HEADS: heads per group, real heads; heads16 counts the padded heads of all groups
-	const float *logits, *correction;  // EXPERT
+	const float *logits, *correction;  // EXPERT (ROUTE: logits unused)
+	const void *router;        // ROUTE: the router's matrix, one tile of 16 outputs, as long in K as W
 	int experts, top;
 	float rscale;
 	int *sel;                  // EXPERT: written by one workgroup; WEIGHTED: read

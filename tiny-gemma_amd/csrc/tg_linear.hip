@@ -3,6 +3,8 @@
 
 #include "tg_linear.h"
 
+#include <type_traits>
+
 namespace {
 
 // ---- packing (load time) -----------------------------------------------------------------------------------------------
@@ -36,6 +38,8 @@ __global__ __launch_bounds__(256) void unpack_f32_kernel(float *dst, int ld, TgP
 
 // ---- one-row products ----------------------------------------------------------------------------------------------------
 constexpr int NT = 256;
+template <int N>
+using Const = std::integral_constant<int, N>;
 
 // Experts by rank: expert e is chosen when fewer than `top` experts have a larger choice score (or the same one and a
 // lower index).  s_sel / s_val (LDS, top entries): the chosen experts in rank order and their scores.
@@ -65,8 +69,8 @@ __device__ __forceinline__ void choose_experts(const float *logits, const float 
 // order, the prologue's arithmetic then runs while the weights are on their way.
 
 // NTL: tiles per wave (2: a gate|up pair); KW: waves that share a tile's K (4), or 1: every wave has tiles of its own;
-// U: fragments in flight per lane and tile
-template <class TR, int PRO, int EPI, int NTL, int KW, int U>
+// U: fragments in flight per lane and tile; VP (prologues with a norm): the vector's length class, see vec_class()
+template <class TR, int PRO, int EPI, int NTL, int KW, int U, int VP>
 __global__ __launch_bounds__(NT) void vec_kernel(TgVec p) {
 	typedef typename TR::T T;
 	typedef typename TR::Frag Frag;
@@ -81,12 +85,12 @@ __global__ __launch_bounds__(NT) void vec_kernel(TgVec p) {
 	const int k0 = kb * TR::KF, kn = nk * TR::KF;
 
 	int zw = z;
-	if constexpr (PRO == TG_VP_EXPERT) {
+	auto choose = [&](const float *logits) {
 		// LDS: choice scores [experts, padded] | selected [top] | their scores [top] behind the vector
 		float *s_choice = reinterpret_cast<float *>(smem + sizeof(T) * (size_t)(per + KW * U) * TR::KF);
 		int *s_sel = reinterpret_cast<int *>(s_choice + ((p.experts + 3) & ~3));
 		float *s_val = reinterpret_cast<float *>(s_sel + p.top);
-		choose_experts(p.logits, p.correction, p.experts, p.top, s_choice, s_sel, s_val);
+		choose_experts(logits, p.correction, p.experts, p.top, s_choice, s_sel, s_val);
 		zw = s_sel[z];
 		if (blockIdx.x == 0 && part == 0 && z == 0) {
 			for (int k = tid; k < p.top; k += NT) {
@@ -96,13 +100,14 @@ __global__ __launch_bounds__(NT) void vec_kernel(TgVec p) {
 				p.wgt[k] = s_val[k] / (sum + 1e-20f) * p.rscale;
 			}
 		}
-	}
+	};
+	if constexpr (PRO == TG_VP_EXPERT) choose(p.logits);
 	if constexpr (EPI == TG_VE_WEIGHTED) zw = p.sel[z];
 
 	const int group = KW == 4 ? (int)blockIdx.x : (int)blockIdx.x * 4 + w;  // tile group of this wave
 	const bool live = group * NTL < p.ntiles;
 	const int tile0 = live ? group * NTL : 0, tiles_here = min(NTL, p.ntiles - tile0);
-	const Frag *W = reinterpret_cast<const Frag *>(p.W) + ((size_t)zw * p.zfrags + (size_t)tile0 * p.kfrags) * 64 + lane;
+	const Frag *W = reinterpret_cast<const Frag *>(p.W) + ((size_t)zw * p.zfrags + (size_t)tile0 * p.kfrags) * 64 + lane;  // (ROUTE: set below)
 	const int step = KW, kf0 = kb + (KW == 4 ? w : 0);
 	Frag wr[NTL][U];
 	auto load = [&](int kf) {
@@ -118,6 +123,20 @@ __global__ __launch_bounds__(NT) void vec_kernel(TgVec p) {
 		}
 	};
 
+	// ROUTE: what is requested behind the inputs is the router's matrix (its rounds as in the product of its own that a router
+	// of more tiles gets, so that the logits are the same); the experts' weights wait for the choice.
+	constexpr int RU = PRO == TG_VP_ROUTE ? 8 : 1;
+	Frag rt[RU];
+	const Frag *R = reinterpret_cast<const Frag *>(p.router) + lane;
+	auto load_router = [&](int kf) {
+#pragma unroll
+		for (int u = 0; u < RU; u++) rt[u] = R[(size_t)min(kf + 4 * u, p.kfrags - 1) * 64];
+	};
+	auto load_first = [&] {
+		if constexpr (PRO == TG_VP_ROUTE) load_router(w);
+		else load(kf0);
+	};
+
 	// the vector's prologue: elements [k0, k0 + kn), then zeros that the surplus steps of the last round multiply
 	if constexpr (PRO == TG_VP_PLAIN || PRO == TG_VP_EXPERT) {
 		const float *x = p.x + (PRO == TG_VP_PLAIN ? (size_t)z * p.x_zstride : 0) + k0;
@@ -130,64 +149,62 @@ __global__ __launch_bounds__(NT) void vec_kernel(TgVec p) {
 			for (int i = 0; i < 2; i++)
 				if (b + 4 * (tid + i * NT) < kn) tg_store4(xs + b + 4 * (tid + i * NT), v[i]);
 		}
-	} else if constexpr (PRO == TG_VP_DYT) {
+	} else if constexpr (PRO == TG_VP_DYT || PRO == TG_VP_ROUTE) {
 		int row = 0;
 		if (p.embed) {
 			row = p.ctr[4];
 			row = row < 0 ? 0 : (row >= p.vocab ? p.vocab - 1 : row);
 		}
-		// two elements per lane and pass; the padding behind the vector is zero in x, the parts, the norm and the table
-		constexpr int PER = 4, PQ = 8;
-		for (int b = 0; b == 0 || b < kn; b += 2 * PER * NT) {
-			float2 x[PER], nw[PER], nb[PER], pq[PER][PQ];
-			int c[PER];
+		// four elements per lane and pass; the padding behind the vector is zero in x, the parts, the norm and the table
+		constexpr int PER = VP == 1 ? 1 : 2;
+		{
+			for (int b = 0; b == 0 || (VP == 3 && b < kn); b += 4 * PER * NT) {
+				f32x4_t x[PER], nw[PER], nb[PER], add[PER];
+				int c[PER];
 #pragma unroll
-			for (int i = 0; i < PER; i++) {
-				const int j = b + 2 * (tid + i * NT);
-				c[i] = k0 + min(j, max(kn - 2, 0));
-				if (p.embed) {
-					const unsigned u = *reinterpret_cast<const unsigned *>((const __bf16 *)p.embed + (size_t)row * p.embed_ld + c[i]);
-					x[i] = float2{__uint_as_float(u << 16), __uint_as_float(u & 0xffff0000u)};
-				} else {
-					x[i] = *reinterpret_cast<const float2 *>(p.x + c[i]);
+				for (int i = 0; i < PER; i++) {
+					c[i] = k0 + min(b + 4 * (tid + i * NT), max(kn - 4, 0));
+					x[i] = p.embed ? tg_load4((const __bf16 *)p.embed + (size_t)row * p.embed_ld + c[i]) : tg_load4(p.x + c[i]);
+					nw[i] = tg_load4(p.nw + c[i]);
+					nb[i] = tg_load4(p.nb + c[i]);
+					add[i] = f32x4_t{0, 0, 0, 0};
 				}
-				nw[i] = *reinterpret_cast<const float2 *>(p.nw + c[i]);
-				nb[i] = *reinterpret_cast<const float2 *>(p.nb + c[i]);
-			}
-			float2 add[PER];
+				auto parts = [&](auto many, int q0) {
+					constexpr int PQ = decltype(many)::value;
+					f32x4_t pq[PER][PQ];
 #pragma unroll
-			for (int i = 0; i < PER; i++) add[i] = float2{0.0f, 0.0f};
-			for (int q0 = 0; q0 < p.nparts; q0 += PQ) {
+					for (int q = 0; q < PQ; q++)
 #pragma unroll
-				for (int q = 0; q < PQ; q++)
+						for (int i = 0; i < PER; i++) pq[i][q] = tg_load4(p.pend + (size_t)min(q0 + q, p.nparts - 1) * p.pend_stride + c[i]);
 #pragma unroll
-					for (int i = 0; i < PER; i++)
-						pq[i][q] = *reinterpret_cast<const float2 *>(p.pend + (size_t)min(q0 + q, p.nparts - 1) * p.pend_stride + c[i]);
-				if (b == 0 && q0 == 0) load(kf0);
+					for (int q = 0; q < PQ; q++)
+						if (q0 + q < p.nparts)
 #pragma unroll
-				for (int q = 0; q < PQ; q++)
-					if (q0 + q < p.nparts)
+							for (int i = 0; i < PER; i++)
 #pragma unroll
-						for (int i = 0; i < PER; i++) {
-							add[i].x += pq[i][q].x;
-							add[i].y += pq[i][q].y;
+								for (int e = 0; e < 4; e++) add[i][e] += pq[i][q][e];
+				};
+				if (p.nparts > 4) {
+					for (int q0 = 0; q0 < p.nparts; q0 += 8) parts(Const<8>(), q0);
+				} else if (p.nparts > 0) {
+					parts(Const<4>(), 0);
+				}
+				if (b == 0) load_first();
+#pragma unroll
+				for (int i = 0; i < PER; i++) {
+					const int j = b + 4 * (tid + i * NT);
+					f32x4_t h;
+#pragma unroll
+					for (int e = 0; e < 4; e++) {
+						if (p.nparts) x[i][e] = x[i][e] + p.mult * add[i][e];
+						h[e] = tanhf(p.alpha * x[i][e]) * nw[i][e] + nb[i][e];
+					}
+					if (j < kn) {
+						tg_store4(xs + j, h);
+						if (blockIdx.x == 0 && z == 0) {
+							if (p.x_out) tg_store4(p.x_out + c[i], x[i]);
+							if (p.h_out) tg_store4(p.h_out + c[i], h);
 						}
-			}
-			if (b == 0 && p.nparts == 0) load(kf0);
-#pragma unroll
-			for (int i = 0; i < PER; i++) {
-				const int j = b + 2 * (tid + i * NT);
-				if (p.nparts) {
-					x[i].x = x[i].x + p.mult * add[i].x;
-					x[i].y = x[i].y + p.mult * add[i].y;
-				}
-				const float2 h = {tanhf(p.alpha * x[i].x) * nw[i].x + nb[i].x, tanhf(p.alpha * x[i].y) * nw[i].y + nb[i].y};
-				if (j < kn) {
-					xs[j] = (T)h.x;
-					xs[j + 1] = (T)h.y;
-					if (blockIdx.x == 0 && z == 0) {
-						if (p.x_out) *reinterpret_cast<float2 *>(p.x_out + c[i]) = x[i];
-						if (p.h_out) *reinterpret_cast<float2 *>(p.h_out + c[i]) = h;
 					}
 				}
 			}
@@ -195,7 +212,6 @@ __global__ __launch_bounds__(NT) void vec_kernel(TgVec p) {
 	} else if constexpr (PRO == TG_VP_RMS) {
 		// The whole vector in every workgroup (ksplit is 1): four elements per lane and pass; the first RP passes stay in
 		// registers, the rest goes through LDS.  The padding is zero in x, the parts, the weights and the table.
-		constexpr int RP = 2, PQ = 8;
 		int row = 0;
 		if (p.embed) {
 			row = p.ctr[4];
@@ -203,7 +219,6 @@ __global__ __launch_bounds__(NT) void vec_kernel(TgVec p) {
 		}
 		float *sv = reinterpret_cast<float *>(smem + sizeof(T) * (size_t)(per + KW * U) * TR::KF);  // [kn], wider vectors only
 		const int npass = (kn + 4 * NT - 1) / (4 * NT);
-		f32x4_t x[RP], add[RP], nw[RP], pw[RP];
 		auto at = [&](int i) { return min(4 * (tid + i * NT), kn - 4); };
 		auto source = [&](int c) {
 			f32x4_t v;
@@ -218,12 +233,12 @@ __global__ __launch_bounds__(NT) void vec_kernel(TgVec p) {
 		};
 		auto parts = [&](int c) {
 			f32x4_t r = {0, 0, 0, 0};
-			for (int q0 = 0; q0 < p.nparts; q0 += PQ) {
-				f32x4_t v[PQ];
+			for (int q0 = 0; q0 < p.nparts; q0 += 8) {
+				f32x4_t v[8];
 #pragma unroll
-				for (int q = 0; q < PQ; q++) v[q] = tg_load4(p.pend + (size_t)min(q0 + q, p.nparts - 1) * p.pend_stride + c);
+				for (int q = 0; q < 8; q++) v[q] = tg_load4(p.pend + (size_t)min(q0 + q, p.nparts - 1) * p.pend_stride + c);
 #pragma unroll
-				for (int q = 0; q < PQ; q++)
+				for (int q = 0; q < 8; q++)
 					if (q0 + q < p.nparts)
 #pragma unroll
 						for (int e = 0; e < 4; e++) r[e] += v[q][e];
@@ -236,82 +251,105 @@ __global__ __launch_bounds__(NT) void vec_kernel(TgVec p) {
 			__syncthreads();
 			return (s_misc[slot] + s_misc[slot + 1]) + (s_misc[slot + 2] + s_misc[slot + 3]);
 		};
+		constexpr int RP = VP == 1 ? 1 : 2;
+		{
+			f32x4_t x[RP], add[RP], nw[RP], pw[RP];
 #pragma unroll
-		for (int i = 0; i < RP; i++) {
-			const int c = at(i);
-			x[i] = source(c);
-			nw[i] = tg_load4(p.nw + c);
-			if (p.nparts) pw[i] = p.post ? tg_load4(p.post + c) : f32x4_t{p.mult, p.mult, p.mult, p.mult};
-		}
-		if (p.nparts) {
-#pragma unroll
-			for (int i = 0; i < RP; i++) add[i] = parts(at(i));
-		}
-		load(kf0);
-		auto wide = [&](int i, auto &&f) {  // f(column, its four values in LDS)
-			for (; i < npass; i++) {
-				const int j = 4 * (tid + i * NT);
-				if (j < kn) f(j);
+			for (int i = 0; i < RP; i++) {
+				const int c = at(i);
+				x[i] = source(c);
+				nw[i] = tg_load4(p.nw + c);
+				if (p.nparts) pw[i] = p.post ? tg_load4(p.post + c) : f32x4_t{p.mult, p.mult, p.mult, p.mult};
 			}
-		};
-		if (p.nparts) {
-			float inv = 1.0f;
-			if (p.post) {
-				float ss = 0.0f;
+			auto first_parts = [&](auto many, int q0) {  // of all passes at once
+				constexpr int PQ = decltype(many)::value;
+				f32x4_t v[RP][PQ];
+#pragma unroll
+				for (int q = 0; q < PQ; q++)
+#pragma unroll
+					for (int i = 0; i < RP; i++) v[i][q] = tg_load4(p.pend + (size_t)min(q0 + q, p.nparts - 1) * p.pend_stride + at(i));
+#pragma unroll
+				for (int q = 0; q < PQ; q++)
+					if (q0 + q < p.nparts)
+#pragma unroll
+						for (int i = 0; i < RP; i++)
+#pragma unroll
+							for (int e = 0; e < 4; e++) add[i][e] += v[i][q][e];
+			};
+#pragma unroll
+			for (int i = 0; i < RP; i++) add[i] = f32x4_t{0, 0, 0, 0};
+			if (p.nparts > 4) {
+				for (int q0 = 0; q0 < p.nparts; q0 += 8) first_parts(Const<8>(), q0);
+			} else if (p.nparts > 0) {
+				first_parts(Const<4>(), 0);
+			}
+			load(kf0);
+			auto wide = [&](int i, auto &&f) {  // f(column, its four values in LDS)
+				if constexpr (VP == 3)
+					for (; i < npass; i++) {
+						const int j = 4 * (tid + i * NT);
+						if (j < kn) f(j);
+					}
+			};
+			if (p.nparts) {
+				float inv = 1.0f;
+				if (p.post) {
+					float ss = 0.0f;
+#pragma unroll
+					for (int i = 0; i < RP; i++)
+						if (4 * (tid + i * NT) < kn)
+#pragma unroll
+							for (int e = 0; e < 4; e++) ss = fmaf(add[i][e], add[i][e], ss);
+					wide(RP, [&](int j) {
+						const f32x4_t v = parts(j);
+#pragma unroll
+						for (int e = 0; e < 4; e++) ss = fmaf(v[e], v[e], ss);
+						tg_store4(sv + j, v);
+					});
+					inv = 1.0f / sqrtf(total(ss, 0) / (float)p.width + p.eps);
+				} else {
+					wide(RP, [&](int j) { tg_store4(sv + j, parts(j)); });
+				}
 #pragma unroll
 				for (int i = 0; i < RP; i++)
-					if (4 * (tid + i * NT) < kn)
 #pragma unroll
-						for (int e = 0; e < 4; e++) ss = fmaf(add[i][e], add[i][e], ss);
+					for (int e = 0; e < 4; e++) x[i][e] += add[i][e] * inv * pw[i][e];
 				wide(RP, [&](int j) {
-					const f32x4_t v = parts(j);
+					f32x4_t v = source(j);
+					const f32x4_t a = tg_load4(sv + j), b = p.post ? tg_load4(p.post + j) : f32x4_t{p.mult, p.mult, p.mult, p.mult};
 #pragma unroll
-					for (int e = 0; e < 4; e++) ss = fmaf(v[e], v[e], ss);
+					for (int e = 0; e < 4; e++) v[e] += a[e] * inv * b[e];
 					tg_store4(sv + j, v);
 				});
-				inv = 1.0f / sqrtf(total(ss, 0) / (float)p.width + p.eps);
 			} else {
-				wide(RP, [&](int j) { tg_store4(sv + j, parts(j)); });
+				wide(RP, [&](int j) { tg_store4(sv + j, source(j)); });
 			}
+			float ss = 0.0f;
 #pragma unroll
 			for (int i = 0; i < RP; i++)
+				if (4 * (tid + i * NT) < kn)
 #pragma unroll
-				for (int e = 0; e < 4; e++) x[i][e] += add[i][e] * inv * pw[i][e];
+					for (int e = 0; e < 4; e++) ss = fmaf(x[i][e], x[i][e], ss);
 			wide(RP, [&](int j) {
-				f32x4_t v = source(j);
-				const f32x4_t a = tg_load4(sv + j), b = p.post ? tg_load4(p.post + j) : f32x4_t{p.mult, p.mult, p.mult, p.mult};
+				const f32x4_t v = tg_load4(sv + j);
 #pragma unroll
-				for (int e = 0; e < 4; e++) v[e] += a[e] * inv * b[e];
-				tg_store4(sv + j, v);
+				for (int e = 0; e < 4; e++) ss = fmaf(v[e], v[e], ss);
 			});
-		} else {
-			wide(RP, [&](int j) { tg_store4(sv + j, source(j)); });
+			const float inv = 1.0f / sqrtf(total(ss, 4) / (float)p.width + p.eps);
+			const bool first = blockIdx.x == 0 && z == 0;
+			auto finish = [&](int j, f32x4_t v, f32x4_t n) {
+				f32x4_t h;
+#pragma unroll
+				for (int e = 0; e < 4; e++) h[e] = v[e] * inv * n[e];
+				tg_store4(xs + j, h);
+				if (first && p.x_out) tg_store4(p.x_out + j, v);
+				if (first && p.h_out) tg_store4(p.h_out + j, h);
+			};
+#pragma unroll
+			for (int i = 0; i < RP; i++)
+				if (4 * (tid + i * NT) < kn) finish(4 * (tid + i * NT), x[i], nw[i]);
+			wide(RP, [&](int j) { finish(j, tg_load4(sv + j), tg_load4(p.nw + j)); });
 		}
-		float ss = 0.0f;
-#pragma unroll
-		for (int i = 0; i < RP; i++)
-			if (4 * (tid + i * NT) < kn)
-#pragma unroll
-				for (int e = 0; e < 4; e++) ss = fmaf(x[i][e], x[i][e], ss);
-		wide(RP, [&](int j) {
-			const f32x4_t v = tg_load4(sv + j);
-#pragma unroll
-			for (int e = 0; e < 4; e++) ss = fmaf(v[e], v[e], ss);
-		});
-		const float inv = 1.0f / sqrtf(total(ss, 4) / (float)p.width + p.eps);
-		const bool first = blockIdx.x == 0 && z == 0;
-		auto finish = [&](int j, f32x4_t v, f32x4_t n) {
-			f32x4_t h;
-#pragma unroll
-			for (int e = 0; e < 4; e++) h[e] = v[e] * inv * n[e];
-			tg_store4(xs + j, h);
-			if (first && p.x_out) tg_store4(p.x_out + j, v);
-			if (first && p.h_out) tg_store4(p.h_out + j, h);
-		};
-#pragma unroll
-		for (int i = 0; i < RP; i++)
-			if (4 * (tid + i * NT) < kn) finish(4 * (tid + i * NT), x[i], nw[i]);
-		wide(RP, [&](int j) { finish(j, tg_load4(sv + j), tg_load4(p.nw + j)); });
 	} else if constexpr (PRO == TG_VP_HEADNORM) {
 		// head by head, a wave each, four elements per lane and pass: sum of squares, then the head's elements that lie in
 		// this part of K
@@ -410,6 +448,45 @@ __global__ __launch_bounds__(NT) void vec_kernel(TgVec p) {
 	}
 	for (int j = kn + tid; j < kn + KW * U * TR::KF; j += NT) xs[j] = (T)0.0f;
 	__syncthreads();
+	if constexpr (PRO == TG_VP_ROUTE) {
+		f32x4_t ra = {0, 0, 0, 0};
+		for (int kf = w; kf < p.kfrags; kf += 4 * RU) {
+			if (kf != w) load_router(kf);
+#pragma unroll
+			for (int u = 0; u < RU; u++) {
+				if (kf + 4 * u >= p.kfrags) break;
+				const Frag xf = *reinterpret_cast<const Frag *>(xs + (size_t)(kf + 4 * u) * TR::KF + (lane >> 4) * TR::KV);
+				ra = TR::mma(xf, rt[u], ra);
+			}
+		}
+		if (lane < 16) s_red[w][lane] = ra[0];
+		__syncthreads();
+		// the choice of choose_experts for at most 16 experts, expert = lane, by every wave for itself: nothing goes through LDS
+		const int e = lane & 15;
+		const float logit = (s_red[0][e] + s_red[1][e]) + (s_red[2][e] + s_red[3][e]);
+		const bool is = e < p.experts;
+		const float val = tg_sigmoid(logit), score = is ? val + p.correction[is ? e : 0] : -INFINITY;
+		int rank = 0;
+#pragma unroll
+		for (int o = 0; o < 16; o++) {
+			const float other = __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)__float_as_uint(score), o));
+			rank += (other > score || (other == score && o < e)) ? 1 : 0;
+		}
+		auto chosen = [&](int k) {  // the lane of the k-th choice (k = 0 .. 15: every rank is there once)
+			return __builtin_ctzll(__ballot(rank == k));
+		};
+		zw = chosen(z);
+		if (blockIdx.x == 0 && part == 0 && z == 0 && w == 0) {
+			float sum = 0.0f;
+			for (int k = 0; k < p.top; k++) sum += __shfl(val, chosen(k), 64);
+			if (lane < 16 && rank < p.top) {
+				p.sel[rank] = e;
+				p.wgt[rank] = val / (sum + 1e-20f) * p.rscale;
+			}
+		}
+		W = reinterpret_cast<const Frag *>(p.W) + ((size_t)zw * p.zfrags + (size_t)tile0 * p.kfrags) * 64 + lane;
+		load(kf0);
+	}
 
 	f32x4_t acc[NTL];
 #pragma unroll
@@ -509,8 +586,15 @@ bool vec_pairs(const TgVec &v, int epi) { return epi == TG_VE_STORE && v.nparts 
 // the norm's vector beyond what the registers of a workgroup hold
 size_t rms_lds(int pro, int k) { return pro == TG_VP_RMS && k > 8 * NT ? sizeof(float) * (size_t)k : 0; }
 
-template <class TR, int PRO, int EPI>
-void launch_vec_t(const TgVec &v, hipStream_t s) {
+// How many passes of 1024 elements a norm's prologue takes: 1, 2, or more (3).  A prologue requests the inputs of all its passes
+// before it uses one, also for lanes behind the vector's end: with two passes of eight parts each for every vector, the 4096
+// workgroups of a head of width 640 read as many bytes for their norms as for the weights (72 us; 66 with what there is).  The
+// classes are instances and not branches because a launch pays for the instructions it fetches: with both in one kernel the
+// 5.2 us products of width 1152 took 6.4.
+int vec_class(int pro, int k) { return pro != TG_VP_DYT && pro != TG_VP_RMS && pro != TG_VP_ROUTE ? 0 : k <= 4 * NT ? 1 : k <= 8 * NT ? 2 : 3; }
+
+template <class TR, int PRO, int EPI, int VP>
+void launch_vec_vp(const TgVec &v, hipStream_t s) {
 	constexpr int NTL = EPI == TG_VE_SWIGLU ? 2 : 1;
 	const int per = (v.kfrags + v.ksplit - 1) / v.ksplit;
 	if constexpr ((PRO == TG_VP_DYT || PRO == TG_VP_RMS) && EPI == TG_VE_STORE) {
@@ -518,8 +602,8 @@ void launch_vec_t(const TgVec &v, hipStream_t s) {
 			const int n = (per + 3) / 4;
 			auto lds = [&](int pad) { return sizeof(typename TR::T) * (size_t)(per + pad) * TR::KF + rms_lds(PRO, per * TR::KF); };
 			const dim3 grid((unsigned)tg_vec_blocks(v, EPI), (unsigned)v.ksplit, (unsigned)v.nz);
-			if (n <= 6) hipLaunchKernelGGL((vec_kernel<TR, PRO, EPI, 2, 4, 6>), grid, dim3(NT), lds(24), s, v);
-			else hipLaunchKernelGGL((vec_kernel<TR, PRO, EPI, 2, 4, 8>), grid, dim3(NT), lds(32), s, v);
+			if (n <= 6) hipLaunchKernelGGL((vec_kernel<TR, PRO, EPI, 2, 4, 6, VP>), grid, dim3(NT), lds(24), s, v);
+			else hipLaunchKernelGGL((vec_kernel<TR, PRO, EPI, 2, 4, 8, VP>), grid, dim3(NT), lds(32), s, v);
 			return;
 		}
 	}
@@ -532,18 +616,30 @@ void launch_vec_t(const TgVec &v, hipStream_t s) {
 	};
 	if constexpr (EPI == TG_VE_STORE || EPI == TG_VE_LOGITS) {
 		if (vec_wide(v, EPI)) {
-			hipLaunchKernelGGL((vec_kernel<TR, PRO, EPI, 1, 1, 8>), dim3(bx, 1, 1), dim3(NT), lds(8), s, v);
+			hipLaunchKernelGGL((vec_kernel<TR, PRO, EPI, 1, 1, 8, VP>), dim3(bx, 1, 1), dim3(NT), lds(8), s, v);
 			return;
 		}
 	}
 	// fragments in flight: all of a wave's where they fit, else in as few equal rounds as possible
 	const dim3 grid(bx, (unsigned)v.ksplit, (unsigned)v.nz);
 	const int n = (per + 3) / 4;
-	if (n <= 2) hipLaunchKernelGGL((vec_kernel<TR, PRO, EPI, NTL, 4, 2>), grid, dim3(NT), lds(8), s, v);
-	else if (n <= 4) hipLaunchKernelGGL((vec_kernel<TR, PRO, EPI, NTL, 4, 4>), grid, dim3(NT), lds(16), s, v);
-	else if (n <= 6 || (n > 9 && n <= 12)) hipLaunchKernelGGL((vec_kernel<TR, PRO, EPI, NTL, 4, 6>), grid, dim3(NT), lds(24), s, v);
-	else if (n <= 8 || (n > 12 && n <= 16) || (n > 18 && n <= 24)) hipLaunchKernelGGL((vec_kernel<TR, PRO, EPI, NTL, 4, 8>), grid, dim3(NT), lds(32), s, v);
-	else hipLaunchKernelGGL((vec_kernel<TR, PRO, EPI, NTL, 4, 9>), grid, dim3(NT), lds(36), s, v);
+	if (n <= 2) hipLaunchKernelGGL((vec_kernel<TR, PRO, EPI, NTL, 4, 2, VP>), grid, dim3(NT), lds(8), s, v);
+	else if (n <= 4) hipLaunchKernelGGL((vec_kernel<TR, PRO, EPI, NTL, 4, 4, VP>), grid, dim3(NT), lds(16), s, v);
+	else if (n <= 6 || (n > 9 && n <= 12)) hipLaunchKernelGGL((vec_kernel<TR, PRO, EPI, NTL, 4, 6, VP>), grid, dim3(NT), lds(24), s, v);
+	else if (n <= 8 || (n > 12 && n <= 16) || (n > 18 && n <= 24)) hipLaunchKernelGGL((vec_kernel<TR, PRO, EPI, NTL, 4, 8, VP>), grid, dim3(NT), lds(32), s, v);
+	else hipLaunchKernelGGL((vec_kernel<TR, PRO, EPI, NTL, 4, 9, VP>), grid, dim3(NT), lds(36), s, v);
+}
+
+template <class TR, int PRO, int EPI>
+void launch_vec_t(const TgVec &v, hipStream_t s) {
+	if constexpr (PRO == TG_VP_DYT || PRO == TG_VP_RMS || PRO == TG_VP_ROUTE) {
+		const int c = vec_class(PRO, (v.kfrags + v.ksplit - 1) / v.ksplit * TR::KF);
+		if (c == 1) launch_vec_vp<TR, PRO, EPI, 1>(v, s);
+		else if (c == 2) launch_vec_vp<TR, PRO, EPI, 2>(v, s);
+		else launch_vec_vp<TR, PRO, EPI, 3>(v, s);
+	} else {
+		launch_vec_vp<TR, PRO, EPI, 0>(v, s);
+	}
 }
 
 template <class TR>
@@ -559,6 +655,7 @@ void launch_vec_dt(const TgVec &v, int pro, int epi, hipStream_t s) {
 	else if (pro == TG_VP_HEADNORM) launch_vec_t<TR, TG_VP_HEADNORM, TG_VE_STORE>(v, s);
 	else if (pro == TG_VP_MERGE) launch_vec_t<TR, TG_VP_MERGE, TG_VE_GATE>(v, s);
 	else if (pro == TG_VP_EXPERT) launch_vec_t<TR, TG_VP_EXPERT, TG_VE_SWIGLU>(v, s);
+	else if (pro == TG_VP_ROUTE) launch_vec_t<TR, TG_VP_ROUTE, TG_VE_SWIGLU>(v, s);
 	else if (pro == TG_VP_PLAIN && epi == TG_VE_GATE) launch_vec_t<TR, TG_VP_PLAIN, TG_VE_GATE>(v, s);
 	else launch_vec_t<TR, TG_VP_PLAIN, TG_VE_WEIGHTED>(v, s);
 }

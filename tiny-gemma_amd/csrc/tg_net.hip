@@ -722,6 +722,12 @@ void norm_prologue(const TgNet *n, TgVec *v, const Norm &nm) {
 	v->width = n->cfg.width;
 	v->embed_scale = n->cfg.embed_scale;
 }
+// A router of one tile is small enough for every workgroup of a decode step's experts' product to do for itself (20 KiB at width
+// 640 in bf16), where a launch of its own is one workgroup that the rest of the chip waits for; larger ones keep theirs.
+constexpr size_t ROUTE_ROW_MAX = 4608;  // bytes of a router's row
+bool routes_in_place(const TgNet *n, const LayerW &w) {
+	return n->cfg.norm == TG_NORM_TANH && w.router.n == 16 && (size_t)w.router.k * tg_dt_bytes(n->dt) <= ROUTE_ROW_MAX;
+}
 int norm_kind(const TgNet *n) { return n->cfg.norm == TG_NORM_RMS ? TG_VP_RMS : TG_VP_DYT; }
 
 // Latent attention of one token: keys per workgroup and the number of parts for a context of ctx keys.
@@ -808,7 +814,7 @@ void tg_net_step_cost(const TgNet *n, double *bytes, int *launches) {
 			k += 2;
 		} else if (c.mlp) {
 			b += (double)w.router.n * w.router.k + (double)c.moe.top * 3.0 * c.moe.ffp() * n->cfg.wp();
-			k += 3;
+			k += routes_in_place(n, w) ? 2 : 3;
 		}
 	}
 	*bytes = b * (double)tg_dt_bytes(n->dt);
@@ -1112,16 +1118,23 @@ struct Step {
 	void experts(int l, float *x_out) {
 		const LayerW &w = n->lw(l);
 		const TgMoeCfg &e = c.layers[(size_t)l].moe;
-		TgVec r = normed(w.router, w.n2, x_out);
-		r.h_out = q->hx;
-		r.y = q->logits;
-		tg_launch_vec(r, dt, norm_kind(n), TG_VE_STORE, s);
-		TgVec g = vec_of(n, w.gate_up);
+		const bool routed = routes_in_place(n, w);
+		TgVec r = normed(w.router, w.n2, x_out), g;
+		if (routed) {
+			g = r;
+			g.router = w.router.w;
+			g.W = w.gate_up.w;
+		} else {
+			r.h_out = q->hx;
+			r.y = q->logits;
+			tg_launch_vec(r, dt, norm_kind(n), TG_VE_STORE, s);
+			g = vec_of(n, w.gate_up);
+			g.x = q->hx;
+			g.logits = q->logits;
+		}
 		g.ntiles = 2 * e.ffp() / 16;
 		g.nz = e.top;
 		g.zfrags = frags(dt, 2 * e.ffp(), Dp);
-		g.x = q->hx;
-		g.logits = q->logits;
 		g.correction = w.correction;
 		g.experts = e.experts;
 		g.top = e.top;
@@ -1130,7 +1143,7 @@ struct Step {
 		g.wgt = q->wgt;
 		g.y = q->u;
 		g.y_zstride = e.ffp();
-		tg_launch_vec(g, dt, TG_VP_EXPERT, TG_VE_SWIGLU, s);
+		tg_launch_vec(g, dt, routed ? TG_VP_ROUTE : TG_VP_EXPERT, TG_VE_SWIGLU, s);
 		TgVec d = vec_of(n, w.down);
 		d.ntiles = Dp / 16;
 		d.nz = e.top;
