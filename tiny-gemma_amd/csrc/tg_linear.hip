@@ -67,11 +67,87 @@ __device__ __forceinline__ void choose_experts(const float *logits, const float 
 // A launch is a chain of dependent memory round trips, so every prologue requests all of its inputs before it uses one
 // (clamped indices, no loads under branches), and the first round of the weight stream right behind them: waits are in
 // order, the prologue's arithmetic then runs while the weights are on their way.
+//
+// The same goes for the arguments.  Read from the descriptor field by field where they are used, they were five scalar round
+// trips in front of the first vector load.  What the first loads need are therefore leading arguments of the kernel, which the
+// dispatcher preloads into scalar registers (VecHot; 14 dwords), and the rest of the descriptor is fetched in one batch behind
+// those loads (fetch_rest).
+
+// v, or +0 where a duplicate of the last part was loaded for an even count: a mask and no condition, behind which the compiler
+// would move the load, with a wait of its own
+__device__ __forceinline__ float masked(float v, bool is) { return __uint_as_float(__float_as_uint(v) & (is ? ~0u : 0u)); }
+
+struct VecHot {
+	const void *a[4];
+	int i[6];
+};
+constexpr size_t VEC_DESC_OFFSET = sizeof(VecHot);  // of the descriptor in the argument block
+static_assert(VEC_DESC_OFFSET % alignof(TgVec) == 0 && sizeof(VecHot) == 56, "leading arguments of vec_kernel");
+
+template <int PRO, int EPI>
+VecHot vec_hot(const TgVec &v) {
+	VecHot h = {{v.x, nullptr, nullptr, nullptr}, {v.kfrags, v.ksplit, 0, 0, 0, 0}};
+	if (PRO == TG_VP_DYT || PRO == TG_VP_ROUTE || PRO == TG_VP_RMS) {
+		h = VecHot{{v.embed ? v.embed : v.x, v.nw, PRO == TG_VP_RMS ? v.post : v.nb, v.pend}, {v.kfrags, v.ksplit, v.nparts, v.pend_stride, v.embed ? 1 : 0, 0}};
+	} else if (PRO == TG_VP_HEADNORM) {
+		h = VecHot{{v.x, v.nw, v.gate, nullptr}, {v.kfrags, v.ksplit, v.vdimp, v.heads16, 0, 0}};
+	} else if (PRO == TG_VP_MERGE || PRO == TG_VP_MERGE_HEADS) {
+		h = VecHot{{v.part_acc, v.part_ml, nullptr, nullptr}, {v.kfrags, v.ksplit, v.nmerge, v.heads16, v.x_zstride, v.group | v.heads << 16}};
+	} else if (PRO == TG_VP_EXPERT) {
+		h = VecHot{{v.x, v.logits, v.correction, nullptr}, {v.kfrags, v.ksplit, v.experts, v.top, 0, 0}};
+	} else {
+		h = VecHot{{v.x, EPI == TG_VE_WEIGHTED ? v.sel : nullptr, nullptr, nullptr}, {v.kfrags, v.ksplit, v.x_zstride, 0, 0, 0}};
+	}
+	return h;
+}
+template <int PRO, int EPI>
+__device__ __forceinline__ TgVec with_hot(const TgVec &v, const void *a0, const void *a1, const void *a2, const void *a3, int i0, int i1, int i2, int i3, int i4,
+                                          int i5) {
+	TgVec p = v;
+	p.kfrags = i0;
+	p.ksplit = i1;
+	p.x = (const float *)a0;
+	if (PRO == TG_VP_DYT || PRO == TG_VP_ROUTE || PRO == TG_VP_RMS) {
+		p.embed = i4 ? a0 : nullptr;
+		p.embed_ld = 0;  // (read where there is a table)
+		p.embed_scale = 0.0f;
+		p.nw = (const float *)a1;
+		p.nb = p.post = (const float *)a2;
+		p.pend = (const float *)a3;
+		p.nparts = i2;
+		p.pend_stride = i3;
+	} else if (PRO == TG_VP_HEADNORM) {
+		p.nw = (const float *)a1;
+		p.gate = (const float *)a2;
+		p.vdimp = i2;
+		p.heads16 = i3;
+	} else if (PRO == TG_VP_MERGE || PRO == TG_VP_MERGE_HEADS) {
+		p.part_acc = (const float *)a0;
+		p.part_ml = (const float *)a1;
+		p.nmerge = i2;
+		p.heads16 = i3;
+		p.x_zstride = i4;
+		p.vdimp = PRO == TG_VP_MERGE_HEADS ? i4 : p.vdimp;
+		p.group = i5 & 0xffff;
+		p.heads = i5 >> 16;
+	} else if (PRO == TG_VP_EXPERT) {
+		p.logits = (const float *)a1;
+		p.correction = (const float *)a2;
+		p.experts = i2;
+		p.top = i3;
+	} else {
+		p.x_zstride = i2;
+		if (EPI == TG_VE_WEIGHTED) p.sel = (int *)a1;
+	}
+	return p;
+}
 
 // NTL: tiles per wave (2: a gate|up pair); KW: waves that share a tile's K (4), or 1: every wave has tiles of its own;
 // U: fragments in flight per lane and tile; VP (prologues with a norm): the vector's length class, see vec_class()
 template <class TR, int PRO, int EPI, int NTL, int KW, int U, int VP>
-__global__ __launch_bounds__(NT) void vec_kernel(TgVec p) {
+__global__ __launch_bounds__(NT) void vec_kernel(const void *a0, const void *a1, const void *a2, const void *a3, int i0, int i1, int i2, int i3, int i4,
+                                                 int i5, const TgVec p_in) {
+	TgVec p = with_hot<PRO, EPI>(p_in, a0, a1, a2, a3, i0, i1, i2, i3, i4, i5);
 	typedef typename TR::T T;
 	typedef typename TR::Frag Frag;
 	extern __shared__ __align__(16) unsigned char smem[];
@@ -102,12 +178,65 @@ __global__ __launch_bounds__(NT) void vec_kernel(TgVec p) {
 		}
 	};
 	if constexpr (PRO == TG_VP_EXPERT) choose(p.logits);
-	if constexpr (EPI == TG_VE_WEIGHTED) zw = p.sel[z];
 
 	const int group = KW == 4 ? (int)blockIdx.x : (int)blockIdx.x * 4 + w;  // tile group of this wave
-	const bool live = group * NTL < p.ntiles;
-	const int tile0 = live ? group * NTL : 0, tiles_here = min(NTL, p.ntiles - tile0);
-	const Frag *W = reinterpret_cast<const Frag *>(p.W) + ((size_t)zw * p.zfrags + (size_t)tile0 * p.kfrags) * 64 + lane;  // (ROUTE: set below)
+	bool live = true;
+	int tile0 = 0, tiles_here = 1;
+	const Frag *W = nullptr;
+	const Frag *R = nullptr;  // ROUTE: the router's matrix
+	float late = 0.0f;        // a factor or an addend of the epilogue, requested with the weights
+	auto weights = [&] { W = reinterpret_cast<const Frag *>(p.W) + ((size_t)zw * p.zfrags + (size_t)tile0 * p.kfrags) * 64 + lane; };
+	// the rest of the descriptor, in one batch, through the address of the argument block: made opaque here, so that no field can be
+	// fetched earlier (which would end with a wait in front of the first loads)
+	typedef const TgVec __attribute__((address_space(4))) *Desc;
+	auto descriptor = [&] {
+		Desc d = (Desc)((const char __attribute__((address_space(4))) *)__builtin_amdgcn_kernarg_segment_ptr() + VEC_DESC_OFFSET);
+		asm volatile("" : "+s"(d) : : "memory");
+		return d;
+	};
+	auto fetch_rest = [&] {
+		const Desc d = descriptor();
+		p.W = d->W;
+		p.ntiles = d->ntiles;
+		p.zfrags = d->zfrags;
+		p.y = d->y;
+		p.y_zstride = d->y_zstride;
+		p.part_stride = d->part_stride;
+		if constexpr (PRO == TG_VP_DYT || PRO == TG_VP_ROUTE || PRO == TG_VP_RMS) {
+			p.mult = d->mult;
+			p.x_out = d->x_out;
+			p.h_out = d->h_out;
+			if constexpr (PRO == TG_VP_RMS) p.width = d->width;
+			else p.alpha = d->alpha;
+		}
+		if constexpr (PRO == TG_VP_RMS || PRO == TG_VP_HEADNORM) p.eps = d->eps;
+		if constexpr (PRO == TG_VP_HEADNORM) {
+			p.vdim = d->vdim;
+			p.gate_sigmoid = d->gate_sigmoid;
+		}
+		if constexpr (PRO == TG_VP_ROUTE) {
+			p.router = d->router;
+			p.correction = d->correction;
+			p.experts = d->experts;
+			p.top = d->top;
+		}
+		if constexpr (EPI == TG_VE_LOGITS) {
+			p.nout = d->nout;
+			p.blk_val = d->blk_val;
+			p.blk_idx = d->blk_idx;
+		}
+		if constexpr (EPI == TG_VE_GATE) p.gate = d->gate;
+		if constexpr (EPI == TG_VE_WEIGHTED) p.wgt = d->wgt;
+		if constexpr (EPI == TG_VE_STORE) p.bias = d->bias;
+		live = group * NTL < p.ntiles;
+		tile0 = live ? group * NTL : 0;
+		tiles_here = min(NTL, p.ntiles - tile0);
+		if constexpr (EPI == TG_VE_WEIGHTED) zw = p.sel[z];
+		if constexpr (PRO != TG_VP_ROUTE) weights();
+		if constexpr (PRO == TG_VP_ROUTE) R = reinterpret_cast<const Frag *>(p.router) + lane;
+		if constexpr (EPI == TG_VE_GATE) late = p.gate[z];
+		if constexpr (EPI == TG_VE_WEIGHTED) late = p.wgt[z];
+	};
 	const int step = KW, kf0 = kb + (KW == 4 ? w : 0);
 	Frag wr[NTL][U];
 	auto load = [&](int kf) {
@@ -127,12 +256,12 @@ __global__ __launch_bounds__(NT) void vec_kernel(TgVec p) {
 	// of more tiles gets, so that the logits are the same); the experts' weights wait for the choice.
 	constexpr int RU = PRO == TG_VP_ROUTE ? 8 : 1;
 	Frag rt[RU];
-	const Frag *R = reinterpret_cast<const Frag *>(p.router) + lane;
 	auto load_router = [&](int kf) {
 #pragma unroll
 		for (int u = 0; u < RU; u++) rt[u] = R[(size_t)min(kf + 4 * u, p.kfrags - 1) * 64];
 	};
 	auto load_first = [&] {
+		fetch_rest();
 		if constexpr (PRO == TG_VP_ROUTE) load_router(w);
 		else load(kf0);
 	};
@@ -144,7 +273,7 @@ __global__ __launch_bounds__(NT) void vec_kernel(TgVec p) {
 			f32x4_t v[2];
 #pragma unroll
 			for (int i = 0; i < 2; i++) v[i] = tg_load4(x + min(b + 4 * (tid + i * NT), max(kn - 4, 0)));
-			if (b == 0) load(kf0);
+			if (b == 0) load_first();
 #pragma unroll
 			for (int i = 0; i < 2; i++)
 				if (b + 4 * (tid + i * NT) < kn) tg_store4(xs + b + 4 * (tid + i * NT), v[i]);
@@ -152,8 +281,11 @@ __global__ __launch_bounds__(NT) void vec_kernel(TgVec p) {
 	} else if constexpr (PRO == TG_VP_DYT || PRO == TG_VP_ROUTE) {
 		int row = 0;
 		if (p.embed) {
-			row = p.ctr[4];
-			row = row < 0 ? 0 : (row >= p.vocab ? p.vocab - 1 : row);
+			const Desc d = descriptor();
+			p.embed_ld = d->embed_ld;
+			p.embed_scale = d->embed_scale;
+			row = d->ctr[4];
+			row = row < 0 ? 0 : (row >= d->vocab ? d->vocab - 1 : row);
 		}
 		// four elements per lane and pass; the padding behind the vector is zero in x, the parts, the norm and the table
 		constexpr int PER = VP == 1 ? 1 : 2;
@@ -176,20 +308,21 @@ __global__ __launch_bounds__(NT) void vec_kernel(TgVec p) {
 					for (int q = 0; q < PQ; q++)
 #pragma unroll
 						for (int i = 0; i < PER; i++) pq[i][q] = tg_load4(p.pend + (size_t)min(q0 + q, p.nparts - 1) * p.pend_stride + c[i]);
+					if (b == 0 && q0 == 0) load_first();
 #pragma unroll
 					for (int q = 0; q < PQ; q++)
-						if (q0 + q < p.nparts)
 #pragma unroll
-							for (int i = 0; i < PER; i++)
+						for (int i = 0; i < PER; i++)
 #pragma unroll
-								for (int e = 0; e < 4; e++) add[i][e] += pq[i][q][e];
+							for (int e = 0; e < 4; e++) add[i][e] += masked(pq[i][q][e], q0 + q < p.nparts);
 				};
 				if (p.nparts > 4) {
 					for (int q0 = 0; q0 < p.nparts; q0 += 8) parts(Const<8>(), q0);
 				} else if (p.nparts > 0) {
 					parts(Const<4>(), 0);
+				} else if (b == 0) {
+					load_first();
 				}
-				if (b == 0) load_first();
 #pragma unroll
 				for (int i = 0; i < PER; i++) {
 					const int j = b + 4 * (tid + i * NT);
@@ -214,8 +347,11 @@ __global__ __launch_bounds__(NT) void vec_kernel(TgVec p) {
 		// registers, the rest goes through LDS.  The padding is zero in x, the parts, the weights and the table.
 		int row = 0;
 		if (p.embed) {
-			row = p.ctr[4];
-			row = row < 0 ? 0 : (row >= p.vocab ? p.vocab - 1 : row);
+			const Desc d = descriptor();
+			p.embed_ld = d->embed_ld;
+			p.embed_scale = d->embed_scale;
+			row = d->ctr[4];
+			row = row < 0 ? 0 : (row >= d->vocab ? d->vocab - 1 : row);
 		}
 		float *sv = reinterpret_cast<float *>(smem + sizeof(T) * (size_t)(per + KW * U) * TR::KF);  // [kn], wider vectors only
 		const int npass = (kn + 4 * NT - 1) / (4 * NT);
@@ -259,7 +395,7 @@ __global__ __launch_bounds__(NT) void vec_kernel(TgVec p) {
 				const int c = at(i);
 				x[i] = source(c);
 				nw[i] = tg_load4(p.nw + c);
-				if (p.nparts) pw[i] = p.post ? tg_load4(p.post + c) : f32x4_t{p.mult, p.mult, p.mult, p.mult};
+				if (p.post) pw[i] = tg_load4(p.post + c);
 			}
 			auto first_parts = [&](auto many, int q0) {  // of all passes at once
 				constexpr int PQ = decltype(many)::value;
@@ -268,22 +404,30 @@ __global__ __launch_bounds__(NT) void vec_kernel(TgVec p) {
 				for (int q = 0; q < PQ; q++)
 #pragma unroll
 					for (int i = 0; i < RP; i++) v[i][q] = tg_load4(p.pend + (size_t)min(q0 + q, p.nparts - 1) * p.pend_stride + at(i));
+				if (VP == 1 && q0 == 0) load_first();
 #pragma unroll
 				for (int q = 0; q < PQ; q++)
-					if (q0 + q < p.nparts)
 #pragma unroll
-						for (int i = 0; i < RP; i++)
+					for (int i = 0; i < RP; i++)
 #pragma unroll
-							for (int e = 0; e < 4; e++) add[i][e] += v[i][q][e];
+						for (int e = 0; e < 4; e++) add[i][e] += masked(v[i][q][e], q0 + q < p.nparts);
 			};
 #pragma unroll
 			for (int i = 0; i < RP; i++) add[i] = f32x4_t{0, 0, 0, 0};
+			// A vector of one pass has its weights requested next to it, a longer one when it is there (1152 columns, 648
+			// workgroups: 9.05 us against 9.45; width 640 in fp32: 5.5 against 5.8)
 			if (p.nparts > 4) {
 				for (int q0 = 0; q0 < p.nparts; q0 += 8) first_parts(Const<8>(), q0);
 			} else if (p.nparts > 0) {
 				first_parts(Const<4>(), 0);
+			} else if (VP == 1) {
+				load_first();
 			}
-			load(kf0);
+			if constexpr (VP != 1) load_first();
+			if (!p.post) {
+#pragma unroll
+				for (int i = 0; i < RP; i++) pw[i] = f32x4_t{p.mult, p.mult, p.mult, p.mult};
+			}
 			auto wide = [&](int i, auto &&f) {  // f(column, its four values in LDS)
 				if constexpr (VP == 3)
 					for (; i < npass; i++) {
@@ -358,7 +502,7 @@ __global__ __launch_bounds__(NT) void vec_kernel(TgVec p) {
 		for (int a = h_lo + w; a <= h_hi; a += 4) {
 			const float *o = p.x + (size_t)a * p.vdimp, *g = p.gate + (size_t)a * p.vdimp;
 			const f32x4_t o0 = tg_load4(o + min(4 * lane, vl)), g0 = tg_load4(g + min(4 * lane, vl)), w0 = tg_load4(p.nw + min(4 * lane, vl));
-			if (first) load(kf0);
+			if (first) load_first();
 			first = false;
 			float ss = 0.0f;
 			for (int v = 4 * lane; v < p.vdimp; v += 256) {  // the padding is zero
@@ -377,7 +521,7 @@ __global__ __launch_bounds__(NT) void vec_kernel(TgVec p) {
 				if (j >= 0 && j < kn) tg_store4(xs + j, r);
 			}
 		}
-		if (first) load(kf0);
+		if (first) load_first();
 		for (int j = tid; j < kn; j += NT)
 			if ((k0 + j) / p.vdimp >= p.heads16) xs[j] = (T)0.0f;
 	} else if constexpr (PRO == TG_VP_MERGE_HEADS) {
@@ -397,7 +541,7 @@ __global__ __launch_bounds__(NT) void vec_kernel(TgVec p) {
 		const float *pa = column(min(tid, max(kn - 1, 0)));
 #pragma unroll
 		for (int b = 0; b < TG_VEC_MERGE_MAX; b++) a[b] = pa[(size_t)min(b, p.nmerge - 1) * step_b];
-		load(kf0);
+		load_first();
 		const bool in = (lane & 15) < p.nmerge;
 		for (int hb = h_lo; hb <= h_hi; hb += 16) {
 			const int h = min(hb + 4 * w + (lane >> 4), h_hi);
@@ -429,7 +573,7 @@ __global__ __launch_bounds__(NT) void vec_kernel(TgVec p) {
 #pragma unroll
 		for (int b = 0; b < TG_VEC_MERGE_MAX; b++)
 			a[b] = pa[(size_t)min(b, p.nmerge - 1) * p.heads16 * p.x_zstride + min(tid, max(kn - 1, 0))];
-		load(kf0);
+		load_first();
 		const bool in = (lane & 15) < p.nmerge;
 		const float m = tg_row16_max(in ? ml.x : -INFINITY);
 		const float f = in ? expf(ml.x - m) : 0.0f;
@@ -484,7 +628,7 @@ __global__ __launch_bounds__(NT) void vec_kernel(TgVec p) {
 				p.wgt[rank] = val / (sum + 1e-20f) * p.rscale;
 			}
 		}
-		W = reinterpret_cast<const Frag *>(p.W) + ((size_t)zw * p.zfrags + (size_t)tile0 * p.kfrags) * 64 + lane;
+		weights();
 		load(kf0);
 	}
 
@@ -531,8 +675,8 @@ __global__ __launch_bounds__(NT) void vec_kernel(TgVec p) {
 					}
 				}
 				if constexpr (EPI == TG_VE_GELU) r = tg_gelu(r);
-				if constexpr (EPI == TG_VE_GATE) r *= tg_sigmoid(p.gate[z]);
-				if constexpr (EPI == TG_VE_WEIGHTED) r *= p.wgt[z];
+				if constexpr (EPI == TG_VE_GATE) r *= tg_sigmoid(late);
+				if constexpr (EPI == TG_VE_WEIGHTED) r *= late;
 				y[group * NTL * 16 + tid] = r;
 				if constexpr (NTL == 2) {
 					if (group * 2 + 1 < p.ntiles) y[group * 32 + 16 + tid] = v[1];
@@ -595,6 +739,10 @@ int vec_class(int pro, int k) { return pro != TG_VP_DYT && pro != TG_VP_RMS && p
 
 template <class TR, int PRO, int EPI, int VP>
 void launch_vec_vp(const TgVec &v, hipStream_t s) {
+	const VecHot h = vec_hot<PRO, EPI>(v);
+#define TG_VEC_LAUNCH(ntl, kw, u, grid, pad)                                                                                                       \
+	hipLaunchKernelGGL((vec_kernel<TR, PRO, EPI, ntl, kw, u, VP>), grid, dim3(NT), lds(pad), s, h.a[0], h.a[1], h.a[2], h.a[3], h.i[0], h.i[1], \
+	                   h.i[2], h.i[3], h.i[4], h.i[5], v)
 	constexpr int NTL = EPI == TG_VE_SWIGLU ? 2 : 1;
 	const int per = (v.kfrags + v.ksplit - 1) / v.ksplit;
 	if constexpr ((PRO == TG_VP_DYT || PRO == TG_VP_RMS) && EPI == TG_VE_STORE) {
@@ -602,8 +750,8 @@ void launch_vec_vp(const TgVec &v, hipStream_t s) {
 			const int n = (per + 3) / 4;
 			auto lds = [&](int pad) { return sizeof(typename TR::T) * (size_t)(per + pad) * TR::KF + rms_lds(PRO, per * TR::KF); };
 			const dim3 grid((unsigned)tg_vec_blocks(v, EPI), (unsigned)v.ksplit, (unsigned)v.nz);
-			if (n <= 6) hipLaunchKernelGGL((vec_kernel<TR, PRO, EPI, 2, 4, 6, VP>), grid, dim3(NT), lds(24), s, v);
-			else hipLaunchKernelGGL((vec_kernel<TR, PRO, EPI, 2, 4, 8, VP>), grid, dim3(NT), lds(32), s, v);
+			if (n <= 6) TG_VEC_LAUNCH(2, 4, 6, (grid), 24);
+			else TG_VEC_LAUNCH(2, 4, 8, (grid), 32);
 			return;
 		}
 	}
@@ -616,19 +764,21 @@ void launch_vec_vp(const TgVec &v, hipStream_t s) {
 	};
 	if constexpr (EPI == TG_VE_STORE || EPI == TG_VE_LOGITS) {
 		if (vec_wide(v, EPI)) {
-			hipLaunchKernelGGL((vec_kernel<TR, PRO, EPI, 1, 1, 8, VP>), dim3(bx, 1, 1), dim3(NT), lds(8), s, v);
+			TG_VEC_LAUNCH(1, 1, 8, (dim3(bx, 1, 1)), 8);
 			return;
 		}
 	}
 	// fragments in flight: all of a wave's where they fit, else in as few equal rounds as possible
 	const dim3 grid(bx, (unsigned)v.ksplit, (unsigned)v.nz);
 	const int n = (per + 3) / 4;
-	if (n <= 2) hipLaunchKernelGGL((vec_kernel<TR, PRO, EPI, NTL, 4, 2, VP>), grid, dim3(NT), lds(8), s, v);
-	else if (n <= 4) hipLaunchKernelGGL((vec_kernel<TR, PRO, EPI, NTL, 4, 4, VP>), grid, dim3(NT), lds(16), s, v);
-	else if (n <= 6 || (n > 9 && n <= 12)) hipLaunchKernelGGL((vec_kernel<TR, PRO, EPI, NTL, 4, 6, VP>), grid, dim3(NT), lds(24), s, v);
-	else if (n <= 8 || (n > 12 && n <= 16) || (n > 18 && n <= 24)) hipLaunchKernelGGL((vec_kernel<TR, PRO, EPI, NTL, 4, 8, VP>), grid, dim3(NT), lds(32), s, v);
-	else hipLaunchKernelGGL((vec_kernel<TR, PRO, EPI, NTL, 4, 9, VP>), grid, dim3(NT), lds(36), s, v);
+	if (n <= 2) TG_VEC_LAUNCH(NTL, 4, 2, (grid), 8);
+	else if (n <= 4) TG_VEC_LAUNCH(NTL, 4, 4, (grid), 16);
+	else if (n <= 6 || (n > 9 && n <= 12)) TG_VEC_LAUNCH(NTL, 4, 6, (grid), 24);
+	else if (n <= 8 || (n > 12 && n <= 16) || (n > 18 && n <= 24)) TG_VEC_LAUNCH(NTL, 4, 8, (grid), 32);
+	else TG_VEC_LAUNCH(NTL, 4, 9, (grid), 36);
 }
+
+#undef TG_VEC_LAUNCH
 
 template <class TR, int PRO, int EPI>
 void launch_vec_t(const TgVec &v, hipStream_t s) {
