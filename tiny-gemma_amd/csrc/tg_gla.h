@@ -24,7 +24,7 @@ struct TgGla {
 	int group;            // heads per q/k head
 };
 // one token: y = the fused product's outputs q | k | v | g | a1 (offsets in floats); o [heads * vdimp]
-void tg_launch_gla_step(const TgGla &g, const float *y, int k_off, int v_off, int a_off, float *o, hipStream_t s);
+void tg_launch_gla_step(const TgGla &g, const float *y, int k_off, int v_off, int a_off, float *o, TgTouch touch, int touch_blocks, hipStream_t s);
 // n tokens: qkv [n][ld] in the model's format (q at column 0, offsets in elements), low [n][ld_low] fp32 (the decay's low-rank input).
 // Scratch: see tg_gla_scratch.  out [n][ld_out]: the normalised, gated heads.
 struct TgGlaScratch {
@@ -50,7 +50,7 @@ struct TgDelta {
 // one token at position host_pos (or ctr[0] where host_pos < 0): y = the fused product's outputs, q | k | v from column 0, the rest
 // at the offsets; o, gate [heads * vdimp]: read-out, and the gate before its sigmoid
 void tg_launch_delta_step(const TgDelta &d, const float *y, int g_off, int b_off, int a_off, const int *ctr, int host_pos, float *o, float *gate,
-                          hipStream_t s);
+                          TgTouch touch, int touch_blocks, hipStream_t s);
 // n tokens behind `past` earlier ones: x [n][ld] q | k | v in the model's format; low [n][ld_low] fp32: step sizes at b_off, the decay's
 // low-rank input at a_off; gate [n][ldg] in the model's format, before its sigmoid; out [n][ld_out]: the normalised, gated heads
 struct TgDeltaScratch {

@@ -18,7 +18,8 @@ __device__ __forceinline__ float pow2(float x) { return __builtin_amdgcn_exp2f(x
 
 // ---- one token -----------------------------------------------------------------------------------------------------------
 // A workgroup owns 32 value columns of a head: lane = 4 columns, 32 groups of key channels.
-__global__ __launch_bounds__(256) void gla_step_kernel(const float *y, TgGla g, int k_off, int v_off, int a_off, float *o) {
+__global__ __launch_bounds__(256) void gla_step_kernel(const float *y, TgGla g, int k_off, int v_off, int a_off, float *o, TgTouch touch) {
+	if (tg_touch(touch)) return;
 	extern __shared__ __align__(16) float sm[];
 	float *s_q = sm, *s_k = sm + g.dimp, *s_a = sm + 2 * g.dimp;
 	__shared__ f32x4_t s_red[4][8];
@@ -780,7 +781,8 @@ __global__ __launch_bounds__(256, 1) void delta_scan_kernel(TgDelta d, const typ
 // ---- one token: 32 value columns of a head per workgroup, lane = 4 columns, 32 groups of key channels (R rows of S per lane) ------
 template <int R>
 __global__ __launch_bounds__(256) void delta_step_kernel(const float *y, TgDelta d, int g_off, int b_off, int a_off, const int *ctr, int host_pos,
-                                                         float *o, float *gate) {
+                                                         float *o, float *gate, TgTouch touch) {
+	if (tg_touch(touch)) return;
 	constexpr int DM = 32 * R;
 	__shared__ __align__(16) float s_q[DM], s_k[DM], s_a[DM], s_z[DM > 256 ? DM : 256], s_v[32], s_g[8][32];
 	__shared__ f32x4_t s_rp[4][8], s_rq[4][8];
@@ -992,9 +994,9 @@ void launch_delta_rows(const TgDelta &d, const void *xv, int ld, const float *lo
 
 }  // namespace
 
-void tg_launch_gla_step(const TgGla &g, const float *y, int k_off, int v_off, int a_off, float *o, hipStream_t s) {
-	hipLaunchKernelGGL(gla_step_kernel, dim3((unsigned)g.heads, (unsigned)(g.vdimp / 32)), dim3(256), sizeof(float) * 3 * (size_t)g.dimp, s, y, g,
-	                   k_off, v_off, a_off, o);
+void tg_launch_gla_step(const TgGla &g, const float *y, int k_off, int v_off, int a_off, float *o, TgTouch touch, int touch_blocks, hipStream_t s) {
+	const dim3 grid = tg_touch_grid(dim3((unsigned)g.heads, (unsigned)(g.vdimp / 32)), &touch, touch_blocks);
+	hipLaunchKernelGGL(gla_step_kernel, grid, dim3(256), sizeof(float) * 3 * (size_t)g.dimp, s, y, g, k_off, v_off, a_off, o, touch);
 }
 
 size_t tg_gla_scratch(const TgGla &g, int n, TgGlaScratch *t, unsigned char *base) {
@@ -1019,9 +1021,9 @@ void tg_launch_gla_rows(const TgGla &g, int dt, const void *qkv, int ld, int k_o
 }
 
 void tg_launch_delta_step(const TgDelta &d, const float *y, int g_off, int b_off, int a_off, const int *ctr, int host_pos, float *o, float *gate,
-                          hipStream_t s) {
-	const dim3 grid((unsigned)d.g.heads, (unsigned)(d.g.vdimp / 32));
-	auto go = [&](auto *kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, y, d, g_off, b_off, a_off, ctr, host_pos, o, gate); };
+                          TgTouch touch, int touch_blocks, hipStream_t s) {
+	const dim3 grid = tg_touch_grid(dim3((unsigned)d.g.heads, (unsigned)(d.g.vdimp / 32)), &touch, touch_blocks);
+	auto go = [&](auto *kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, y, d, g_off, b_off, a_off, ctr, host_pos, o, gate, touch); };
 	if (d.g.dimp <= 64) go(delta_step_kernel<2>);
 	else if (d.g.dimp <= 128) go(delta_step_kernel<4>);
 	else go(delta_step_kernel<8>);

@@ -50,6 +50,8 @@ struct TgLatentStep {
 	int host_pos;                  // the position, or -1: read the counter
 	int chunk, nb;                 // keys per part (multiple of TG_LATENT_TILE), parts
 	float *part_acc, *part_ml;     // [nb][groups * heads16][rankp], [nb][groups * heads16][2]; heads16: heads padded to 16
+	TgTouch touch;
+	int touch_blocks;
 	int rowp() const { return rankp + rotp; }
 };
 void tg_launch_latent_step(const TgLatentStep &a, int dt, hipStream_t s);

@@ -46,6 +46,7 @@ __device__ __forceinline__ int div_by(int e, unsigned m) { return (int)(((unsign
 // NC: column tiles of the value part per wave (4 NC tiles of 16 per workgroup).
 template <class TR, bool ROT, int NC>
 __global__ __launch_bounds__(256) void latent_step_kernel(TgLatentStep a) {
+	if (tg_touch(a.touch)) return;
 	typedef typename TR::T T;
 	typedef typename TR::Frag Frag;
 	extern __shared__ __align__(16) unsigned char smem[];
@@ -57,7 +58,7 @@ __global__ __launch_bounds__(256) void latent_step_kernel(TgLatentStep a) {
 	__shared__ float s_corr[16], s_sq[4];
 	const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, lr = lane & 15, lg = lane >> 4;
 	const int blocks = (a.heads + 15) / 16, grp = (int)blockIdx.y / blocks, hb = (int)blockIdx.y - grp * blocks;
-	const int part = blockIdx.x, h0 = hb * 16, heads16 = (int)gridDim.y * 16, g0 = grp * a.heads;  // (h0: inside the group)
+	const int part = blockIdx.x, h0 = hb * 16, heads16 = a.groups * blocks * 16, g0 = grp * a.heads;  // (h0: inside the group)
 	const int pos = a.host_pos >= 0 ? a.host_pos : a.ctr[0], ctx = pos + 1, lo = max(0, ctx - a.window);
 	const int kb = lo + part * a.chunk, ke = min(ctx, kb + a.chunk);
 	const size_t key_bytes = (size_t)a.groups * row;
@@ -619,11 +620,12 @@ void launch_attention(const TgLatentRows &a, hipStream_t s) {
 namespace {
 template <class TR>
 void launch_step(const TgLatentStep &a, hipStream_t s) {
-	const dim3 grid((unsigned)a.nb, (unsigned)(a.groups * ((a.heads + 15) / 16)), (unsigned)((a.rankp + 511) / 512));
+	TgLatentStep t = a;
+	const dim3 grid = tg_touch_grid(dim3((unsigned)a.nb, (unsigned)(a.groups * ((a.heads + 15) / 16)), (unsigned)((a.rankp + 511) / 512)), &t.touch, a.touch_blocks);
 	const size_t lds = latent_step_lds<TR>(a.rowp());
 	auto go = [&](auto *kernel) {
 		if (lds > 48 * 1024) (void)hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-		hipLaunchKernelGGL(kernel, grid, dim3(256), lds, s, a);
+		hipLaunchKernelGGL(kernel, grid, dim3(256), lds, s, t);
 	};
 	if (a.rotp && a.rankp <= 128) go(latent_step_kernel<TR, true, 2>);
 	else if (a.rotp && a.rankp <= 256) go(latent_step_kernel<TR, true, 4>);

@@ -58,6 +58,50 @@ __device__ __forceinline__ f32x4_t tg_load4(const float *p) { return *reinterpre
 __device__ __forceinline__ f32x4_t tg_load4(const __bf16 *p) { return __builtin_convertvector(*reinterpret_cast<const bf16x4_t *>(p), f32x4_t); }
 #endif
 
+// Weights that a launch with few workgroups touches for the launches behind it, so that these find them in the memory-side cache.
+struct TgTouch {
+	const unsigned char *ptr = nullptr;  // null: nothing
+	unsigned slab = 0;                   // bytes of a tile of 16 outputs, a multiple of 128
+	int tiles = 0;                       // tile t is read by the workgroups of XCD t % 8, as its consumer's workgroups are dealt
+	int first = 0;                       // rows of workgroups (blockIdx.y) in front of the touching ones
+};
+#if defined(__HIPCC__)
+// workgroups of 256 threads, appended to a grid along y; one dword per line of 128 bytes, four in flight per lane
+__device__ __forceinline__ bool tg_touch(const TgTouch &t) {
+	if (t.ptr == nullptr || (int)blockIdx.y < t.first) return false;
+	if (blockIdx.z != 0) return true;
+	const int pb = ((int)blockIdx.y - t.first) * (int)gridDim.x + (int)blockIdx.x, nb = ((int)gridDim.y - t.first) * (int)gridDim.x;
+	const unsigned x = (unsigned)(t.first * (int)gridDim.x + pb) & 7u, q = (unsigned)pb >> 3, Q = (unsigned)nb >> 3;
+	if ((int)x >= t.tiles || q >= Q) return true;
+	const unsigned lps = t.slab >> 7, total = (((unsigned)t.tiles - x + 7u) >> 3) * lps, per = (total + Q - 1) / Q, lo = q * per, hi = min(lo + per, total);
+	for (unsigned i0 = lo + threadIdx.x; i0 < hi; i0 += 4u * 256u) {
+		int sink = 0;
+#pragma unroll
+		for (unsigned k = 0; k < 4; k++) {
+			unsigned i = i0 + k * 256u;
+			i = i < hi ? i : i0;
+			const unsigned j = i / lps, line = i - j * lps;
+			sink += *(const int *)(t.ptr + (size_t)(x + 8 * j) * t.slab + (size_t)line * 128u);
+		}
+		asm volatile("" ::"v"(sink));  // the values are not needed, the loads are
+	}
+	return true;
+}
+#endif
+
+// the grid with at least `blocks` touching workgroups behind its own, a multiple of 8
+inline dim3 tg_touch_grid(dim3 grid, TgTouch *t, int blocks) {
+	t->first = (int)grid.y;
+	if (t->ptr == nullptr || blocks <= 0) {
+		t->ptr = nullptr;
+		return grid;
+	}
+	unsigned rows = ((unsigned)blocks + grid.x - 1) / grid.x;
+	while (rows * grid.x % 8) rows++;
+	grid.y += rows;
+	return grid;
+}
+
 // A packed matrix (see above); n, k are the padded sizes.
 struct TgMat {
 	void *w = nullptr;
