@@ -325,6 +325,8 @@ struct tg_session {
 	float *blk_val = nullptr;
 	int *blk_idx = nullptr;
 	bool counted = false;     // this session is included in m->n_sessions
+	bool kv_clean = false;    // the caches were zero as a whole once (at the first reset)
+	int kv_hi = 0;            // positions that prompts since the last reset have written, or begun to
 	unsigned graph_epoch = 0; // g_knob_epoch the cached graphs were captured under
 	float *zeros = nullptr;   // [hidden] of 0: as the pending block output of a post-norm + residual prologue it adds nothing
 	float *blk_x = nullptr, *blk_y = nullptr;  // [hidden] input / output of the block-level entry points
@@ -1038,18 +1040,22 @@ int tg_session_reset(tg_session *s) {
 	if (!s) return tg_fail(TG_ERR_BAD_ARG, "null session");
 	const tg_config &c = s->m->cfg;
 	if (s->seq && !s->m->loaded) return tg_fail(TG_ERR_STATE, "the session's model has been destroyed");
-	TG_HIP(hipStreamSynchronize(g_stream));
+	// cache rows that may have been written since the last reset (a step that failed on the way may have written the next ones)
+	const size_t rows = s->kv_clean ? (size_t)std::max(s->kv_hi, s->pos + 8) : (size_t)c.n_pos;
+	std::vector<TgClear> list;
 	for (size_t l = 0; l < s->kc.size(); l++) {
-		const size_t bytes = sizeof(float) * (size_t)s->max_pos[l] * c.head_dim;
-		TG_HIP(hipMemset(s->kc[l], 0, bytes));
-		TG_HIP(hipMemset(s->vc[l], 0, bytes));
+		const size_t bytes = sizeof(float) * std::min(rows, (size_t)s->max_pos[l]) * c.head_dim;
+		list.push_back(TgClear{s->kc[l], bytes});
+		list.push_back(TgClear{s->vc[l], bytes});
 	}
-	TG_HIP(hipMemset(s->ctr, 0, sizeof(int) * 8));
-	if (s->seq) {
-		if (int rc = tg_net_seq_reset(s->seq)) return rc;
-	} else
-		TG_HIP(hipMemset(s->xr, 0, sizeof(float) * (size_t)(2 * c.n_layers + 1) * c.hidden_size));
-	TG_HIP(hipDeviceSynchronize());
+	list.push_back(TgClear{s->ctr, sizeof(int) * 8});
+	if (s->seq) tg_net_seq_reset(s->seq, &list);
+	else list.push_back(TgClear{s->xr, sizeof(float) * (size_t)(2 * c.n_layers + 1) * c.hidden_size});
+	tg_launch_clear(list.data(), (int)list.size(), g_stream);
+	TG_HIP(hipGetLastError());
+	TG_HIP(hipStreamSynchronize(g_stream));
+	s->kv_clean = true;
+	s->kv_hi = 0;
 	s->pos = s->bp_local = s->bp_global = s->steps = 0;
 	s->pick_pending = false;
 	s->taps = nullptr;
@@ -2225,6 +2231,7 @@ int prefill_setup(tg_session *s, int n, PrefillCtx *ctx, bool with_taps, int at 
 		TG_HIP(hipMalloc(&s->pf_ws, need));
 		s->pf_ws_bytes = need;
 	}
+	s->kv_hi = std::max(s->kv_hi, (at < 0 ? 0 : at) + n);
 	uint8_t *ws = (uint8_t *)s->pf_ws;
 	ctx->s = s;
 	ctx->n = n;
@@ -2516,6 +2523,7 @@ int tg_session_kv_prefill(tg_session *s, int layer, const float *keys, const flo
 	if (int rc = block_args_ok(s, layer, keys, rows)) return rc;
 	if (!values) return tg_fail(TG_ERR_BAD_ARG, "null argument");
 	if (s->pos != 0 && s->pos != rows) return tg_fail(TG_ERR_STATE, "the session's position counter is shared by all layers: reset it, or give every layer the same number of rows");
+	s->kv_hi = std::max(s->kv_hi, rows);
 	const int hd = s->m->cfg.head_dim, mp = s->max_pos[(size_t)layer];
 	const int start = rows >= mp ? rows - mp : 0;  // decode.hpp:84-86: the tail of a context longer than the cache
 	const size_t bytes = sizeof(float) * (size_t)(rows - start) * hd;

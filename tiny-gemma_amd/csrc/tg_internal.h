@@ -301,6 +301,11 @@ void tg_launch_gemm(float *C, const float *A, const int8_t *Wp, const float *sca
                     const float *lut, float gmin, float geps, int lut_size, hipStream_t s);
 
 void tg_launch_copy(void *dst, const void *src, size_t bytes, hipStream_t s);
+struct TgClear {
+	void *p;
+	size_t bytes;  // a multiple of 4
+};
+void tg_launch_clear(const TgClear *list, int n, hipStream_t s);  // zeros, one launch for up to TG_CLEAR_MAX buffers
 
 // Load-time re-tiling on the device.  A matrix of N virtual columns is assembled from up to three
 // row-major int8 sources (device pointers, reference layout [K][n[i]], scales[i] per source column):

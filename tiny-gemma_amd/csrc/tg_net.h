@@ -77,7 +77,7 @@ int tg_net_vocab_padded(const TgNet *n);
 void tg_net_step_cost(const TgNet *n, double *bytes, int *launches);
 
 int tg_net_seq_create(TgNet *n, int capacity, TgNetSeq **out);
-int tg_net_seq_reset(TgNetSeq *q);
+void tg_net_seq_reset(TgNetSeq *q, std::vector<TgClear> *clear);  // adds what has to be zero for an empty sequence
 void tg_net_seq_free(TgNetSeq *q);
 void tg_net_seq_release_workspace(TgNetSeq *q);
 // n tokens behind pos earlier ones.  want: positions among them whose logits go to `logits` (host, [n_want][vocab]).

@@ -914,17 +914,16 @@ int tg_net_seq_create(TgNet *n, int capacity, TgNetSeq **out) {
 	for (auto &p : parts) *p.first = (char *)q->ws + p.second;
 	if (hipMemset(q->ws, 0, off) != hipSuccess) return fail("step buffers");
 	*out = q;
-	return tg_net_seq_reset(q);
+	return TG_OK;
 }
 
-int tg_net_seq_reset(TgNetSeq *q) {
+void tg_net_seq_reset(TgNetSeq *q, std::vector<TgClear> *clear) {
 	// Latent rows need no clearing: a row is written before it is read.  Recurrent state starts at zero.
 	for (size_t r = 0; r < q->state.size(); r++) {
 		const int kind = q->net->cfg.layers[(size_t)q->net->cfg.runs[r]].mix.kind;
-		if (kind == TG_MIX_GLA || kind == TG_MIX_DELTA) TG_HIP(hipMemset(q->state[r], 0, q->state_bytes[r]));
+		if (kind == TG_MIX_GLA || kind == TG_MIX_DELTA) clear->push_back(TgClear{q->state[r], q->state_bytes[r]});
 	}
 	q->tap_rows = 0;
-	return TG_OK;
 }
 
 void tg_net_seq_release_workspace(TgNetSeq *q) {
