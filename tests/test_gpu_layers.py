@@ -207,6 +207,23 @@ def test_norm_and_head_alone(tg, folder):
     rows_close(np.concatenate([s.forward([t])[1] for t in ids]), want, F32_TOL, "head, token by token")
 
 
+@pytest.mark.parametrize("heads,n", [(2, 130), (5, 1000), (16, 1030)])
+@pytest.mark.parametrize("kind", ["gla", "delta"])
+def test_chunk_workgroups(tg, folder, kind, heads, n):
+    """Chunks whose outputs take 16, 32 and 64 tokens per workgroup, key sizes of five slabs in groups of four."""
+    if kind == "gla":
+        cfg = nm.config(40, 97, [nm.layer(nm.gla(heads, 130, 130))])
+    else:
+        cfg = nm.tutelix(40, 97, [nm.layer(nm.delta(heads, heads, 130, 130, 3))])
+    path, om = folder(("chunks", kind, heads), cfg, seed=19)
+    ids = ids_of(cfg, n)
+    taps = []
+    want = om.step(om.state(), ids, taps)
+    s = tg.Transformer.from_dir(path, "float32").open_session(n)
+    places = np.unique(np.concatenate([np.arange(0, n, 37), np.arange(n - 20, n)]))
+    rows_close(s.forward(ids, places)[1], want[places], 4 * F32_TOL, f"{kind}, {heads} heads, {n} tokens")
+
+
 # ---- whole models ------------------------------------------------------------------------------------------------------------
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("name", nm.MODELS)

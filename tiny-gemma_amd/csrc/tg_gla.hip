@@ -132,6 +132,8 @@ __global__ __launch_bounds__(256) void gla_decay_kernel(const float *low, int ld
 }
 
 // ---- A: a workgroup per chunk and head, a wave per block of 16 rows ---------------------------------------------------------
+// NS groups of four waves take the slabs of key channels in turn and add their sums at the end: a portion of 130 tokens with four
+// heads has 12 workgroups, and each was a chain of four slabs (30 us with one group at key size 128, 17.5 with four).
 constexpr int SL = 32, SLP = 36;  // key channels per slab, row pitch
 
 // DELTA: also k . k with the decay between them, T = beta (k . k) below the diagonal, of which it leaves -T outside the 16 x 16
@@ -142,18 +144,22 @@ struct DeltaIntra {
 	float *t;           // [chunks][heads][64][64]
 };
 
-template <class TR, bool DELTA>
-__global__ __launch_bounds__(256) void gla_intra_kernel(const typename TR::T *qkv, int ld, int k_off, TgGla g, int n, const float *b, float *A,
-                                                        DeltaIntra x) {
-	__shared__ __align__(16) float s_q[C][SLP], s_k[C][SLP], s_b[C][SLP];
-	const int ch = blockIdx.x, h = blockIdx.y, kh = DELTA ? h / g.group : h, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+template <class TR, bool DELTA, int NS>
+__global__ __launch_bounds__(256 * NS) void gla_intra_kernel(const typename TR::T *qkv, int ld, int k_off, TgGla g, int n, const float *b, float *A,
+                                                             DeltaIntra x) {
+	typedef float Slab[C][SLP];
+	__shared__ __align__(16) float s_all[NS][3][C][SLP];
+	const int ch = blockIdx.x, h = blockIdx.y, kh = DELTA ? h / g.group : h, sg = threadIdx.x >> 8, tid = threadIdx.x & 255, lane = tid & 63, w = tid >> 6;
+	Slab &s_q = s_all[sg][0], &s_k = s_all[sg][1], &s_b = s_all[sg][2];
 	const int lr = lane & 15, lg = lane >> 4, hd = g.heads * g.dimp, t0 = ch * C;
 	f32x4_t off[3], dia = {0, 0, 0, 0}, koff[3], kdia = {0, 0, 0, 0};
 #pragma unroll
 	for (int j = 0; j < 3; j++) off[j] = koff[j] = f32x4_t{0, 0, 0, 0};
-	for (int d0 = 0; d0 < g.dimp; d0 += SL) {
+	for (int base = 0; base < g.dimp; base += SL * NS) {
+		const int d0 = base + SL * sg;
+		const bool has = d0 < g.dimp;  // (uniform over the group)
 		__syncthreads();
-		for (int e = tid; e < C * SL / 4; e += 256) {
+		for (int e = tid; has && e < C * SL / 4; e += 256) {
 			const int r = e / (SL / 4), c4 = (e % (SL / 4)) * 4, t = t0 + r;
 			const size_t col = (size_t)h * g.dimp + d0 + c4, kcol = (size_t)kh * g.dimp + d0 + c4;
 			f32x4_t q = tg_load4(qkv + (size_t)min(t, n - 1) * ld + kcol), k = tg_load4(qkv + (size_t)min(t, n - 1) * ld + k_off + kcol);
@@ -167,6 +173,7 @@ __global__ __launch_bounds__(256) void gla_intra_kernel(const typename TR::T *qk
 			tg_store4(&s_b[r][c4], tg_load4(b + (size_t)t * hd + col));
 		}
 		__syncthreads();
+		if (!has) continue;
 		const int qi = 16 * w + lr;
 		if (w > 0) {
 			for (int st = 0; st < SL / 4; st++) {
@@ -201,6 +208,27 @@ __global__ __launch_bounds__(256) void gla_intra_kernel(const typename TR::T *qk
 			}
 		}
 	}
+	if constexpr (NS > 1) {  // the groups' sums, in order
+		constexpr int NV = DELTA ? 8 : 4;
+		static_assert(sizeof(s_all) >= sizeof(f32x4_t) * (NS - 1) * NV * 256, "the sums take the slabs' place");
+		f32x4_t(*sum)[NV][256] = reinterpret_cast<f32x4_t(*)[NV][256]>(&s_all[0][0][0][0]);
+		__syncthreads();
+		auto each = [&](auto f) {
+#pragma unroll
+			for (int j = 0; j < 3; j++) f(j, off[j]);
+			f(3, dia);
+			if constexpr (DELTA) {
+#pragma unroll
+				for (int j = 0; j < 3; j++) f(4 + j, koff[j]);
+				f(7, kdia);
+			}
+		};
+		if (sg > 0) each([&](int i, f32x4_t &v) { sum[sg - 1][i][tid] = v; });
+		__syncthreads();
+		if (sg > 0) return;
+#pragma unroll
+		for (int o = 0; o < NS - 1; o++) each([&](int i, f32x4_t &v) { v += sum[o][i][tid]; });
+	}
 	float *out = A + ((size_t)ch * g.heads + h) * C * C;
 #pragma unroll
 	for (int j = 0; j < 4; j++) {
@@ -227,7 +255,7 @@ __global__ __launch_bounds__(256) void gla_intra_kernel(const typename TR::T *qk
 #pragma unroll
 				for (int e = 0; e < 4; e++) T[(size_t)(16 * w + 4 * lg + e) * C + 16 * j + lr] = -beta_r[e] * koff[j][e];
 			}
-		__syncthreads();
+		__builtin_amdgcn_wave_barrier();  // a wave reads what it wrote itself
 		float m[16];
 #pragma unroll
 		for (int r = 0; r < 16; r++) {
@@ -434,29 +462,33 @@ __global__ __launch_bounds__(256) void gla_scan_kernel(float *U, const float *b,
 	g.state[e] = s;
 }
 
-// ---- o = (q e^b)^T S + A v, the head's root mean square norm and silu(gate): 64 tokens x the whole head per workgroup -------------
-// 8 waves: 16 tokens x half of the value columns each.  Slabs of 32: first the key channels (rows q e^b, columns of S), then
+// ---- o = (q e^b)^T S + A v, the head's root mean square norm and silu(gate): TB tokens x the whole head per workgroup -------------
+// 8 waves: 16 tokens x 1 / NC of the value columns each (64 tokens: half of them; fewer tokens where there are few chunks, see
+// launch_out_vb).  Slabs of 32: first the key channels (rows q e^b, columns of S), then
 // the chunk's own tokens (rows A, columns v); a slab's loads are in flight during the one before it.
 // (delta rule: v is u, the states are tiles (value columns, key channels) like u's, the gate's function is the sigmoid)
 struct OutIn {
 	const void *q, *v, *gate;
 	int ldq, ldv, ldg;
 };
-template <class TI, class TR, int VB, bool DELTA>
+template <class TI, class TR, int VB, bool DELTA, int TB>
 __global__ __launch_bounds__(512) void gla_out_kernel(OutIn in, TgGla g, int n, const float *b, const float *A, const float *U, typename TR::T *out,
                                                       int ld_out) {
 	const typename TI::T *Q = (const typename TI::T *)in.q + (size_t)(DELTA ? blockIdx.y / g.group : blockIdx.y) * g.dimp,
 	                     *V = (const typename TI::T *)in.v + (DELTA ? ((size_t)blockIdx.x * g.heads + blockIdx.y) * g.vdimp * C : (size_t)blockIdx.y * g.vdimp);
 	// (delta rule: v and S come transposed and are turned on their way into LDS; the pitch keeps those writes apart)
-	constexpr int XP = 36, YP = VB + (DELTA ? 18 : 16), NI = VB / 32, NY = 32 * VB / 4 / 512;
-	__shared__ __align__(16) float s_x[C][XP], s_y[32][YP];
-	__shared__ float s_sq[2][C];
-	const int ch = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, w = tid >> 6, wt = (w & 3) * 16, wv = (w >> 2) * (VB / 2);
-	const int lr = lane & 15, lg = lane >> 4, hd = g.heads * g.dimp, t0 = ch * C;
+	constexpr int NTT = TB / 16, NC = 8 / NTT;  // token tiles, groups of columns
+	constexpr int XP = 36, YP = VB + (DELTA ? 18 : 16), NI = VB / 16 / NC, NY = 32 * VB / 4 / 512;
+	static_assert(NI >= 1, "a wave has a tile of columns");
+	__shared__ __align__(16) float s_x[TB][XP], s_y[32][YP];
+	__shared__ float s_sq[NC][TB];
+	const int ch = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, w = tid >> 6, wt = (w % NTT) * 16, wc = w / NTT, wv = wc * (VB / NC);
+	const int lr = lane & 15, lg = lane >> 4, hd = g.heads * g.dimp, c0 = ch * C, b0 = (int)blockIdx.z * TB, t0 = c0 + b0;
+	if (t0 >= n) return;  // a part of the last chunk behind the end
 	const float *S = U + ((size_t)ch * g.heads + h) * g.dimp * g.vdimp;
 	const int slabs = g.dimp / 32;  // dimp is a multiple of 32
 	f32x4_t x, bx, y[NY];
-	const int xr = tid >> 3, xc = (tid & 7) * 4;
+	const int xr = (tid >> 3) % TB, xc = (tid & 7) * 4;  // (TB < 64: the first threads' pieces again, not stored)
 	auto fetch = [&](int sl) {
 		if (sl < slabs) {
 			const size_t qc = (size_t)h * g.dimp + sl * 32 + xc;
@@ -470,12 +502,12 @@ __global__ __launch_bounds__(512) void gla_out_kernel(OutIn in, TgGla g, int n, 
 			}
 		} else {
 			const int j0 = (sl - slabs) * 32;
-			x = tg_load4(A + (((size_t)ch * g.heads + h) * C + xr) * C + j0 + xc);
+			x = tg_load4(A + (((size_t)ch * g.heads + h) * C + b0 + xr) * C + j0 + xc);
 #pragma unroll
 			for (int i = 0; i < NY; i++) {
 				const int e = tid + 512 * i, r = e / (VB / 4), c4 = (e % (VB / 4)) * 4;
 				if constexpr (DELTA) y[i] = tg_load4(V + ((size_t)(min(e >> 3, g.vdimp - 1) >> 4) * 4 + j0 / 16 + ((e >> 2) & 1)) * 256 + ((e >> 3) & 15) * 4 + (e & 3) * 64);
-				else y[i] = tg_load4(V + (size_t)min(t0 + j0 + r, n - 1) * in.ldv + (c4 < g.vdimp ? c4 : 0));
+				else y[i] = tg_load4(V + (size_t)min(c0 + j0 + r, n - 1) * in.ldv + (c4 < g.vdimp ? c4 : 0));
 			}
 		}
 	};
@@ -484,7 +516,7 @@ __global__ __launch_bounds__(512) void gla_out_kernel(OutIn in, TgGla g, int n, 
 #pragma unroll
 			for (int e = 0; e < 4; e++) x[e] = x[e] * g.qscale * pow2(bx[e]);
 		}
-		tg_store4(&s_x[xr][xc], x);
+		if (TB == 64 || tid < 8 * TB) tg_store4(&s_x[xr][xc], x);
 #pragma unroll
 		for (int i = 0; i < NY; i++) {
 			const int e = tid + 512 * i, r = e / (VB / 4), c4 = (e % (VB / 4)) * 4;
@@ -521,11 +553,14 @@ __global__ __launch_bounds__(512) void gla_out_kernel(OutIn in, TgGla g, int n, 
 		for (int e = 0; e < 4; e++) ss = fmaf(acc[j][e], acc[j][e], ss);
 	ss += tg_red_partner<32>(ss);
 	ss += tg_red_partner<16>(ss);
-	if (lg == 0) s_sq[w >> 2][wt + lr] = ss;
+	if (lg == 0) s_sq[wc][wt + lr] = ss;
 	__syncthreads();
 	const int t = t0 + wt + lr;
 	if (t >= n) return;
-	const float inv = 1.0f / sqrtf((s_sq[0][wt + lr] + s_sq[1][wt + lr]) / (float)g.vdim + g.eps);
+	float sq = s_sq[0][wt + lr];
+#pragma unroll
+	for (int i = 1; i < NC; i++) sq += s_sq[i][wt + lr];
+	const float inv = 1.0f / sqrtf(sq / (float)g.vdim + g.eps);
 	typename TR::T *dst = out + (size_t)t * ld_out + (size_t)h * g.vdimp;
 	const typename TR::T *gate = (const typename TR::T *)in.gate + (size_t)t * in.ldg + (size_t)h * g.vdimp;
 #pragma unroll
@@ -540,13 +575,30 @@ __global__ __launch_bounds__(512) void gla_out_kernel(OutIn in, TgGla g, int n, 
 		}
 	}
 	if (h == g.heads - 1)  // the columns behind the heads
-		for (int v = g.heads * g.vdimp + (w >> 2) * 16 + 4 * lg; v < ld_out; v += 32) tg_store4(out + (size_t)t * ld_out + v, f32x4_t{0, 0, 0, 0});
+		for (int v = g.heads * g.vdimp + wc * 16 + 4 * lg; v < ld_out; v += 16 * NC) tg_store4(out + (size_t)t * ld_out + v, f32x4_t{0, 0, 0, 0});
+}
+
+template <class TR, bool DELTA>
+void launch_intra(const typename TR::T *qkv, int ld, int k_off, const TgGla &g, int n, const float *b, float *A, const DeltaIntra &x, hipStream_t s) {
+	const dim3 grid((unsigned)((n + C - 1) / C), (unsigned)g.heads);
+	auto go = [&](auto *kernel, int groups) { hipLaunchKernelGGL(kernel, grid, dim3(256 * groups), 0, s, qkv, ld, k_off, g, n, b, A, x); };
+	if (g.dimp <= 32) go(gla_intra_kernel<TR, DELTA, 1>, 1);
+	else if (g.dimp < 128) go(gla_intra_kernel<TR, DELTA, 2>, 2);
+	else go(gla_intra_kernel<TR, DELTA, 4>, 4);
 }
 
 template <class TI, class TR, int VB, bool DELTA>
 void launch_out_vb(const TgGla &g, const OutIn &in, int n, const float *b, const float *A, const float *U, void *out, int ld_out, hipStream_t s) {
-	hipLaunchKernelGGL((gla_out_kernel<TI, TR, VB, DELTA>), dim3((unsigned)((n + C - 1) / C), (unsigned)g.heads), dim3(512), 0, s, in, g, n, b, A, U,
-	                   (typename TR::T *)out, ld_out);
+	// A workgroup's time is its chain of slabs; with few chunks and heads the tokens of a chunk go to several workgroups, each with
+	// a part of the matrix instructions and all of the chunk's states and values (3 chunks, 4 heads, 128 x 256: 24.7 us with 64
+	// tokens, 13.7 with 16; 16 chunks, 4 heads, 64 x 128: 12.8 with 64, 9.2 with 32).
+	const unsigned chunks = (unsigned)((n + C - 1) / C), H = (unsigned)g.heads;
+	auto go = [&](auto *kernel, int tokens) { hipLaunchKernelGGL(kernel, dim3(chunks, H, C / tokens), dim3(512), 0, s, in, g, n, b, A, U, (typename TR::T *)out, ld_out); };
+	if constexpr (VB >= 128) {
+		if (chunks * H < 64) return go(gla_out_kernel<TI, TR, VB, DELTA, 16>, 16);
+	}
+	if (chunks * H < 256) go(gla_out_kernel<TI, TR, VB, DELTA, 32>, 32);
+	else go(gla_out_kernel<TI, TR, VB, DELTA, 64>, 64);
 }
 template <class TI, class TR, bool DELTA>
 void launch_out(const TgGla &g, const OutIn &in, int n, const float *b, const float *A, const float *U, void *out, int ld_out, hipStream_t s) {
@@ -563,7 +615,7 @@ void launch_rows(const TgGla &g, const void *qkv, int ld, int k_off, int v_off, 
 	const T *x = (const T *)qkv;
 	const unsigned chunks = (unsigned)((n + C - 1) / C), H = (unsigned)g.heads, hd = (unsigned)(g.heads * g.dimp), nd = (unsigned)((g.dimp + 127) / 128);
 	hipLaunchKernelGGL(gla_decay_kernel, dim3(chunks, (hd + 63) / 64), dim3(256), 0, s, low, ld_low, g, n, t.b);
-	hipLaunchKernelGGL((gla_intra_kernel<TR, false>), dim3(chunks, H), dim3(256), 0, s, x, ld, k_off, g, n, t.b, t.a, DeltaIntra{});
+	launch_intra<TR, false>(x, ld, k_off, g, n, t.b, t.a, DeltaIntra{}, s);
 	if (g.vdimp <= 64)
 		hipLaunchKernelGGL((gla_state_kernel<TR, 64>), dim3(chunks, H, nd), dim3(512), 0, s, x, ld, k_off, v_off, g, n, t.b, t.u);
 	else
@@ -977,8 +1029,7 @@ void launch_delta_rows(const TgDelta &d, const void *xv, int ld, const float *lo
 	else if (d.taps == 3) prep(delta_prep_kernel<TR, 3>);
 	else prep(delta_prep_kernel<TR, 0>);
 	hipLaunchKernelGGL(gla_decay_kernel, dim3(chunks, (unsigned)((hd + 63) / 64)), dim3(256), 0, s, low + a_off, ld_low, g, n, t.b);
-	hipLaunchKernelGGL((gla_intra_kernel<TgF32, true>), dim3(chunks, (unsigned)g.heads), dim3(256), 0, s, t.qk, 2 * qc, qc, g, n, t.b, t.a,
-	                   DeltaIntra{low + b_off, ld_low, t.t});
+	launch_intra<TgF32, true>(t.qk, 2 * qc, qc, g, n, t.b, t.a, DeltaIntra{low + b_off, ld_low, t.t}, s);
 	const DeltaSolve solve = {t.qk, t.b, t.t, low + b_off, 2 * qc, qc, ld_low, t.v, t.u, t.wk, t.kt};
 	hipLaunchKernelGGL(delta_solve_kernel, dim3(chunks, (unsigned)g.heads, (unsigned)((g.dimp + g.vdimp + 127) / 128)), dim3(256), 0, s, solve, g, n);
 	const dim3 grid((unsigned)g.heads, (unsigned)(g.vdimp / 16));
