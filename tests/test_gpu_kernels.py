@@ -207,6 +207,26 @@ def test_qgemm_two_workgroups_per_unit_equal_the_other_kernels_and_the_closed_fo
     assert np.array_equal(out[0], _digit_plane_closed_form(A, W, s))
 
 
+@pytest.mark.parametrize("m, i, n, few", [(449, 6912, 1152, True), (777, 6912, 1152, True), (896, 256, 1152, True), (897, 256, 1152, False),
+                                          (1632, 640, 640, True), (1633, 640, 640, False), (1009, 2048, 256, True), (4096, 256, 256, True),
+                                          (4097, 256, 256, False)])
+def test_qgemm_one_round_of_the_few_row_kernel(tg, m, i, n, few):
+    """More than 448 rows run on the few-row kernel while its workgroups (32 rows x 128 columns) are at most the 256
+    compute units, and on the plain tiling from one more on: both sides of the line at three widths, with K of one stage a
+    wave up to 27, rows that fill no group of eight and no tile, and rows of very small, very large and no magnitude.
+    Integer sums and one rounding: equal to the closed form bit for bit."""
+    A, W, s = gi.gemm_inputs(m, i, n, 41)
+    A[1] *= np.float32(1e-5)
+    A[m // 2] = 0
+    A[m - 1] *= np.float32(3e4)
+    C = np.full((m, n), np.nan, np.float32)
+    before = tg.gemm_launches()
+    tg.launch_qgemm(C, A, W, s, m, i, n)
+    ran = tuple(b - a for a, b in zip(before, tg.gemm_launches()))
+    assert ran[0] == (1 if few else 0) and sum(ran) == 1
+    assert np.array_equal(C, _digit_plane_closed_form(A, W, s))
+
+
 def test_device_resident_gemv_matches_host_entry(tg, oracle):
     x, W, s = gi.gemv_inputs(1152, 6912, 9)
     w = tg.QWeight(W, s)

@@ -65,48 +65,77 @@ __device__ __forceinline__ float gelu_lut(float x, const float *lut, float gmin,
 	return lut[idx];
 }
 
-// One wave per row: mul[m] = 2^s with max|A[m][:]| * 2^s in [2^21, 2^22), inv[m] = 2^-s.
-__global__ __launch_bounds__(GNT) void row_scale_kernel(const float *A, int lda, int M, int K, float *mul, float *inv, int Mpad) {
-	const int lane = threadIdx.x & 63, m = blockIdx.x * 4 + (threadIdx.x >> 6);
-	if (m >= Mpad) return;
-	float amax = 0.0f;
-	if (m < M) {
-		const f32x4 *row = reinterpret_cast<const f32x4 *>(A + (size_t)m * lda);
-		for (int i = lane; i < (K >> 2); i += 64) {
-			const f32x4 a = row[i];
-			amax = fmaxf(amax, fmaxf(fmaxf(fabsf(a[0]), fabsf(a[1])), fmaxf(fabsf(a[2]), fabsf(a[3]))));
-		}
+// A [M][lda] fp32 -> digit planes in A-operand order and the row factors mul[m] = 2^s with max|A[m][:]| * 2^s in
+// [2^21, 2^22), inv[m] = 2^-s.  Workgroup = ROWS rows whole, LANES lanes along K with 16 consecutive k each, NG times:
+// the rows stay in registers between the pass that finds their maxima and the one that forms the planes, so A is read
+// once and in one launch.  Bound by the latency of its one read and the conversions (fewer rows a workgroup spread them
+// over more compute units), from a few thousand rows on by memory.  777 rows of 1152 take 4.9 us and of 6912 9.0 us, where a
+// launch for the maxima and one for the planes took 10.4 and 13.4 us; eight rows of 6912 a workgroup 16.0 us (with the
+// digits taken one at a time).
+template <int ROWS, int LANES, int NG>
+__global__ __launch_bounds__(ROWS * LANES) void quant_rows_kernel(const float *A, int lda, int M, int K, int8_t *Apack, float *mul_out, float *inv_out) {
+	constexpr int NW = ROWS * LANES / 64;
+	static_assert(ROWS == 4 || ROWS == 8, "the rows of a wave's lanes");
+	__shared__ float smax[NW][ROWS];
+	const int tid = threadIdx.x, r = tid & (ROWS - 1), kq = tid / ROWS, m = blockIdx.x * ROWS + r;
+	const int ngrp = K >> 4;
+	const float *row = A + (size_t)(m < M ? m : M - 1) * lda;
+	f32x4 v[NG][4];
+#pragma unroll
+	for (int g = 0; g < NG; g++) {
+		const int k = kq + g * LANES;
+		const f32x4 *src = reinterpret_cast<const f32x4 *>(row + 16 * (k < ngrp ? k : ngrp - 1));  // past K: the last group again, which changes no maximum
+#pragma unroll
+		for (int q = 0; q < 4; q++) v[g][q] = src[q];
 	}
-	amax = tg_wave_max(amax);
-	if (lane == 0) {
-		float s, r;
-		tg_row_factors(amax, s, r);
-		mul[m] = s;
-		inv[m] = r;
+	float amax = 0.0f;
+#pragma unroll
+	for (int g = 0; g < NG; g++)
+#pragma unroll
+		for (int q = 0; q < 4; q++)
+#pragma unroll
+			for (int i = 0; i < 4; i++) amax = fmaxf(amax, fabsf(v[g][q][i]));
+	amax = fmaxf(amax, tg_red_partner<32>(amax));
+	amax = fmaxf(amax, tg_red_partner<16>(amax));
+	amax = fmaxf(amax, tg_red_partner<8>(amax));
+	if constexpr (ROWS == 4) amax = fmaxf(amax, tg_red_partner<4>(amax));
+	if ((tid & 63) < ROWS) smax[tid >> 6][r] = amax;
+	__syncthreads();
+#pragma unroll
+	for (int w = 0; w < NW; w++) amax = fmaxf(amax, smax[w][r]);
+	float factor = 1.0f, rcp = 1.0f;
+	if (m < M) tg_row_factors(amax, factor, rcp);  // rows of the padding: factors of 1, planes of 0
+	if (kq == 0) {
+		mul_out[m] = factor;
+		inv_out[m] = rcp;
+	}
+#pragma unroll
+	for (int g = 0; g < NG; g++) {
+		const int k = kq + g * LANES;
+		i32x4 pl[3] = {i32x4{0, 0, 0, 0}, i32x4{0, 0, 0, 0}, i32x4{0, 0, 0, 0}};
+		if (m < M) tg_quant16(reinterpret_cast<const float *>(&v[g][0]), factor, pl);
+		if (k < ngrp) {
+			i32x4 *dst = tg_plane_dst(Apack, m, 16 * k, K);
+#pragma unroll
+			for (int p = 0; p < 3; p++) dst[p * 64] = pl[p];
+		}
 	}
 }
 
-// A [M][lda] fp32 -> digit planes in A-operand order.  Workgroup = 32 rows x 128 k; thread = one lane's 16
-// bytes of one (k step, half): row r = tid % 32, k = 128 blockIdx.y + 16 (tid / 32) .. + 15.
-// FROM_MAX: `mul` holds the rows' maxima instead (left by the producer of A): the factors are formed here, and the
-// workgroups of the first 128 k also store them for the product's epilogue (mul_out, inv_out).
-template <bool FROM_MAX>
-__global__ __launch_bounds__(GNT) void quant_pack_kernel(const float *A, int lda, int M, int K, const float *mul, int8_t *Apack,
+// The same from row maxima that the producer of A left.  Workgroup = 32 rows x 128 k; thread = one lane's 16 bytes of
+// one (k step, half): row r = tid % 32, k = 128 blockIdx.y + 16 (tid / 32) .. + 15.  The workgroups of the first 128 k
+// also store the factors for the product's epilogue (mul_out, inv_out).
+__global__ __launch_bounds__(GNT) void quant_pack_kernel(const float *A, int lda, int M, int K, const float *amax, int8_t *Apack,
                                                          float *mul_out, float *inv_out) {
 	const int tid = threadIdx.x, r = tid & 31, kq = tid >> 5;
 	const int mtile = blockIdx.x, m = mtile * 32 + r;
 	const int k0 = blockIdx.y * 128 + 16 * kq;
 	i32x4 pl[3] = {i32x4{0, 0, 0, 0}, i32x4{0, 0, 0, 0}, i32x4{0, 0, 0, 0}};
-	float factor = 1.0f;
-	if (FROM_MAX) {
-		float rcp;
-		tg_row_factors(m < M ? mul[m] : 0.0f, factor, rcp);  // rows of the padding were never written
-		if (blockIdx.y == 0 && kq == 0) {
-			mul_out[m] = factor;
-			inv_out[m] = rcp;
-		}
-	} else if (m < M) {
-		factor = mul[m];
+	float factor, rcp;
+	tg_row_factors(m < M ? amax[m] : 0.0f, factor, rcp);  // rows of the padding were never written
+	if (blockIdx.y == 0 && kq == 0) {
+		mul_out[m] = factor;
+		inv_out[m] = rcp;
 	}
 	if (m < M) {
 		const f32x4 *src = reinterpret_cast<const f32x4 *>(A + (size_t)m * lda + k0);
@@ -704,19 +733,31 @@ size_t tg_gemm_mfma_rows(int M) { return (size_t)((M + 127) / 128) * 128; }
 // rowmax != nullptr: [tg_gemm_mfma_rows(M)] row maxima left by the producer of A (no pass over A for them).
 void tg_launch_quant_pack(const float *A, int lda, int M, int K, int8_t *apack, float *rowfac, const float *rowmax, hipStream_t s) {
 	const int Mpad = (int)tg_gemm_mfma_rows(M);
-	const dim3 grid((unsigned)(Mpad / 32), (unsigned)(K / 128));
 	if (rowmax != nullptr) {
-		hipLaunchKernelGGL(quant_pack_kernel<true>, grid, dim3(GNT), 0, s, A, lda, M, K, rowmax, apack, rowfac, rowfac + Mpad);
+		hipLaunchKernelGGL(quant_pack_kernel, dim3((unsigned)(Mpad / 32), (unsigned)(K / 128)), dim3(GNT), 0, s, A, lda, M, K, rowmax, apack, rowfac,
+		                   rowfac + Mpad);
 		return;
 	}
-	hipLaunchKernelGGL(row_scale_kernel, dim3((unsigned)(Mpad / 4)), dim3(GNT), 0, s, A, lda, M, K, rowfac, rowfac + Mpad, Mpad);
-	hipLaunchKernelGGL(quant_pack_kernel<false>, grid, dim3(GNT), 0, s, A, lda, M, K, rowfac, apack, (float *)nullptr, (float *)nullptr);
+	if (K <= 2048)  // 128 lanes of 16 values
+		hipLaunchKernelGGL((quant_rows_kernel<4, 128, 1>), dim3((unsigned)(Mpad / 4)), dim3(512), 0, s, A, lda, M, K, apack, rowfac, rowfac + Mpad);
+	else  // K is at most 6912
+		hipLaunchKernelGGL((quant_rows_kernel<4, 256, 2>), dim3((unsigned)(Mpad / 4)), dim3(1024), 0, s, A, lda, M, K, apack, rowfac, rowfac + Mpad);
+}
+
+// Whether a product of M rows in ntiles column tiles and kparts parts of K runs on the few-row kernel, which splits K over
+// a workgroup's waves and has four workgroups where the plain tiling has one.  It is the better one while its grid is one
+// round of workgroups (one fits a compute unit): 256 rows of K take it 0.76 us, the plain tiling 2.2 us.  Few rows are its
+// case in any number of rounds that TG_GEMM_SKINNY_BLOCKS allows.  Measured, 777 rows of the 1B shape, K = 6912, 9 column
+// tiles: 25.4 us here, 60 us in the plain tiling.
+static bool tg_gemm_skinny_taken(int M, int ntiles, int kparts, int n_cu) {
+	if (M <= TG_GEMM_SKINNY_ROWS && ntiles * ((M + 127) / 128) < TG_GEMM_SKINNY_BLOCKS) return true;
+	return (long)ntiles * ((M + 31) / 32) * kparts <= n_cu;
 }
 
 // whether a product of M rows, K deep, ntiles column tiles runs on gemm_i8_lds_kernel (K in whole groups of four k steps)
 static bool tg_gemm_lds_taken(int M, int K, int ntiles) {
 	const int tiles = ntiles * ((M + 127) / 128);
-	if (M <= TG_GEMM_SKINNY_ROWS && tiles < TG_GEMM_SKINNY_BLOCKS) return false;  // the few-row kernel's case
+	if (tg_gemm_skinny_taken(M, ntiles, 1, g_gemm_lds_cus)) return false;
 	return g_gemm_lds > 0 && (K & 127) == 0 && 2 * tiles >= g_gemm_lds * g_gemm_lds_cus;
 }
 
@@ -733,8 +774,7 @@ void tg_launch_gemm_mfma(float *C, const int8_t *apack, const float *rowfac, con
 	const bool geglu = epi == TG_EPI_GEGLU, lutlds = geglu && lut_size <= LUT_LDS_MAX;
 	const int ldc = geglu ? ntiles * (TG_CT / 2) : ntiles * TG_CT;
 	float *rmp = geglu ? rowmax_part : nullptr;
-	// few rows and few column tiles: split K over the waves instead of leaving most compute units idle
-	if (M <= TG_GEMM_SKINNY_ROWS && (int)mblocks * ntiles < TG_GEMM_SKINNY_BLOCKS) {
+	if (tg_gemm_skinny_taken(M, ntiles, geglu ? 1 : kparts, g_gemm_lds_cus)) {
 		g_gemm_launches[0]++;
 		const dim3 grid((unsigned)ntiles, (unsigned)((M + 31) / 32), (unsigned)(geglu ? 1 : kparts)), block(GNT);
 		if (geglu && lutlds)
@@ -789,17 +829,21 @@ void tg_launch_gemm_mfma(float *C, const int8_t *apack, const float *rowfac, con
 
 // In how many parts of K (1, 2 or 4) a STORE product of M rows, K deep, ntiles column tiles should run; the parts
 // write separate partial results which the consumer adds.
-//   * the few-row kernel: as many parts as leave each at least 8 stages (the down projection of a 178-token prompt:
-//     54 workgroups walking 6912 rows of K become 216 walking 1728);
+//   * the few-row kernel: as many parts as leave each at least 8 stages and fit in one round of workgroups (the down
+//     projection of a 178-token prompt: 54 workgroups walking 6912 rows of K become 216 walking 1728; prompts of 225, 300
+//     and 448 tokens of the 1B shape 2.42, 2.81 and 3.05 ms, with parts in two rounds 2.52, 2.93 and 3.19 ms).  Whole
+//     where one round takes more than 448 rows of a long K or fills two thirds of the chip: 777 tokens of the 1B shape
+//     4.30 ms, with the output projection in halves of the plain tiling 4.40 ms, with both products so 4.68 ms;
 //   * the tiled kernel: 2 when that fills the last round of workgroups noticeably better (whole pairs of stages per half).
 int tg_gemm_mfma_k_parts(int M, int K, int ntiles, int n_cu) {
 	const int nstage = K / KSTAGE;
-	if (M <= TG_GEMM_SKINNY_ROWS && ((M + 127) / 128) * ntiles < TG_GEMM_SKINNY_BLOCKS) {
-		if (nstage % 4 == 0 && nstage / 4 >= 8) return 4;
-		if (nstage % 2 == 0 && nstage / 2 >= 8) return 2;
+	if (M <= TG_GEMM_SKINNY_ROWS && tg_gemm_skinny_taken(M, ntiles, 1, n_cu)) {
+		for (int parts = 4; parts > 1; parts /= 2)
+			if (nstage % parts == 0 && nstage / parts >= 8 && (long)ntiles * ((M + 31) / 32) * parts <= n_cu) return parts;
 		return 1;
 	}
 	if (M <= TG_GEMM_SKINNY_ROWS || nstage % 4 != 0) return 1;
+	if (tg_gemm_skinny_taken(M, ntiles, 1, n_cu) && (nstage >= 32 || 3 * ntiles * ((M + 31) / 32) > 2 * n_cu)) return 1;
 	if (tg_gemm_lds_taken(M, K, ntiles)) {
 		// Two workgroups per compute unit.  With more tiles than compute units but well under two per unit, most units
 		// would hold one workgroup and a few two, and those few set the pace: two half-K copies fill both slots of
