@@ -1461,7 +1461,7 @@ static void flush_pick(tg_session *s) {
 static void finish_pick(tg_session *s, bool may_stay) {
 	if (s->sampling)
 		tg_launch_minp(s->logits, s->m->cfg.n_vocab, s->s_minp, s->s_temp, s->randf, -1, s->rand_base, s->probs, s->seg, s->bsum, s->bmax,
-		               s->ctr, s->tok_log, 0, nullptr, g_stream);
+		               s->blk_val, head_blocks(s), s->ctr, s->tok_log, 0, nullptr, g_stream);
 	else if (may_stay)
 		s->pick_pending = true;
 	else
@@ -2697,7 +2697,7 @@ int tg_minp_logits(const float *logits, int n_vocab, float minp, float temp, flo
 	    hipMemcpy(d_rand, &randf, sizeof(float), hipMemcpyHostToDevice) != hipSuccess)
 		rc = tg_fail(TG_ERR_HIP, "upload failed");
 	if (rc == TG_OK) {
-		tg_launch_minp(d_logits, n_vocab, minp, temp, d_rand, 0, 0, d_probs, d_seg, d_bsum, d_bmax, nullptr, nullptr, 2, d_tok, g_stream);
+		tg_launch_minp(d_logits, n_vocab, minp, temp, d_rand, 0, 0, d_probs, d_seg, d_bsum, d_bmax, nullptr, 0, nullptr, nullptr, 2, d_tok, g_stream);
 		if (hipStreamSynchronize(g_stream) != hipSuccess || hipMemcpy(token_out, d_tok, sizeof(int), hipMemcpyDeviceToHost) != hipSuccess)
 			rc = tg_fail(TG_ERR_HIP, "sampler launch failed");
 	}
@@ -2736,7 +2736,7 @@ int tg_generate(tg_session *s, const int32_t *prompt, int n_prompt, int n_decode
 	if (int rc = tg_forward_prefill(s, prompt, n_prompt, nullptr, &tok)) return rc;
 	// the prefill logits are still on the device: draw the first token from them (transformer.hpp:208-211)
 	if (int rc = sampler_prepare(s, randf, 1)) return rc;
-	tg_launch_minp(s->logits, s->m->cfg.n_vocab, minp, temp, s->randf, 0, 0, s->probs, s->seg, s->bsum, s->bmax, s->ctr, s->tok_log, 1,
+	tg_launch_minp(s->logits, s->m->cfg.n_vocab, minp, temp, s->randf, 0, 0, s->probs, s->seg, s->bsum, s->bmax, nullptr, 0, s->ctr, s->tok_log, 1,
 	               nullptr, g_stream);
 	TG_HIP(hipStreamSynchronize(g_stream));
 	auto t1 = clk::now();

@@ -184,7 +184,8 @@ size_t tg_minp_blocks(int n);
 size_t tg_minp_padded(int n);
 size_t tg_minp_segments(int n);
 void tg_launch_minp(const float *logits, int n, float minp, float temp, const float *randf, int rand_idx, int rand_base, float *probs,
-                    float *seg, float *bsum, float *bmax, int *ctr, int *tok_log, int mode, int *out_tok, hipStream_t s);
+                    float *seg, float *bsum, float *bmax, const float *head_max, int head_n, int *ctr, int *tok_log, int mode, int *out_tok,
+                    hipStream_t s);
 
 // ---- one-kernel decode step (tg_decode_fused.hip) --------------------------------------------------------------
 // All layers of a decode step in ONE launch of resident workgroups: `ng` GEMV workgroups that own fixed column tiles of

@@ -13,9 +13,11 @@
 // can differ from the reference's only where randf lies within fp32 summation error of a boundary of the
 // cumulative distribution.
 //
-// Three launches per token: block maxima; probabilities + masked block sums + sums of 256-element
-// segments; one workgroup that finds the crossing segment, re-scans it and does the per-token bookkeeping
-// tg_argmax_finish does on the greedy branch.
+// Two launches per token behind a head that left its workgroups' maxima, three without: block maxima; probabilities +
+// masked block sums + sums of 256-element segments; one workgroup that finds the crossing segment, re-scans it and does
+// the per-token bookkeeping tg_argmax_finish does on the greedy branch.
+// Each is bound by its launch and the memory round trips in series.  The head's maxima serve a decode step as they are:
+// a division by temp > 0 is monotonic, so max(l) / temp is max(l / temp) bit for bit.
 
 #include "tg_internal.h"
 
@@ -53,19 +55,26 @@ __global__ __launch_bounds__(SNT) void minp_max_kernel(const float *logits, int 
 	if (tid == 0) bmax[blockIdx.x] = fmaxf(fmaxf(sm[0], sm[1]), fmaxf(sm[2], sm[3]));
 }
 
-// probs[i] = exp(logits[i] / temp - rowmax); seg[s] = sum of segment s; bsum[b] = sum of the workgroup's
+// probs[i] = exp(logits[i] / temp - rowmax), rowmax the largest of bmax[nblocks] divided by bdiv (temp for maxima of the
+// logits themselves, 1 for those of minp_max_kernel); seg[s] = sum of segment s; bsum[b] = sum of the workgroup's
 // probabilities that are >= cut.  maxp is exp(0) = 1 (the maximum element itself), so cut = minp.
 __global__ __launch_bounds__(SNT) void minp_prob_kernel(const float *logits, int n, float temp, float minp, const float *bmax, int nblocks,
-                                                        float *probs, float *seg, float *bsum) {
+                                                        float bdiv, float *probs, float *seg, float *bsum) {
 	__shared__ float sm[SNT / 64], ss[SNT / 64];
 	const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
 	const f32x4 l = load_logits(logits, (int)blockIdx.x * SCHUNK + 4 * tid, n);
 	float m = -INFINITY;
-	for (int i = tid; i < nblocks; i += SNT) m = fmaxf(m, bmax[i]);
+	for (int i0 = 0; i0 < nblocks; i0 += 8 * SNT) {  // eight loads in flight; past the end the last one again
+		float b[8];
+#pragma unroll
+		for (int u = 0; u < 8; u++) b[u] = bmax[min(i0 + u * SNT + tid, nblocks - 1)];
+#pragma unroll
+		for (int u = 0; u < 8; u++) m = fmaxf(m, b[u]);
+	}
 	m = wave_max(m);
 	if (lane == 0) sm[w] = m;
 	__syncthreads();
-	const float rowmax = fmaxf(fmaxf(sm[0], sm[1]), fmaxf(sm[2], sm[3]));
+	const float rowmax = fmaxf(fmaxf(sm[0], sm[1]), fmaxf(sm[2], sm[3])) / bdiv;
 	const float cut = minp * 1.0f;
 	f32x4 p;
 	float all = 0.0f, kept = 0.0f;
@@ -94,35 +103,35 @@ __global__ __launch_bounds__(SNT) void minp_prob_kernel(const float *logits, int
 __global__ __launch_bounds__(FNT) void minp_finish_kernel(const float *probs, const float *seg, const float *bsum, int nblocks, int nseg,
                                                           const float *randf, int rand_idx, int rand_base, int *ctr, int *tok_log,
                                                           int mode, int *out_tok, int n) {
-	__shared__ float s_w[FNT / 64];
-	__shared__ float s_scan[FNT / 64];
-	__shared__ int s_seg;
-	__shared__ float s_start, s_inv;
+	constexpr int NW = FNT / 64;
+	__shared__ __attribute__((aligned(16))) float s_w[NW], s_scan[2][NW], s_start[2][NW];
+	__shared__ __attribute__((aligned(16))) int s_seg[2][NW];
 	const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
 
-	// denominator: fixed-order sum of the masked block sums
-	float d = 0.0f;
+	// Everything that does not wait for another result is requested here, in one round trip: the block sums, the first
+	// FNT segment sums, the counters and, behind them, the draw.
+	float q = seg[min(tid, nseg - 1)], d = 0.0f;
 	for (int i = tid; i < nblocks; i += FNT) d += bsum[i];
+	int c0 = 0, c1 = 0, c2 = 0, c3 = 0;
+	if (mode != 2) { c0 = ctr[0]; c1 = ctr[1]; c2 = ctr[2]; c3 = ctr[3]; }
+	const float r = randf[rand_idx >= 0 ? rand_idx : c3 - rand_base - (mode == 1 ? 1 : 0)];
+
+	// denominator: fixed-order sum of the masked block sums
 	d = wave_sum(d);
 	if (lane == 0) s_w[w] = d;
-	if (tid == 0) s_seg = NONE;
 	__syncthreads();
-	if (tid == 0) {
-		float denom = 0.0f;
-		for (int i = 0; i < FNT / 64; i++) denom += s_w[i];
-		s_inv = (float)(1.0 / (double)denom);  // ops.hpp:836
-	}
-	__syncthreads();
-	const float inv = s_inv;
-	int ri = rand_idx;
-	if (ri < 0) ri = ctr[3] - rand_base - (mode == 1 ? 1 : 0);
-	const float r = randf[ri];
+	float denom = 0.0f;
+#pragma unroll
+	for (int i = 0; i < NW; i++) denom += s_w[i];
+	const float inv = (float)(1.0 / (double)denom);  // ops.hpp:836
 
 	// running sum over the segments, FNT at a time (nseg <= FNT for a 262144-entry vocabulary)
-	float base = 0.0f;
-	for (int s0 = 0; s0 < nseg && s_seg == NONE; s0 += FNT) {
+	float base = 0.0f, start = 0.0f;
+	int cs = NONE;
+	for (int s0 = 0, it = 0; s0 < nseg && cs == NONE; s0 += FNT, it ^= 1) {
 		const int s = s0 + tid;
-		const float q = (s < nseg) ? seg[s] * inv : 0.0f;
+		if (s0 > 0) q = seg[min(s, nseg - 1)];
+		q = (s < nseg) ? q * inv : 0.0f;
 		// inclusive scan inside the wave, then across the 16 waves
 		float incl = q;
 #pragma unroll
@@ -130,23 +139,35 @@ __global__ __launch_bounds__(FNT) void minp_finish_kernel(const float *probs, co
 			const float t = __shfl_up(incl, o, 64);
 			if (lane >= o) incl += t;
 		}
-		if (lane == 63) s_scan[w] = incl;
+		if (lane == 63) s_scan[it][w] = incl;
 		__syncthreads();
-		float woff = base;
-		for (int i = 0; i < w; i++) woff += s_scan[i];
-		const float end = woff + incl, start = end - q;
-		// the crossing segment is the first one whose running sum reaches r, as in the sequential scan
-		if (s < nseg && end >= r) atomicMin(&s_seg, s);
-		float total = base;
-		for (int i = 0; i < FNT / 64; i++) total += s_scan[i];
+		float woff = base, total = base;
+#pragma unroll
+		for (int i = 0; i < NW; i++) {  // all sixteen read at once, the ones behind this wave added as 0
+			const float t = s_scan[it][i];
+			woff += i < w ? t : 0.0f;
+			total += t;
+		}
+		const float end = woff + incl;
+		// the crossing segment is the first one whose running sum reaches r, as in the sequential scan: every wave leaves
+		// its first, and the first wave that has one gives the answer
+		const unsigned long long hit = __ballot(s < nseg && end >= r);
+		const int first = hit ? __ffsll(hit) - 1 : 0;
+		if (lane == first) {
+			s_seg[it][w] = hit ? s : NONE;
+			s_start[it][w] = end - q;
+		}
 		__syncthreads();
-		if (s_seg == s) s_start = start;
+#pragma unroll
+		for (int i = NW - 1; i >= 0; i--) {
+			const int si = s_seg[it][i];
+			const float st = s_start[it][i];
+			if (si != NONE) { cs = si; start = st; }
+		}
 		base = total;
-		__syncthreads();
 	}
 
 	int token = 0;  // ops.hpp:850: index stays 0 when the running sum never reaches randf
-	const int cs = s_seg;
 	if (cs != NONE && w == 0) {
 		// re-scan the crossing segment with the stored probabilities: 4 consecutive elements per lane
 		const f32x4 p = *reinterpret_cast<const f32x4 *>(probs + (size_t)cs * SEG + 4 * lane);
@@ -158,7 +179,7 @@ __global__ __launch_bounds__(FNT) void minp_finish_kernel(const float *probs, co
 			const float t = __shfl_up(incl, o, 64);
 			if (lane >= o) incl += t;
 		}
-		float c = s_start + (incl - lsum);
+		float c = start + (incl - lsum);
 		int first = NONE;
 		c += q0;
 		if (c >= r) first = 4 * lane;
@@ -177,15 +198,14 @@ __global__ __launch_bounds__(FNT) void minp_finish_kernel(const float *probs, co
 		if (out_tok) *out_tok = token;
 		if (mode == 0) {
 			ctr[4] = token;
-			const int st = ctr[3];
-			tok_log[st] = token;
-			ctr[3] = st + 1;
-			ctr[0] += 1;
-			ctr[1] += 1;
-			ctr[2] += 1;
+			tok_log[c3] = token;
+			ctr[3] = c3 + 1;
+			ctr[0] = c0 + 1;
+			ctr[1] = c1 + 1;
+			ctr[2] = c2 + 1;
 		} else if (mode == 1) {
 			ctr[4] = token;
-			tok_log[ctr[3] - 1] = token;
+			tok_log[c3 - 1] = token;
 		}
 	}
 }
@@ -196,12 +216,20 @@ size_t tg_minp_blocks(int n) { return ((size_t)n + SCHUNK - 1) / SCHUNK; }
 size_t tg_minp_padded(int n) { return tg_minp_blocks(n) * SCHUNK; }
 size_t tg_minp_segments(int n) { return tg_minp_padded(n) / SEG; }
 
-// logits[n] -> token; probs[tg_minp_padded(n)], seg[tg_minp_segments(n)], bsum and bmax[tg_minp_blocks(n)] are scratch
+// logits[n] -> token; probs[tg_minp_padded(n)], seg[tg_minp_segments(n)], bsum and bmax[tg_minp_blocks(n)] are scratch;
+// head_max != nullptr: the logits' maxima over head_n workgroups of the head's launch, which spare the launch that finds them
+// (measured, vocabulary of 262144: 10.0 us with them and 17.1 us with that launch and one round trip after another in the last)
 void tg_launch_minp(const float *logits, int n, float minp, float temp, const float *randf, int rand_idx, int rand_base, float *probs,
-                    float *seg, float *bsum, float *bmax, int *ctr, int *tok_log, int mode, int *out_tok, hipStream_t s) {
+                    float *seg, float *bsum, float *bmax, const float *head_max, int head_n, int *ctr, int *tok_log, int mode, int *out_tok,
+                    hipStream_t s) {
 	const int nb = (int)tg_minp_blocks(n), nseg = (int)tg_minp_segments(n);
-	hipLaunchKernelGGL(minp_max_kernel, dim3((unsigned)nb), dim3(SNT), 0, s, logits, n, temp, bmax);
-	hipLaunchKernelGGL(minp_prob_kernel, dim3((unsigned)nb), dim3(SNT), 0, s, logits, n, temp, minp, bmax, nb, probs, seg, bsum);
+	const dim3 grid((unsigned)nb), block(SNT);
+	if (head_max == nullptr) {
+		hipLaunchKernelGGL(minp_max_kernel, grid, block, 0, s, logits, n, temp, bmax);
+		hipLaunchKernelGGL(minp_prob_kernel, grid, block, 0, s, logits, n, temp, minp, bmax, nb, 1.0f, probs, seg, bsum);
+	} else {
+		hipLaunchKernelGGL(minp_prob_kernel, grid, block, 0, s, logits, n, temp, minp, head_max, head_n, temp, probs, seg, bsum);
+	}
 	hipLaunchKernelGGL(minp_finish_kernel, dim3(1), dim3(FNT), 0, s, probs, seg, bsum, nb, nseg, randf, rand_idx, rand_base, ctr, tok_log,
 	                   mode, out_tok, n);
 }
