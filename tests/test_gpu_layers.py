@@ -224,6 +224,36 @@ def test_chunk_workgroups(tg, folder, kind, heads, n):
     rows_close(s.forward(ids, places)[1], want[places], F32_TOL, f"{kind}, {heads} heads, {n} tokens")
 
 
+@pytest.mark.parametrize("width", [1024, 1025, 2048, 2049])
+@pytest.mark.parametrize("design", ["madevik", "tutelix"])
+def test_norms_of_every_length(tg, folder, design, width):
+    """Decode steps whose norms take a vector of 1, 2 and 3 length classes, at the classes' ends; routers of one tile (inside
+    the experts' product) and of more (a launch of their own)."""
+    if design == "madevik":
+        cfg = nm.config(width, 50, [nm.layer(nm.gla(2, 16, 16), nm.moe(5, 2, 64)), nm.layer(nm.latent(2, 16, 16, 32, 0.25), nm.moe(20, 3, 32))])
+    else:
+        cfg = nm.tutelix(width, 50, [nm.layer(nm.delta(2, 1, 16, 16, 3), nm.dense(96)), nm.layer(nm.key_values(2, 1, 16, 8, 5, 0.25), nm.dense(40))])
+    path, om = folder(("norms", design, width), cfg, seed=23)
+    ids = ids_of(cfg, 8)
+    want = om.step(om.state(), ids)
+    s = tg.Transformer.from_dir(path, "float32").open_session(8)
+    rows_close(np.concatenate([s.forward([t])[1] for t in ids]), want, F32_TOL, "token by token")
+
+
+@pytest.mark.parametrize("mixer", [nm.delta(2, 1, 32, 32, 3), nm.key_values(4, 2, 32, 16, 7, 0.2), nm.rot_latent(3, 16, 16, 32, 40, 48, 9, 0.2)])
+def test_decoding_before_a_large_feed_forward(tg, folder, mixer):
+    """A feed-forward of more than 12 MB, part of which the launches of the mixer read ahead: nothing of it may show, in the
+    vector's own result or in a session that is reset in between."""
+    cfg = nm.tutelix(644, 50, [nm.layer(mixer, nm.dense(5100)), nm.layer(mixer, nm.dense(5100))])
+    path, om = folder(("large_ff", mixer["type"]), cfg, seed=24)
+    ids = ids_of(cfg, 12)
+    want = om.step(om.state(), ids)
+    s = tg.Transformer.from_dir(path, "float32").open_session(12)
+    for n in (7, 12):  # after the reset nothing of the first seven tokens may be left
+        s.reset()
+        rows_close(np.concatenate([s.forward([t])[1] for t in ids[:n]]), want[:n], F32_TOL, f"{n} tokens, one by one")
+
+
 # ---- whole models ------------------------------------------------------------------------------------------------------------
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("name", nm.MODELS)
