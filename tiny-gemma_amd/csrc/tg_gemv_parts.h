@@ -191,14 +191,14 @@ __device__ __forceinline__ void attn_merge_prologue(float *xs, float (*wgt)[TG_A
 		m = part_ml[((size_t)b * 4 + h) * 2];
 		l = part_ml[((size_t)b * 4 + h) * 2 + 1];
 	}
-	// Loads through a descriptor of exactly nb partials: one past them reads as 0 and takes no cache access, and none is
-	// under a branch, at whose end it would be waited for (as many round trips as loads).  From a clamped index instead
-	// every workgroup fetches sixteen partials however few there are: 128 steps behind 64 tokens of the 270m shape 43.7 ms,
-	// 43.3 ms this way.
-	const uint32_t bytes = (uint32_t)nb * 4096u;
-	const __amdgpu_buffer_rsrc_t ra = make_rsrc(part_acc, bytes);
 #pragma unroll
-	for (int b = 0; b < TG_ATTN_MERGE_MAX; b++) a[b] = ldx(ra, (uint32_t)tid * 16u, min((uint32_t)b * 4096u, bytes));
+	for (int b = 0; b < TG_ATTN_MERGE_MAX; b++) {
+		// unconditional load from a clamped index, select afterwards: a load under a branch is waited for
+		// at the end of that branch, which would turn these loads into as many round trips
+		const int bb = b < nb ? b : 0;
+		const f32x4 val = *reinterpret_cast<const f32x4 *>(part_acc + ((size_t)bb * 4 + w) * 256 + 4 * lane);
+		a[b] = (b < nb) ? val : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+	}
 	after_loads();
 	if (tid < 4 * TG_ATTN_MERGE_MAX) {
 		const int h = tid / TG_ATTN_MERGE_MAX, b = tid % TG_ATTN_MERGE_MAX;
