@@ -1289,6 +1289,8 @@ __global__ __launch_bounds__(PNT) void attn_prefill_merge_kernel(float *o, int S
 // per row: heads 0-1 and 2-3).  Rows of whole query tiles are read from o, where their workgroup wrote them.
 // cr (a later portion of a sequence, else cr.k is null): the rows' keys and values go into the cache here, the last
 // cr.ring of them, row i into slot (cr.slot + i) mod cr.ring.
+// NP parts are requested at a time.
+template <int NP>
 __global__ __launch_bounds__(PNT) void attn_prefill_finish_kernel(const float *o, int S, int ldo, const int2 *tiles, const float *part_o,
                                                                  const float *part_ml, int tq, int8_t *apack, float *rowfac, int Mpad,
                                                                  TgCacheRows cr) {
@@ -1296,13 +1298,10 @@ __global__ __launch_bounds__(PNT) void attn_prefill_finish_kernel(const float *o
 	const int tid = threadIdx.x, t = tid & 127, half = tid >> 7;
 	const int row = 2 * (int)blockIdx.x + half, qrow = row < S ? row : S - 1;  // the odd last row is computed twice, written once
 	const int head = t >> 5, d0 = 8 * (t & 31);
-	if (cr.k != nullptr && row < S && row >= S - cr.ring) {  // a portion's keys and values enter the cache behind its attention
-		int r = cr.slot + row % cr.ring;
-		r = r < cr.ring ? r : r - cr.ring;
-		const int at = 4 * (t & 63);
-		const float *src = (t < 64 ? cr.k : cr.v) + (size_t)row * cr.ld + at;
-		*reinterpret_cast<f32x4 *>((t < 64 ? cr.kc : cr.vc) + (size_t)r * HD + at) = *reinterpret_cast<const f32x4 *>(src);
-	}
+	// a portion's keys and values enter the cache behind its attention: fetched here, stored at the end (nothing to copy: any row)
+	const bool enters = cr.k != nullptr && row < S && row >= S - cr.ring;
+	const int at = 4 * (t & 63);
+	const f32x4 entry = *reinterpret_cast<const f32x4 *>(enters ? (t < 64 ? cr.k : cr.v) + (size_t)row * cr.ld + at : o + (size_t)qrow * ldo + at);
 	int2 ti = int2{-1, 1};
 	if (tiles != nullptr) ti = tiles[qrow / tq];
 	float v[8];
@@ -1315,17 +1314,50 @@ __global__ __launch_bounds__(PNT) void attn_prefill_finish_kernel(const float *o
 			v[4 + e] = b[e];
 		}
 	} else {
-		const int qi = qrow % tq;
+		// all values of NP parts are requested before the first is used, the parts past the last as the last again and left
+		// out of the sums
+		const int qi = qrow % tq, np = ti.y;
+		const size_t r0 = ((size_t)ti.x * tq + qi) * NH + head, step = (size_t)tq * NH;
+		float2 ml[NP];
+		f32x4 pa[NP], pb[NP];
+		auto fetch = [&](int c0) {
+#pragma unroll
+			for (int u = 0; u < NP; u++) {
+				const size_t r = r0 + (size_t)min(c0 + u, np - 1) * step;
+				ml[u] = *reinterpret_cast<const float2 *>(part_ml + r * 2);
+				pa[u] = *reinterpret_cast<const f32x4 *>(part_o + r * HD + d0);
+				pb[u] = *reinterpret_cast<const f32x4 *>(part_o + r * HD + d0 + 4);
+			}
+		};
+		fetch(0);
 		float M = -INFINITY;
-		for (int ch = 0; ch < ti.y; ch++) M = fmaxf(M, part_ml[(((size_t)(ti.x + ch) * tq + qi) * NH + head) * 2]);
+#pragma unroll
+		for (int u = 0; u < NP; u++) M = fmaxf(M, ml[u].x);
+		for (int c0 = NP; c0 < np; c0 += NP) {
+			float m[NP];
+#pragma unroll
+			for (int u = 0; u < NP; u++) m[u] = part_ml[(r0 + (size_t)min(c0 + u, np - 1) * step) * 2];
+#pragma unroll
+			for (int u = 0; u < NP; u++) M = fmaxf(M, m[u]);
+		}
 		float L = 0.0f;
 		f32x4 a = f32x4{0.0f, 0.0f, 0.0f, 0.0f}, b = a;
-		for (int ch = 0; ch < ti.y; ch++) {
-			const size_t r = ((size_t)(ti.x + ch) * tq + qi) * NH + head;
-			const float wgt = expf(part_ml[r * 2] - M);
-			L = fmaf(part_ml[r * 2 + 1], wgt, L);
-			a += *reinterpret_cast<const f32x4 *>(part_o + r * HD + d0) * wgt;
-			b += *reinterpret_cast<const f32x4 *>(part_o + r * HD + d0 + 4) * wgt;
+		for (int c0 = 0;;) {
+#pragma unroll
+			for (int u = 0; u < NP; u++) {
+				const bool in = c0 + u < np;
+				const float wgt = expf(ml[u].x - M);
+				L = in ? fmaf(ml[u].y, wgt, L) : L;
+				const f32x4 an = a + pa[u] * wgt, bn = b + pb[u] * wgt;
+#pragma unroll
+				for (int e = 0; e < 4; e++) {
+					a[e] = in ? an[e] : a[e];
+					b[e] = in ? bn[e] : b[e];
+				}
+			}
+			c0 += NP;
+			if (c0 >= np) break;
+			fetch(c0);
 		}
 		const float Linv = 1.0f / L;
 		a = a * Linv;
@@ -1356,6 +1388,11 @@ __global__ __launch_bounds__(PNT) void attn_prefill_finish_kernel(const float *o
 	uint2 *dst = reinterpret_cast<uint2 *>(tg_plane_dst(apack, row, k0 & ~15, NH * HD)) + ((k0 >> 3) & 1);
 #pragma unroll
 	for (int p = 0; p < 3; p++) dst[p * 128] = pl[p];  // planes are 64 pieces of 16 bytes apart
+	if (enters) {
+		int r = cr.slot + row % cr.ring;
+		r = r < cr.ring ? r : r - cr.ring;
+		*reinterpret_cast<f32x4 *>((t < 64 ? cr.kc : cr.vc) + (size_t)r * HD + at) = entry;
+	}
 }
 
 }  // namespace
@@ -1616,7 +1653,15 @@ void tg_launch_attn_extend(float *o, const float *q, const float *k, const float
 void tg_launch_attn_prefill_finish(const float *o, int S, int ldo, const TgAttnPrefillPlan *plan, int n_cu, int8_t *apack, float *rowfac,
                                    hipStream_t s, const TgCacheRows &rows) {
 	const int tq = tg_attn_prefill_query_tile(S, n_cu);
-	hipLaunchKernelGGL(attn_prefill_finish_kernel, dim3((unsigned)((S + 1) / 2)), dim3(PNT), 0, s, o, S, ldo,
-	                   plan ? plan->tiles : nullptr, plan ? plan->part_o : nullptr, plan ? plan->part_ml : nullptr, tq, apack, rowfac,
-	                   (int)tg_gemm_mfma_rows(S), rows);
+	auto launch = [&](auto kernel) {
+		hipLaunchKernelGGL(kernel, dim3((unsigned)((S + 1) / 2)), dim3(PNT), 0, s, o, S, ldo, plan ? plan->tiles : nullptr,
+		                   plan ? plan->part_o : nullptr, plan ? plan->part_ml : nullptr, tq, apack, rowfac, (int)tg_gemm_mfma_rows(S), rows);
+	};
+	// Four parts at a time while no compute unit has more than four of the workgroups: their registers halve how many it
+	// could hold, which beyond that costs more (4096 rows: 17.1 us, one part at a time 13.7 us; 300 rows: 7.0 and 9.1 us; a
+	// portion of 61: 6.8 and 10.6 us)
+	if (S <= 8 * n_cu)
+		launch(attn_prefill_finish_kernel<4>);
+	else
+		launch(attn_prefill_finish_kernel<1>);
 }
