@@ -536,6 +536,23 @@ def test_sampled_generation(tg, folder):
     assert np.array_equal(greedy, s.greedy(prompt, 40)[0])
 
 
+@pytest.mark.parametrize("vocab,temp", [(1024, 0.3), (33792, 1.0), (33792, 3.0)])
+def test_sampled_steps_equal_the_sampler_on_their_logits(tg, folder, vocab, temp):
+    """A sampled step takes the maximum from the head's workgroups (16 columns each, 64 in a large vocabulary); the sampler by
+    itself finds it in the logits.  The same token, draw for draw."""
+    cfg = nm.config(40, vocab, [nm.layer(nm.gla(2, 16, 16))])
+    path, _ = folder(("sampled", vocab), cfg, seed=25)
+    model = tg.Transformer.from_dir(path, "float32")
+    a, b = model.open_session(40), model.open_session(40)
+    prompt = ids_of(cfg, 5)
+    randf = np.random.default_rng(vocab).uniform(0, 1, 21).astype(np.float32)
+    ids, _, _ = a.generate(prompt, 20, 0.01, temp, randf)
+    _, lg = b.prefill(prompt)
+    for i, t in enumerate(ids):
+        assert tg.minp_logits(lg, 0.01, temp, float(randf[i])) == t
+        _, lg = b.decode(t)
+
+
 def test_prefill_and_decode_entry_points(tg, folder):
     cfg = nm.MODELS["ragged"]
     path, om = folder("ragged", cfg, seed=20)
