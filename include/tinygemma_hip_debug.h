@@ -42,7 +42,7 @@ int tg_set_gemm_mode(int mfma);
  * partial results where that keeps more compute units busy (a badly filled last round of workgroups at a few thousand
  * tokens; the long-K products of a short prompt); the following norm adds the parts.  0 = never */
 int tg_set_gemm_split(int enable);
-/* n > 0 (default 2): prefill products of more than 448 rows with at least n / 2 output tiles per compute unit run two workgroups per compute
+/* n > 0 (default 2): products outside the few-row kernel's case with at least n / 2 output tiles per compute unit run two workgroups per compute
  * unit with both operands staged through LDS (same bits as the other kernels); 0: one workgroup per compute unit always.
  * n + 64: the same without the two half-K copies that products filling under 3/4 of the workgroup slots otherwise run as */
 int tg_set_gemm_lds(int half_tiles_per_cu);

@@ -558,7 +558,7 @@ __global__ __launch_bounds__(GNT, 2) void gemm_i8_lds_kernel(float *C, const int
 }
 
 // ---- few rows (a short prompt): the same product with the reduction split over the four waves ----------------
-// With a few hundred rows (up to 448: measured crossover between 400 and 512) the kernel above has only a handful of
+// With a few hundred rows (which products: tg_gemm_skinny_taken) the kernel above has only a handful of
 // workgroups (two row blocks x 9 column tiles for the down
 // projection of the 1B shape) and each walks all of K alone.  Here a workgroup owns 32 rows x 128 columns and its
 // four waves take the K stages round-robin (stage w, w + 4, ...), each with a private register pipeline: no LDS and
