@@ -224,6 +224,45 @@ def test_chunk_workgroups(tg, folder, kind, heads, n):
     rows_close(s.forward(ids, places)[1], want[places], F32_TOL, f"{kind}, {heads} heads, {n} tokens")
 
 
+@pytest.mark.parametrize("dim", [64, 128])
+def test_sums_over_key_channels_keep_their_order(tg, folder, dim):
+    """Channel 0 of every score is cancelled by channel 32, and channel 36 is all that is left of it: exact where the channels are
+    added in order, gone where slabs of 32 channels are summed by themselves (2^30 + 1 is 2^30 in fp32).  One chunk, no decay."""
+    def edit(t):
+        for name in "qk":
+            w = np.zeros_like(t[f"l0.mix.{name}"])
+            w[36] = t[f"l0.mix.{name}"][36]
+            w[0, 0] = 2.0 ** 15
+            w[32, 0] = -2.0 ** 15 if name == "q" else 2.0 ** 15
+            t[f"l0.mix.{name}"] = w
+        t["l0.norm1"][0], t["l0.norm1.b"][0] = 0.0, 1.0  # the normed vector's first entry is 1
+        t["l0.mix.a2"] = np.zeros_like(t["l0.mix.a2"])
+        t["l0.mix.a2.b"] = np.full_like(t["l0.mix.a2.b"], 200.0)
+
+    cfg = nm.config(40, 97, [nm.layer(nm.gla(1, dim, 16))])
+    path, om = folder(("order", dim), cfg, seed=26, edit=edit)
+    ids = ids_of(cfg, 60)
+    want = om.step(om.state(), ids)
+    s = tg.Transformer.from_dir(path, "float32").open_session(60)
+    rows_close(s.forward(ids, np.arange(60))[1], want, F32_TOL, f"key size {dim}")
+
+
+@pytest.mark.parametrize("kind,vdim", [("gla", 16), ("gla", 128), ("gla", 200), ("delta", 64), ("delta", 130)])
+def test_rows_do_not_depend_on_the_workgroups(tg, folder, kind, vdim):
+    """The chunks' outputs take 16, 32 or 64 tokens per workgroup by the number of chunks: a prompt's first rows are the same bits,
+    however long it goes on."""
+    mixer = nm.gla(4, 96, vdim) if kind == "gla" else nm.delta(4, 2, 96, vdim, 3)
+    layer = nm.layer(mixer)
+    cfg = nm.config(40, 97, [layer]) if kind == "gla" else nm.tutelix(40, 97, [layer])
+    path, _ = folder(("workgroups", kind, vdim), cfg, seed=27)
+    s = tg.Transformer.from_dir(path, "float32").open_session(4200)
+    ids, places, rows = ids_of(cfg, 4200), np.arange(0, 129, 3), []
+    for n in (130, 1100, 4200):
+        s.reset()
+        rows.append(s.forward(ids[:n], places)[1])
+    assert np.array_equal(rows[0], rows[1]) and np.array_equal(rows[0], rows[2])
+
+
 @pytest.mark.parametrize("width", [1024, 1025, 2048, 2049])
 @pytest.mark.parametrize("design", ["madevik", "tutelix"])
 def test_norms_of_every_length(tg, folder, design, width):

@@ -132,8 +132,10 @@ __global__ __launch_bounds__(256) void gla_decay_kernel(const float *low, int ld
 }
 
 // ---- A: a workgroup per chunk and head, a wave per block of 16 rows ---------------------------------------------------------
-// NS groups of four waves take the slabs of key channels in turn and add their sums at the end: a portion of 130 tokens with four
-// heads has 12 workgroups, and each was a chain of four slabs (30 us with one group at key size 128, 17.5 with four).
+// NS groups of four waves stage a slab of key channels each, and each then takes all of these slabs, in order, for its own
+// share of the sums (block columns of A, columns of the diagonal block).  No sum is split, so its bits do not depend on NS: a
+// router behind these rows picks another expert at a near-tie for one of the last place.  A portion of 130 tokens with four
+// heads has 12 workgroups, each a chain of four slabs: 30 us with one group at key size 128, 16.8 with four.
 constexpr int SL = 32, SLP = 36;  // key channels per slab, row pitch
 
 // DELTA: also k . k with the decay between them, T = beta (k . k) below the diagonal, of which it leaves -T outside the 16 x 16
@@ -148,18 +150,21 @@ template <class TR, bool DELTA, int NS>
 __global__ __launch_bounds__(256 * NS) void gla_intra_kernel(const typename TR::T *qkv, int ld, int k_off, TgGla g, int n, const float *b, float *A,
                                                              DeltaIntra x) {
 	typedef float Slab[C][SLP];
+	constexpr int OWN = 4 / NS;
 	__shared__ __align__(16) float s_all[NS][3][C][SLP];
 	const int ch = blockIdx.x, h = blockIdx.y, kh = DELTA ? h / g.group : h, sg = threadIdx.x >> 8, tid = threadIdx.x & 255, lane = tid & 63, w = tid >> 6;
-	Slab &s_q = s_all[sg][0], &s_k = s_all[sg][1], &s_b = s_all[sg][2];
-	const int lr = lane & 15, lg = lane >> 4, hd = g.heads * g.dimp, t0 = ch * C;
-	f32x4_t off[3], dia = {0, 0, 0, 0}, koff[3], kdia = {0, 0, 0, 0};
+	const int lr = lane & 15, lg = lane >> 4, hd = g.heads * g.dimp, t0 = ch * C, qi = 16 * w + lr, j0 = sg * OWN;
+	f32x4_t off[OWN], koff[OWN];
+	float dia[OWN], kdia[OWN];
 #pragma unroll
-	for (int j = 0; j < 3; j++) off[j] = koff[j] = f32x4_t{0, 0, 0, 0};
+	for (int o = 0; o < OWN; o++) {
+		off[o] = koff[o] = f32x4_t{0, 0, 0, 0};
+		dia[o] = kdia[o] = 0.0f;
+	}
 	for (int base = 0; base < g.dimp; base += SL * NS) {
 		const int d0 = base + SL * sg;
-		const bool has = d0 < g.dimp;  // (uniform over the group)
 		__syncthreads();
-		for (int e = tid; has && e < C * SL / 4; e += 256) {
+		for (int e = tid; d0 < g.dimp && e < C * SL / 4; e += 256) {
 			const int r = e / (SL / 4), c4 = (e % (SL / 4)) * 4, t = t0 + r;
 			const size_t col = (size_t)h * g.dimp + d0 + c4, kcol = (size_t)kh * g.dimp + d0 + c4;
 			f32x4_t q = tg_load4(qkv + (size_t)min(t, n - 1) * ld + kcol), k = tg_load4(qkv + (size_t)min(t, n - 1) * ld + k_off + kcol);
@@ -168,94 +173,75 @@ __global__ __launch_bounds__(256 * NS) void gla_intra_kernel(const typename TR::
 				q[i] = t < n ? q[i] * g.qscale : 0.0f;
 				k[i] = t < n ? k[i] : 0.0f;
 			}
-			tg_store4(&s_q[r][c4], q);
-			tg_store4(&s_k[r][c4], k);
-			tg_store4(&s_b[r][c4], tg_load4(b + (size_t)t * hd + col));
+			tg_store4(&s_all[sg][0][r][c4], q);
+			tg_store4(&s_all[sg][1][r][c4], k);
+			tg_store4(&s_all[sg][2][r][c4], tg_load4(b + (size_t)t * hd + col));
 		}
 		__syncthreads();
-		if (!has) continue;
-		const int qi = 16 * w + lr;
-		if (w > 0) {
-			for (int st = 0; st < SL / 4; st++) {
-				const int d = 4 * st + lg;
-				const float ref = s_b[16 * w - 1][d];
-				const float fade = pow2(s_b[qi][d] - ref), qv = s_q[qi][d] * fade, kq = DELTA ? s_k[qi][d] * fade : 0.0f;
+		for (int sl = 0; sl < NS && base + SL * sl < g.dimp; sl++) {
+			const Slab &s_q = s_all[sl][0], &s_k = s_all[sl][1], &s_b = s_all[sl][2];
+			if (j0 < w) {
+				for (int st = 0; st < SL / 4; st++) {
+					const int d = 4 * st + lg;
+					const float ref = s_b[16 * w - 1][d];
+					const float fade = pow2(s_b[qi][d] - ref), qv = s_q[qi][d] * fade, kq = DELTA ? s_k[qi][d] * fade : 0.0f;
 #pragma unroll
-				for (int j = 0; j < 3; j++)
-					if (j < w) {
-						const float kv = s_k[16 * j + lr][d] * pow2(ref - s_b[16 * j + lr][d]);
-						off[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(qv, kv, off[j], 0, 0, 0);
-						if constexpr (DELTA) koff[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kq, kv, koff[j], 0, 0, 0);
-					}
+					for (int o = 0; o < OWN; o++)
+						if (j0 + o < w) {
+							const float kv = s_k[16 * (j0 + o) + lr][d] * pow2(ref - s_b[16 * (j0 + o) + lr][d]);
+							off[o] = __builtin_amdgcn_mfma_f32_16x16x4f32(qv, kv, off[o], 0, 0, 0);
+							if constexpr (DELTA) koff[o] = __builtin_amdgcn_mfma_f32_16x16x4f32(kq, kv, koff[o], 0, 0, 0);
+						}
+				}
 			}
-		}
-		for (int d = 0; d < SL; d += 4) {
-			const f32x4_t q = tg_load4(&s_q[qi][d]), bi = tg_load4(&s_b[qi][d]);
-			f32x4_t ki = {0, 0, 0, 0};
-			if constexpr (DELTA) ki = tg_load4(&s_k[qi][d]);
+			for (int d = 0; d < SL; d += 4) {
+				const f32x4_t q = tg_load4(&s_q[qi][d]), bi = tg_load4(&s_b[qi][d]);
+				f32x4_t ki = {0, 0, 0, 0};
+				if constexpr (DELTA) ki = tg_load4(&s_k[qi][d]);
 #pragma unroll
-			for (int j = 0; j < 4; j++) {
-				const int kj = 16 * w + 4 * lg + j;
-				const f32x4_t k = tg_load4(&s_k[kj][d]), bj = tg_load4(&s_b[kj][d]);
-				if (kj <= qi) {
+				for (int o = 0; o < OWN; o++) {
+					const int kj = 16 * w + 4 * lg + j0 + o;
+					const f32x4_t k = tg_load4(&s_k[kj][d]), bj = tg_load4(&s_b[kj][d]);
+					if (kj <= qi) {
 #pragma unroll
-					for (int e = 0; e < 4; e++) {
-						const float fade = pow2(bi[e] - bj[e]);
-						dia[j] = fmaf(q[e] * k[e], fade, dia[j]);
-						if constexpr (DELTA) kdia[j] = fmaf(ki[e] * k[e], fade, kdia[j]);
+						for (int e = 0; e < 4; e++) {
+							const float fade = pow2(bi[e] - bj[e]);
+							dia[o] = fmaf(q[e] * k[e], fade, dia[o]);
+							if constexpr (DELTA) kdia[o] = fmaf(ki[e] * k[e], fade, kdia[o]);
+						}
 					}
 				}
 			}
 		}
 	}
-	if constexpr (NS > 1) {  // the groups' sums, in order
-		constexpr int NV = DELTA ? 8 : 4;
-		static_assert(sizeof(s_all) >= sizeof(f32x4_t) * (NS - 1) * NV * 256, "the sums take the slabs' place");
-		f32x4_t(*sum)[NV][256] = reinterpret_cast<f32x4_t(*)[NV][256]>(&s_all[0][0][0][0]);
-		__syncthreads();
-		auto each = [&](auto f) {
-#pragma unroll
-			for (int j = 0; j < 3; j++) f(j, off[j]);
-			f(3, dia);
-			if constexpr (DELTA) {
-#pragma unroll
-				for (int j = 0; j < 3; j++) f(4 + j, koff[j]);
-				f(7, kdia);
-			}
-		};
-		if (sg > 0) each([&](int i, f32x4_t &v) { sum[sg - 1][i][tid] = v; });
-		__syncthreads();
-		if (sg > 0) return;
-#pragma unroll
-		for (int o = 0; o < NS - 1; o++) each([&](int i, f32x4_t &v) { v += sum[o][i][tid]; });
-	}
 	float *out = A + ((size_t)ch * g.heads + h) * C * C;
 #pragma unroll
-	for (int j = 0; j < 4; j++) {
-		if (j == w) {
-			tg_store4(out + (size_t)(16 * w + lr) * C + 16 * w + 4 * lg, dia);
-		} else {
+	for (int o = 0; o < OWN; o++) {
+		const int j = j0 + o;
+		out[(size_t)qi * C + 16 * w + 4 * lg + j] = dia[o];
+		if (j != w)
 #pragma unroll
-			for (int e = 0; e < 4; e++) out[(size_t)(16 * w + 4 * lg + e) * C + 16 * j + lr] = j < w ? off[j < 3 ? j : 0][e] : 0.0f;
-		}
+			for (int e = 0; e < 4; e++) out[(size_t)(16 * w + 4 * lg + e) * C + 16 * j + lr] = j < w ? off[o][e] : 0.0f;
 	}
 	if constexpr (DELTA) {
 		__shared__ __align__(16) float s_t[4][16][20];
 		float *T = x.t + ((size_t)ch * g.heads + h) * C * C;
 		float beta_q = 0.0f, beta_r[4];
 		auto step = [&](int r) { return t0 + r < n ? tg_sigmoid(x.beta[(size_t)(t0 + r) * x.ld_beta + h]) : 0.0f; };
-		beta_q = step(16 * w + lr);
+		beta_q = step(qi);
 #pragma unroll
 		for (int e = 0; e < 4; e++) beta_r[e] = step(16 * w + 4 * lg + e);
 #pragma unroll
-		for (int j = 0; j < 4; j++) s_t[w][lr][4 * lg + j] = 4 * lg + j < lr ? beta_q * kdia[j] : 0.0f;
-#pragma unroll
-		for (int j = 0; j < 3; j++)
+		for (int o = 0; o < OWN; o++) {
+			const int j = j0 + o;
+			s_t[w][lr][4 * lg + j] = 4 * lg + j < lr ? beta_q * kdia[o] : 0.0f;
 			if (j < w) {
 #pragma unroll
-				for (int e = 0; e < 4; e++) T[(size_t)(16 * w + 4 * lg + e) * C + 16 * j + lr] = -beta_r[e] * koff[j][e];
+				for (int e = 0; e < 4; e++) T[(size_t)(16 * w + 4 * lg + e) * C + 16 * j + lr] = -beta_r[e] * koff[o][e];
 			}
-		__builtin_amdgcn_wave_barrier();  // a wave reads what it wrote itself
+		}
+		__syncthreads();
+		if (sg > 0) return;
 		float m[16];
 #pragma unroll
 		for (int r = 0; r < 16; r++) {
@@ -481,7 +467,7 @@ __global__ __launch_bounds__(512) void gla_out_kernel(OutIn in, TgGla g, int n, 
 	constexpr int XP = 36, YP = VB + (DELTA ? 18 : 16), NI = VB / 16 / NC, NY = 32 * VB / 4 / 512;
 	static_assert(NI >= 1, "a wave has a tile of columns");
 	__shared__ __align__(16) float s_x[TB][XP], s_y[32][YP];
-	__shared__ float s_sq[NC][TB];
+	__shared__ float s_sq[2][TB], s_chain[2][NTT][64];
 	const int ch = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, w = tid >> 6, wt = (w % NTT) * 16, wc = w / NTT, wv = wc * (VB / NC);
 	const int lr = lane & 15, lg = lane >> 4, hd = g.heads * g.dimp, c0 = ch * C, b0 = (int)blockIdx.z * TB, t0 = c0 + b0;
 	if (t0 >= n) return;  // a part of the last chunk behind the end
@@ -545,21 +531,29 @@ __global__ __launch_bounds__(512) void gla_out_kernel(OutIn in, TgGla g, int n, 
 		}
 		tg_lds_barrier();
 	}
-	// a lane holds token wt + lr, value columns wv + 16 j + 4 lg ...
+	// A lane holds token wt + lr, value columns wv + 16 j + 4 lg ...  Its squares are one chain over the columns of a half of the
+	// head, handed from wave to wave where several share the half: the same bits for every TB.
+	constexpr int HW = NC / 2;
+	const int half = wc / HW;
 	float ss = 0.0f;
+	for (int i = 0; i < HW; i++) {
+		if (wc % HW == i) {
+			if (i > 0) ss = s_chain[half][w % NTT][lane];
 #pragma unroll
-	for (int j = 0; j < NI; j++)
+			for (int j = 0; j < NI; j++)
 #pragma unroll
-		for (int e = 0; e < 4; e++) ss = fmaf(acc[j][e], acc[j][e], ss);
+				for (int e = 0; e < 4; e++) ss = fmaf(acc[j][e], acc[j][e], ss);
+			if (i + 1 < HW) s_chain[half][w % NTT][lane] = ss;
+		}
+		if (i + 1 < HW) __syncthreads();
+	}
 	ss += tg_red_partner<32>(ss);
 	ss += tg_red_partner<16>(ss);
-	if (lg == 0) s_sq[wc][wt + lr] = ss;
+	if (wc % HW == HW - 1 && lg == 0) s_sq[half][wt + lr] = ss;
 	__syncthreads();
 	const int t = t0 + wt + lr;
 	if (t >= n) return;
-	float sq = s_sq[0][wt + lr];
-#pragma unroll
-	for (int i = 1; i < NC; i++) sq += s_sq[i][wt + lr];
+	const float sq = s_sq[0][wt + lr] + s_sq[1][wt + lr];
 	const float inv = 1.0f / sqrtf(sq / (float)g.vdim + g.eps);
 	typename TR::T *dst = out + (size_t)t * ld_out + (size_t)h * g.vdimp;
 	const typename TR::T *gate = (const typename TR::T *)in.gate + (size_t)t * in.ldg + (size_t)h * g.vdimp;
@@ -591,7 +585,7 @@ template <class TI, class TR, int VB, bool DELTA>
 void launch_out_vb(const TgGla &g, const OutIn &in, int n, const float *b, const float *A, const float *U, void *out, int ld_out, hipStream_t s) {
 	// A workgroup's time is its chain of slabs; with few chunks and heads the tokens of a chunk go to several workgroups, each with
 	// a part of the matrix instructions and all of the chunk's states and values (3 chunks, 4 heads, 128 x 256: 24.7 us with 64
-	// tokens, 13.7 with 16; 16 chunks, 4 heads, 64 x 128: 12.8 with 64, 9.2 with 32).
+	// tokens, 13.9 with 16; 16 chunks, 4 heads, 64 x 128: 12.8 with 64, 10.1 with 32).
 	const unsigned chunks = (unsigned)((n + C - 1) / C), H = (unsigned)g.heads;
 	auto go = [&](auto *kernel, int tokens) { hipLaunchKernelGGL(kernel, dim3(chunks, H, C / tokens), dim3(512), 0, s, in, g, n, b, A, U, (typename TR::T *)out, ld_out); };
 	if constexpr (VB >= 128) {
