@@ -129,6 +129,24 @@ def test_block_entry_points_reject_bad_calls(tg, oracle, block_models, tables):
     assert e.value.code == -7
 
 
+@pytest.mark.parametrize("rows", [32, 250])
+def test_decode_attention_adds_groups_of_sixteen_keys(tg, weight_images, rows):
+    """Up to 256 keys, a decode step's sums are those of 16 keys each, added up afterwards: sampled draws follow from their last
+    bits.  Two values of 2^30 that cancel inside the second group leave no trace; in one sum with the first group's they would."""
+    model = tg.Transformer(tg.named_config("270m", 1))
+    model.read_weights_mem(weight_images("270m", 1, 31))
+    x = np.random.default_rng(6).standard_normal((1, 640)).astype(np.float32)
+    keys, values = np.zeros((2, rows, 256), np.float32)
+    values[:16] = np.random.default_rng(7).standard_normal((16, 256))
+    out = []
+    for big in (0.0, 2.0 ** 30):
+        values[16], values[24] = big, -big
+        s = model.session()
+        s.kv_prefill(0, keys, values)
+        out.append(s.block_attention(0, x))
+    assert np.array_equal(out[0], out[1])
+
+
 # ---- teacher-forced random-token streams through the full models ----
 
 @pytest.mark.parametrize("name", list(gi.STREAM_CASES))

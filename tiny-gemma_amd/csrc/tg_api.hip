@@ -1109,17 +1109,15 @@ static int head_blocks(const tg_session *s) { return s->m->net ? tg_net_head_blo
 // context, the output projection merges their partials in its prologue.  Longer contexts are bound by how long one
 // workgroup walks its keys, so they are spread over up to TG_ATTN_MAX_BLOCKS workgroups (32 keys each or more) and a
 // merge launch folds every TG_ATTN_FOLD partials into one first: the extra launch costs less than a few dozen keys per workgroup.
-// At least ATTN_CHUNK_MIN keys: a workgroup's pass takes 32 keys whether or not its chunk has them, and fewer partials
-// are fewer rows for every workgroup of the output projection to fetch.  Measured at 32 and at 16: 16 steps after 9
-// tokens of the 270m shape 6.97 and 7.09 ms, 128 steps after 64 tokens 43.80 and 44.12 ms, 128 steps after 178 tokens
-// of the 1B shape 81.10 and 81.39 ms.
-static constexpr int ATTN_CHUNK_MIN = 32;
+// Chunks of 16 keys up to 256 of them: with 32 at least, 16 steps after 9 tokens of the 270m shape take 6.88 instead of 7.12 ms
+// (128 steps after 64 tokens 43.7 and 44.0), but the regrouped sums move the logits of every such step (2e-3 behind the stepped
+// GeLU table) and with them the draws of sampled requests.
 static int attn_chunk_for(int valid, bool *needs_merge) {
 	auto up16 = [](int x) { return (x + 15) / 16 * 16; };
 	const int c = up16((valid + TG_ATTN_MERGE_MAX - 1) / TG_ATTN_MERGE_MAX);
 	*needs_merge = c > g_attn_merge_chunk;
-	if (!*needs_merge) return std::max(ATTN_CHUNK_MIN, c);
-	return std::max(ATTN_CHUNK_MIN, up16((valid + TG_ATTN_MAX_BLOCKS - 1) / TG_ATTN_MAX_BLOCKS));
+	if (!*needs_merge) return c;
+	return std::max(32, up16((valid + TG_ATTN_MAX_BLOCKS - 1) / TG_ATTN_MAX_BLOCKS));
 }
 
 // Event pool for tg_decode_profile: one event before every launch of a step plus one at the end.
@@ -1158,7 +1156,7 @@ static TgFusedMat fused_mat(const PackedMat &p) { return TgFusedMat{p.K, p.C, p.
 // TG_ATTN_MERGE_MAX * g_attn_merge_chunk keys that is what the launch path does as well; 0: too many keys for it.
 static int fused_chunk(int valid) {
 	const int c = (valid + TG_FUSED_ATTN_WGS - 1) / TG_FUSED_ATTN_WGS;
-	const int c16 = std::max(ATTN_CHUNK_MIN, (c + 15) / 16 * 16);  // as attn_chunk_for: the same partials, the same bits
+	const int c16 = (c + 15) / 16 * 16;
 	return c16 <= 256 ? c16 : 0;
 }
 
