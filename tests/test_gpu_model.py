@@ -475,6 +475,27 @@ def test_short_prompt_k_parts_equal_the_unsplit_products(tg, oracle):
     assert not np.array_equal(lg_a, lg_b)
 
 
+@pytest.mark.parametrize("n", [416, 417, 448, 449, 800, 801, 1632, 1633])
+def test_parts_of_k_in_turn_equal_the_unsplit_products(tg, weight_images, n):
+    """Parts of K on the few-row kernel: a workgroup for each while that is one round of workgroups (down projection of the 270m shape: up
+    to 416 rows in four parts, 800 in two), two in turn beyond, and the plain tiling from 1633 rows on.  Same id and logits to the
+    rounding of the additions, with a table of 2^20 entries as above."""
+    model = tg.Transformer(tg.named_config("270m", 1))
+    model.read_weights_mem(weight_images("270m", 1, 31))
+    sess = model.session(gsize=1 << 20)
+    out = []
+    try:
+        for split in (1, 0):
+            tg.check(tg.lib().tg_set_gemm_split(split))
+            sess.reset()
+            out.append(sess.prefill(gi.prompt_ids(36, n)))
+    finally:
+        tg.check(tg.lib().tg_set_gemm_split(1))
+    rel = normrel(out[0][1], out[1][1])
+    print(f"{n} rows: logits rel {rel:.2e}")
+    assert out[0][0] == out[1][0] and rel < 2e-5
+
+
 @pytest.mark.parametrize("gsize", [1024, 8192])
 def test_two_gemm_workgroups_per_unit_change_no_bit_of_a_long_prefill(tg, oracle, gsize):
     """3000 tokens through two layers of the 270m shape with tg_set_gemm_lds(1): the up|gate product (fused

@@ -253,6 +253,14 @@ def test_gemm_k_parts_rule(pkg):
         assert pkg.lib().tg_set_gemm_lds(2) == 0
 
 
+@pytest.mark.parametrize("m, i, o, parts", [(224, 6912, 1152, 4), (225, 6912, 1152, 4), (448, 6912, 1152, 4), (449, 6912, 1152, 2), (777, 6912, 1152, 2),
+                                            (777, 1024, 1152, 2), (900, 1024, 1152, 2), (417, 2048, 640, 4), (1000, 2048, 640, 2), (1000, 1024, 640, 2)])
+def test_parts_of_k_do_not_follow_the_kernel(pkg, m, i, o, parts):
+    """The number of parts decides the last bits of a prompt's logits, and with them a sampled request's draws: it stays the
+    same on both sides of the lines at which a product changes its kernel or its number of workgroups."""
+    assert pkg.lib().tg_plan_gemm_k_parts(m, i, o, 256) == parts
+
+
 def test_bench_refuses_more_than_one_gpu():
     """This path runs on one GPU: `bench.py --gpus N` with N above 1 says so and exits (no GPU needed for that)."""
     import subprocess

@@ -565,14 +565,15 @@ __global__ __launch_bounds__(GNT, 2) void gemm_i8_lds_kernel(float *C, const int
 // no barrier in the main loop, weights fetched straight from global memory in operand order (32 lanes x 16 bytes =
 // 512 contiguous bytes per fragment).  The integer partial sums are added through LDS at the end (exact, so the
 // result equals the unsplit one bit for bit) and every wave finishes a quarter of each column block.
-// gridDim.z > 1 (plain epilogue only): K is also cut into gridDim.z equal parts over workgroups; part z writes its own
-// partial result C + z * part_stride and the consumer adds them (a long K with few rows and few column tiles would
-// otherwise run on a few dozen compute units, each pulling megabytes of weights through its own L1).
+// kparts > 1 (plain epilogue only): K is also cut into kparts equal parts; part z has a partial result of its own, C + z *
+// part_stride, and the consumer adds them (a long K with few rows and few column tiles would otherwise run on a few dozen
+// compute units, each pulling megabytes of weights through its own L1).  gridDim.z workgroups share the parts of a tile: all of
+// them where that is one round of workgroups, else one takes 2 or 4 parts in turn.
 template <bool GEGLU, bool LUTLDS>
 __global__ __launch_bounds__(GNT) void gemm_i8_skinny_kernel(float *C, const int8_t *Apack, const float *rowinv, const int8_t *Wg,
                                                              const float *scales, int M, int K, int ldc, const float *lut, float gmin,
                                                              float geps, float ginv, int lut_size, float *rowmax_part, int Mpad,
-                                                             size_t part_stride) {
+                                                             size_t part_stride, int kparts) {
 	__shared__ __attribute__((aligned(16))) i32x4 red[4][3][4][64];  // [wave][plane][quarter of the 16 registers][lane]
 	__shared__ float lut_lds[(GEGLU && LUTLDS) ? LUT_LDS_MAX : 1];
 	__shared__ float pmax[4][32];
@@ -593,133 +594,142 @@ __global__ __launch_bounds__(GNT) void gemm_i8_skinny_kernel(float *C, const int
 		tile = t % ntiles;
 		z = t / ntiles;
 	}
-	const int nstage = K / KSTAGE / (int)gridDim.z, last = nstage - 1;  // stages of this workgroup's part of K
+	const int nstage = K / KSTAGE / (GEGLU ? 1 : kparts), last = nstage - 1;  // stages of a part of K
+	const int turns = GEGLU ? 1 : kparts / (int)gridDim.z;      // parts of this workgroup
 	if (GEGLU && LUTLDS) {  // visible after the barriers of the reduction
 		for (int i = tid; i < lut_size; i += GNT) lut_lds[i] = lut[i];
 	}
+	z *= turns;
 	C += (size_t)z * part_stride;
 	const i32x4 *bsrc =
 	    reinterpret_cast<const i32x4 *>(Wg + (size_t)tile * (size_t)K * TG_CT) + hb * TG_CT + c + (size_t)z * nstage * 4 * TG_CT;
 	const i32x4 *asrc =
 	    reinterpret_cast<const i32x4 *>(Apack) + (size_t)mtile * (size_t)(K >> 5) * 3 * 64 + lane + (size_t)z * nstage * 6 * 64;
+	for (int turn = 0;;) {
 
-	// ring of three stages: loads go to ordinary vector registers only, and 3 x 56 of them is what fits beside the
-	// addresses (the 192 accumulators live in the accumulation registers)
-	i32x4 areg[3][6];  // [ring slot][k step * 3 + plane]
-	i32x4 breg[3][8];  // [ring slot][k step * 4 + column block]
-	auto load = [&](int st, i32x4 *ar, i32x4 *br) {
-		st = st < last ? st : last;  // unconditional loads: surplus ones land in ring slots nobody reads again
+		// ring of three stages: loads go to ordinary vector registers only, and 3 x 56 of them is what fits beside the
+		// addresses (the 192 accumulators live in the accumulation registers)
+		i32x4 areg[3][6];  // [ring slot][k step * 3 + plane]
+		i32x4 breg[3][8];  // [ring slot][k step * 4 + column block]
+		auto load = [&](int st, i32x4 *ar, i32x4 *br) {
+			st = st < last ? st : last;  // unconditional loads: surplus ones land in ring slots nobody reads again
 #pragma unroll
-		for (int i = 0; i < 6; i++) ar[i] = asrc[(size_t)(st * 6 + i) * 64];
+			for (int i = 0; i < 6; i++) ar[i] = asrc[(size_t)(st * 6 + i) * 64];
 #pragma unroll
-		for (int ks = 0; ks < 2; ks++)
+			for (int ks = 0; ks < 2; ks++)
 #pragma unroll
-			for (int j = 0; j < 4; j++) br[ks * 4 + j] = bsrc[(size_t)(st * 4 + 2 * ks) * TG_CT + 32 * j];
-	};
-	i32x16 acc[3][4];
-#pragma unroll
-	for (int p = 0; p < 3; p++)
-#pragma unroll
-		for (int j = 0; j < 4; j++)
-#pragma unroll
-			for (int i = 0; i < 16; i++) acc[p][j][i] = 0;
-
-	// iteration i of wave w is stage w + 4 i; every wave runs the same number of iterations, a stage beyond K
-	// contributes zeros (its activation fragments are cleared: no branch around the matrix instructions)
-	auto stage = [&](int i, auto uc) {
-		constexpr int u = decltype(uc)::value;
-		load(w + 4 * (i + 2), areg[(u + 2) % 3], breg[(u + 2) % 3]);
-		const bool valid = w + 4 * i < nstage;
-#pragma unroll
-		for (int ks = 0; ks < 2; ks++)
-#pragma unroll
-			for (int p = 0; p < 3; p++) {
-				i32x4 a = areg[u][ks * 3 + p];
-				if (!valid) a = i32x4{0, 0, 0, 0};
-#pragma unroll
-				for (int j = 0; j < 4; j++) acc[p][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(breg[u][ks * 4 + j], a, acc[p][j], 0, 0, 0);
-			}
-		// Where the stage's 14 loads go among its 24 matrix instructions is fixed here.  Left to itself the scheduler
-		// sank the loads of two of every three unrolled stages to the end of the stage that needs their data and
-		// waited there for everything in flight (vmcnt(0)): one stage in flight instead of two, 1.1 us per
-		// iteration.  All loads in front of the matrix instructions: 0.76 us, but the first stage waits behind three
-		// stages of requests.  One load ahead of every two matrix instructions: the same pace and the first stage 0.7 us
-		// sooner (the four waves share one request path that takes a 16-byte-per-lane load every 16 clocks).
-		__builtin_amdgcn_sched_group_barrier(0x020, 2, 0);
-		__builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-#pragma unroll
-		for (int g = 0; g < 12; g++) {
-			__builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-			__builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-		}
-		__builtin_amdgcn_sched_barrier(0);
-	};
-	load(w, areg[0], breg[0]);
-	load(w + 4, areg[1], breg[1]);
-	const int n_it = (nstage + 3) / 4;
-	int i0 = 0;
-	for (; i0 + 3 <= n_it; i0 += 3) {
-		stage(i0, std::integral_constant<int, 0>{});
-		stage(i0 + 1, std::integral_constant<int, 1>{});
-		stage(i0 + 2, std::integral_constant<int, 2>{});
-	}
-	if (i0 < n_it) stage(i0, std::integral_constant<int, 0>{});
-	if (i0 + 1 < n_it) stage(i0 + 1, std::integral_constant<int, 1>{});
-
-	// reduction over the waves, one column block per round: every wave leaves its partial sums of the block in LDS and
-	// adds up one quarter of it (registers 4 w .. 4 w + 3 of each plane, from all four waves).  After the four
-	// rounds wave w holds, of every column block j, the four consecutive output columns 32 j + 8 w + 4 (lane / 32) ..
-	fin_t fin[4][3];
-#pragma unroll
-	for (int j = 0; j < 4; j++) {
+				for (int j = 0; j < 4; j++) br[ks * 4 + j] = bsrc[(size_t)(st * 4 + 2 * ks) * TG_CT + 32 * j];
+		};
+		i32x16 acc[3][4];
 #pragma unroll
 		for (int p = 0; p < 3; p++)
 #pragma unroll
-			for (int qq = 0; qq < 4; qq++)
-				red[w][p][qq][lane] = i32x4{acc[p][j][4 * qq], acc[p][j][4 * qq + 1], acc[p][j][4 * qq + 2], acc[p][j][4 * qq + 3]};
-		__syncthreads();
+			for (int j = 0; j < 4; j++)
 #pragma unroll
-		for (int p = 0; p < 3; p++) fin[j][p] = (red[0][p][w][lane] + red[1][p][w][lane]) + (red[2][p][w][lane] + red[3][p][w][lane]);
-		if (j < 3) __syncthreads();
-	}
+				for (int i = 0; i < 16; i++) acc[p][j][i] = 0;
 
-	const int m = mtile * 32 + c;
-	const float rs = rowinv[m];
-	auto value = [&](const fin_t *f, int e, float scale) {
-		const float v = fmaf((float)f[2][e], 65536.0f, fmaf((float)f[1][e], 256.0f, (float)f[0][e]));
-		return (v * rs) * scale;
-	};
-	float omax = 0.0f;
-	const int col = 8 * w + 4 * hb;  // of a column block
-	f32x4 sc[4];
+		// iteration i of wave w is stage w + 4 i; every wave runs the same number of iterations, a stage beyond K
+		// contributes zeros (its activation fragments are cleared: no branch around the matrix instructions)
+		auto stage = [&](int i, auto uc) {
+			constexpr int u = decltype(uc)::value;
+			load(w + 4 * (i + 2), areg[(u + 2) % 3], breg[(u + 2) % 3]);
+			const bool valid = w + 4 * i < nstage;
 #pragma unroll
-	for (int j = 0; j < 4; j++) sc[j] = *reinterpret_cast<const f32x4 *>(scales + tile * TG_CT + 32 * j + col);
-	if (m < M) {
-		float *crow = C + (size_t)m * ldc + (size_t)tile * (GEGLU ? TG_CT / 2 : TG_CT) + col;
+			for (int ks = 0; ks < 2; ks++)
 #pragma unroll
-		for (int j = 0; j < (GEGLU ? 2 : 4); j++) {  // GEGLU: blocks 0 and 1 are up, 2 and 3 their gates
-			f32x4 o;
+				for (int p = 0; p < 3; p++) {
+					i32x4 a = areg[u][ks * 3 + p];
+					if (!valid) a = i32x4{0, 0, 0, 0};
 #pragma unroll
-			for (int e = 0; e < 4; e++) {
-				if (GEGLU) {
-					const float gate = value(fin[j + 2], e, sc[j + 2][e]);
-					o[e] = (LUTLDS ? gelu_lut(gate, lut_lds, gmin, geps, ginv, lut_size) : gelu_lut(gate, lut, gmin, geps, ginv, lut_size)) *
-					       value(fin[j], e, sc[j][e]);
-					omax = fmaxf(omax, fabsf(o[e]));
-				} else {
-					o[e] = value(fin[j], e, sc[j][e]);
+					for (int j = 0; j < 4; j++) acc[p][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(breg[u][ks * 4 + j], a, acc[p][j], 0, 0, 0);
 				}
+			// Where the stage's 14 loads go among its 24 matrix instructions is fixed here.  Left to itself the scheduler
+			// sank the loads of two of every three unrolled stages to the end of the stage that needs their data and
+			// waited there for everything in flight (vmcnt(0)): one stage in flight instead of two, 1.1 us per
+			// iteration.  All loads in front of the matrix instructions: 0.76 us, but the first stage waits behind three
+			// stages of requests.  One load ahead of every two matrix instructions: the same pace and the first stage 0.7 us
+			// sooner (the four waves share one request path that takes a 16-byte-per-lane load every 16 clocks).
+			__builtin_amdgcn_sched_group_barrier(0x020, 2, 0);
+			__builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+#pragma unroll
+			for (int g = 0; g < 12; g++) {
+				__builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+				__builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
 			}
-			*reinterpret_cast<f32x4 *>(crow + 32 * j) = o;
+			__builtin_amdgcn_sched_barrier(0);
+		};
+		load(w, areg[0], breg[0]);
+		load(w + 4, areg[1], breg[1]);
+		const int n_it = (nstage + 3) / 4;
+		int i0 = 0;
+		for (; i0 + 3 <= n_it; i0 += 3) {
+			stage(i0, std::integral_constant<int, 0>{});
+			stage(i0 + 1, std::integral_constant<int, 1>{});
+			stage(i0 + 2, std::integral_constant<int, 2>{});
 		}
-	}
-	if (GEGLU && rowmax_part != nullptr) {
-		omax = fmaxf(omax, tg_red_partner<32>(omax));
-		if (hb == 0) pmax[w][c] = omax;
-		__syncthreads();
-		if (w == 0 && hb == 0 && m < M)
-			atomicMax(reinterpret_cast<unsigned *>(rowmax_part) + m,
-			          __float_as_uint(fmaxf(fmaxf(pmax[0][c], pmax[1][c]), fmaxf(pmax[2][c], pmax[3][c]))));
+		if (i0 < n_it) stage(i0, std::integral_constant<int, 0>{});
+		if (i0 + 1 < n_it) stage(i0 + 1, std::integral_constant<int, 1>{});
+
+		// reduction over the waves, one column block per round: every wave leaves its partial sums of the block in LDS and
+		// adds up one quarter of it (registers 4 w .. 4 w + 3 of each plane, from all four waves).  After the four
+		// rounds wave w holds, of every column block j, the four consecutive output columns 32 j + 8 w + 4 (lane / 32) ..
+		fin_t fin[4][3];
+#pragma unroll
+		for (int j = 0; j < 4; j++) {
+#pragma unroll
+			for (int p = 0; p < 3; p++)
+#pragma unroll
+				for (int qq = 0; qq < 4; qq++)
+					red[w][p][qq][lane] = i32x4{acc[p][j][4 * qq], acc[p][j][4 * qq + 1], acc[p][j][4 * qq + 2], acc[p][j][4 * qq + 3]};
+			__syncthreads();
+#pragma unroll
+			for (int p = 0; p < 3; p++) fin[j][p] = (red[0][p][w][lane] + red[1][p][w][lane]) + (red[2][p][w][lane] + red[3][p][w][lane]);
+			if (j < 3) __syncthreads();
+		}
+
+		const int m = mtile * 32 + c;
+		const float rs = rowinv[m];
+		auto value = [&](const fin_t *f, int e, float scale) {
+			const float v = fmaf((float)f[2][e], 65536.0f, fmaf((float)f[1][e], 256.0f, (float)f[0][e]));
+			return (v * rs) * scale;
+		};
+		float omax = 0.0f;
+		const int col = 8 * w + 4 * hb;  // of a column block
+		f32x4 sc[4];
+#pragma unroll
+		for (int j = 0; j < 4; j++) sc[j] = *reinterpret_cast<const f32x4 *>(scales + tile * TG_CT + 32 * j + col);
+		if (m < M) {
+			float *crow = C + (size_t)m * ldc + (size_t)tile * (GEGLU ? TG_CT / 2 : TG_CT) + col;
+#pragma unroll
+			for (int j = 0; j < (GEGLU ? 2 : 4); j++) {  // GEGLU: blocks 0 and 1 are up, 2 and 3 their gates
+				f32x4 o;
+#pragma unroll
+				for (int e = 0; e < 4; e++) {
+					if (GEGLU) {
+						const float gate = value(fin[j + 2], e, sc[j + 2][e]);
+						o[e] = (LUTLDS ? gelu_lut(gate, lut_lds, gmin, geps, ginv, lut_size) : gelu_lut(gate, lut, gmin, geps, ginv, lut_size)) *
+						       value(fin[j], e, sc[j][e]);
+						omax = fmaxf(omax, fabsf(o[e]));
+					} else {
+						o[e] = value(fin[j], e, sc[j][e]);
+					}
+				}
+				*reinterpret_cast<f32x4 *>(crow + 32 * j) = o;
+			}
+		}
+		if (GEGLU && rowmax_part != nullptr) {
+			omax = fmaxf(omax, tg_red_partner<32>(omax));
+			if (hb == 0) pmax[w][c] = omax;
+			__syncthreads();
+			if (w == 0 && hb == 0 && m < M)
+				atomicMax(reinterpret_cast<unsigned *>(rowmax_part) + m,
+				          __float_as_uint(fmaxf(fmaxf(pmax[0][c], pmax[1][c]), fmaxf(pmax[2][c], pmax[3][c]))));
+		}
+		if (++turn == turns) break;
+		C += part_stride;
+		bsrc += (size_t)nstage * 4 * TG_CT;
+		asrc += (size_t)nstage * 6 * 64;
+		__syncthreads();  // the sums of this part have been read by all
 	}
 }
 
@@ -744,20 +754,24 @@ void tg_launch_quant_pack(const float *A, int lda, int M, int K, int8_t *apack, 
 		hipLaunchKernelGGL((quant_rows_kernel<4, 256, 2>), dim3((unsigned)(Mpad / 4)), dim3(1024), 0, s, A, lda, M, K, apack, rowfac, rowfac + Mpad);
 }
 
-// Whether a product of M rows in ntiles column tiles and kparts parts of K runs on the few-row kernel, which splits K over
-// a workgroup's waves and has four workgroups where the plain tiling has one.  It is the better one while its grid is one
-// round of workgroups (one fits a compute unit): 256 rows of K take it 0.76 us, the plain tiling 2.2 us.  Few rows are its
-// case in any number of rounds that TG_GEMM_SKINNY_BLOCKS allows.  Measured, 777 rows of the 1B shape, K = 6912, 9 column
-// tiles: 25.4 us here, 60 us in the plain tiling.
-static bool tg_gemm_skinny_taken(int M, int ntiles, int kparts, int n_cu) {
+// Whether a product of M rows in ntiles column tiles and kparts parts of K runs on the few-row kernel, which splits K over a
+// workgroup's waves and has four workgroups where the plain tiling has one.  It is the better one while its grid is one round of
+// workgroups (one fits a compute unit): 256 rows of K take it 0.76 us, the plain tiling 2.2 us.  Few rows are its case in any
+// number of rounds that TG_GEMM_SKINNY_BLOCKS allows.  Measured, 777 rows of the 1B shape, K = 6912, 9 column tiles: 25.4 us
+// here, 60 us in the plain tiling.  Parts in turn want 16 stages each: prompts of 300 and 777 tokens of the 1B shape 2.83 and
+// 4.44 ms, with a workgroup for every part 2.89 and with halves in the plain tiling 4.59 ms; 1000 tokens of the 270m shape,
+// whose output projection has 8 stages a part, 1.95 ms with that one in the plain tiling, 2.02 ms here.
+static bool tg_gemm_skinny_taken(int M, int K, int ntiles, int kparts, int n_cu) {
 	if (M <= TG_GEMM_SKINNY_ROWS && ntiles * ((M + 127) / 128) < TG_GEMM_SKINNY_BLOCKS) return true;
-	return (long)ntiles * ((M + 31) / 32) * kparts <= n_cu;
+	const long tiles = (long)ntiles * ((M + 31) / 32);
+	return tiles * kparts <= n_cu || (tiles <= n_cu && K / KSTAGE / kparts >= 16);
 }
 
-// whether a product of M rows, K deep, ntiles column tiles runs on gemm_i8_lds_kernel (K in whole groups of four k steps)
+// whether a product of M rows, K deep, ntiles column tiles that the few-row kernel does not take runs on gemm_i8_lds_kernel (K in
+// whole groups of four k steps)
 static bool tg_gemm_lds_taken(int M, int K, int ntiles) {
 	const int tiles = ntiles * ((M + 127) / 128);
-	if (tg_gemm_skinny_taken(M, ntiles, 1, g_gemm_lds_cus)) return false;
+	if (M <= TG_GEMM_SKINNY_ROWS && tiles < TG_GEMM_SKINNY_BLOCKS) return false;
 	return g_gemm_lds > 0 && (K & 127) == 0 && 2 * tiles >= g_gemm_lds * g_gemm_lds_cus;
 }
 
@@ -774,18 +788,21 @@ void tg_launch_gemm_mfma(float *C, const int8_t *apack, const float *rowfac, con
 	const bool geglu = epi == TG_EPI_GEGLU, lutlds = geglu && lut_size <= LUT_LDS_MAX;
 	const int ldc = geglu ? ntiles * (TG_CT / 2) : ntiles * TG_CT;
 	float *rmp = geglu ? rowmax_part : nullptr;
-	if (tg_gemm_skinny_taken(M, ntiles, geglu ? 1 : kparts, g_gemm_lds_cus)) {
+	if (tg_gemm_skinny_taken(M, K, ntiles, geglu ? 1 : kparts, g_gemm_lds_cus)) {
 		g_gemm_launches[0]++;
-		const dim3 grid((unsigned)ntiles, (unsigned)((M + 31) / 32), (unsigned)(geglu ? 1 : kparts)), block(GNT);
+		const int rows32 = (M + 31) / 32, parts = geglu ? 1 : kparts;
+		int groups = parts;  // workgroups that share a tile's parts
+		while (groups > 1 && (long)ntiles * rows32 * groups > g_gemm_lds_cus) groups /= 2;
+		const dim3 grid((unsigned)ntiles, (unsigned)rows32, (unsigned)groups), block(GNT);
 		if (geglu && lutlds)
 			hipLaunchKernelGGL((gemm_i8_skinny_kernel<true, true>), grid, block, 0, s, C, apack, rowinv, Wg, scales, M, K, ldc, lut, gmin, geps,
-			                   ginv, lut_size, rmp, Mpad, (size_t)0);
+			                   ginv, lut_size, rmp, Mpad, (size_t)0, 1);
 		else if (geglu)
 			hipLaunchKernelGGL((gemm_i8_skinny_kernel<true, false>), grid, block, 0, s, C, apack, rowinv, Wg, scales, M, K, ldc, lut, gmin, geps,
-			                   ginv, lut_size, rmp, Mpad, (size_t)0);
+			                   ginv, lut_size, rmp, Mpad, (size_t)0, 1);
 		else
 			hipLaunchKernelGGL((gemm_i8_skinny_kernel<false, false>), grid, block, 0, s, C, apack, rowinv, Wg, scales, M, K, ldc, lut, gmin,
-			                   geps, ginv, lut_size, rmp, Mpad, part_stride);
+			                   geps, ginv, lut_size, rmp, Mpad, part_stride, parts);
 		return;
 	}
 	// kparts == 2 (STORE only; see tg_gemm_mfma_k_parts): two half-K copies of the grid, the second writes C + part_stride
@@ -828,22 +845,19 @@ void tg_launch_gemm_mfma(float *C, const int8_t *apack, const float *rowfac, con
 }
 
 // In how many parts of K (1, 2 or 4) a STORE product of M rows, K deep, ntiles column tiles should run; the parts
-// write separate partial results which the consumer adds.
-//   * the few-row kernel: as many parts as leave each at least 8 stages and fit in one round of workgroups (the down
-//     projection of a 178-token prompt: 54 workgroups walking 6912 rows of K become 216 walking 1728; prompts of 225, 300
-//     and 448 tokens of the 1B shape 2.42, 2.81 and 3.05 ms, with parts in two rounds 2.52, 2.93 and 3.19 ms).  Whole
-//     where one round takes more than 448 rows of a long K or fills two thirds of the chip: 777 tokens of the 1B shape
-//     4.30 ms, with the output projection in halves of the plain tiling 4.40 ms, with both products so 4.68 ms;
-//   * the tiled kernel: 2 when that fills the last round of workgroups noticeably better (whole pairs of stages per half).
+// write separate partial results which the consumer adds.  The parts are part of the result, whose last bits depend on them;
+// which kernel runs them, and with how many workgroups, is not.
+//   * few rows: as many parts as leave each at least 8 stages (the down projection of a 178-token prompt: 54 workgroups
+//     walking 6912 rows of K become 216 walking 1728);
+//   * the tiled kernels: 2 when that fills the last round of workgroups noticeably better (whole pairs of stages per half).
 int tg_gemm_mfma_k_parts(int M, int K, int ntiles, int n_cu) {
 	const int nstage = K / KSTAGE;
-	if (M <= TG_GEMM_SKINNY_ROWS && tg_gemm_skinny_taken(M, ntiles, 1, n_cu)) {
-		for (int parts = 4; parts > 1; parts /= 2)
-			if (nstage % parts == 0 && nstage / parts >= 8 && (long)ntiles * ((M + 31) / 32) * parts <= n_cu) return parts;
+	if (M <= TG_GEMM_SKINNY_ROWS && ((M + 127) / 128) * ntiles < TG_GEMM_SKINNY_BLOCKS) {
+		if (nstage % 4 == 0 && nstage / 4 >= 8) return 4;
+		if (nstage % 2 == 0 && nstage / 2 >= 8) return 2;
 		return 1;
 	}
 	if (M <= TG_GEMM_SKINNY_ROWS || nstage % 4 != 0) return 1;
-	if (tg_gemm_skinny_taken(M, ntiles, 1, n_cu) && (nstage >= 32 || 3 * ntiles * ((M + 31) / 32) > 2 * n_cu)) return 1;
 	if (tg_gemm_lds_taken(M, K, ntiles)) {
 		// Two workgroups per compute unit.  With more tiles than compute units but well under two per unit, most units
 		// would hold one workgroup and a few two, and those few set the pace: two half-K copies fill both slots of
