@@ -279,6 +279,20 @@ def test_norms_of_every_length(tg, folder, design, width):
     rows_close(np.concatenate([s.forward([t])[1] for t in ids]), want, F32_TOL, "token by token")
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("width", [1, 32, 64])
+def test_routed_experts_of_narrow_models(tg, folder, width, dtype):
+    """Vectors so short that waves of the experts' product have no weights of their own and reach its last sums while others
+    still read the router's: the choice of eight layers, token by token, is the oracle's."""
+    cfg = nm.config(width, 50, [nm.layer(nm.gla(1, 8, 8), nm.moe(13, 3, 24)) for _ in range(8)], residual_mult=0.2)
+    path, om = folder(("narrow", width), cfg, seed=28)
+    ids = ids_of(cfg, 200)
+    want = om.step(om.state(), ids)
+    s = tg.Transformer.from_dir(path, dtype).open_session(200)
+    got = np.concatenate([s.forward([t])[1] for t in ids])
+    rows_close(got, want, TOL[dtype], f"width {width}, token by token", 0.0 if dtype == "float32" else 0.15)
+
+
 @pytest.mark.parametrize("mixer", [nm.delta(2, 1, 32, 32, 3), nm.key_values(4, 2, 32, 16, 7, 0.2), nm.rot_latent(3, 16, 16, 32, 40, 48, 9, 0.2)])
 def test_decoding_before_a_large_feed_forward(tg, folder, mixer):
     """A feed-forward of more than 12 MB, part of which the launches of the mixer read ahead: nothing of it may show, in the

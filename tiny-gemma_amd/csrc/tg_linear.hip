@@ -603,11 +603,11 @@ __global__ __launch_bounds__(NT) void vec_kernel(const void *a0, const void *a1,
 				ra = TR::mma(xf, rt[u], ra);
 			}
 		}
-		if (lane < 16) s_red[w][lane] = ra[0];
+		if (lane < 16) s_misc[16 * w + lane] = ra[0];  // (not s_red: a wave without weights of its own may be in the epilogue while another reads these)
 		__syncthreads();
 		// the choice of choose_experts for at most 16 experts, expert = lane, by every wave for itself: nothing goes through LDS
 		const int e = lane & 15;
-		const float logit = (s_red[0][e] + s_red[1][e]) + (s_red[2][e] + s_red[3][e]);
+		const float logit = (s_misc[e] + s_misc[16 + e]) + (s_misc[32 + e] + s_misc[48 + e]);
 		const bool is = e < p.experts;
 		const float val = tg_sigmoid(logit), score = is ? val + p.correction[is ? e : 0] : -INFINITY;
 		int rank = 0;
