@@ -293,6 +293,30 @@ def test_routed_experts_of_narrow_models(tg, folder, width, dtype):
     rows_close(got, want, TOL[dtype], f"width {width}, token by token", 0.0 if dtype == "float32" else 0.15)
 
 
+@pytest.mark.parametrize("bad", [[0], [1, 2, 5], "all"])
+@pytest.mark.parametrize("experts,top", [(6, 2), (16, 3), (20, 3)])
+def test_experts_whose_score_is_no_number_come_last(tg, folder, experts, top, bad):
+    """Scores that are NaN count as the lowest, the lower index first among them: a choice is an expert in the experts' product (up to
+    16 experts), in a router of its own and in a prompt.  The oracle has a correction of -1e30 in their place."""
+    cfg = nm.config(72, 50, [nm.layer(nm.gla(1, 8, 8), nm.moe(experts, top, 24)), nm.layer(nm.latent(2, 16, 16, 32, 0.25), nm.moe(experts, top, 24))])
+    which = slice(None) if bad == "all" else bad
+
+    def edit(value):
+        def f(t):
+            for i in range(2):
+                t[f"l{i}.mlp.correction"][which] = value
+        return f
+
+    _, om = folder(("lowest", experts, str(bad)), cfg, seed=29, edit=edit(-1e30))
+    path, _ = folder(("nan", experts, str(bad)), cfg, seed=29, edit=edit(np.nan))
+    ids = ids_of(cfg, 40)
+    want = om.step(om.state(), ids)
+    s = tg.Transformer.from_dir(path, "float32").open_session(40)
+    rows_close(s.forward(ids, np.arange(40))[1], want, F32_TOL, "prompt")
+    s.reset()
+    rows_close(np.concatenate([s.forward([t])[1] for t in ids]), want, F32_TOL, "token by token")
+
+
 @pytest.mark.parametrize("mixer", [nm.delta(2, 1, 32, 32, 3), nm.key_values(4, 2, 32, 16, 7, 0.2), nm.rot_latent(3, 16, 16, 32, 40, 48, 9, 0.2)])
 def test_decoding_before_a_large_feed_forward(tg, folder, mixer):
     """A feed-forward of more than 12 MB, part of which the launches of the mixer read ahead: nothing of it may show, in the

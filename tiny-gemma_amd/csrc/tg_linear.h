@@ -58,6 +58,15 @@ __device__ __forceinline__ f32x4_t tg_load4(const float *p) { return *reinterpre
 __device__ __forceinline__ f32x4_t tg_load4(const __bf16 *p) { return __builtin_convertvector(*reinterpret_cast<const bf16x4_t *>(p), f32x4_t); }
 #endif
 
+#if defined(__HIPCC__)
+// What a router's experts are ordered by.  NaN counts as the lowest score: the ranks stay a permutation, and every choice is
+// an expert whose weights exist.
+__device__ __forceinline__ float tg_choice_score(float score, float correction) {
+	const float c = score + correction;
+	return c == c ? c : -INFINITY;
+}
+#endif
+
 // Weights that a launch with few workgroups touches for the launches behind it, so that these find them in the memory-side cache.
 struct TgTouch {
 	const unsigned char *ptr = nullptr;  // null: nothing

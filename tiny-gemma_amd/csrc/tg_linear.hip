@@ -46,7 +46,7 @@ using Const = std::integral_constant<int, N>;
 __device__ __forceinline__ void choose_experts(const float *logits, const float *correction, int E, int top, float *s_choice, int *s_sel,
                                                float *s_val) {
 	const int E4 = (E + 3) & ~3;  // s_choice has room for a multiple of four
-	for (int e = threadIdx.x; e < E4; e += NT) s_choice[e] = e < E ? tg_sigmoid(logits[e]) + correction[e] : -INFINITY;
+	for (int e = threadIdx.x; e < E4; e += NT) s_choice[e] = e < E ? tg_choice_score(tg_sigmoid(logits[e]), correction[e]) : -INFINITY;
 	__syncthreads();
 	for (int e = threadIdx.x; e < E; e += NT) {
 		const float c = s_choice[e];
@@ -609,14 +609,14 @@ __global__ __launch_bounds__(NT) void vec_kernel(const void *a0, const void *a1,
 		const int e = lane & 15;
 		const float logit = (s_misc[e] + s_misc[16 + e]) + (s_misc[32 + e] + s_misc[48 + e]);
 		const bool is = e < p.experts;
-		const float val = tg_sigmoid(logit), score = is ? val + p.correction[is ? e : 0] : -INFINITY;
+		const float val = tg_sigmoid(logit), score = is ? tg_choice_score(val, p.correction[is ? e : 0]) : -INFINITY;
 		int rank = 0;
 #pragma unroll
 		for (int o = 0; o < 16; o++) {
 			const float other = __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)__float_as_uint(score), o));
 			rank += (other > score || (other == score && o < e)) ? 1 : 0;
 		}
-		auto chosen = [&](int k) {  // the lane of the k-th choice (k = 0 .. 15: every rank is there once)
+		auto chosen = [&](int k) {  // the lane of the k-th choice (every rank of 0 .. 15 is there once, the padding's behind the experts')
 			return __builtin_ctzll(__ballot(rank == k));
 		};
 		zw = chosen(z);

@@ -17,7 +17,7 @@ __global__ __launch_bounds__(256) void moe_route_kernel(TgMoeRoute r) {
 		const int t = blockIdx.x * TG_MOE_BLOCK + i;
 		if (t < r.n) {
 			const float *lg = r.logits + (size_t)t * r.ld;
-			for (int e = lane; e < E; e += 64) s_choice[e] = tg_sigmoid(lg[e]) + r.correction[e];
+			for (int e = lane; e < E; e += 64) s_choice[e] = tg_choice_score(tg_sigmoid(lg[e]), r.correction[e]);
 			__builtin_amdgcn_wave_barrier();
 			asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 			for (int e = lane; e < E; e += 64) {
