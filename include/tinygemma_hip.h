@@ -159,7 +159,8 @@ int tg_forward_decode(tg_session *s, int32_t id, float *logits, int32_t *argmax)
  * want[n_want]: ascending places among them whose logits go to logits (host, [n_want][n_vocab]); argmax (may be NULL): the pick
  * behind the last one.  The result does not depend on how a sequence is cut into portions, beyond rounding.  A portion of
  * more than one token (of a Gemma model: of three tokens or more) runs through the prefill kernels, behind whatever the
- * session holds; a Gemma model's shorter portions go token by token.  Afterwards the token log (tg_session_read_ids) starts
+ * session holds, with a fourth digit plane, so that its rows are no less exact than those of single tokens; a Gemma model's
+ * shorter portions go token by token.  Afterwards the token log (tg_session_read_ids) starts
  * with this pick, as behind a prefill, unless the portion went token by token. */
 int tg_forward_tokens(tg_session *s, const int32_t *ids, int n, const int32_t *want, int n_want, float *logits, int32_t *argmax);
 /* greedy branch of gemma::generate (transformer.hpp:204-250) without tokenizer/EOS stop:

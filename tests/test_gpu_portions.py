@@ -65,6 +65,88 @@ def test_portions_equal_single_tokens(sessions, prompt, portions):
     assert a.read_ids(64).size == 8
 
 
+def layer_in_64_bits(image, cos, sin, ids, past, table):
+    """Residual stream in front of, inside and behind the one layer of a 270m-shaped image for tokens behind `past` (its keys and
+    values), and their keys and values; table: the session's GeLU table over [-4, 4)."""
+    h, f, qo, at = 640, 2048, 1024, 0
+
+    def take(count, dtype):
+        nonlocal at
+        a = np.frombuffer(image, dtype, count, at)
+        at += a.nbytes
+        return a
+
+    def matrix(rows, cols):
+        return take(rows * cols, np.int8).reshape(rows, cols), take(cols, np.float32)
+
+    wte, wte_scales = matrix(262144, h)
+    take(h, np.float32)
+    m = {name: matrix(*shape) for name, shape in (("q", (h, qo)), ("k", (h, 256)), ("v", (h, 256)), ("o", (qo, h)))}
+    qn, kn, apre, apost = (1.0 + take(n, np.float32).astype(np.float64) for n in (256, 256, h, h))
+    m.update({name: matrix(*shape) for name, shape in (("up", (h, f)), ("gate", (h, f)), ("down", (f, h)))})
+    mpre, mpost = (1.0 + take(h, np.float32).astype(np.float64) for _ in range(2))
+    w = {name: a.astype(np.float64) * s.astype(np.float64) for name, (a, s) in m.items()}
+    n, n_past = len(ids), past[0].shape[0]
+
+    def rms(x, wt):
+        return x / np.sqrt((x * x).mean(-1, keepdims=True) + 1e-6) * wt
+
+    def rope(x):
+        c, s = (t.reshape(-1, 256)[n_past:n_past + n, :128].astype(np.float64).reshape(n, *[1] * (x.ndim - 2), 128) for t in (cos, sin))
+        u, v = x[..., :128], x[..., 128:]
+        return np.concatenate([c * u - s * v, c * v + s * u], -1)
+
+    x0 = np.sqrt(np.float64(h)) * wte[ids].astype(np.float64) * wte_scales.astype(np.float64)
+    a = rms(x0, apre)
+    q = rope(rms((a @ w["q"]).reshape(n, 4, 256), qn)) / 16.0
+    k, v = rope(rms(a @ w["k"], kn)), a @ w["v"]
+    keys, values = np.concatenate([past[0], k]), np.concatenate([past[1], v])
+    scores = np.einsum("nhd,jd->nhj", q, keys)
+    scores[np.broadcast_to((np.arange(n_past + n) > n_past + np.arange(n)[:, None])[:, None], scores.shape)] = -np.inf
+    p = np.exp(scores - scores.max(-1, keepdims=True))
+    att = np.einsum("nhj,jd->nhd", p / p.sum(-1, keepdims=True), values).reshape(n, qo)
+    x1 = x0 + rms(att @ w["o"], apost)
+    a = rms(x1, mpre)
+    gate, up = a @ w["gate"], a @ w["up"]
+    i = np.trunc((gate + 4.0) * (table.size / 8.0)).astype(np.int64)
+    act = np.where(i < 0, 0.0, np.where(i < table.size, table.astype(np.float64)[np.clip(i, 0, table.size - 1)], gate))
+    return x0, x1, x1 + rms((act * up) @ w["down"], mpost), k, v
+
+
+@pytest.mark.parametrize("prompt,n", [(3, 5), (200, 61), (400, 100)])
+def test_portions_are_as_exact_as_single_tokens(tg, oracle, weight_images, prompt, n):
+    """The error of a portion's rows against 64 bits is not larger than that of the same tokens one by one, behind the same cached keys
+    and values: of the portion's own keys and values, behind the attention and behind the feed-forward.  Gates far
+    outside the table's range, so that its steps play no part; rows with few large entries, as a feed-forward's inside is."""
+    image = weight_images("270m", 1, 31).copy()
+    h, f = 640, 2048
+    gate_scales = 262144 * h + 4 * h + 4 * h + sum(a * b + 4 * b for a, b in ((h, 1024), (h, 256), (h, 256), (1024, h), (h, f))) + 4 * (512 + 2 * h) + h * f
+    image[gate_scales:gate_scales + 4 * f].view(np.float32)[:] *= 1e4
+    model = tg.Transformer(tg.named_config("270m", 1))
+    model.read_weights_mem(image)
+    table = oracle.gelu_table(-4.0, 4.0, 1 << 20)
+    cos, sin = oracle.rope_tables(10000.0, 32768)
+    a, b = [model.session(rope_sw=(cos, sin), gelu_table=table) for _ in range(2)]
+    for s in (a, b):
+        s.prefill(gi.prompt_ids(9, prompt))
+    past = [t[:prompt].astype(np.float64) for t in a.kv(0)[:2]]
+    ids = np.random.default_rng(n).integers(0, 262144, n).astype(np.int32)
+    x0, x1, x2, k, v = layer_in_64_bits(image, cos, sin, ids, past, table)
+    a.forward(ids)
+    got = {"portion": [a.tap(1, rows=n), a.tap(2, rows=n)], "steps": [[], []]}
+    for t in ids:
+        b.decode(int(t), want_logits=False)
+        for i in range(2):
+            got["steps"][i].append(b.tap(i + 1)[0])
+    err = {}
+    for name, s in (("portion", a), ("steps", b)):
+        kk, vv = (t[prompt:prompt + n] for t in s.kv(0)[:2])
+        y1, y2 = (np.array(t, np.float64) for t in got[name])
+        err[name] = [normrel(kk, k), normrel(vv, v), normrel(y1 - x0, x1 - x0), normrel(y2 - y1, x2 - x1)]
+    print(f"{prompt} + {n}: " + "; ".join(f"{name} {' '.join(f'{e:.2e}' for e in es)}" for name, es in err.items()), flush=True)
+    assert all(p <= 1.1 * q for p, q in zip(err["portion"], err["steps"]))
+
+
 def test_short_portions_go_token_by_token(sessions):
     a, b = sessions
     for s in (a, b):

@@ -168,11 +168,11 @@ TgGemv gemv_base(const PackedMat &p) {
 //               part p's partial result goes to C + p * part_stride and the consumer adds them
 void launch_gemm(float *C, const float *A, int lda, const PackedMat &p, int m, int epi, const float *lut, float gmin, float geps,
                  int lut_size, int8_t *apack, float *rowscale, bool prepacked = false, const float *amax_in = nullptr,
-                 float *amax_out = nullptr, int kparts = 1, size_t part_stride = 0) {
+                 float *amax_out = nullptr, int kparts = 1, size_t part_stride = 0, int digits = 3) {
 	if (g_gemm_mfma) {
-		if (!prepacked) tg_launch_quant_pack(A, lda, m, p.K, apack, rowscale, amax_in, g_stream);
+		if (!prepacked) tg_launch_quant_pack(A, lda, m, p.K, apack, rowscale, amax_in, g_stream, digits);
 		tg_launch_gemm_mfma(C, apack, rowscale, p.Wg, p.scales_g, m, p.K, p.ntiles_g, epi, lut, gmin, geps, lut_size, amax_out, kparts,
-		                    part_stride, g_stream);
+		                    part_stride, g_stream, digits);
 	} else {
 		(void)lda;  // the exact kernel reads dense rows (lda == K at every call site)
 		tg_launch_gemm(C, A, p.W, p.scales, m, p.K, p.ntiles, p.C, epi, lut, gmin, geps, lut_size, g_stream);
@@ -378,9 +378,9 @@ struct tg_session {
 namespace {
 constexpr int ATTN_MAX_BLOCKS = TG_ATTN_MAX_BLOCKS;
 constexpr int PREFILL_TAP_MAX_ROWS = 1024;
-// A later portion of a Gemma model goes through the kernels of a prompt from this many tokens on, below it token by token:
-// behind 300 tokens the kernels of a prompt take 1.97 ms for up to 16 tokens of the 1B shape and 1.15 ms of the 270m shape,
-// two tokens one by one 1.49 and 0.89 ms, three 2.24 and 1.30 ms.
+// A later portion of a Gemma model goes through the kernels of a prompt from this many tokens on, below it token by token.  Those
+// kernels take 2.2 ms for 3 to 16 tokens of the 1B shape behind 300 keys and 2.45 ms behind 16,000 (270m: 1.33 and 1.55 ms), three
+// tokens one by one 2.3 and 2.4 ms (1.37 and 1.5 ms), four 3.0 and 3.2 ms (1.78 and 1.98 ms).
 constexpr int TG_EXTEND_MIN = 3;
 
 bool layer_is_local(const tg_config &c, int l) { return (l % c.window_pattern) != (c.window_pattern - 1); }  // transformer.hpp:43
@@ -2202,6 +2202,7 @@ struct PrefillCtx {
 	int o_parts = 1, d_parts = 1;
 	size_t tpart = 0;
 	int at = -1;             // position of the first row of a later portion (-1: a whole prompt from an empty session)
+	int digits = 3;          // digit planes of the products' rows (a later portion: 4)
 };
 
 int prefill_setup(tg_session *s, int n, PrefillCtx *ctx, bool with_taps, int at = -1) {
@@ -2210,6 +2211,7 @@ int prefill_setup(tg_session *s, int n, PrefillCtx *ctx, bool with_taps, int at 
 	const int L = c.n_layers, h = c.hidden_size, f = c.intermediate_size, hd = c.head_dim;
 	const int qo = c.n_head * hd, nq = qo + 2 * hd;
 	const size_t S = (size_t)n;
+	const int digits = at < 0 ? 3 : 4;
 	// taps: every row of a short prompt, the last row of a long one
 	const int tap_rows = !(g_keep_taps && with_taps) ? 0 : (n <= PREFILL_TAP_MAX_ROWS ? n : 1);
 	size_t need = 0;
@@ -2221,7 +2223,7 @@ int prefill_setup(tg_session *s, int n, PrefillCtx *ctx, bool with_taps, int at 
 	const size_t o_ids = carve(sizeof(int) * S), o_x = carve(sizeof(float) * S * h), o_xn = carve(sizeof(float) * S * h),
 	             o_qkv = carve(sizeof(float) * S * nq), o_ao = carve(sizeof(float) * S * qo), o_t = carve(sizeof(float) * 4 * S * h),  // up to 4 partial results
 	             o_hb = carve(sizeof(float) * S * f),
-	             o_apack = carve(g_gemm_mfma ? tg_gemm_mfma_apack_bytes(n, std::max(std::max(f, qo), h)) : 0),
+	             o_apack = carve(g_gemm_mfma ? tg_gemm_mfma_apack_bytes(n, std::max(std::max(f, qo), h), digits) : 0),
 	             o_rs = carve(g_gemm_mfma ? sizeof(float) * 2 * tg_gemm_mfma_rows(n) : 0),
 	             o_amax = carve(g_gemm_mfma ? sizeof(float) * tg_gemm_mfma_rows(n) : 0),
 	             o_taps = carve(sizeof(float) * (size_t)(2 * L + 1) * (size_t)tap_rows * h),
@@ -2256,6 +2258,7 @@ int prefill_setup(tg_session *s, int n, PrefillCtx *ctx, bool with_taps, int at 
 	s->taps = tap_rows ? (float *)(ws + o_taps) : nullptr;
 	s->tap_rows = tap_rows;
 	ctx->at = at;
+	ctx->digits = digits;
 	if (at < 0) {
 		// Work lists of the attention launches.  A local layer whose window covers the whole prompt is a causal layer.
 		const bool local_is_causal = n <= c.n_pos_local + 1;
@@ -2291,7 +2294,7 @@ hipError_t prefill_tap(const PrefillCtx &p, int b) {
 void prefill_first_norm(const PrefillCtx &p, const float *w_pre, bool clear_amax) {
 	const int h = p.s->m->cfg.hidden_size;
 	tg_launch_norm_rows(p.pk ? nullptr : p.xn, p.x, 1, 0, w_pre, nullptr, nullptr, nullptr, p.n, h, p.pk ? p.apack : nullptr, p.rowscale, g_stream,
-	                    clear_amax ? p.amax : nullptr);
+	                    clear_amax ? p.amax : nullptr, p.digits);
 }
 
 // modules::attention, prefill branch (modules.hpp:98-133), from the pre-normalised rows to the output projection's
@@ -2304,7 +2307,7 @@ void prefill_attention_launches(const PrefillCtx &p, int l) {
 	const LayerDev &Ld = m->L[(size_t)l];
 	const int mp = s->max_pos[(size_t)l];
 	// Q|K|V (modules.hpp:106-108)
-	launch_gemm(p.qkv, p.xn, h, Ld.qkv, n, TG_EPI_STORE, nullptr, 0, 0, 0, p.apack, p.rowscale, p.pk);
+	launch_gemm(p.qkv, p.xn, h, Ld.qkv, n, TG_EPI_STORE, nullptr, 0, 0, 0, p.apack, p.rowscale, p.pk, nullptr, nullptr, 1, 0, p.digits);
 	if (p.at >= 0) {
 		// A later portion sees what its tokens would see one by one: the keys of the cache, in a local layer at most
 		// n_pos_local with the token's own, and enters the cache in the slots it would take then (KVCache::update_single,
@@ -2330,8 +2333,8 @@ void prefill_attention_launches(const PrefillCtx &p, int l) {
 		rows.ld = nq;
 		rows.slot = slot;
 		rows.ring = mp;
-		tg_launch_attn_prefill_finish(p.ao, n, qo, plan, g_n_cu, p.apack, p.rowscale, g_stream, rows);
-		launch_gemm(p.t, p.ao, qo, Ld.o, n, TG_EPI_STORE, nullptr, 0, 0, 0, p.apack, p.rowscale, p.pk, nullptr, nullptr, p.o_parts, p.tpart);
+		tg_launch_attn_extend_finish(p.ao, n, qo, plan, g_n_cu, p.apack, p.rowscale, rows, g_stream);
+		launch_gemm(p.t, p.ao, qo, Ld.o, n, TG_EPI_STORE, nullptr, 0, 0, 0, p.apack, p.rowscale, p.pk, nullptr, nullptr, p.o_parts, p.tpart, p.digits);
 		return;
 	}
 	// q/k norm + RoPE from position 0, KV write (modules.hpp:115-121)
@@ -2355,8 +2358,8 @@ void prefill_mlp_launches(const PrefillCtx &p, int l) {
 	const LayerDev &Ld = s->m->L[(size_t)l];
 	const int h = c.hidden_size, f = c.intermediate_size, n = p.n;
 	// up|gate + gelu*up (modules.hpp:190-195), down (modules.hpp:196-197)
-	launch_gemm(p.hb, p.xn, h, Ld.ug, n, TG_EPI_GEGLU, s->lut, s->gmin, s->geps, s->lut_size, p.apack, p.rowscale, p.pk, nullptr, p.amax);
-	launch_gemm(p.t, p.hb, f, Ld.d, n, TG_EPI_STORE, nullptr, 0, 0, 0, p.apack, p.rowscale, false, p.amax, nullptr, p.d_parts, p.tpart);
+	launch_gemm(p.hb, p.xn, h, Ld.ug, n, TG_EPI_GEGLU, s->lut, s->gmin, s->geps, s->lut_size, p.apack, p.rowscale, p.pk, nullptr, p.amax, 1, 0, p.digits);
+	launch_gemm(p.t, p.hb, f, Ld.d, n, TG_EPI_STORE, nullptr, 0, 0, 0, p.apack, p.rowscale, false, p.amax, nullptr, p.d_parts, p.tpart, p.digits);
 }
 
 // x = rmsnorm(t, w_post) + x, then xn (or its digit planes) = rmsnorm(x, next_pre)  (modules.hpp:130-132, 188, 199-201)
@@ -2364,7 +2367,7 @@ void prefill_block_end(const PrefillCtx &p, int nparts, const float *w_post, con
 	const int h = p.s->m->cfg.hidden_size;
 	const bool planes = p.pk && !want_fp32;
 	tg_launch_norm_rows(planes ? nullptr : p.xn, p.t, nparts, p.tpart, next_pre, w_post, p.x, p.x, p.n, h, planes ? p.apack : nullptr, p.rowscale,
-	                    g_stream, clear_amax ? p.amax : nullptr);
+	                    g_stream, clear_amax ? p.amax : nullptr, p.digits);
 }
 
 // Embedding and all layers of the context's rows: p.xn = rmsnorm(x, RMSw), the rows that the LM head takes
@@ -2435,7 +2438,8 @@ static int net_extend(tg_session *s, const int32_t *ids, int n, const int32_t *w
 	return TG_OK;
 }
 
-// A portion of several tokens of a Gemma model behind whatever the session holds, through the kernels of a prompt.  The token
+// A portion of several tokens of a Gemma model behind whatever the session holds, through the kernels of a prompt, with one digit
+// plane more than a prompt's rows have (a portion stands in for decode steps and is to be as exact as those).  The token
 // log starts anew with the portion's pick, as behind a prefill.
 static int gemma_extend(tg_session *s, const int32_t *ids, int n, const int32_t *want, int n_want, float *logits, int32_t *argmax) {
 	const size_t V = (size_t)s->m->cfg.n_vocab;

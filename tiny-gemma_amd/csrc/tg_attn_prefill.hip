@@ -294,7 +294,7 @@ __device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) { return __
 __device__ __forceinline__ f32x4 mfma16(f16x8 a, f16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
 // acc += a . b with the significant cross terms, smallest first
 template <typename F>
-__device__ __forceinline__ f32x4 mfma_terms(const PlanesT<F> &a, const PlanesT<F> &b, f32x4 acc) {
+__device__ __forceinline__ f32x4 mfma_cross_terms(const PlanesT<F> &a, const PlanesT<F> &b, f32x4 acc) {
 	if constexpr (F::NP == 3) {
 		acc = mfma16(a.p[2], b.p[0], acc);
 		acc = mfma16(a.p[0], b.p[2], acc);
@@ -302,8 +302,11 @@ __device__ __forceinline__ f32x4 mfma_terms(const PlanesT<F> &a, const PlanesT<F
 	}
 	acc = mfma16(a.p[1], b.p[0], acc);
 	acc = mfma16(a.p[0], b.p[1], acc);
-	acc = mfma16(a.p[0], b.p[0], acc);
 	return acc;
+}
+template <typename F>
+__device__ __forceinline__ f32x4 mfma_terms(const PlanesT<F> &a, const PlanesT<F> &b, f32x4 acc) {
+	return mfma16(a.p[0], b.p[0], mfma_cross_terms<F>(a, b, acc));
 }
 // largest magnitude among 8 values about to be converted (formats with a limited range only)
 template <typename F>
@@ -339,6 +342,9 @@ constexpr int NT32 = HD / 32;  // k steps of a score product
 // Key j of the launch is then cache row (past.slot0 + j) mod past.ring for j < past.n and row j - past.n of k / v (the
 // portion's own keys, not yet in the cache: a local layer's ring still holds the keys they will overwrite, which the first
 // queries need) from there on; the key ranges of the work list count from the first cached key.
+// Such a portion stands in for decode steps and may not be less exact: its sums are rounded less often.  The cross terms, 2^-8 of
+// the leading products, have accumulators of their own, and a tile's values are summed before they join the others' (error
+// behind the attention against 64 bits, 61 tokens behind 200: 2.0e-7, with every term in one accumulator 2.8e-7, steps 2.4e-7).
 template <int QG, typename F, bool PAST>
 __global__ __launch_bounds__(256 * QG) void attn_prefill_split_kernel(float *o, const float *q, const float *k, const float *v, int S, int ldq,
                                                                 int ldkv, int ldo, int is_sw, int window, const int4 *items,
@@ -459,9 +465,9 @@ __global__ __launch_bounds__(256 * QG) void attn_prefill_split_kernel(float *o, 
 		if (kb + tile * TK > np + q0w + 15) continue;
 
 		// ---- scores of the tile's two groups of 16 keys; even and odd k steps in separate accumulators ----
-		f32x4 sa[2][2];
+		f32x4 sa[2][2], cross[2];
 #pragma unroll
-		for (int hf = 0; hf < 2; hf++) sa[hf][0] = sa[hf][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+		for (int hf = 0; hf < 2; hf++) sa[hf][0] = sa[hf][1] = cross[hf] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
 		for (int t = 0; t < NT32; t++) {
 #pragma unroll
@@ -469,10 +475,19 @@ __global__ __launch_bounds__(256 * QG) void attn_prefill_split_kernel(float *o, 
 				Planes kf;
 #pragma unroll
 				for (int pn = 0; pn < F::NP; pn++) kf.p[pn] = Kb[pn][t][16 * hf + c][g];
-				sa[hf][t & 1] = mfma_terms<F>(kf, qp[t], sa[hf][t & 1]);
+				if constexpr (PAST) {
+					sa[hf][t & 1] = mfma16(kf.p[0], qp[t].p[0], sa[hf][t & 1]);
+					cross[hf] = mfma_cross_terms<F>(kf, qp[t], cross[hf]);
+				} else {
+					sa[hf][t & 1] = mfma_terms<F>(kf, qp[t], sa[hf][t & 1]);
+				}
 			}
 		}
 		f32x4 s0 = (sa[0][0] + sa[0][1]) * F::SSCALE, s1 = (sa[1][0] + sa[1][1]) * F::SSCALE;
+		if constexpr (PAST) {
+			s0 += cross[0] * F::SSCALE;
+			s1 += cross[1] * F::SSCALE;
+		}
 		// ---- mask + online softmax for query c ----
 		const int j0 = kb + tile * TK + 4 * g;
 		float tmax = -INFINITY;
@@ -515,7 +530,8 @@ __global__ __launch_bounds__(256 * QG) void attn_prefill_split_kernel(float *o, 
 			Planes vf;
 #pragma unroll
 			for (int pn = 0; pn < F::NP; pn++) vf.p[pn] = Vb[pn][g][16 * dt + c];
-			oacc[dt] = mfma_terms<F>(pp, vf, oacc[dt]);
+			if constexpr (PAST) oacc[dt] += mfma_terms<F>(pp, vf, f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+			else oacc[dt] = mfma_terms<F>(pp, vf, oacc[dt]);
 		}
 	}
 
@@ -1289,8 +1305,8 @@ __global__ __launch_bounds__(PNT) void attn_prefill_merge_kernel(float *o, int S
 // per row: heads 0-1 and 2-3).  Rows of whole query tiles are read from o, where their workgroup wrote them.
 // cr (a later portion of a sequence, else cr.k is null): the rows' keys and values go into the cache here, the last
 // cr.ring of them, row i into slot (cr.slot + i) mod cr.ring.
-// NP parts are requested at a time.
-template <int NP>
+// NP parts are requested at a time; P digit planes.
+template <int NP, int P>
 __global__ __launch_bounds__(PNT) void attn_prefill_finish_kernel(const float *o, int S, int ldo, const int2 *tiles, const float *part_o,
                                                                  const float *part_ml, int tq, int8_t *apack, float *rowfac, int Mpad,
                                                                  TgCacheRows cr) {
@@ -1377,17 +1393,17 @@ __global__ __launch_bounds__(PNT) void attn_prefill_finish_kernel(const float *o
 	amax = fmaxf(wmax[2 * half], wmax[2 * half + 1]);
 	if (row >= S) return;
 	float mul, inv;
-	tg_row_factors(amax, mul, inv);
+	tg_row_factors<P>(amax, mul, inv);
 	if (t == 0) {
 		rowfac[row] = mul;
 		rowfac[Mpad + row] = inv;
 	}
-	uint2 pl[3];
-	tg_quant8(v, mul, pl);
+	uint2 pl[P];
+	tg_quant8<P>(v, mul, pl);
 	const int k0 = head * HD + d0;
-	uint2 *dst = reinterpret_cast<uint2 *>(tg_plane_dst(apack, row, k0 & ~15, NH * HD)) + ((k0 >> 3) & 1);
+	uint2 *dst = reinterpret_cast<uint2 *>(tg_plane_dst<P>(apack, row, k0 & ~15, NH * HD)) + ((k0 >> 3) & 1);
 #pragma unroll
-	for (int p = 0; p < 3; p++) dst[p * 128] = pl[p];  // planes are 64 pieces of 16 bytes apart
+	for (int p = 0; p < P; p++) dst[p * 128] = pl[p];  // planes are 64 pieces of 16 bytes apart
 	if (enters) {
 		int r = cr.slot + row % cr.ring;
 		r = r < cr.ring ? r : r - cr.ring;
@@ -1628,7 +1644,7 @@ void tg_launch_attn_prefill(float *o, const float *q, const float *k, const floa
 
 // A later portion of a sequence: S queries behind past.n cached keys.  The planes are the three bf16 ones, whose exponent range
 // is fp32's: a portion has no operand that it could not take, as the decode steps that would otherwise take it have none.
-// Split query tiles are merged by tg_launch_attn_prefill_finish.
+// Split query tiles are merged by tg_launch_attn_extend_finish.
 void tg_launch_attn_extend(float *o, const float *q, const float *k, const float *v, int S, int ldq, int ldkv, int ldo, int is_sw, int window,
                            const TgAttnPrefillPlan *plan, const TgAttnPast &past, int n_cu, hipStream_t s) {
 	static bool lds_set = false;
@@ -1650,8 +1666,10 @@ void tg_launch_attn_extend(float *o, const float *q, const float *k, const float
 		                   po, pml, nullptr, past);
 }
 
-void tg_launch_attn_prefill_finish(const float *o, int S, int ldo, const TgAttnPrefillPlan *plan, int n_cu, int8_t *apack, float *rowfac,
-                                   hipStream_t s, const TgCacheRows &rows) {
+namespace {
+template <int P>
+void launch_finish(const float *o, int S, int ldo, const TgAttnPrefillPlan *plan, int n_cu, int8_t *apack, float *rowfac, const TgCacheRows &rows,
+                   hipStream_t s) {
 	const int tq = tg_attn_prefill_query_tile(S, n_cu);
 	auto launch = [&](auto kernel) {
 		hipLaunchKernelGGL(kernel, dim3((unsigned)((S + 1) / 2)), dim3(PNT), 0, s, o, S, ldo, plan ? plan->tiles : nullptr,
@@ -1661,7 +1679,18 @@ void tg_launch_attn_prefill_finish(const float *o, int S, int ldo, const TgAttnP
 	// could hold, which beyond that costs more (4096 rows: 17.1 us, one part at a time 13.7 us; 300 rows: 7.0 and 9.1 us; a
 	// portion of 61: 6.8 and 10.6 us)
 	if (S <= 8 * n_cu)
-		launch(attn_prefill_finish_kernel<4>);
+		launch(attn_prefill_finish_kernel<4, P>);
 	else
-		launch(attn_prefill_finish_kernel<1>);
+		launch(attn_prefill_finish_kernel<1, P>);
+}
+}  // namespace
+
+void tg_launch_attn_prefill_finish(const float *o, int S, int ldo, const TgAttnPrefillPlan *plan, int n_cu, int8_t *apack, float *rowfac,
+                                   hipStream_t s) {
+	launch_finish<3>(o, S, ldo, plan, n_cu, apack, rowfac, TgCacheRows(), s);
+}
+
+void tg_launch_attn_extend_finish(const float *o, int S, int ldo, const TgAttnPrefillPlan *plan, int n_cu, int8_t *apack, float *rowfac,
+                                  const TgCacheRows &rows, hipStream_t s) {
+	launch_finish<4>(o, S, ldo, plan, n_cu, apack, rowfac, rows, s);
 }

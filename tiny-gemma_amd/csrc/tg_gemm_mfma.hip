@@ -125,14 +125,17 @@ __global__ __launch_bounds__(ROWS * LANES) void quant_rows_kernel(const float *A
 // The same from row maxima that the producer of A left.  Workgroup = 32 rows x 128 k; thread = one lane's 16 bytes of
 // one (k step, half): row r = tid % 32, k = 128 blockIdx.y + 16 (tid / 32) .. + 15.  The workgroups of the first 128 k
 // also store the factors for the product's epilogue (mul_out, inv_out).
+template <int P>
 __global__ __launch_bounds__(GNT) void quant_pack_kernel(const float *A, int lda, int M, int K, const float *amax, int8_t *Apack,
                                                          float *mul_out, float *inv_out) {
 	const int tid = threadIdx.x, r = tid & 31, kq = tid >> 5;
 	const int mtile = blockIdx.x, m = mtile * 32 + r;
 	const int k0 = blockIdx.y * 128 + 16 * kq;
-	i32x4 pl[3] = {i32x4{0, 0, 0, 0}, i32x4{0, 0, 0, 0}, i32x4{0, 0, 0, 0}};
+	i32x4 pl[P];
+#pragma unroll
+	for (int p = 0; p < P; p++) pl[p] = i32x4{0, 0, 0, 0};
 	float factor, rcp;
-	tg_row_factors(m < M ? amax[m] : 0.0f, factor, rcp);  // rows of the padding were never written
+	tg_row_factors<P>(m < M ? amax[m] : 0.0f, factor, rcp);  // rows of the padding were never written
 	if (blockIdx.y == 0 && kq == 0) {
 		mul_out[m] = factor;
 		inv_out[m] = rcp;
@@ -146,11 +149,11 @@ __global__ __launch_bounds__(GNT) void quant_pack_kernel(const float *A, int lda
 #pragma unroll
 			for (int i = 0; i < 4; i++) v[4 * q + i] = a[i];
 		}
-		tg_quant16(v, factor, pl);
+		tg_quant16<P>(v, factor, pl);
 	}
-	i32x4 *dst = tg_plane_dst(Apack, m, k0, K);
+	i32x4 *dst = tg_plane_dst<P>(Apack, m, k0, K);
 #pragma unroll
-	for (int p = 0; p < 3; p++) dst[p * 64] = pl[p];
+	for (int p = 0; p < P; p++) dst[p * 64] = pl[p];
 }
 
 // GEGLU: fused up|gate tile with gelu(gate) * up; LUTLDS: the GeLU table is small enough to be staged in LDS
@@ -569,12 +572,14 @@ __global__ __launch_bounds__(GNT, 2) void gemm_i8_lds_kernel(float *C, const int
 // part_stride, and the consumer adds them (a long K with few rows and few column tiles would otherwise run on a few dozen
 // compute units, each pulling megabytes of weights through its own L1).  gridDim.z workgroups share the parts of a tile: all of
 // them where that is one round of workgroups, else one takes 2 or 4 parts in turn.
-template <bool GEGLU, bool LUTLDS>
+// P = 4 (a later portion's rows): every product of such rows runs here, whatever their number (a portion of 61 tokens of the 1B
+// shape 2.55 ms, with three planes 2.40 ms; 4096 tokens 31.8 ms, on the tiled kernels with three planes 17.0 ms, one by one 2.5 s).
+template <bool GEGLU, bool LUTLDS, int P>
 __global__ __launch_bounds__(GNT) void gemm_i8_skinny_kernel(float *C, const int8_t *Apack, const float *rowinv, const int8_t *Wg,
                                                              const float *scales, int M, int K, int ldc, const float *lut, float gmin,
                                                              float geps, float ginv, int lut_size, float *rowmax_part, int Mpad,
                                                              size_t part_stride, int kparts) {
-	__shared__ __attribute__((aligned(16))) i32x4 red[4][3][4][64];  // [wave][plane][quarter of the 16 registers][lane]
+	__shared__ __attribute__((aligned(16))) i32x4 red[4][P][4][64];  // [wave][plane][quarter of the 16 registers][lane]
 	__shared__ float lut_lds[(GEGLU && LUTLDS) ? LUT_LDS_MAX : 1];
 	__shared__ float pmax[4][32];
 	typedef i32x4 fin_t;
@@ -595,7 +600,7 @@ __global__ __launch_bounds__(GNT) void gemm_i8_skinny_kernel(float *C, const int
 		z = t / ntiles;
 	}
 	const int nstage = K / KSTAGE / (GEGLU ? 1 : kparts), last = nstage - 1;  // stages of a part of K
-	const int turns = GEGLU ? 1 : kparts / (int)gridDim.z;      // parts of this workgroup
+	const int turns = GEGLU || P == 4 ? 1 : kparts / (int)gridDim.z;  // parts of this workgroup (four planes leave no registers for the loop)
 	if (GEGLU && LUTLDS) {  // visible after the barriers of the reduction
 		for (int i = tid; i < lut_size; i += GNT) lut_lds[i] = lut[i];
 	}
@@ -604,25 +609,25 @@ __global__ __launch_bounds__(GNT) void gemm_i8_skinny_kernel(float *C, const int
 	const i32x4 *bsrc =
 	    reinterpret_cast<const i32x4 *>(Wg + (size_t)tile * (size_t)K * TG_CT) + hb * TG_CT + c + (size_t)z * nstage * 4 * TG_CT;
 	const i32x4 *asrc =
-	    reinterpret_cast<const i32x4 *>(Apack) + (size_t)mtile * (size_t)(K >> 5) * 3 * 64 + lane + (size_t)z * nstage * 6 * 64;
+	    reinterpret_cast<const i32x4 *>(Apack) + (size_t)mtile * (size_t)(K >> 5) * P * 64 + lane + (size_t)z * nstage * 2 * P * 64;
 	for (int turn = 0;;) {
 
 		// ring of three stages: loads go to ordinary vector registers only, and 3 x 56 of them is what fits beside the
 		// addresses (the 192 accumulators live in the accumulation registers)
-		i32x4 areg[3][6];  // [ring slot][k step * 3 + plane]
+		i32x4 areg[3][2 * P];  // [ring slot][k step * P + plane]
 		i32x4 breg[3][8];  // [ring slot][k step * 4 + column block]
 		auto load = [&](int st, i32x4 *ar, i32x4 *br) {
 			st = st < last ? st : last;  // unconditional loads: surplus ones land in ring slots nobody reads again
 #pragma unroll
-			for (int i = 0; i < 6; i++) ar[i] = asrc[(size_t)(st * 6 + i) * 64];
+			for (int i = 0; i < 2 * P; i++) ar[i] = asrc[(size_t)(st * 2 * P + i) * 64];
 #pragma unroll
 			for (int ks = 0; ks < 2; ks++)
 #pragma unroll
 				for (int j = 0; j < 4; j++) br[ks * 4 + j] = bsrc[(size_t)(st * 4 + 2 * ks) * TG_CT + 32 * j];
 		};
-		i32x16 acc[3][4];
+		i32x16 acc[P][4];
 #pragma unroll
-		for (int p = 0; p < 3; p++)
+		for (int p = 0; p < P; p++)
 #pragma unroll
 			for (int j = 0; j < 4; j++)
 #pragma unroll
@@ -637,8 +642,8 @@ __global__ __launch_bounds__(GNT) void gemm_i8_skinny_kernel(float *C, const int
 #pragma unroll
 			for (int ks = 0; ks < 2; ks++)
 #pragma unroll
-				for (int p = 0; p < 3; p++) {
-					i32x4 a = areg[u][ks * 3 + p];
+				for (int p = 0; p < P; p++) {
+					i32x4 a = areg[u][ks * P + p];
 					if (!valid) a = i32x4{0, 0, 0, 0};
 #pragma unroll
 					for (int j = 0; j < 4; j++) acc[p][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(breg[u][ks * 4 + j], a, acc[p][j], 0, 0, 0);
@@ -652,7 +657,7 @@ __global__ __launch_bounds__(GNT) void gemm_i8_skinny_kernel(float *C, const int
 			__builtin_amdgcn_sched_group_barrier(0x020, 2, 0);
 			__builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
 #pragma unroll
-			for (int g = 0; g < 12; g++) {
+			for (int g = 0; g < 6 + 2 * P; g++) {
 				__builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
 				__builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
 			}
@@ -673,24 +678,25 @@ __global__ __launch_bounds__(GNT) void gemm_i8_skinny_kernel(float *C, const int
 		// reduction over the waves, one column block per round: every wave leaves its partial sums of the block in LDS and
 		// adds up one quarter of it (registers 4 w .. 4 w + 3 of each plane, from all four waves).  After the four
 		// rounds wave w holds, of every column block j, the four consecutive output columns 32 j + 8 w + 4 (lane / 32) ..
-		fin_t fin[4][3];
+		fin_t fin[4][P];
 #pragma unroll
 		for (int j = 0; j < 4; j++) {
 #pragma unroll
-			for (int p = 0; p < 3; p++)
+			for (int p = 0; p < P; p++)
 #pragma unroll
 				for (int qq = 0; qq < 4; qq++)
 					red[w][p][qq][lane] = i32x4{acc[p][j][4 * qq], acc[p][j][4 * qq + 1], acc[p][j][4 * qq + 2], acc[p][j][4 * qq + 3]};
 			__syncthreads();
 #pragma unroll
-			for (int p = 0; p < 3; p++) fin[j][p] = (red[0][p][w][lane] + red[1][p][w][lane]) + (red[2][p][w][lane] + red[3][p][w][lane]);
+			for (int p = 0; p < P; p++) fin[j][p] = (red[0][p][w][lane] + red[1][p][w][lane]) + (red[2][p][w][lane] + red[3][p][w][lane]);
 			if (j < 3) __syncthreads();
 		}
 
 		const int m = mtile * 32 + c;
 		const float rs = rowinv[m];
 		auto value = [&](const fin_t *f, int e, float scale) {
-			const float v = fmaf((float)f[2][e], 65536.0f, fmaf((float)f[1][e], 256.0f, (float)f[0][e]));
+			float v = fmaf((float)f[2][e], 65536.0f, fmaf((float)f[1][e], 256.0f, (float)f[0][e]));
+			if constexpr (P == 4) v = fmaf((float)f[P - 1][e], 16777216.0f, v);
 			return (v * rs) * scale;
 		};
 		float omax = 0.0f;
@@ -728,7 +734,7 @@ __global__ __launch_bounds__(GNT) void gemm_i8_skinny_kernel(float *C, const int
 		if (++turn == turns) break;
 		C += part_stride;
 		bsrc += (size_t)nstage * 4 * TG_CT;
-		asrc += (size_t)nstage * 6 * 64;
+		asrc += (size_t)nstage * 2 * P * 64;
 		__syncthreads();  // the sums of this part have been read by all
 	}
 }
@@ -736,16 +742,19 @@ __global__ __launch_bounds__(GNT) void gemm_i8_skinny_kernel(float *C, const int
 }  // namespace
 
 // scratch sizes for M rows of K: digit planes (bytes) and row factors (floats, two arrays of this length)
-size_t tg_gemm_mfma_apack_bytes(int M, int K) { return (size_t)((M + 127) / 128) * 128 * (size_t)K * 3; }
+size_t tg_gemm_mfma_apack_bytes(int M, int K, int digits) { return (size_t)((M + 127) / 128) * 128 * (size_t)K * (size_t)digits; }
 size_t tg_gemm_mfma_rows(int M) { return (size_t)((M + 127) / 128) * 128; }
 
 // A [M][lda] fp32 -> digit planes + row factors; rowfac holds 2 * tg_gemm_mfma_rows(M) floats (multipliers, then inverses).
 // rowmax != nullptr: [tg_gemm_mfma_rows(M)] row maxima left by the producer of A (no pass over A for them).
-void tg_launch_quant_pack(const float *A, int lda, int M, int K, int8_t *apack, float *rowfac, const float *rowmax, hipStream_t s) {
+void tg_launch_quant_pack(const float *A, int lda, int M, int K, int8_t *apack, float *rowfac, const float *rowmax, hipStream_t s, int digits) {
 	const int Mpad = (int)tg_gemm_mfma_rows(M);
 	if (rowmax != nullptr) {
-		hipLaunchKernelGGL(quant_pack_kernel, dim3((unsigned)(Mpad / 32), (unsigned)(K / 128)), dim3(GNT), 0, s, A, lda, M, K, rowmax, apack, rowfac,
-		                   rowfac + Mpad);
+		auto go = [&](auto *kernel) {
+			hipLaunchKernelGGL(kernel, dim3((unsigned)(Mpad / 32), (unsigned)(K / 128)), dim3(GNT), 0, s, A, lda, M, K, rowmax, apack, rowfac, rowfac + Mpad);
+		};
+		if (digits == 4) go(quant_pack_kernel<4>);
+		else go(quant_pack_kernel<3>);
 		return;
 	}
 	if (K <= 2048)  // 128 lanes of 16 values
@@ -779,7 +788,7 @@ static bool tg_gemm_lds_taken(int M, int K, int ntiles) {
 // rowmax_part (GEGLU only, may be null): [tg_gemm_mfma_rows(M)] floats cleared by the caller; max|C[m][:]| is folded into it
 void tg_launch_gemm_mfma(float *C, const int8_t *apack, const float *rowfac, const int8_t *Wg, const float *scales, int M, int K,
                          int ntiles, int epi, const float *lut, float gmin, float geps, int lut_size, float *rowmax_part,
-                         int kparts, size_t part_stride, hipStream_t s) {
+                         int kparts, size_t part_stride, hipStream_t s, int digits) {
 	const unsigned mblocks = (unsigned)((M + 127) / 128);
 	const int Mpad = (int)tg_gemm_mfma_rows(M);
 	const float *rowinv = rowfac + Mpad;
@@ -788,21 +797,24 @@ void tg_launch_gemm_mfma(float *C, const int8_t *apack, const float *rowfac, con
 	const bool geglu = epi == TG_EPI_GEGLU, lutlds = geglu && lut_size <= LUT_LDS_MAX;
 	const int ldc = geglu ? ntiles * (TG_CT / 2) : ntiles * TG_CT;
 	float *rmp = geglu ? rowmax_part : nullptr;
-	if (tg_gemm_skinny_taken(M, K, ntiles, geglu ? 1 : kparts, g_gemm_lds_cus)) {
+	if (digits == 4 || tg_gemm_skinny_taken(M, K, ntiles, geglu ? 1 : kparts, g_gemm_lds_cus)) {
 		g_gemm_launches[0]++;
 		const int rows32 = (M + 31) / 32, parts = geglu ? 1 : kparts;
 		int groups = parts;  // workgroups that share a tile's parts
-		while (groups > 1 && (long)ntiles * rows32 * groups > g_gemm_lds_cus) groups /= 2;
+		while (digits == 3 && groups > 1 && (long)ntiles * rows32 * groups > g_gemm_lds_cus) groups /= 2;
 		const dim3 grid((unsigned)ntiles, (unsigned)rows32, (unsigned)groups), block(GNT);
-		if (geglu && lutlds)
-			hipLaunchKernelGGL((gemm_i8_skinny_kernel<true, true>), grid, block, 0, s, C, apack, rowinv, Wg, scales, M, K, ldc, lut, gmin, geps,
-			                   ginv, lut_size, rmp, Mpad, (size_t)0, 1);
-		else if (geglu)
-			hipLaunchKernelGGL((gemm_i8_skinny_kernel<true, false>), grid, block, 0, s, C, apack, rowinv, Wg, scales, M, K, ldc, lut, gmin, geps,
-			                   ginv, lut_size, rmp, Mpad, (size_t)0, 1);
-		else
-			hipLaunchKernelGGL((gemm_i8_skinny_kernel<false, false>), grid, block, 0, s, C, apack, rowinv, Wg, scales, M, K, ldc, lut, gmin,
-			                   geps, ginv, lut_size, rmp, Mpad, part_stride, parts);
+		auto go = [&](auto *kernel) {
+			hipLaunchKernelGGL(kernel, grid, block, 0, s, C, apack, rowinv, Wg, scales, M, K, ldc, lut, gmin, geps, ginv, lut_size, rmp, Mpad, part_stride,
+			                   parts);
+		};
+		auto rows = [&](auto planes) {
+			constexpr int P = decltype(planes)::value;
+			if (geglu && lutlds) go(gemm_i8_skinny_kernel<true, true, P>);
+			else if (geglu) go(gemm_i8_skinny_kernel<true, false, P>);
+			else go(gemm_i8_skinny_kernel<false, false, P>);
+		};
+		if (digits == 4) rows(std::integral_constant<int, 4>());
+		else rows(std::integral_constant<int, 3>());
 		return;
 	}
 	// kparts == 2 (STORE only; see tg_gemm_mfma_k_parts): two half-K copies of the grid, the second writes C + part_stride

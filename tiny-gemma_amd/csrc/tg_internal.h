@@ -252,7 +252,7 @@ void tg_launch_embed_rows(float *x, const int *ids, int S, const int8_t *wte, co
 // tg_launch_gemm_mfma (rowfac as tg_launch_quant_pack lays it out for S rows)
 void tg_launch_norm_rows(float *out, const float *in, int nparts, size_t part_stride, const float *w_pre, const float *w_post, const float *resid,
                          float *resid_out, int S, int dim, int8_t *apack, float *rowfac, hipStream_t s,
-                         float *clear_rows = nullptr);  // clear_rows: S floats set to 0 (row maxima the next product folds into)
+                         float *clear_rows = nullptr, int digits = 3);  // clear_rows: S floats set to 0 (row maxima the next product folds into); digits: planes
 void tg_launch_qk_norm_rope_rows(float *q, float *k, const float *v, const float *rms_q, const float *rms_k, const float *cos_t,
                                  const float *sin_t, float *kc, float *vc, int max_pos, int S, int n_head, int hd, int ldq, int ldkv,
                                  hipStream_t s);  // cos_t / sin_t: the tables' row of the first token; kc null: nothing goes into a cache
@@ -283,13 +283,16 @@ size_t tg_attn_prefill_planes_bytes(int S);
 // The rows of o (S x 1024, 4 heads x 256) -> digit planes + row factors of the int8 MFMA GEMM, merging the partial
 // results of split query tiles on the way (instead of attn_prefill_merge_kernel + the two quantising launches);
 // tg_launch_attn_prefill must then have been called with finish_later = true
-struct TgCacheRows {  // rows that the finishing launch copies into a layer's cache (k null: none)
+struct TgCacheRows {  // rows that a finishing launch copies into a layer's cache (k null: none)
 	const float *k = nullptr, *v = nullptr;
 	float *kc = nullptr, *vc = nullptr;
 	int ld = 0, slot = 0, ring = 1;  // row stride of k and v, slot of row 0, rows of the cache
 };
 void tg_launch_attn_prefill_finish(const float *o, int S, int ldo, const TgAttnPrefillPlan *plan, int n_cu, int8_t *apack, float *rowfac,
-                                   hipStream_t s, const TgCacheRows &rows = TgCacheRows());
+                                   hipStream_t s);
+// the same of a later portion, whose keys and values enter the layer's cache; four digit planes
+void tg_launch_attn_extend_finish(const float *o, int S, int ldo, const TgAttnPrefillPlan *plan, int n_cu, int8_t *apack, float *rowfac,
+                                  const TgCacheRows &rows, hipStream_t s);
 // Attention of a later portion of a sequence: the n keys in front of it are rows (slot0 + j) mod ring of the cache
 struct TgAttnPast {
 	const float *kc = nullptr, *vc = nullptr;
@@ -322,13 +325,14 @@ struct TgColMap {
 void tg_launch_retile_gemv(int8_t *dst, float *dst_scales, const TgColMap &m, int K, int N, int C, hipStream_t s);
 void tg_launch_retile_mfma(int8_t *dst, float *dst_scales, const TgColMap &m, int K, int N, hipStream_t s);
 
-// int8 MFMA prefill GEMM (tg_gemm_mfma.hip): A is first quantised per row into three int8 digit planes in operand order
-size_t tg_gemm_mfma_apack_bytes(int M, int K);
+// int8 MFMA prefill GEMM (tg_gemm_mfma.hip): A is first quantised per row into int8 digit planes in operand order
+size_t tg_gemm_mfma_apack_bytes(int M, int K, int digits = 3);
 size_t tg_gemm_mfma_rows(int M);  // rowfac scratch holds twice this many floats
-void tg_launch_quant_pack(const float *A, int lda, int M, int K, int8_t *apack, float *rowfac, const float *rowmax, hipStream_t s);
+// digits = 4: with rowmax only
+void tg_launch_quant_pack(const float *A, int lda, int M, int K, int8_t *apack, float *rowfac, const float *rowmax, hipStream_t s, int digits = 3);
 void tg_launch_gemm_mfma(float *C, const int8_t *apack, const float *rowfac, const int8_t *Wg, const float *scales, int M, int K,
                          int ntiles, int epi, const float *lut, float gmin, float geps, int lut_size, float *rowmax_part,
-                         int kparts, size_t part_stride, hipStream_t s);
+                         int kparts, size_t part_stride, hipStream_t s, int digits = 3);
 extern int g_gemm_lds, g_gemm_lds_cus, g_gemm_lds_ksplit;
 int tg_gemm_clk_begin(unsigned long long **buf, int n, hipStream_t s);
 int tg_gemm_clk_end(unsigned long long *buf, int n, double *clock_mhz, double *workgroup_us, int *workgroups);
@@ -416,17 +420,22 @@ __device__ __forceinline__ float tg_row16_max(float v) {
 // ---- activation quantisation of the int8 MFMA GEMM (shared by the stand-alone pre-pass and fused producers) ----
 // A row is scaled by a power of two so that its largest magnitude lies in [2^21, 2^22), rounded to an integer and
 // written as three signed base-256 digits (int8 planes), 16 consecutive k per lane, in MFMA operand order:
-//   planes [tile of 32 rows][K/32][3][64 lanes][16 bytes], lane = row % 32 + 32 * ((k % 32) / 16).
+//   planes [tile of 32 rows][K/32][P][64 lanes][16 bytes], lane = row % 32 + 32 * ((k % 32) / 16).
+// P = 4 (largest magnitude in [2^29, 2^30)) for the rows of a later portion, which stand in for decode steps and may not be
+// less exact than those.  Norm-relative error of a product against 64 bits: one row in fp32 (a decode step) 0.9e-7 .. 1.3e-7,
+// three planes 2.9e-7 of a normed row and 1.2e-6 of a gated one.
 #if defined(__HIPCC__)
-constexpr int TG_QBITS = 22;
+template <int P = 3>
 __device__ __forceinline__ void tg_row_factors(float amax, float &mul, float &inv) {
+	constexpr int QBITS = 8 * P - 2;
 	mul = 1.0f;
 	inv = 1.0f;
 	if (amax > 0.0f && amax < INFINITY) {
 		int e;
 		(void)frexpf(amax, &e);  // amax = f * 2^e, f in [0.5, 1)
-		mul = ldexpf(1.0f, TG_QBITS - e);
-		inv = ldexpf(1.0f, e - TG_QBITS);
+		e = e < QBITS - 126 ? QBITS - 126 : e;  // (both factors stay normal numbers)
+		mul = ldexpf(1.0f, QBITS - e);
+		inv = ldexpf(1.0f, e - QBITS);
 	}
 }
 typedef int tg_i32x4 __attribute__((ext_vector_type(4)));
@@ -434,38 +443,48 @@ typedef int tg_i32x4 __attribute__((ext_vector_type(4)));
 // digits a0 + 256 a1 + 65536 a2 of a value are its bytes, without carries between them: bytes 0 and 1 with the top bit
 // flipped back, byte 2 as it is.  4 operations a value and 9 for the four bytes of three planes, where one digit at a
 // time took 15 a value; the same bytes for every value, saturated conversions included.  4096 tokens of the 1B shape: 13.51
-// ms, one digit at a time 13.76 ms.
-__device__ __forceinline__ void tg_quant4(const float *v, float mul, unsigned d[3]) {
+// ms, one digit at a time 13.76 ms.  (P = 4: the same with a third lower digit.)
+template <int P = 3>
+__device__ __forceinline__ void tg_quant4(const float *v, float mul, unsigned *d) {
 	unsigned t[4];
 #pragma unroll
-	for (int i = 0; i < 4; i++) t[i] = (unsigned)(int)rintf(v[i] * mul) + 0x8080u;
+	for (int i = 0; i < 4; i++) t[i] = (unsigned)(int)rintf(v[i] * mul) + (P == 4 ? 0x808080u : 0x8080u);
 	const unsigned lo = __builtin_amdgcn_perm(t[1], t[0], 0x05010400u), hi = __builtin_amdgcn_perm(t[3], t[2], 0x05010400u);
 	d[0] = __builtin_amdgcn_perm(hi, lo, 0x05040100u) ^ 0x80808080u;
 	d[1] = __builtin_amdgcn_perm(hi, lo, 0x07060302u) ^ 0x80808080u;
-	d[2] = __builtin_amdgcn_perm(t[1], t[0], 0x0c0c0602u) | __builtin_amdgcn_perm(t[3], t[2], 0x06020c0cu);
+	if constexpr (P == 3) {
+		d[2] = __builtin_amdgcn_perm(t[1], t[0], 0x0c0c0602u) | __builtin_amdgcn_perm(t[3], t[2], 0x06020c0cu);
+	} else {
+		const unsigned lo2 = __builtin_amdgcn_perm(t[1], t[0], 0x07030602u), hi2 = __builtin_amdgcn_perm(t[3], t[2], 0x07030602u);
+		d[2] = __builtin_amdgcn_perm(hi2, lo2, 0x05040100u) ^ 0x80808080u;
+		d[3] = __builtin_amdgcn_perm(hi2, lo2, 0x07060302u);
+	}
 }
 // v[16] consecutive k of one row -> the lane's 16 bytes of each plane
-__device__ __forceinline__ void tg_quant16(const float *v, float mul, tg_i32x4 pl[3]) {
+template <int P = 3>
+__device__ __forceinline__ void tg_quant16(const float *v, float mul, tg_i32x4 *pl) {
 #pragma unroll
 	for (int q = 0; q < 4; q++) {
-		unsigned d[3];
-		tg_quant4(v + 4 * q, mul, d);
+		unsigned d[P];
+		tg_quant4<P>(v + 4 * q, mul, d);
 #pragma unroll
-		for (int p = 0; p < 3; p++) pl[p][q] = (int)d[p];
+		for (int p = 0; p < P; p++) pl[p][q] = (int)d[p];
 	}
 }
 // v[8] consecutive k of one row -> the 8 bytes of each plane (half of a lane's piece)
-__device__ __forceinline__ void tg_quant8(const float *v, float mul, uint2 pl[3]) {
-	unsigned d[2][3];
+template <int P = 3>
+__device__ __forceinline__ void tg_quant8(const float *v, float mul, uint2 *pl) {
+	unsigned d[2][P];
 #pragma unroll
-	for (int q = 0; q < 2; q++) tg_quant4(v + 4 * q, mul, d[q]);
+	for (int q = 0; q < 2; q++) tg_quant4<P>(v + 4 * q, mul, d[q]);
 #pragma unroll
-	for (int p = 0; p < 3; p++) pl[p] = uint2{d[0][p], d[1][p]};
+	for (int p = 0; p < P; p++) pl[p] = uint2{d[0][p], d[1][p]};
 }
 // where the 16 bytes of (row m, k0 = multiple of 16) of plane 0 go; planes are 64 pieces apart
+template <int P = 3>
 __device__ __forceinline__ tg_i32x4 *tg_plane_dst(int8_t *apack, int m, int k0, int K) {
 	const int kb = k0 >> 5, hb = (k0 >> 4) & 1;
-	return reinterpret_cast<tg_i32x4 *>(apack) + ((size_t)(m >> 5) * (size_t)(K >> 5) + kb) * 3 * 64 + ((m & 31) + 32 * hb);
+	return reinterpret_cast<tg_i32x4 *>(apack) + ((size_t)(m >> 5) * (size_t)(K >> 5) + kb) * P * 64 + ((m & 31) + 32 * hb);
 }
 #endif
 

@@ -10,6 +10,8 @@
 
 #include "tg_internal.h"
 
+#include <type_traits>
+
 namespace {
 
 constexpr int RNT = 256;
@@ -47,7 +49,7 @@ __global__ __launch_bounds__(RNT) void embed_rows_kernel(float *x, const int *id
 // [post-norm + residual (+ residual out)] + pre-norm.  The normalised row goes out as fp32 (out != nullptr) and/or
 // straight as the int8 digit planes + row factors of the MFMA GEMM that consumes it (apack != nullptr): the same bits
 // the stand-alone quantising pre-pass would produce from the fp32 row.
-template <int ROUNDS, int NPARTS>
+template <int ROUNDS, int NPARTS, int P>
 __global__ __launch_bounds__(RNT) void norm_rows_kernel(float *out, const float *in, size_t part_stride, const float *w_pre,
                                                         const float *w_post, const float *resid, float *resid_out, int S, int dim,
                                                         int8_t *apack, float *rowfac, int Mpad, float *clear_rows) {
@@ -147,7 +149,7 @@ __global__ __launch_bounds__(RNT) void norm_rows_kernel(float *out, const float 
 	if (apack == nullptr) return;
 	amax = tg_wave_max(amax);
 	float mul, inv;
-	tg_row_factors(amax, mul, inv);
+	tg_row_factors<P>(amax, mul, inv);
 	if (lane == 0) {
 		rowfac[s] = mul;
 		rowfac[Mpad + s] = inv;
@@ -160,13 +162,13 @@ __global__ __launch_bounds__(RNT) void norm_rows_kernel(float *out, const float 
 		for (int q = 0; q < 2; q++)
 #pragma unroll
 			for (int e = 0; e < 4; e++) y[4 * q + e] = v[r][q][e];
-		uint2 pl[3];
-		tg_quant8(y, mul, pl);
+		uint2 pl[P];
+		tg_quant8<P>(y, mul, pl);
 		// two neighbouring lanes share a 16-byte piece of every plane
 		const int k0 = (int)off[r];
-		uint2 *dst = reinterpret_cast<uint2 *>(tg_plane_dst(apack, s, k0 & ~15, dim)) + ((k0 >> 3) & 1);
+		uint2 *dst = reinterpret_cast<uint2 *>(tg_plane_dst<P>(apack, s, k0 & ~15, dim)) + ((k0 >> 3) & 1);
 #pragma unroll
-		for (int p = 0; p < 3; p++) dst[p * 128] = pl[p];  // planes are 64 pieces of 16 bytes apart
+		for (int p = 0; p < P; p++) dst[p * 128] = pl[p];  // planes are 64 pieces of 16 bytes apart
 	}
 }
 
@@ -296,23 +298,27 @@ void tg_launch_embed_rows(float *x, const int *ids, int S, const int8_t *wte, co
 // in: nparts (1, 2 or 4) addends of every row, part_stride floats apart
 void tg_launch_norm_rows(float *out, const float *in, int nparts, size_t part_stride, const float *w_pre, const float *w_post,
                          const float *resid, float *resid_out, int S, int dim, int8_t *apack, float *rowfac, hipStream_t s,
-                         float *clear_rows) {
+                         float *clear_rows, int digits) {
 	const int Mpad = (int)tg_gemm_mfma_rows(S);
 	const dim3 grid((unsigned)((S + RNT / 64 - 1) / (RNT / 64))), block(RNT);
 	// dim is a legal row dimension: a multiple of 16, at most 1536 where a norm is applied (hidden sizes 640 and 1152)
-#define TG_NORM_ROWS(R, P)                                                                                                        \
-	hipLaunchKernelGGL((norm_rows_kernel<R, P>), grid, block, 0, s, out, in, part_stride, w_pre, w_post, resid, resid_out, S, dim, apack, \
-	                   rowfac, Mpad, clear_rows)
-	if (dim <= 1024) {
-		if (nparts == 4) TG_NORM_ROWS(2, 4);
-		else if (nparts == 2) TG_NORM_ROWS(2, 2);
-		else TG_NORM_ROWS(2, 1);
-	} else {
-		if (nparts == 4) TG_NORM_ROWS(3, 4);
-		else if (nparts == 2) TG_NORM_ROWS(3, 2);
-		else TG_NORM_ROWS(3, 1);
-	}
-#undef TG_NORM_ROWS
+	auto go = [&](auto *kernel) {
+		hipLaunchKernelGGL(kernel, grid, block, 0, s, out, in, part_stride, w_pre, w_post, resid, resid_out, S, dim, apack, rowfac, Mpad, clear_rows);
+	};
+	auto rows = [&](auto planes) {
+		constexpr int P = decltype(planes)::value;
+		if (dim <= 1024) {
+			if (nparts == 4) go(norm_rows_kernel<2, 4, P>);
+			else if (nparts == 2) go(norm_rows_kernel<2, 2, P>);
+			else go(norm_rows_kernel<2, 1, P>);
+		} else {
+			if (nparts == 4) go(norm_rows_kernel<3, 4, P>);
+			else if (nparts == 2) go(norm_rows_kernel<3, 2, P>);
+			else go(norm_rows_kernel<3, 1, P>);
+		}
+	};
+	if (digits == 4) rows(std::integral_constant<int, 4>());
+	else rows(std::integral_constant<int, 3>());
 }
 
 // Wp/scales: GEMV tiling of the matrix (ntiles tiles of Ct columns); C gets ntiles * Ct columns, or half of that for GEGLU
