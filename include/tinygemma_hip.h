@@ -160,8 +160,9 @@ int tg_forward_decode(tg_session *s, int32_t id, float *logits, int32_t *argmax)
  * behind the last one.  The result does not depend on how a sequence is cut into portions, beyond rounding.  A portion of
  * more than one token (of a Gemma model: of three tokens or more) runs through the prefill kernels, behind whatever the
  * session holds, with a fourth digit plane, so that its rows are no less exact than those of single tokens; a Gemma model's
- * shorter portions go token by token.  Afterwards the token log (tg_session_read_ids) starts
- * with this pick, as behind a prefill, unless the portion went token by token. */
+ * shorter portions go token by token.  The token log (tg_session_read_ids) of a model opened from a folder then starts with
+ * this pick, as behind a prefill; that of a Gemma model goes on, with this pick or, where the portion went token by token, with
+ * one for each of its tokens. */
 int tg_forward_tokens(tg_session *s, const int32_t *ids, int n, const int32_t *want, int n_want, float *logits, int32_t *argmax);
 /* greedy branch of gemma::generate (transformer.hpp:204-250) without tokenizer/EOS stop:
  * out_ids gets n_decode+1 ids (the first from the prefill logits); seconds are wall clock around

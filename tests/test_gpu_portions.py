@@ -30,9 +30,11 @@ def test_portions_equal_single_tokens(sessions, prompt, portions):
     rng = np.random.default_rng(1000 + prompt)
     for s in (a, b):
         s.reset()
+    log = []
     if prompt:
         ids = gi.prompt_ids(50 + prompt, prompt)
-        assert a.prefill(ids)[0] == b.prefill(ids)[0]
+        log = [a.prefill(ids)[0]]
+        assert log == [b.prefill(ids)[0]]
     for n in portions:
         ids = rng.integers(0, a.cfg.n_vocab, n).astype(np.int32)
         want = np.unique([0, n // 2, n - 2, n - 1] if n != 5 else [1, 3])  # once without the last place
@@ -54,7 +56,8 @@ def test_portions_equal_single_tokens(sessions, prompt, portions):
             n_valid = min(pa, ka.shape[0])
             assert normrel(ka[:n_valid], kb[:n_valid]) < TOL and normrel(va[:n_valid], vb[:n_valid]) < TOL
             assert np.abs(ka - kb).max() < 1e-3 and np.abs(va - vb).max() < 1e-3  # every slot, also the untouched ones
-        assert a.read_ids(1 << 15).tolist() == [arg]  # the log starts with the portion's pick
+        log += [arg]
+        assert a.read_ids(1 << 15).tolist() == log  # the log goes on with the portion's pick
     # both go on: steps that read every slot the portions wrote
     tok = int(rng.integers(0, a.cfg.n_vocab))
     for _ in range(2):
@@ -62,7 +65,7 @@ def test_portions_equal_single_tokens(sessions, prompt, portions):
         assert normrel(la, lb) < TOL
         tok = pa
     a.decode_enqueue(5)
-    assert a.read_ids(64).size == 8
+    assert a.read_ids(1 << 15)[:len(log)].tolist() == log and a.read_ids(1 << 15).size == len(log) + 7
 
 
 def layer_in_64_bits(image, cos, sin, ids, past, table):
@@ -170,3 +173,29 @@ def test_context_end(sessions):
     assert a.position == n
     with pytest.raises(Exception, match="context is full"):
         a.forward([1, 2, 3])
+
+
+def test_the_log_keeps_earlier_answers(sessions):
+    """Prompt, answer, next turn, answer, sampled tokens: the log read once at the end holds all picks in order."""
+    a, b = sessions
+    for s in (a, b):
+        s.reset()
+    prompt, turn = gi.prompt_ids(9, 20), gi.prompt_ids(10, 30)
+    randf = np.random.default_rng(3).uniform(0, 1, 6).astype(np.float32)
+    log = [a.prefill(prompt)[0]]
+    a.decode_enqueue(5)
+    log = a.read_ids(64).tolist()
+    assert len(log) == 6
+    log.append(a.forward(np.concatenate([[log[-1]], turn]).astype(np.int32))[0])
+    a.decode_enqueue(4)
+    a.decode_enqueue_sampled(6, 0.05, 1.0, randf)
+    got = a.read_ids(64).tolist()
+    assert got[:7] == log and len(got) == 17
+    # the same with a read behind every call
+    b.prefill(prompt)
+    b.decode_enqueue(5)
+    b.forward(np.concatenate([b.read_ids(64)[-1:], turn]).astype(np.int32))
+    b.decode_enqueue(4)
+    assert b.read_ids(64).tolist() == got[:11]
+    b.decode_enqueue_sampled(6, 0.05, 1.0, randf)
+    assert b.read_ids(64).tolist() == got

@@ -2440,9 +2440,10 @@ static int net_extend(tg_session *s, const int32_t *ids, int n, const int32_t *w
 
 // A portion of several tokens of a Gemma model behind whatever the session holds, through the kernels of a prompt, with one digit
 // plane more than a prompt's rows have (a portion stands in for decode steps and is to be as exact as those).  The token
-// log starts anew with the portion's pick, as behind a prefill.
+// log goes on with the portion's pick.
 static int gemma_extend(tg_session *s, const int32_t *ids, int n, const int32_t *want, int n_want, float *logits, int32_t *argmax) {
 	const size_t V = (size_t)s->m->cfg.n_vocab;
+	if (s->steps >= s->tok_log_cap) return tg_fail(TG_ERR_STATE, "token log is full");
 	PrefillCtx p;
 	if (int rc = prefill_setup(s, n, &p, true, s->pos)) return rc;
 	if (int rc = prefill_rows(p, ids)) return rc;
@@ -2454,8 +2455,8 @@ static int gemma_extend(tg_session *s, const int32_t *ids, int n, const int32_t 
 	s->pos += n;
 	s->bp_local += n;
 	s->bp_global += n;
-	s->steps = 1;
-	const int ctr[4] = {s->pos, s->bp_local, s->bp_global, 0};
+	s->steps += 1;
+	const int ctr[3] = {s->pos, s->bp_local, s->bp_global};
 	TG_HIP(hipMemcpyAsync(s->ctr, ctr, sizeof(ctr), hipMemcpyHostToDevice, g_stream));
 	tg_launch_argmax_finish(s->blk_val, s->blk_idx, s->m->lm.ntiles, s->ctr, s->tok_log, 0, g_stream);
 	TG_HIP(hipGetLastError());
