@@ -158,7 +158,7 @@ int tg_forward_decode(tg_session *s, int32_t id, float *logits, int32_t *argmax)
 /* The next n tokens of the session's sequence, at whatever position it is: a prompt may come in portions of any size.
  * want[n_want]: ascending places among them whose logits go to logits (host, [n_want][n_vocab]); argmax (may be NULL): the pick
  * behind the last one.  The result does not depend on how a sequence is cut into portions, beyond rounding.  A portion of
- * more than one token (of a Gemma model: of three tokens or more) runs through the prefill kernels, behind whatever the
+ * more than one token (of a Gemma model: of four tokens or more) runs through the prefill kernels, behind whatever the
  * session holds, with a fourth digit plane, so that its rows are no less exact than those of single tokens; a Gemma model's
  * shorter portions go token by token.  The token log (tg_session_read_ids) of a model opened from a folder then starts with
  * this pick, as behind a prefill; that of a Gemma model goes on, with this pick or, where the portion went token by token, with

@@ -23,7 +23,7 @@ def sessions(tg, oracle, weight_images):
 # a portion of an empty session with several wanted places; portions in front of, at and across the 512 slots of the
 # local rings; one longer than a ring; counts around the tiles of 16 and 32 queries; a long past for few queries; a portion of more
 # rows than the last pass of the attention takes four parts at a time for
-@pytest.mark.parametrize("prompt,portions", [(0, [40]), (3, [4, 17, 16]), (9, [3]), (480, [31, 5, 33]), (511, [32]), (512, [40]), (700, [33]), (300, [530]),
+@pytest.mark.parametrize("prompt,portions", [(0, [40]), (3, [4, 17, 16]), (9, [3, 4]), (480, [31, 5, 33]), (511, [32]), (512, [40]), (700, [33]), (300, [530]),
                                              (1, [600, 65]), (2500, [21, 4]), (5, [2060])])
 def test_portions_equal_single_tokens(sessions, prompt, portions):
     a, b = sessions
@@ -56,8 +56,8 @@ def test_portions_equal_single_tokens(sessions, prompt, portions):
             n_valid = min(pa, ka.shape[0])
             assert normrel(ka[:n_valid], kb[:n_valid]) < TOL and normrel(va[:n_valid], vb[:n_valid]) < TOL
             assert np.abs(ka - kb).max() < 1e-3 and np.abs(va - vb).max() < 1e-3  # every slot, also the untouched ones
-        log += [arg]
-        assert a.read_ids(1 << 15).tolist() == log  # the log goes on with the portion's pick
+        log += [arg] if n > 3 else b.read_ids(1 << 15)[-n:].tolist()
+        assert a.read_ids(1 << 15).tolist() == log  # the log goes on with the portion's pick, or with those of its single tokens
     # both go on: steps that read every slot the portions wrote
     tok = int(rng.integers(0, a.cfg.n_vocab))
     for _ in range(2):
@@ -156,7 +156,8 @@ def test_short_portions_go_token_by_token(sessions):
         s.reset()
         s.prefill(gi.prompt_ids(7, 30))
     a.forward([5, 6])
-    for t in (5, 6):
+    a.forward([7, 8, 9])
+    for t in range(5, 10):
         b.decode(t)
     assert np.array_equal(a.read_ids(64), b.read_ids(64)) and np.array_equal(a.kv(0)[0], b.kv(0)[0])
 

@@ -381,7 +381,7 @@ constexpr int PREFILL_TAP_MAX_ROWS = 1024;
 // A later portion of a Gemma model goes through the kernels of a prompt from this many tokens on, below it token by token.  Those
 // kernels take 2.2 ms for 3 to 16 tokens of the 1B shape behind 300 keys and 2.45 ms behind 16,000 (270m: 1.33 and 1.55 ms), three
 // tokens one by one 2.3 and 2.4 ms (1.37 and 1.5 ms), four 3.0 and 3.2 ms (1.78 and 1.98 ms).
-constexpr int TG_EXTEND_MIN = 3;
+constexpr int TG_EXTEND_MIN = 4;
 
 bool layer_is_local(const tg_config &c, int l) { return (l % c.window_pattern) != (c.window_pattern - 1); }  // transformer.hpp:43
 
