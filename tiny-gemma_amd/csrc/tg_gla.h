@@ -24,7 +24,7 @@ struct TgGla {
 	int group;            // heads per q/k head
 };
 // one token: y = the fused product's outputs q | k | v | g | a1 (offsets in floats); o [heads * vdimp]
-void tg_launch_gla_step(const TgGla &g, const float *y, int k_off, int v_off, int a_off, float *o, TgTouch touch, int touch_blocks, hipStream_t s);
+void tg_launch_gla_step(const TgGla &g, const float *y, int k_off, int v_off, int a_off, float *o, hipStream_t s);
 // n tokens: qkv [n][ld] in the model's format (q at column 0, offsets in elements), low [n][ld_low] fp32 (the decay's low-rank input).
 // Scratch: see tg_gla_scratch.  out [n][ld_out]: the normalised, gated heads.
 struct TgGlaScratch {

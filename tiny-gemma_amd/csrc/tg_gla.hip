@@ -18,8 +18,7 @@ __device__ __forceinline__ float pow2(float x) { return __builtin_amdgcn_exp2f(x
 
 // ---- one token -----------------------------------------------------------------------------------------------------------
 // A workgroup owns 32 value columns of a head: lane = 4 columns, 32 groups of key channels.
-__global__ __launch_bounds__(256) void gla_step_kernel(const float *y, TgGla g, int k_off, int v_off, int a_off, float *o, TgTouch touch) {
-	if (tg_touch(touch)) return;
+__global__ __launch_bounds__(256) void gla_step_kernel(const float *y, TgGla g, int k_off, int v_off, int a_off, float *o) {
 	extern __shared__ __align__(16) float sm[];
 	float *s_q = sm, *s_k = sm + g.dimp, *s_a = sm + 2 * g.dimp;
 	__shared__ f32x4_t s_red[4][8];
@@ -1039,9 +1038,9 @@ void launch_delta_rows(const TgDelta &d, const void *xv, int ld, const float *lo
 
 }  // namespace
 
-void tg_launch_gla_step(const TgGla &g, const float *y, int k_off, int v_off, int a_off, float *o, TgTouch touch, int touch_blocks, hipStream_t s) {
-	const dim3 grid = tg_touch_grid(dim3((unsigned)g.heads, (unsigned)(g.vdimp / 32)), &touch, touch_blocks);
-	hipLaunchKernelGGL(gla_step_kernel, grid, dim3(256), sizeof(float) * 3 * (size_t)g.dimp, s, y, g, k_off, v_off, a_off, o, touch);
+void tg_launch_gla_step(const TgGla &g, const float *y, int k_off, int v_off, int a_off, float *o, hipStream_t s) {
+	hipLaunchKernelGGL(gla_step_kernel, dim3((unsigned)g.heads, (unsigned)(g.vdimp / 32)), dim3(256), sizeof(float) * 3 * (size_t)g.dimp, s, y, g,
+	                   k_off, v_off, a_off, o);
 }
 
 size_t tg_gla_scratch(const TgGla &g, int n, TgGlaScratch *t, unsigned char *base) {

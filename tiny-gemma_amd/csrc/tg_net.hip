@@ -947,7 +947,7 @@ void tg_net_seq_free(TgNetSeq *q) {
 // ---- one token -------------------------------------------------------------------------------------------------------------------
 namespace {
 
-constexpr size_t TOUCH_MIN_BYTES = (size_t)12 << 20;
+constexpr size_t TOUCH_MIN_BYTES = (size_t)12 << 20, TOUCH_MAX_BYTES = (size_t)14 << 20;
 constexpr int TOUCH_BLOCKS = 128;
 
 // One decode step: the launches of a mixer and of a feed-forward, and the residual stream between them (x, and parts that the next
@@ -995,7 +995,7 @@ struct Step {
 	void gla(int l, int r, TgVec o) {
 		const TgMixerCfg &m = c.layers[(size_t)l].mix;
 		const LayerW &w = n->lw(l);
-		tg_launch_gla_step(gla_of(n, l, q, r), q->yin, row_k_off(m), row_v_off(m), w.n_split, q->mix, touch, touch_blocks, s);
+		tg_launch_gla_step(gla_of(n, l, q, r), q->yin, row_k_off(m), row_v_off(m), w.n_split, q->mix, s);
 		o.gate = q->yin + row_g_off(m);
 		head_norm(m, w, o);
 	}
@@ -1196,13 +1196,15 @@ struct Step {
 			// The state or attention launch of a layer leaves most of the chip and the memory idle for 7 to 12 us: workgroups behind its
 			// own touch the first part of a wide feed-forward's matrix for the launch after next.  24 MB (width 1152, ff 10368): that
 			// launch 8.2 -> 6.0 us, the state launch 6.9 -> 7.4; 600 tokens and 24 steps 42.7 -> 41.8 ms with 60 % of the matrix, 42.9
-			// with all of it.  6 MB (width 640 in fp32, of which the memory-side cache keeps some): no difference.
+			// with all of it.  6 MB (width 640 in fp32, of which the memory-side cache keeps some): no difference.  At most 14 MB, what the
+			// idle time fetches: steps of 8 layer runs with matrices of 48, 111 and 198 MB 334, 571 and 801 us, with 60 % of the matrix
+			// 333, 600 and 895, without 383, 618 and 869 us.
 			touch = TgTouch();
 			touch_blocks = 0;
 			if (lc.mlp == TG_FF_DENSE && (size_t)w.gate_up.n * w.gate_up.k * tg_dt_bytes(dt) >= TOUCH_MIN_BYTES) {
 				touch.ptr = (const unsigned char *)w.gate_up.w;
 				touch.slab = (unsigned)(w.gate_up.k / frag_k(dt) * 1024);
-				touch.tiles = w.gate_up.n / 16 * 3 / 5;
+				touch.tiles = (int)std::min((size_t)(w.gate_up.n / 16 * 3 / 5), TOUCH_MAX_BYTES / touch.slab);
 				touch_blocks = TOUCH_BLOCKS;
 			}
 			switch (lc.mix.kind) {
