@@ -111,6 +111,8 @@ inline dim3 tg_touch_grid(dim3 grid, TgTouch *t, int blocks) {
 	return grid;
 }
 
+#define TG_ROUTE_ROW_MAX 4608
+
 // A packed matrix (see above); n, k are the padded sizes.
 struct TgMat {
 	void *w = nullptr;
@@ -150,7 +152,7 @@ enum {
 	TG_VP_MERGE,       // merged attention partials of head z
 	TG_VP_MERGE_HEADS, // the same of all heads, side by side (vdimp elements each): groups of `group` heads, each padded to 16
 	TG_VP_EXPERT,      // x, for the z-th of the experts that the router's logits select
-	TG_VP_ROUTE        // DYT, then the router's product on its result, then EXPERT: routers of one tile (at most 16 experts)
+	TG_VP_ROUTE        // DYT, then the router's product on its result, then EXPERT: routers of one tile (at most 16 experts), rows of TG_ROUTE_ROW_MAX bytes at most
 };
 enum {
 	TG_VE_STORE = 0,

@@ -737,8 +737,23 @@ size_t rms_lds(int pro, int k) { return pro == TG_VP_RMS && k > 8 * NT ? sizeof(
 // 5.2 us products of width 1152 took 6.4.
 int vec_class(int pro, int k) { return pro != TG_VP_DYT && pro != TG_VP_RMS && pro != TG_VP_ROUTE ? 0 : k <= 4 * NT ? 1 : k <= 8 * NT ? 2 : 3; }
 
+// Fragments in flight for n of them a wave: all where they fit, else as few equal rounds as possible; whether some n of a range
+// gets u (instances that no length of a class reaches are not built: a third of the library's size).
+constexpr int vec_depth(int n) {
+	return n <= 2 ? 2 : n <= 4 ? 4 : n <= 6 || (n > 9 && n <= 12) ? 6 : n <= 8 || (n > 12 && n <= 16) || (n > 18 && n <= 24) ? 8 : 9;
+}
+constexpr bool vec_reaches(int u, int n_min, int n_max) {
+	for (int n = n_min; n <= n_max && n <= n_min + 32; n++)
+		if (vec_depth(n) == u) return true;
+	return false;
+}
+
 template <class TR, int PRO, int EPI, int VP>
 void launch_vec_vp(const TgVec &v, hipStream_t s) {
+	// fragments a wave in this class
+	constexpr int PASS = 4 * NT / TR::KF / 4, ROUTED = (TG_ROUTE_ROW_MAX / (int)sizeof(typename TR::T) / TR::KF + 3) / 4;
+	constexpr int N_MIN = VP == 3 ? 2 * PASS + 1 : VP == 2 ? PASS + 1 : 1, N_CLASS = VP == 1 ? PASS : VP == 2 ? 2 * PASS : 1 << 16;
+	constexpr int N_MAX = PRO == TG_VP_ROUTE && ROUTED < N_CLASS ? ROUTED : N_CLASS;
 	const VecHot h = vec_hot<PRO, EPI>(v);
 #define TG_VEC_LAUNCH(ntl, kw, u, grid, pad)                                                                                                       \
 	hipLaunchKernelGGL((vec_kernel<TR, PRO, EPI, ntl, kw, u, VP>), grid, dim3(NT), lds(pad), s, h.a[0], h.a[1], h.a[2], h.a[3], h.i[0], h.i[1], \
@@ -750,8 +765,13 @@ void launch_vec_vp(const TgVec &v, hipStream_t s) {
 			const int n = (per + 3) / 4;
 			auto lds = [&](int pad) { return sizeof(typename TR::T) * (size_t)(per + pad) * TR::KF + rms_lds(PRO, per * TR::KF); };
 			const dim3 grid((unsigned)tg_vec_blocks(v, EPI), (unsigned)v.ksplit, (unsigned)v.nz);
-			if (n <= 6) TG_VEC_LAUNCH(2, 4, 6, (grid), 24);
-			else TG_VEC_LAUNCH(2, 4, 8, (grid), 32);
+			if constexpr (N_MIN <= 6) {
+				if (n <= 6) {
+					TG_VEC_LAUNCH(2, 4, 6, (grid), 24);
+					return;
+				}
+			}
+			TG_VEC_LAUNCH(2, 4, 8, (grid), 32);
 			return;
 		}
 	}
@@ -768,14 +788,19 @@ void launch_vec_vp(const TgVec &v, hipStream_t s) {
 			return;
 		}
 	}
-	// fragments in flight: all of a wave's where they fit, else in as few equal rounds as possible
 	const dim3 grid(bx, (unsigned)v.ksplit, (unsigned)v.nz);
-	const int n = (per + 3) / 4;
-	if (n <= 2) TG_VEC_LAUNCH(NTL, 4, 2, (grid), 8);
-	else if (n <= 4) TG_VEC_LAUNCH(NTL, 4, 4, (grid), 16);
-	else if (n <= 6 || (n > 9 && n <= 12)) TG_VEC_LAUNCH(NTL, 4, 6, (grid), 24);
-	else if (n <= 8 || (n > 12 && n <= 16) || (n > 18 && n <= 24)) TG_VEC_LAUNCH(NTL, 4, 8, (grid), 32);
-	else TG_VEC_LAUNCH(NTL, 4, 9, (grid), 36);
+	const int depth = vec_depth((per + 3) / 4);
+	auto go = [&](auto u) {
+		constexpr int U = decltype(u)::value;
+		if constexpr (vec_reaches(U, N_MIN, N_MAX)) {
+			if (depth == U) TG_VEC_LAUNCH(NTL, 4, U, (grid), 4 * U);
+		}
+	};
+	go(Const<2>());
+	go(Const<4>());
+	go(Const<6>());
+	go(Const<8>());
+	go(Const<9>());
 }
 
 #undef TG_VEC_LAUNCH

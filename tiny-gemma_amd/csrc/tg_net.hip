@@ -724,9 +724,8 @@ void norm_prologue(const TgNet *n, TgVec *v, const Norm &nm) {
 }
 // A router of one tile is small enough for every workgroup of a decode step's experts' product to do for itself (20 KiB at width
 // 640 in bf16), where a launch of its own is one workgroup that the rest of the chip waits for; larger ones keep theirs.
-constexpr size_t ROUTE_ROW_MAX = 4608;  // bytes of a router's row
 bool routes_in_place(const TgNet *n, const LayerW &w) {
-	return n->cfg.norm == TG_NORM_TANH && w.router.n == 16 && (size_t)w.router.k * tg_dt_bytes(n->dt) <= ROUTE_ROW_MAX;
+	return n->cfg.norm == TG_NORM_TANH && w.router.n == 16 && (size_t)w.router.k * tg_dt_bytes(n->dt) <= TG_ROUTE_ROW_MAX;
 }
 int norm_kind(const TgNet *n) { return n->cfg.norm == TG_NORM_RMS ? TG_VP_RMS : TG_VP_DYT; }
 
