@@ -200,3 +200,42 @@ def test_the_log_keeps_earlier_answers(sessions):
     assert b.read_ids(64).tolist() == got[:11]
     b.decode_enqueue_sampled(6, 0.05, 1.0, randf)
     assert b.read_ids(64).tolist() == got
+
+
+def test_reset_leaves_empty_caches(sessions):
+    """A reset clears the rows written since the last one: behind a prompt longer than the local rings, portions, single tokens, steps and
+    rows set one layer at a time, then behind a shorter request."""
+    a, _ = sessions
+    rng = np.random.default_rng(12)
+
+    def rows(n):
+        return rng.standard_normal((n, 256)).astype(np.float32)
+
+    def long_request():
+        a.prefill(gi.prompt_ids(11, 700))
+        a.forward(gi.prompt_ids(12, 40))
+        a.forward([1, 2])
+        a.decode_enqueue(9)
+        a.decode_enqueue_sampled(3, 0.1, 1.0, rng.uniform(0, 1, 3).astype(np.float32))
+
+    def short_request():
+        a.prefill(gi.prompt_ids(13, 20))
+        a.decode_enqueue(2)
+
+    def by_layer():
+        for layer in (0, 5):
+            a.kv_prefill(layer, rows(600), rows(600))
+        for _ in range(3):
+            a.block_attention(0, rng.standard_normal((1, 640)).astype(np.float32))
+
+    def by_block():
+        a.block_attention(5, rng.standard_normal((50, 640)).astype(np.float32))
+
+    a.reset()
+    for fill in (long_request, short_request, by_layer, by_block, short_request):
+        fill()
+        assert any(a.kv(layer)[0].any() for layer in range(6))
+        a.reset()
+        for layer in range(6):
+            k, v, pos, _ = a.kv(layer)
+            assert pos == 0 and not k.any() and not v.any(), (fill.__name__, layer)
