@@ -575,9 +575,12 @@ template <class TR, bool DELTA>
 void launch_intra(const typename TR::T *qkv, int ld, int k_off, const TgGla &g, int n, const float *b, float *A, const DeltaIntra &x, hipStream_t s) {
 	const dim3 grid((unsigned)((n + C - 1) / C), (unsigned)g.heads);
 	auto go = [&](auto *kernel, int groups) { hipLaunchKernelGGL(kernel, grid, dim3(256 * groups), 0, s, qkv, ld, k_off, g, n, b, A, x); };
+	// Four groups fill a compute unit; with more workgroups than units two share one (delta rule, key size 128: 256 workgroups 19.4
+	// us with four groups, 21.2 with two, 31.1 with one; 512: 36.0, 31.7 and 37.0; 1024: 71.3, 56.5 and 55.6; key size 64,
+	// 256: 13.4, 13.8 and 18.7)
 	if (g.dimp <= 32) go(gla_intra_kernel<TR, DELTA, 1>, 1);
-	else if (g.dimp < 128) go(gla_intra_kernel<TR, DELTA, 2>, 2);
-	else go(gla_intra_kernel<TR, DELTA, 4>, 4);
+	else if (grid.x * grid.y <= 256) go(gla_intra_kernel<TR, DELTA, 4>, 4);
+	else go(gla_intra_kernel<TR, DELTA, 2>, 2);
 }
 
 template <class TI, class TR, int VB, bool DELTA>
