@@ -612,8 +612,8 @@ __global__ __launch_bounds__(GNT) void gemm_i8_skinny_kernel(float *C, const int
 	    reinterpret_cast<const i32x4 *>(Apack) + (size_t)mtile * (size_t)(K >> 5) * P * 64 + lane + (size_t)z * nstage * 2 * P * 64;
 	for (int turn = 0;;) {
 
-		// ring of three stages: loads go to ordinary vector registers only, and 3 x 56 of them is what fits beside the
-		// addresses (the 192 accumulators live in the accumulation registers)
+		// ring of three stages: loads go to ordinary vector registers only, and 3 x 56 of them (64 with four planes) is what fits
+		// beside the addresses (the 192 or 256 accumulators live in the accumulation registers)
 		i32x4 areg[3][2 * P];  // [ring slot][k step * P + plane]
 		i32x4 breg[3][8];  // [ring slot][k step * 4 + column block]
 		auto load = [&](int st, i32x4 *ar, i32x4 *br) {
