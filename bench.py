@@ -21,8 +21,8 @@ rotating over 512 MB of distinct copies) and `prefill.long_prompt` (a 4096-token
 model: the matrix-matrix path on the int8 matrix cores).
 `settle_ms` is the pause between the warm-up's synchronisation and the timed region (the host's first launches right
 behind a long wait are slow), `host_pace` the time the host needs to issue 32 steps against the time the device needs to
-run them, and `gemma3_270m` the 270m shape in the launch form the library chooses for it (a replayed graph whose
-position-dependent nodes are updated every step) with the same steps as stream launches beside it.
+run them, and `gemma3_270m` the 270m shape in the launch form the library chooses (the resident step) with the same steps
+as a replayed graph and as stream launches beside it.
 `cpu_baseline` times the reference's single-threaded AVX2 path (oracle/_ref, built from the
 reference's own sources) — or, where that library is absent, the scalar C restatement — on
 this machine's host cores over a bounded sample of the same workload.
@@ -322,9 +322,9 @@ def main():
     from tiny_gemma_amd import weights as tgw
 
     dev = tg.init(0)
-    # the headline model's steps: stream launches unless --graphs; the library's own choice (-1) would be the same for the
-    # 1B shape and updated-graph replay for the 270m shape (its section below runs both)
-    if tg.lib().tg_set_graphs(1 if args.graphs else (0 if (args.model == "1B" or args.stream_launches) else -1)) != 0:
+    # the headline model's steps: the library's own choice (-1: the resident step) unless --graphs or --stream-launches
+    own_mode = 1 if args.graphs else (0 if args.stream_launches else -1)
+    if tg.lib().tg_set_graphs(own_mode) != 0:
         print("bench.py: " + tg.lib().tg_last_error().decode(), file=sys.stderr)
         sys.exit(2)
     if args.prefetch_blocks is not None:
@@ -656,7 +656,7 @@ def main():
                                                    "body": float((t[:, 17] - t[:, 16]).mean() / 100.0),
                                                    "arrive": float((t[:, 18] - t[:, 17]).mean() / 100.0),
                                                    "gemv_wg0_sees_it_after": float((t[:, 4] - t[:, 18]).mean() / 100.0)}
-            L.tg_set_fused_decode(0, 0, 0)
+            L.tg_set_fused_decode(-1, 0, 0)
         launch_floor["one_kernel_step"] = fused
         if not args.graphs and L.tg_set_graphs(1) == 0:
             rates = {}
@@ -670,6 +670,7 @@ def main():
                 tg.synchronize()
                 rates["graph_replay_tok_s" if mode else "stream_tok_s"] = 256 / (1e-3 * ev.elapsed_ms(e0, e1))
             launch_floor.update(rates)
+            L.tg_set_graphs(own_mode)
 
     # ---- long-prompt prefill (the matrix-matrix path) on a fresh session ----
     long_prefill = None
@@ -727,13 +728,14 @@ def main():
             return {"prompt_tokens": n_prompt_s, "prefill_ms": 1e3 * tp, "prefill_tok_s": n_prompt_s / tp, "decode_steps": n_steps,
                     "decode_tok_s": n_steps / td, "ms_per_step": 1e3 * td / n_steps, "host_enqueue_ms_per_step": 1e3 * te / n_steps}
 
-        # The library's own choice for this shape (tg_set_graphs(-1)): replay of a captured step whose position-dependent
-        # nodes are updated before every replay, one graph launch and 36 node updates per step on the host instead of 91
-        # kernel launches.  Beside it the same 256 steps as stream launches, which follow the host wherever the launching
-        # thread sits on a slow core (`host_enqueue_ms_per_step` = `ms_per_step`).
+        # The library's own choice (the resident step).  Beside it the same 256 steps as replay of a captured step whose
+        # position-dependent nodes are updated before every replay, and as stream launches, which follow the host wherever
+        # the launching thread sits on a slow core (`host_enqueue_ms_per_step` = `ms_per_step`).
         L.tg_set_graphs(-1)
         short, long_ctx = run(64, 256), run(16384, 256)
-        short["launch"] = long_ctx["launch"] = "updated hipGraph replay (library default for this shape)"
+        short["launch"] = long_ctx["launch"] = "library default (resident step)"
+        if L.tg_set_graphs(2) == 0:
+            short["updated_graph_replay"] = {k: v for k, v in run(64, 256).items() if k in ("decode_tok_s", "ms_per_step", "host_enqueue_ms_per_step")}
         L.tg_set_graphs(0)
         short["stream_launches"] = {k: v for k, v in run(64, 256).items() if k in ("decode_tok_s", "ms_per_step", "host_enqueue_ms_per_step")}
         short["weight_stream_GBps"] = s_bytes * short["decode_tok_s"] / 1e9
@@ -771,7 +773,7 @@ def main():
             "prompt_tokens": n_prompt,
             "decode_position_start": n_prompt + args.warmup,
             "seed": args.seed,
-            "launch": "hipGraph replay" if args.graphs else ("stream" if (args.model == "1B" or args.stream_launches) else "library default (updated hipGraph replay; stream launches under a profiler)"),
+            "launch": "hipGraph replay" if args.graphs else ("stream" if args.stream_launches else "library default (resident step)"),
         },
         "roofline": {
             "kernel": "tg_gemv_lmhead_argmax",

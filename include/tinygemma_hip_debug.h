@@ -111,13 +111,19 @@ int tg_debug_launch_chain(int n_launches, int workgroups, double *us_per_launch)
 int tg_debug_handover(int rounds, int workgroups, int barrier, int data, int words_per_wg, int max_spins, double *us_per_round,
                       int *timed_out, int *wrong_sums, int *xcd_of_wg);
 /* enable = 1: tg_decode_enqueue / tg_forward_decode run all layers of a decode step as ONE launch of resident workgroups
- * that hand over through device memory (the LM head stays a launch of its own) instead of five launches per layer.
- * Bit-identical results; off by default because it is slower on this machine (a hand-over through memory costs more
- * than a launch boundary).  gemv_workgroups: 0 = one per compute unit less the 16 attention workgroups; max_spins: polls
+ * that hand over through device memory (the LM head stays a launch of its own) instead of five launches per layer, with the
+ * launch path's bits; 0: five launches per layer; -1 (default): left to the library (tg_set_resident_decode).  Slower than
+ * the launches on this machine (a hand-over of everything to everybody costs more than a launch boundary).  gemv_workgroups: 0 = one per compute unit less the 16 attention workgroups; max_spins: polls
  * before a wait between workgroups gives up (0 = 2^20, at most 2^22).  When a wait gives up the next read-back returns
  * TG_ERR_STATE, the decode steps since the previous read-back are invalid, and the session stays on the launch path.
  * Used up to 4096 cached keys; longer contexts take the launch path by themselves. */
 int tg_set_fused_decode(int enable, int gemv_workgroups, int max_spins);
+/* enable = 1 (default): decode steps of the 270m and 1B widths run their layers as one launch of resident workgroups that hand
+ * over inside an XCD where they can (the LM head stays a launch of its own), unless tg_set_graphs or tg_set_fused_decode name
+ * another path, the stream is being captured, or the device is not one of 8 XCDs with 32 compute units.  Sums run in another
+ * order than on the launch path.  max_spins: polls before a wait between workgroups gives up (0 = 2^20, at most 2^22); the
+ * steps since the last read-back are then done again with one launch per product, and the session keeps to that. */
+int tg_set_resident_decode(int enable, int max_spins);
 /* One decode step of the session on the one-kernel path with timestamps of the 100 MHz counter: out[n_layers][24];
  * entries 0..15 of a layer: GEMV workgroup 0 at layer start, after the norms, after its Q|K|V tiles, after arriving, after
  * the wait for the attention, after the merge, after its O tiles, after arriving, after the wait, after the norms, after

@@ -46,9 +46,12 @@ bool g_gemm_split = true;       // prefill: products that would leave most compu
 int g_attn_merge_chunk = 64;  // decode attention: past this many keys per workgroup, use more workgroups and a merge launch
 bool g_chain_picks = true;  // inside a batch of greedy decode steps the next step's first launch finishes the previous pick
 bool g_keep_taps = false;  // prefill keeps a copy of the residual stream after every block (parity checks)
-// Decode: all layers of a step in one launch of resident workgroups (tg_decode_fused.hip) instead of 5 launches per layer.
+// Decode: all layers of a step in one launch of workgroups that keep the launch path's order of sums (tg_decode_fused.hip): 0 no,
+// 1 yes, -1 (default) left to the library, which then takes the resident step (tg_decode_resident.hip) where it can.
 // g_fused_ng: GEMV workgroups of that launch (0: one per compute unit, less the attention workgroups).
-int g_fused = 0, g_fused_ng = 0, g_fused_spins = 1 << 20;
+int g_fused = -1, g_fused_ng = 0, g_fused_spins = 1 << 20;
+bool g_resident = true;              // the resident step may be taken
+int g_resident_spins = 1 << 20;      // polls before one of its waits gives up (0.5 s and more)
 unsigned long long *g_fused_ts = nullptr;  // device buffer of tg_debug_fused_timestamps while it runs
 // Counts changes of the tuning knobs.  A captured decode step bakes the knobs of its capture into its launches
 // (prefetch workgroups, grid limits, attention geometry), so a session drops its captured graphs when this has moved.
@@ -373,6 +376,18 @@ struct tg_session {
 	float *fused_xch = nullptr;
 	unsigned *fused_sync = nullptr;
 	unsigned fused_all = 0, fused_attn = 0;  // host mirrors of the arrival counters
+	// resident decode step (tg_decode_resident.hip): built on first use; state as fused_state
+	int res_state = 0;
+	TgResident res;                    // the launch-independent fields
+	TgResidentLayer *res_layers = nullptr;
+	unsigned *res_xch = nullptr, *res_err = nullptr;
+	struct ResidentSteps {             // steps enqueued since the error block was last read, in runs with the same picks
+		int first, n;                  // log index of the first
+		bool sampling;
+		float minp, temp;
+		int rand_base;
+	};
+	std::vector<ResidentSteps> res_steps;
 };
 
 namespace {
@@ -941,7 +956,7 @@ void tg_session_destroy(tg_session *s) {
 	void *ps[] = {s->cos_g, s->sin_g, s->cos_l, s->sin_l, s->lut, s->xr, s->qkv, s->attn_out, s->o_out, s->hbuf, s->d_out,
 	              s->logits, s->part_acc, s->part_ml, s->merged_acc, s->merged_ml, s->blk_val, s->blk_idx, s->ctr,
 	              s->tok_log, s->pf_ws, s->probs, s->seg, s->bsum, s->bmax, s->randf, s->zeros, s->blk_x, s->blk_y, s->fused_layers,
-	              s->fused_xch, s->fused_sync};
+	              s->fused_xch, s->fused_sync, s->res_layers, s->res_xch, s->res_err};
 	for (void *p : ps)
 		if (p) (void)hipFree(p);
 	s->pf_plan.release();
@@ -1056,6 +1071,12 @@ int tg_session_reset(tg_session *s) {
 	tg_launch_clear(list.data(), (int)list.size(), g_stream);
 	TG_HIP(hipGetLastError());
 	TG_HIP(hipStreamSynchronize(g_stream));
+	if (!s->res_steps.empty()) {  // nothing to do again, but a wait that gave up ends the resident steps of this session
+		unsigned err = 0;
+		s->res_steps.clear();
+		TG_HIP(hipMemcpy(&err, s->res_err, sizeof(err), hipMemcpyDeviceToHost));
+		if (err) s->res_state = -1;
+	}
 	s->kv_clean = true;
 	s->kv_hi = 0;
 	s->pos = s->bp_local = s->bp_global = s->steps = 0;
@@ -1148,6 +1169,8 @@ static int session_usable(const tg_session *s) {
 	if (!s->m || !s->m->loaded) return tg_fail(TG_ERR_STATE, "the session's model has no weights (destroyed, or a load failed)");
 	return TG_OK;
 }
+
+static int enqueue_decode_step(tg_session *s, StepProfile *prof, bool full_grid, const StepOnly *only = nullptr, bool chain = false);
 
 // ---- the one-kernel decode step ---------------------------------------------------------------------------
 static TgFusedMat fused_mat(const PackedMat &p) { return TgFusedMat{p.K, p.C, p.lc_shift, p.ntiles}; }
@@ -1244,7 +1267,7 @@ static int fused_prepare(tg_session *s) {
 
 // Whether the next decode step of the session can run as one launch, and its attention geometry if so.
 static bool fused_usable(tg_session *s, int *chunk_local, int *chunk_global) {
-	if (!g_fused || s->fused_state != 1) return false;
+	if (g_fused <= 0 || s->fused_state != 1) return false;
 	if (s->fused_epoch != g_knob_epoch) {  // the knobs have moved: workgroups of the launch, kernel instantiation
 		s->fused_epoch = g_knob_epoch;
 		s->fused.ng = g_fused_ng > 0 ? g_fused_ng : g_n_cu - TG_FUSED_ATTN_WGS;
@@ -1306,6 +1329,152 @@ static int fused_check(tg_session *s) {
 	TG_HIP(hipMemset(s->fused_sync, 0, sizeof(unsigned) * TG_FUSED_SYNC_WORDS));
 	return tg_fail(TG_ERR_STATE, "one-kernel decode step: a bounded wait between workgroups gave up (the workgroups were not all resident, or the device "
 	                             "is shared); the decode steps since the last read-back are not valid.  Reset the session; it now uses one launch per projection");
+}
+
+// ---- the resident decode step ----------------------------------------------------------------------------------
+// Whether workgroups are dealt to the XCDs of this device as the launch needs it: a fact of the device, asked once.
+static bool resident_device() {
+	static int known_for = -2;
+	static bool known = false;
+	if (known_for != g_device) {
+		known = tg_resident_device(g_n_cu, g_stream);
+		known_for = g_device;
+	}
+	return known;
+}
+
+// Builds the per-session tables of the resident step on first use.  Leaves res_state at 1 (usable) or -1.
+static int resident_prepare(tg_session *s) {
+	if (s->res_state != 0) return TG_OK;
+	s->res_state = -1;
+	tg_model *m = s->m;
+	const tg_config &c = m->cfg;
+	const int L = c.n_layers;
+	if (!tg_resident_shape(c.hidden_size, c.intermediate_size) || !resident_device()) return TG_OK;
+	std::vector<TgResidentLayer> hl((size_t)L);
+	for (int l = 0; l < L; l++) {
+		const LayerDev &Ld = m->L[(size_t)l];
+		hl[(size_t)l] = TgResidentLayer{Ld.qkv.Wg, Ld.o.Wg, Ld.ug.Wg, Ld.d.Wg, Ld.qkv.scales_g, Ld.o.scales_g, Ld.ug.scales_g, Ld.d.scales_g,
+		                                Ld.apre, Ld.apost, Ld.mpre, Ld.mpost, Ld.rms_q, Ld.rms_k, s->kc[(size_t)l], s->vc[(size_t)l], Ld.is_sw ? 1 : 0};
+	}
+	const size_t words = tg_resident_exchange_words(c.hidden_size);
+	TG_HIP(hipMalloc((void **)&s->res_layers, sizeof(TgResidentLayer) * (size_t)L));
+	TG_HIP(hipMalloc((void **)&s->res_xch, sizeof(unsigned) * words));
+	TG_HIP(hipMalloc((void **)&s->res_err, sizeof(unsigned) * 8));
+	TG_HIP(hipMemcpy(s->res_layers, hl.data(), sizeof(TgResidentLayer) * (size_t)L, hipMemcpyHostToDevice));
+	TG_HIP(hipMemset(s->res_xch, 0xff, sizeof(unsigned) * words));
+	TG_HIP(hipMemset(s->res_err, 0, sizeof(unsigned) * 8));
+	TG_HIP(hipDeviceSynchronize());  // the fills are not on the library's stream
+	TgResident &f = s->res;
+	memset(&f, 0, sizeof(f));
+	f.layers = s->res_layers;
+	f.L = L;
+	f.wte = m->wte;
+	f.wte_scales = m->wte_scales;
+	f.vocab = c.n_vocab;
+	f.emb_scale = (float)sqrt((double)c.hidden_size);  // ops.hpp:586
+	f.cos_g = s->cos_g;
+	f.sin_g = s->sin_g;
+	f.cos_l = s->cos_l;
+	f.sin_l = s->sin_l;
+	f.n_pos = c.n_pos;
+	f.n_pos_local = c.n_pos_local;
+	f.lut = s->lut;
+	f.gmin = s->gmin;
+	f.geps = s->geps;
+	f.lut_size = s->lut_size;
+	f.xr = s->xr;
+	f.pend = s->d_out;
+	f.xch = s->res_xch;
+	f.err = s->res_err;
+	s->res_state = 1;
+	return TG_OK;
+}
+
+// Whether the session's next decode step runs as one resident launch: left to the library (a setting of graphs or of the
+// one-kernel step names another path), on a device and for widths it is made for, and not while the stream is captured (a
+// replay would run again with the same place in the exchange buffer).
+static int resident_usable(tg_session *s, bool *yes) {
+	*yes = false;
+	if (!g_resident || g_fused >= 0 || g_use_graphs >= 0 || s->m->net || s->res_state < 0) return TG_OK;
+	hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+	if (hipStreamIsCapturing(g_stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return TG_OK;
+	if (int rc = resident_prepare(s)) return rc;
+	*yes = s->res_state == 1;
+	return TG_OK;
+}
+
+// The layers of a decode step; the LM head follows as a launch of its own.
+static void launch_resident_layers(tg_session *s) {
+	const tg_config &c = s->m->cfg;
+	TgResident f = s->res;
+	f.tok = s->ctr + 4;
+	if (s->pick_pending) {  // this launch finishes the previous step's greedy pick
+		f.am_val = s->blk_val;
+		f.am_idx = s->blk_idx;
+		f.am_n = s->m->lm.ntiles;
+		f.am_ctr = s->ctr;
+		f.am_log = s->tok_log;
+		s->pick_pending = false;
+	}
+	f.pos = s->pos;
+	f.bp_local = s->bp_local;
+	f.bp_global = s->bp_global;
+	f.step = s->steps;
+	f.max_spins = g_resident_spins;
+	tg_launch_decode_resident(f, c.hidden_size, g_stream);
+	s->res.ring = (s->res.ring + c.n_layers) & 3;
+	auto &runs = s->res_steps;
+	const tg_session::ResidentSteps run{s->steps, 1, s->sampling, s->s_minp, s->s_temp, s->rand_base};
+	if (!runs.empty() && runs.back().first + runs.back().n == run.first && runs.back().sampling == run.sampling && runs.back().rand_base == run.rand_base)
+		runs.back().n += 1;
+	else
+		runs.push_back(run);
+}
+
+// After a stream synchronisation: has a wait inside a resident launch given up (the device is shared with something that holds
+// compute units)?  Then that step and all behind it are done again with one launch per product, which the session keeps to from here on.
+static int resident_check(tg_session *s) {
+	if (s->res_steps.empty()) return TG_OK;
+	std::vector<tg_session::ResidentSteps> runs;
+	runs.swap(s->res_steps);
+	unsigned err[8];
+	TG_HIP(hipMemcpy(err, s->res_err, sizeof(err), hipMemcpyDeviceToHost));
+	if (err[0] == 0u) return TG_OK;
+	s->res_state = -1;
+	const int tok = (int)err[1], first = (int)err[3], n = s->steps - first;
+	if (n < 1 || first < runs.front().first) return tg_fail(TG_ERR_STATE, "resident decode step: the error block names no step since the last read-back");
+	s->pos = (int)err[2];
+	s->bp_local -= n;
+	s->bp_global -= n;
+	s->steps = first;
+	const int ctr[5] = {s->pos, s->bp_local, s->bp_global, s->steps, tok};
+	TG_HIP(hipMemcpy(s->ctr, ctr, sizeof(ctr), hipMemcpyHostToDevice));
+	if (err[4]) TG_HIP(hipMemcpy(s->tok_log + first - 1, &tok, sizeof(int), hipMemcpyHostToDevice));  // the pick that launch was to record
+	const bool sampling = s->sampling;
+	const float minp = s->s_minp, temp = s->s_temp;
+	const int rand_base = s->rand_base;
+	int rc = TG_OK;
+	for (size_t r = 0; r < runs.size() && rc == TG_OK; r++) {
+		s->sampling = runs[r].sampling;
+		s->s_minp = runs[r].minp;
+		s->s_temp = runs[r].temp;
+		s->rand_base = runs[r].rand_base;
+		while (s->steps < runs[r].first + runs[r].n && rc == TG_OK) rc = enqueue_decode_step(s, nullptr, false);
+	}
+	s->sampling = sampling;
+	s->s_minp = minp;
+	s->s_temp = temp;
+	s->rand_base = rand_base;
+	if (rc != TG_OK) return rc;
+	TG_HIP(hipStreamSynchronize(g_stream));
+	return TG_OK;
+}
+// For calls that go on from the session's state without reading it back.
+static int resident_settle(tg_session *s) {
+	if (!s || s->res_steps.empty()) return TG_OK;
+	TG_HIP(hipStreamSynchronize(g_stream));
+	return resident_check(s);
 }
 
 // ---- the launches of a decode step, one function per kernel (modules.hpp:135-220, 242-246) ----
@@ -1470,7 +1639,7 @@ static void finish_pick(tg_session *s, bool may_stay) {
 
 // One decode step.  chain: the greedy pick may stay pending for the next step's first launch to finish (the caller
 // flushes after its last step); otherwise the step ends with the finishing launch.
-static int enqueue_decode_step(tg_session *s, StepProfile *prof, bool full_grid, const StepOnly *only = nullptr, bool chain = false) {
+static int enqueue_decode_step(tg_session *s, StepProfile *prof, bool full_grid, const StepOnly *only, bool chain) {
 	if (int rc = session_usable(s)) return rc;
 	tg_model *m = s->m;
 	const tg_config &c = m->cfg;
@@ -1500,16 +1669,21 @@ static int enqueue_decode_step(tg_session *s, StepProfile *prof, bool full_grid,
 	// all layers in one launch where that is possible (not when single kernels are timed or repeated, not in a captured step)
 	int fch_l = 0, fch_g = 0;
 	bool fused = false;
-	if (g_fused && !prof && !only && !full_grid) {
+	if (g_fused > 0 && !prof && !only && !full_grid) {
 		if (int rc = fused_prepare(s)) return rc;
 		fused = fused_usable(s, &fch_l, &fch_g);
 	}
 	const float *last_pend = s->d_out;
+	bool resident = false;
+	if (!prof && !only && !full_grid) {
+		if (int rc = resident_usable(s, &resident)) return rc;
+	}
+	if (resident) launch_resident_layers(s);
 	if (fused) {
 		launch_fused_layers(s, fch_l, fch_g);
 		last_pend = s->fused_xch + (size_t)(L - 1) * s->fused.layer_stride + s->fused.off_d;
 	}
-	for (int l = 0; l < L && !fused; l++) {
+	for (int l = 0; l < L && !fused && !resident; l++) {
 		float *xr_in = s->xr + (size_t)(2 * l) * h, *xr_mid = s->xr + (size_t)(2 * l + 1) * h;
 		TG_MARK(TG_KC_QKV);
 		if (l == 0) {
@@ -1546,13 +1720,24 @@ static int enqueue_decode_step(tg_session *s, StepProfile *prof, bool full_grid,
 
 int tg_forward_decode(tg_session *s, int32_t id, float *logits, int32_t *argmax) {
 	if (int rc = session_usable(s)) return rc;
+	if (int rc = resident_settle(s)) return rc;
 	TG_HIP(hipMemcpyAsync(s->ctr + 4, &id, sizeof(int), hipMemcpyHostToDevice, g_stream));
 	if (int rc = enqueue_decode_step(s, nullptr, false)) return rc;
-	if (logits) TG_HIP(hipMemcpyAsync(logits, s->logits, sizeof(float) * (size_t)s->m->cfg.n_vocab, hipMemcpyDeviceToHost, g_stream));
 	int32_t tok = -1;
-	TG_HIP(hipMemcpyAsync(&tok, s->ctr + 4, sizeof(int), hipMemcpyDeviceToHost, g_stream));
-	TG_HIP(hipStreamSynchronize(g_stream));
+	auto fetch = [&]() -> int {
+		if (logits) TG_HIP(hipMemcpyAsync(logits, s->logits, sizeof(float) * (size_t)s->m->cfg.n_vocab, hipMemcpyDeviceToHost, g_stream));
+		TG_HIP(hipMemcpyAsync(&tok, s->ctr + 4, sizeof(int), hipMemcpyDeviceToHost, g_stream));
+		TG_HIP(hipStreamSynchronize(g_stream));
+		return TG_OK;
+	};
+	if (int rc = fetch()) return rc;
 	if (int rc = fused_check(s)) return rc;
+	if (!s->res_steps.empty()) {
+		if (int rc = resident_check(s)) return rc;
+		if (s->res_state < 0) {  // the step was done again
+			if (int rc = fetch()) return rc;
+		}
+	}
 	if (argmax) *argmax = tok;
 	if (s->taps) {  // taps now describe the decode step
 		s->taps = nullptr;
@@ -1795,6 +1980,8 @@ int tg_decode_enqueue(tg_session *s, int n_steps) {
 		s->graph_epoch = g_knob_epoch;
 	}
 	for (int i = 0; i < n_steps; i++) {
+		bool resident = false;
+		if (int rc = resident_usable(s, &resident)) return rc;
 		if (s->m->net && graph_mode && !s->graphs_failed) {
 			if (s->pos >= s->capacity || s->steps >= s->tok_log_cap) return tg_fail(TG_ERR_STATE, "context is full (n_pos)");
 			const int bound = net_context_bound(s);
@@ -1806,7 +1993,7 @@ int tg_decode_enqueue(tg_session *s, int n_steps) {
 			(void)hipGetLastError();  // a capture the runtime refuses leaves nothing enqueued: plain launches from here on
 			s->graphs_failed = true;
 		}
-		if (s->m->net || !graph_mode || (graph_mode == 2 && g_fused)) {
+		if (s->m->net || !graph_mode || resident || (graph_mode == 2 && g_fused > 0)) {
 			if (int rc = enqueue_decode_step(s, nullptr, false, nullptr, g_chain_picks)) {
 				flush_pick(s);
 				return rc;
@@ -2042,7 +2229,7 @@ int tg_set_chain_picks(int enable) {
 
 int tg_set_fused_decode(int enable, int gemv_workgroups, int max_spins) {
 	if (gemv_workgroups < 0 || max_spins < 0 || max_spins > (1 << 22)) return tg_fail(TG_ERR_BAD_ARG, "bad argument (max_spins <= 2^22)");
-	g_fused = enable != 0;
+	g_fused = enable < 0 ? -1 : enable != 0;
 	g_fused_ng = gemv_workgroups;
 	g_fused_spins = max_spins > 0 ? max_spins : 1 << 20;
 	g_knob_epoch++;
@@ -2067,8 +2254,17 @@ int tg_debug_fused_timestamps(tg_session *s, unsigned long long *out, int n_laye
 	return rc;
 }
 
+int tg_set_resident_decode(int enable, int max_spins) {
+	if (max_spins < 0 || max_spins > (1 << 22)) return tg_fail(TG_ERR_BAD_ARG, "bad argument (max_spins <= 2^22)");
+	g_resident = enable != 0;
+	g_resident_spins = max_spins > 0 ? max_spins : 1 << 20;
+	return TG_OK;
+}
+
 int tg_reset_knobs() {
-	g_fused = 0;
+	g_resident = true;
+	g_resident_spins = 1 << 20;
+	g_fused = -1;
 	g_fused_ng = 0;
 	g_fused_spins = 1 << 20;
 	g_gemm_mfma = 1;
@@ -2105,7 +2301,7 @@ int tg_decode_profile(tg_session *s, int n_steps, double *ms_sum, int *launches)
 		launches[k] = 0;
 	}
 	StepProfile prof;
-	int rc = TG_OK;
+	int rc = resident_settle(s);
 	for (int i = 0; i < n_steps && rc == TG_OK; i++) {
 		prof.used = 0;
 		rc = enqueue_decode_step(s, &prof, false);
@@ -2132,6 +2328,7 @@ int tg_session_read_ids(tg_session *s, int32_t *ids, int max_ids, int *n_out) {
 	if (!s || !ids) return tg_fail(TG_ERR_BAD_ARG, "null argument");
 	TG_HIP(hipStreamSynchronize(g_stream));
 	if (int rc = fused_check(s)) return rc;
+	if (int rc = resident_check(s)) return rc;
 	const int n = std::min(max_ids, s->steps);
 	if (n > 0) TG_HIP(hipMemcpy(ids, s->tok_log, sizeof(int) * (size_t)n, hipMemcpyDeviceToHost));
 	if (n_out) *n_out = n;
@@ -2478,6 +2675,7 @@ int tg_forward_tokens(tg_session *s, const int32_t *ids, int n, const int32_t *w
 		if (want[i] < 0 || want[i] >= n || (i > 0 && want[i] <= want[i - 1])) return tg_fail(TG_ERR_BAD_ARG, "wanted places must ascend within the portion");
 	if (s->pos + n > s->capacity) return tg_fail(TG_ERR_STATE, "context is full (n_pos)");
 	flush_pick(s);
+	if (int rc = resident_settle(s)) return rc;
 	if (s->m->net && n > 1) return net_extend(s, ids, n, want, n_want, logits, nullptr, argmax);
 	// a whole prompt of which only the end is wanted is a prefill
 	if (!s->m->net && s->pos == 0 && n > 1 && (n_want == 0 || (n_want == 1 && want[0] == n - 1)))
@@ -2526,7 +2724,7 @@ static int block_args_ok(tg_session *s, int layer, const float *x, int rows) {
 	const tg_config &c = s->m->cfg;
 	if (!x || rows < 1 || layer < 0 || layer >= c.n_layers) return tg_fail(TG_ERR_BAD_ARG, "bad argument");
 	if (rows > c.n_pos) return tg_fail(TG_ERR_STATE, "more rows than n_pos");
-	return TG_OK;
+	return resident_settle(s);
 }
 
 int tg_session_kv_prefill(tg_session *s, int layer, const float *keys, const float *values, int rows) {
@@ -2670,6 +2868,7 @@ int sampler_prepare(tg_session *s, const float *randf, int n) {
 		TG_HIP(hipMalloc((void **)&s->bmax, sizeof(float) * tg_minp_blocks(c.n_vocab)));
 	}
 	if (n > s->randf_cap) {
+		if (int rc = resident_settle(s)) return rc;
 		TG_HIP(hipStreamSynchronize(g_stream));
 		if (s->randf) (void)hipFree(s->randf);
 		s->randf = nullptr;
@@ -2679,6 +2878,7 @@ int sampler_prepare(tg_session *s, const float *randf, int n) {
 	}
 	// the previous batch of draws may still be in use by launches in flight
 	TG_HIP(hipStreamSynchronize(g_stream));
+	if (int rc = resident_check(s)) return rc;  // which may have to be done again with them
 	TG_HIP(hipMemcpy(s->randf, randf, sizeof(float) * (size_t)n, hipMemcpyHostToDevice));
 	return TG_OK;
 }
@@ -2764,6 +2964,7 @@ int tg_session_tap(tg_session *s, int b, float *out, int rows) {
 	if (b < 0 || b > 2 * c.n_layers) return tg_fail(TG_ERR_BAD_ARG, "no such block");
 	TG_HIP(hipStreamSynchronize(g_stream));
 	if (int rc = fused_check(s)) return rc;
+	if (int rc = resident_check(s)) return rc;
 	if (s->seq) return s->m->loaded ? tg_net_tap(s->seq, b, out, rows) : tg_fail(TG_ERR_STATE, "the session's model has been destroyed");
 	const size_t h = (size_t)c.hidden_size;
 	if (s->taps) {
@@ -2784,6 +2985,7 @@ int tg_session_kv(tg_session *s, int layer, float *keys, float *values, int *pos
 	if (s->seq) return tg_fail(TG_ERR_BAD_ARG, "the session's model has no key/value cache");
 	TG_HIP(hipStreamSynchronize(g_stream));
 	if (int rc = fused_check(s)) return rc;
+	if (int rc = resident_check(s)) return rc;
 	const size_t bytes = sizeof(float) * (size_t)s->max_pos[(size_t)layer] * c.head_dim;
 	if (keys) TG_HIP(hipMemcpy(keys, s->kc[(size_t)layer], bytes, hipMemcpyDeviceToHost));
 	if (values) TG_HIP(hipMemcpy(values, s->vc[(size_t)layer], bytes, hipMemcpyDeviceToHost));

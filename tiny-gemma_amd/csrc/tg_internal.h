@@ -244,6 +244,45 @@ int tg_fused_variant(const TgFused &f);
 bool tg_fused_supported(int n_cu);
 void tg_launch_decode_fused(const TgFused &f, int variant, hipStream_t s);
 
+// ---- resident decode step (tg_decode_resident.hip) --------------------------------------------------------------
+struct TgResidentLayer {
+	const int8_t *Wqkv, *Wo, *Wug, *Wd;      // MFMA tile layout
+	const float *sqkv, *so, *sug, *sd;       // column scales, tile order
+	const float *apre, *apost, *mpre, *mpost, *rms_q, *rms_k;
+	float *kc, *vc;
+	int is_sw;
+};
+struct TgResident {
+	const TgResidentLayer *layers;  // device array [L]
+	int L;
+	int ring;                       // layers run through the exchange buffer before this step, modulo 4
+	// first layer: embedding of the device-side token, or of the previous step's pending greedy pick (see TgGemv)
+	const int8_t *wte;
+	const float *wte_scales;
+	const int *tok;
+	const float *am_val;
+	const int *am_idx;
+	int am_n;
+	int *am_ctr, *am_log;
+	int vocab;
+	float emb_scale;
+	const float *cos_g, *sin_g, *cos_l, *sin_l;  // [n_pos][128]
+	int pos, bp_local, bp_global, n_pos, n_pos_local;
+	int step;                       // token-log index of the token this step picks
+	const float *lut;
+	float gmin, geps;
+	int lut_size;
+	float *xr;                      // [2L+1][hidden] residual stream after every block (all but the last row, which is the head's)
+	float *pend;                    // [hidden] output of the last block, still to be normed and added
+	unsigned *xch;                  // tg_resident_exchange_words; every word 0xffffffff before the first step
+	unsigned *err;                  // [4]: 1 once a wait has given up, then that step's token, position and log index
+	int max_spins;                  // polls before a wait gives up
+};
+bool tg_resident_device(int n_cu, hipStream_t s);
+bool tg_resident_shape(int hidden, int ff);  // widths that have an instance
+size_t tg_resident_exchange_words(int hidden);
+void tg_launch_decode_resident(const TgResident &f, int hidden, hipStream_t s);
+
 // ---- prefill kernels (rows = prompt positions) -----------------------------------------------
 void tg_launch_embed_rows(float *x, const int *ids, int S, const int8_t *wte, const float *scales, int hidden, int vocab,
                           hipStream_t s);
