@@ -496,6 +496,29 @@ def test_decoding_where_the_partials_need_a_fold(tg, folder, n):
     rows_close(s.forward(ids[-1:])[1], want, F32_TOL, f"{n} keys")
 
 
+@pytest.mark.parametrize("n", [63, 64, 65, 128, 2048, 2049, 3072, 3073])
+def test_decoding_at_the_edges_of_tiles_and_parts(tg, folder, n):
+    """A step's tiles hold 64 keys; up to 1024 keys a part is one tile, up to 3072 at most three, behind that the parts are folded."""
+    cfg, path, om, prompt = standout_case(folder, "latent")
+    ids, plain = prompt(n, n // 2)
+    t = om.t
+    h = om.norm("l0.norm1", t["embed"][ids])
+    cache = list(layers.rms_norm(h[:-1] @ t["l0.mix.dkv"].T, t["l0.mix.dkv.norm"], cfg["norm"]["eps"]))
+    want = om.step([cache], ids[-1:], [])
+    s = tg.Transformer.from_dir(path, "float32").open_session(n)
+    s.forward(ids[:-1])
+    rows_close(s.forward(ids[-1:])[1], want, F32_TOL, f"{n} keys")
+
+
+@pytest.mark.parametrize("rank", [192, 193, 512, 513, 768])
+def test_rows_of_every_width_a_step_is_made_for(tg, folder, rank):
+    """768 bytes: three pieces a wave; 2048: eight; wider rows go in tiles of 32 keys."""
+    cfg = nm.config(84, 97, [nm.layer(nm.latent(3, 32, 16, rank, 0.2))])
+    path, om = folder(("row", rank), cfg, seed=12, gain=2.0)
+    check_block(tg, cfg, path, om, "float32", 70)
+
+
+
 def test_long_context_over_several_passes(tg, folder):
     """16,500 tokens: several passes of a prefill, more than 64 keys per workgroup in a decode step.  The last query against
     the oracle (latent attention) and decoding against a portion (both mixers)."""

@@ -830,7 +830,7 @@ __global__ __launch_bounds__(256, 1) void delta_scan_kernel(TgDelta d, const typ
 template <int R>
 __global__ __launch_bounds__(256) void delta_step_kernel(const float *y, TgDelta d, int g_off, int b_off, int a_off, const int *ctr, int host_pos,
                                                          float *o, float *gate, TgTouch touch) {
-	if (tg_touch(touch)) return;
+	if (tg_touch<256>(touch)) return;
 	constexpr int DM = 32 * R;
 	__shared__ __align__(16) float s_q[DM], s_k[DM], s_a[DM], s_z[DM > 256 ? DM : 256], s_v[32], s_g[8][32];
 	__shared__ f32x4_t s_rp[4][8], s_rq[4][8];

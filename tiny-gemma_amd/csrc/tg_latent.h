@@ -18,8 +18,8 @@
 
 #define TG_LATENT_MAX_PARTS TG_VEC_MERGE_MAX  // partials that the value product merges in its prologue
 #define TG_LATENT_MAX_BLOCKS 128   // key parts per launch
-#define TG_LATENT_TILE 32
-#define TG_LATENT_LDS_MAX (150 * 1024)
+#define TG_LATENT_TILE 64          // keys of a part are a multiple of it
+#define TG_LATENT_ROW_MAX 3189     // bytes of a row that is accepted (the step takes up to 3584)
 #define TG_LATENT_HEAD_MAX 256     // largest padded head size of the tiled kernel, and rotated part of a row
 
 // Rotary positions: dims / 2 pairs of a vector, (2i, 2i + 1) or (i, i + dims / 2); elements behind them pass unchanged.
@@ -55,7 +55,6 @@ struct TgLatentStep {
 	int rowp() const { return rankp + rotp; }
 };
 void tg_launch_latent_step(const TgLatentStep &a, int dt, hipStream_t s);
-size_t tg_latent_step_lds(int rowp, int dt);  // LDS the step asks for, besides its static 7 KiB
 // folds nb partials into one (heads: of all groups, padded); out: instead of a partial the normalised sums of the real heads,
 // [groups * heads][out_stride]
 void tg_launch_latent_fold(const float *acc, const float *ml, int nb, int heads_padded, int rankp, float *out_acc, float *out_ml, hipStream_t s);

@@ -5,19 +5,26 @@
 namespace {
 
 // ---- one token -------------------------------------------------------------------------------------------------------------
-// A workgroup takes one part of the keys for 16 heads, tile by tile of 32.  A tile's latent rows go to LDS in one round trip
-// (the first tile's loads are requested before anything else is done), row pitch 16 bytes more than the row.  Scores: wave w
-// takes keys 16 (w % 2) ... and half w / 2 of the latent; the running softmax is a wave's work for 4 heads; the value sum is
-// a product of the probabilities [16 heads x 32 keys] (in the bf16 format two planes, value and remainder) with the tile,
-// wave w the column tiles w, w + 4, ..., NC of them; wider rows take several workgroups (blockIdx.z).
-constexpr int ST = 32;         // keys per tile
-template <bool ROT>
-constexpr int ST_LOADS = ROT ? 10 : 8;  // 16-byte pieces per lane and round of the tile copy
+// A workgroup of 16 waves takes one part of the keys for 16 heads, tile by tile of ST keys.  Scores: wave = 16 keys and a slice of
+// the row; the keys come from memory in operand order (lane = key, 16 bytes of its row), queries and the new token's row
+// through LDS.  The loaded pieces then go to LDS for the value sum, a product of the probabilities
+// [16 heads x ST keys] (in the bf16 format two planes, value and remainder) with the tile, wave = column tiles; wider rows take
+// several workgroups (blockIdx.z).  In between four waves do the softmax, a row of 16 lanes per head.
+// The launch has few workgroups and is a chain of dependent stages: arguments, position, one round trip to memory, three stages
+// behind barriers.  What bounds it beside these latencies is bytes through the unit's L1 (64 a clock: a query row loaded by every
+// wave for itself, 147 KB a workgroup, took 2,300 clocks) and a wave's own issue (four waves that divided a linear index to find a
+// piece's row took 7,600 to 15,700 clocks in front of the first product).  Against four waves and tiles of 32 keys whose scores
+// came from LDS: 1000 keys, 4 heads, rows of 256 bytes 8.2 -> 5.2 us and no fold (3.0); 8 heads, rows of 640 bytes in bf16 11.9 ->
+// 7.4; 4 heads, rows of 640 bytes in fp32 11.0 -> 7.1; a key group of 96 in fp32 8.0 -> 5.9.  Sixteen waves in the softmax are not
+// faster than four (1,450 and 1,060 clocks): there it is the issue of their 16 rows of 64 lanes.
+template <int ST>
+constexpr int ST_SLICES = 256 / ST;  // of the rows in the scores
+constexpr size_t ST_WIDE_LDS = 136 * 1024;  // tiles of 64 keys: LDS beside the static 22 KiB
 
 template <class TR>
-size_t latent_step_lds(int rowp) {  // q' fragments | tile
-	const size_t row = (size_t)rowp * sizeof(typename TR::T);
-	return 16 * row + ST * (row + 16);
+size_t latent_step_lds(int rankp, int rotp, int keys) {  // tile | queries, of wide rows their rotated parts | the new token's row
+	const size_t value = (size_t)rankp * sizeof(typename TR::T), rot = (size_t)rotp * sizeof(typename TR::T);
+	return (size_t)keys * (value + 16) + 16 * ((keys == 64 ? value : 0) + rot + 16) + value + rot;
 }
 
 // Element i of a rotated vector: itself, turned with its partner.
@@ -40,201 +47,208 @@ __device__ __forceinline__ float rotated(const V *x, int i, const float2 *turn, 
 	const Turn r(i, dims, half_layout);
 	return r((float)x[i], (float)x[r.other], turn[r.pair]);
 }
-// e / d for e * d < 2^22, m = 2^22 / d rounded up
-__device__ __forceinline__ int div_by(int e, unsigned m) { return (int)(((unsigned)e * m) >> 22); }
-
-// NC: column tiles of the value part per wave (4 NC tiles of 16 per workgroup).
-template <class TR, bool ROT, int NC>
-__global__ __launch_bounds__(256) void latent_step_kernel(TgLatentStep a) {
-	if (tg_touch(a.touch)) return;
+// MF: pieces of 64 bytes of a row per wave; NC: column tiles of the value part per wave (16 NC tiles of 16 per workgroup).
+template <class TR, bool ROT, int ST, int MF, int NC>
+__global__ __launch_bounds__(1024) void latent_step_kernel(const float *q_rows, const void *cache_rows, const int *ctr, const float *kv_rows, int host_pos, int chunk,
+                                                           int window, int heads, int sizes, int key_bytes, TgLatentStep a) {
+	if (tg_touch<1024>(a.touch)) return;
 	typedef typename TR::T T;
 	typedef typename TR::Frag Frag;
+	constexpr int NS = ST_SLICES<ST>, KT = ST / 16, PLANES = TR::DT == TG_DT_BF16 ? 2 : 1, ROW = 64;
+	constexpr bool SHARE = ST == 64;  // queries meet in LDS: every wave's own copies would be 16 times their bytes through the unit's L1
 	extern __shared__ __align__(16) unsigned char smem[];
-	const int rowp = a.rankp + (ROT ? a.rotp : 0), row = rowp * (int)sizeof(T), pitch = row + 16, ppr = row / 16;  // bytes; 16-byte pieces per row
-	Frag *s_q = reinterpret_cast<Frag *>(smem);  // [rowp / KF][64]
-	unsigned char *s_c = smem + 16 * row;
-	__shared__ float s_half[2][ST][16];
-	__shared__ __align__(16) float s_p[16][ST + 4];
-	__shared__ float s_corr[16], s_sq[4];
-	const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, lr = lane & 15, lg = lane >> 4;
-	const int blocks = (a.heads + 15) / 16, grp = (int)blockIdx.y / blocks, hb = (int)blockIdx.y - grp * blocks;
-	const int part = blockIdx.x, h0 = hb * 16, heads16 = a.groups * blocks * 16, g0 = grp * a.heads;  // (h0: inside the group)
-	const int pos = a.host_pos >= 0 ? a.host_pos : a.ctr[0], ctx = pos + 1, lo = max(0, ctx - a.window);
-	const int kb = lo + part * a.chunk, ke = min(ctx, kb + a.chunk);
-	const size_t key_bytes = (size_t)a.groups * row;
-	unsigned char *cache = (unsigned char *)a.cache + (size_t)grp * row;
-	const float2 *turn = ROT ? a.rot.table + (size_t)pos * (a.rot.dims / 2) : nullptr;
-	constexpr int SL = ST_LOADS<ROT>;
-	const unsigned mppr = ((1u << 22) + (unsigned)ppr - 1) / (unsigned)ppr;  // (32 ppr^2 < 2^22: rows below 5 KiB)
-	typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-	u32x4 piece[SL];
-	// pieces [base, base + 256 * SL) of a tile; the new token's row is not in memory yet: it is written to LDS below
-	auto request = [&](int k0, int base) {
-#pragma unroll
-		for (int i = 0; i < SL; i++) {
-			const int e = min(base + tid + 256 * i, ST * ppr - 1), r = div_by(e, mppr), key = max(min(min(k0 + r, ke - 1), pos - 1), 0);
-			piece[i] = *reinterpret_cast<const u32x4 *>(cache + (size_t)key * key_bytes + (e - r * ppr) * 16);
-		}
-	};
-	auto place = [&](int base) {
-#pragma unroll
-		for (int i = 0; i < SL; i++) {
-			const int e = base + tid + 256 * i, r = div_by(e, mppr);
-			if (e < ST * ppr) *reinterpret_cast<u32x4 *>(s_c + (size_t)r * pitch + (e - r * ppr) * 16) = piece[i];
-		}
-	};
-	const bool mine = pos >= kb && pos < kb + a.chunk;
-	const float *kv = a.kv + (size_t)grp * a.kv_stride;
-	float raw[2], nrm[2];
-#pragma unroll
-	for (int i = 0; i < 2; i++) {
-		const int j = min(tid + 256 * i, a.rank - 1);
-		raw[i] = kv[j];
-		nrm[i] = a.norm ? a.norm[j] : 1.0f;
+	const int rankp = sizes & 0xffff, rotp = ROT ? sizes >> 16 : 0;
+	const int pitch = rankp * (int)sizeof(T) + 16, q0 = SHARE ? 0 : rankp, qpitch = (rankp + rotp - q0) * (int)sizeof(T) + 16;
+	unsigned char *s_c = smem, *s_q = s_c + ST * pitch, *s_new = s_q + 16 * qpitch;  // s_q: [16][qpitch], rows from element q0 on
+	__shared__ __align__(16) float s_part[NS][16][ST + 4];
+	__shared__ __align__(16) T s_p[PLANES][16][ST + TR::KV];
+	__shared__ float s_corr[16];
+	const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 15, lg = lane >> 4;
+	// (read as a scalar: the wave's addresses depend on it)
+	const int pos = host_pos >= 0 ? host_pos : *(const __attribute__((address_space(4))) int *)(unsigned long long)ctr;
+	int grp = blockIdx.y, hb = 0, blocks = 1;
+	if (heads > 16) {
+		blocks = (heads + 15) / 16;
+		grp = (int)blockIdx.y / blocks;
+		hb = (int)blockIdx.y - grp * blocks;
 	}
-	// rotated parts: of the queries (16 * rotp elements, RB of them per lane and pass) and of the new row
-	constexpr int RB = 4;
-	float rx[RB], ro[RB], kx = 0.0f, ko = 0.0f;
-	float2 rt[RB], kt = {0.0f, 0.0f};
-	unsigned mrot = 0;
-	auto rot_request = [&](int base) {
-#pragma unroll
-		for (int i = 0; i < RB; i++) {
-			const int e = min(base + tid + 256 * i, 16 * a.rotp - 1), h = div_by(e, mrot), j = min(e - h * a.rotp, a.rot_size - 1);
-			const Turn r(j, a.rot.dims, a.rot.half_layout);
-			const float *x = a.qr + (size_t)(g0 + min(h0 + h, a.heads - 1)) * a.qr_stride;
-			rx[i] = x[j];
-			ro[i] = x[r.other];
-			rt[i] = turn[r.pair];
-		}
-	};
-	auto rot_place = [&](int base) {
-#pragma unroll
-		for (int i = 0; i < RB; i++) {
-			const int e = base + tid + 256 * i, h = div_by(min(e, 16 * a.rotp - 1), mrot), j = e - h * a.rotp, c = a.rankp + j;
-			const Turn r(j, a.rot.dims, a.rot.half_layout);
-			const float v = j < a.rot_size && h0 + h < a.heads ? r(rx[i], ro[i], rt[i]) : 0.0f;
-			if (e < 16 * a.rotp)
-				reinterpret_cast<T *>(s_q)[((size_t)(c / TR::KF) * 64 + h + 16 * ((c % TR::KF) / TR::KV)) * TR::KV + c % TR::KV] = (T)v;
-		}
-	};
-	if constexpr (ROT) {
-		mrot = ((1u << 22) + (unsigned)a.rotp - 1) / (unsigned)a.rotp;
-		const int j = min(tid, a.rot_size - 1);
-		const Turn r(j, a.rot.dims, a.rot.half_layout);
-		const float *x = a.kr + (size_t)grp * a.kr_stride;
-		kx = x[j];
-		ko = x[r.other];
-		kt = turn[r.pair];
-		rot_request(0);
-	}
-	request(kb, 0);
+	const int g0 = grp * heads, nh = min(heads - hb * 16, 16);
+	const int kfr = (rankp + rotp) / TR::KF, kfv = rankp / TR::KF, kh = (kfr + NS - 1) / NS, slice = w / KT, kt16 = 16 * (w % KT);
+	const int kf_lo = min(slice * kh, kfr), nf = min(kfr - kf_lo, kh);  // (at most MF)
 
-	// q' in operand order: lane = head, 16 bytes of the row
-	const int r4 = a.rankp / 4;
-	const unsigned mr4 = ((1u << 22) + (unsigned)r4 - 1) / (unsigned)r4;
-	for (int base = 0; base < 16 * r4; base += 256 * 8) {
-		f32x4_t v[8];
+	// the queries; no address of them needs the position.  SHARE: wave = head, 4 elements per lane and round; else in operand order
+	const float *q = q_rows + (size_t)(g0 + hb * 16 + min(SHARE ? w : lr, nh - 1)) * a.q_stride + (SHARE ? 4 * lane : lg * TR::KV);
+	f32x4_t q4 = {0, 0, 0, 0};
+	Frag qf[MF];
+	if constexpr (SHARE) {
+		if (w < nh && 4 * lane < rankp) q4 = tg_load4(q);
+	} else {
 #pragma unroll
-		for (int i = 0; i < 8; i++) {
-			const int e = min(base + tid + 256 * i, 16 * r4 - 1), h = div_by(e, mr4);
-			v[i] = tg_load4(a.q + (size_t)(g0 + min(h0 + h, a.heads - 1)) * a.q_stride + (e - h * r4) * 4);
+		for (int i = 0; i < MF; i++) {
+			if (i >= nf || kf_lo + i >= kfv) break;
+#pragma unroll
+			for (int e = 0; e < TR::KV / 4; e++) {
+				const f32x4_t v = tg_load4(q + (kf_lo + i) * TR::KF + 4 * e);
+#pragma unroll
+				for (int c = 0; c < 4; c++) qf[i][4 * e + c] = (T)(lr >= nh || (ROT && (kf_lo + i) * TR::KF + lg * TR::KV + 4 * e + c < a.q_zero) ? 0.0f : v[c]);
+			}
 		}
+	}
+	const int ctx = pos + 1, lo = max(0, ctx - window), part = blockIdx.x, kb = lo + part * chunk, ke = min(ctx, kb + chunk);
+	const bool mine = pos >= kb && pos < kb + chunk;
+	unsigned char *cache = (unsigned char *)const_cast<void *>(cache_rows) + (size_t)grp * (kfr * ROW);
+	// rows past the part's end repeat its last row, with probability 0; the new token's row is not in memory yet
+	Frag tile[MF];
+	auto request = [&](int k0) {
+		const unsigned char *row = cache + (size_t)max(min(min(k0 + kt16 + lr, ke - 1), pos - 1), 0) * (size_t)key_bytes + lg * 16;
 #pragma unroll
-		for (int i = 0; i < 8; i++) {
-			const int e = base + tid + 256 * i, h = div_by(min(e, 16 * r4 - 1), mr4), j = (e - h * r4) * 4;
-			if (h0 + h >= a.heads) v[i] = f32x4_t{0, 0, 0, 0};
+		for (int i = 0; i < MF; i++) {
+			if (i >= nf) break;
+			tile[i] = *reinterpret_cast<const Frag *>(row + (kf_lo + i) * ROW);
+		}
+	};
+	if (kb < ke) request(kb);
+
+	// Element j of a rotated part, requested in front of everything that waits.
+	const float2 *turn = ROT ? a.rot.table + (size_t)pos * (a.rot.dims / 2) : nullptr;
+	struct Rotated {
+		float x, o;
+		float2 t;
+	};
+	auto rot_request = [&](const float *x, int j0) {
+		const int j = min(j0, a.rot_size - 1);
+		const Turn r(j, a.rot.dims, a.rot.half_layout);
+		return Rotated{x[j], x[r.other], turn[r.pair]};
+	};
+	auto rot_value = [&](const Rotated &v, int j) {
+		const Turn r(min(j, a.rot_size - 1), a.rot.dims, a.rot.half_layout);
+		return (T)(j < a.rot_size ? r(v.x, v.o, v.t) : 0.0f);
+	};
+	const float *qr = ROT ? a.qr + (size_t)(g0 + hb * 16 + min(w, nh - 1)) * a.qr_stride : nullptr;
+	Rotated rq = {}, rk = {};
+	float x = 0.0f, g = 1.0f, sq[4];
+	const float *kv = kv_rows + (size_t)grp * a.kv_stride;
+	if (mine) {
+		x = kv[min(tid, a.rank - 1)];
+		if (a.norm) {
+			g = a.norm[min(tid, a.rank - 1)];
+#pragma unroll
+			for (int i = 0; i < 4; i++) sq[i] = kv[min(lane + 64 * i, a.rank - 1)];
+		}
+	}
+	if constexpr (ROT) {
+		if (mine && tid < rotp) rk = rot_request(a.kr + (size_t)grp * a.kr_stride, tid);
+		if (w < nh && lane < rotp) rq = rot_request(qr, lane);
+	}
+	if (mine) {  // the new token's row, its latent normalised, by the workgroups whose part it ends
+		T *dst = reinterpret_cast<T *>(cache + (size_t)pos * (size_t)key_bytes), *row = reinterpret_cast<T *>(s_new);
+		float inv = 1.0f;
+		if (a.norm) {  // (the sum by every wave for itself)
+			float ss = 0.0f;
+#pragma unroll
+			for (int i = 0; i < 4; i++) ss = lane + 64 * i < a.rank ? fmaf(sq[i], sq[i], ss) : ss;
+			for (int j = lane + 256; j < a.rank; j += 64) ss = fmaf(kv[j], kv[j], ss);
+			inv = 1.0f / sqrtf(tg_wave_sum(ss) / (float)a.rank + a.eps);
+		}
+		for (int j = tid; j < rankp; j += 1024) {
+			if (j >= 1024) {
+				x = kv[min(j, a.rank - 1)];
+				g = a.norm ? a.norm[min(j, a.rank - 1)] : 1.0f;
+			}
+			const T c = (T)(j < a.rank ? x * inv * g : 0.0f);
+			row[j] = c;
+			dst[j] = c;
+		}
+		if constexpr (ROT) {
+			if (tid < rotp) {  // (rotp is at most 256)
+				const T c = rot_value(rk, tid);
+				row[rankp + tid] = c;
+				dst[rankp + tid] = c;
+			}
+		}
+	}
+	if constexpr (SHARE) {
+		for (int j = 4 * lane; j < rankp; j += 256) {
+			if (j >= 256 && w < nh) q4 = tg_load4(q + (j - 4 * lane));
 			if constexpr (ROT) {
 #pragma unroll
 				for (int c = 0; c < 4; c++)
-					if (j + c < a.q_zero) v[i][c] = 0.0f;
+					if (j + c < a.q_zero) q4[c] = 0.0f;
 			}
-			if (e < 16 * r4)
-				tg_store4(reinterpret_cast<T *>(s_q) + ((size_t)(j / TR::KF) * 64 + h + 16 * ((j % TR::KF) / TR::KV)) * TR::KV + j % TR::KV, v[i]);
+			tg_store4(reinterpret_cast<T *>(s_q + w * qpitch) + j, q4);
 		}
 	}
 	if constexpr (ROT) {
-		rot_place(0);
-		for (int base = 256 * RB; base < 16 * a.rotp; base += 256 * RB) {
-			rot_request(base);
-			rot_place(base);
+		for (int j = lane; j < rotp; j += 64) {
+			if (j >= 64 && w < nh) rq = rot_request(qr, j);
+			reinterpret_cast<T *>(s_q + w * qpitch)[rankp - q0 + j] = w < nh ? rot_value(rq, j) : (T)0.0f;
 		}
 	}
-	// the new token's latent, normalised, by the workgroups whose part it ends
-	float inv = 1.0f;
-	if (mine && a.norm) {
-		float ss = 0.0f;
-		for (int j = tid, i = 0; j < a.rank; j += 256, i++) {
-			const float x = i < 2 ? raw[i & 1] : kv[j];
-			ss = fmaf(x, x, ss);
-		}
-		ss = tg_wave_sum(ss);
-		if (lane == 0) s_sq[w] = ss;
-		__syncthreads();
-		inv = 1.0f / sqrtf(((s_sq[0] + s_sq[1]) + (s_sq[2] + s_sq[3])) / (float)a.rank + a.eps);
+	if (SHARE || ROT || mine) tg_lds_barrier();
+#pragma unroll
+	for (int i = 0; i < MF; i++) {
+		if (i >= nf) break;
+		if (SHARE || (ROT && kf_lo + i >= kfv)) qf[i] = *reinterpret_cast<const Frag *>(s_q + lr * qpitch + (kf_lo + i) * ROW - q0 * (int)sizeof(T) + lg * 16);
 	}
 
-	const int ct0 = blockIdx.z * (4 * NC) + w, nct = a.rankp / 16;
+	const int ct0 = blockIdx.z * (16 * NC) + w, nct = rankp / 16;
 	f32x4_t acc[NC];
 #pragma unroll
 	for (int c = 0; c < NC; c++) acc[c] = f32x4_t{0, 0, 0, 0};
-	float m[2], l[2];
-#pragma unroll
-	for (int i = 0; i < 2; i++) { m[i] = -INFINITY; l[i] = 0.0f; }
-	const int kfr = rowp / TR::KF, kh = (kfr + 1) / 2, kf_lo = (w >> 1) * kh, kf_hi = min(kfr, kf_lo + kh);
+	float m = -INFINITY, l = 0.0f;
 	for (int k0 = kb; k0 < ke; k0 += ST) {
-		for (int base = 0; base < ST * ppr; base += 256 * SL) {
-			if (base) request(k0, base);
-			place(base);
-		}
-		__syncthreads();
-		if (mine && pos < k0 + ST) {
-			T *dst = reinterpret_cast<T *>(cache + (size_t)pos * key_bytes), *tile = reinterpret_cast<T *>(s_c + (size_t)(pos - k0) * pitch);
-			for (int j = tid, i = 0; j < a.rankp; j += 256, i++) {
-				const int jc = j < a.rank ? j : 0;
-				const float x = i < 2 ? raw[i & 1] : kv[jc], g = i < 2 ? nrm[i & 1] : (a.norm ? a.norm[jc] : 1.0f);
-				const T c = (T)(j < a.rank ? x * inv * g : 0.0f);
-				tile[j] = c;
-				dst[j] = c;
-			}
-			if constexpr (ROT) {
-				if (tid < a.rotp) {  // (rotp is at most 256)
-					const Turn r(tid, a.rot.dims, a.rot.half_layout);
-					const T c = (T)(tid < a.rot_size ? r(kx, ko, kt) : 0.0f);
-					tile[a.rankp + tid] = c;
-					dst[a.rankp + tid] = c;
-				}
-			}
-			__syncthreads();
-		}
-		if (k0 + ST < ke) request(k0 + ST, 0);
-		{
-			const unsigned char *rp = s_c + (size_t)(16 * (w & 1) + lr) * pitch + lg * 16;
-			f32x4_t sc = {0, 0, 0, 0};
-			for (int kf = kf_lo; kf < kf_hi; kf++) sc = TR::mma(*reinterpret_cast<const Frag *>(rp + kf * 64), s_q[kf * 64 + lane], sc);
+		if (mine && (unsigned)(pos - k0 - kt16) < 16u) {
 #pragma unroll
-			for (int e = 0; e < 4; e++) s_half[w >> 1][16 * (w & 1) + 4 * lg + e][lr] = sc[e];
-		}
-		__syncthreads();
-		{
-			// lane: key lane % 32, heads 4 w + lane / 32 and 4 w + 2 + lane / 32
-			const int key = lane & 31;
-#pragma unroll
-			for (int i = 0; i < 2; i++) {
-				const int h = 4 * w + 2 * i + (lane >> 5);
-				const float s = k0 + key < ke ? (s_half[0][key][h] + s_half[1][key][h]) * a.scale : -INFINITY;
-				float mx = fmaxf(s, tg_red_partner<16>(s));
-				mx = tg_row16_max(mx);
-				const float mn = fmaxf(m[i], mx), f = expf(m[i] - mn), p = expf(s - mn);
-				float sum = p + tg_red_partner<16>(p);
-				sum = tg_row16_sum(sum);
-				s_p[h][key] = p;
-				l[i] = l[i] * f + sum;
-				m[i] = mn;
-				if (key == 0) s_corr[h] = f;
+			for (int i = 0; i < MF; i++) {
+				if (i >= nf) break;
+				const Frag f = *reinterpret_cast<const Frag *>(s_new + (kf_lo + i) * ROW + lg * 16);
+				if (k0 + kt16 + lr == pos) tile[i] = f;
 			}
 		}
-		__syncthreads();
+		f32x4_t sc = {0, 0, 0, 0};
+#pragma unroll
+		for (int i = 0; i < MF; i++) {
+			if (i >= nf) break;
+			sc = TR::mma(tile[i], qf[i], sc);
+			if (kf_lo + i < kfv) *reinterpret_cast<Frag *>(s_c + (kt16 + lr) * pitch + (kf_lo + i) * ROW + lg * 16) = tile[i];
+		}
+		tg_store4(&s_part[slice][lr][kt16 + 4 * lg], sc);
+		tg_lds_barrier();
+		if (k0 + ST < ke) request(k0 + ST);
+		if (w < 4) {  // heads 4 w + lg; lane lr: keys KT lr ...
+			const int h = 4 * w + lg;
+			typedef float vec __attribute__((ext_vector_type(KT)));
+			typedef T tvec __attribute__((ext_vector_type(KT)));
+			vec s = *reinterpret_cast<const vec *>(&s_part[0][h][KT * lr]), p;
+#pragma unroll
+			for (int i = 1; i < NS; i++) s += *reinterpret_cast<const vec *>(&s_part[i][h][KT * lr]);
+			float mx = -INFINITY;
+#pragma unroll
+			for (int i = 0; i < KT; i++) {
+				s[i] = k0 + KT * lr + i < ke ? s[i] * a.scale : -INFINITY;
+				mx = fmaxf(mx, s[i]);
+			}
+			const float mn = fmaxf(m, tg_row16_max(mx)), f = expf(m - mn);
+			float sum = 0.0f;
+			tvec hi;
+#pragma unroll
+			for (int i = 0; i < KT; i++) {
+				p[i] = expf(s[i] - mn);
+				hi[i] = (T)p[i];
+				sum += p[i];
+			}
+			*reinterpret_cast<tvec *>(&s_p[0][h][KT * lr]) = hi;
+			if constexpr (PLANES == 2) {
+				tvec rest;
+#pragma unroll
+				for (int i = 0; i < KT; i++) rest[i] = (T)(p[i] - (float)hi[i]);
+				*reinterpret_cast<tvec *>(&s_p[1][h][KT * lr]) = rest;
+			}
+			if (lr == 0) s_corr[h] = f;
+			l = l * f + tg_row16_sum(sum);
+			m = mn;
+		}
+		tg_lds_barrier();
 		if (k0 > kb) {
 #pragma unroll
 			for (int e = 0; e < 4; e++) {
@@ -243,50 +257,36 @@ __global__ __launch_bounds__(256) void latent_step_kernel(TgLatentStep a) {
 				for (int c = 0; c < NC; c++) acc[c][e] *= f;
 			}
 		}
-		// rows past the part's end repeat its last row, with probability 0
+		if (ct0 < nct) {
 #pragma unroll
-		for (int b = 0; b < ST / TR::KF; b++) {
-			Frag ph, pl;
-			f32x4_t pv[TR::KV / 4];
+			for (int b = 0; b < ST / TR::KF; b++) {
+				Frag pf[PLANES];
 #pragma unroll
-			for (int i = 0; i < TR::KV / 4; i++) pv[i] = tg_load4(&s_p[lr][b * TR::KF + lg * TR::KV + 4 * i]);
+				for (int i = 0; i < PLANES; i++) pf[i] = *reinterpret_cast<const Frag *>(&s_p[i][lr][b * TR::KF + lg * TR::KV]);
 #pragma unroll
-			for (int i = 0; i < TR::KV; i++) {
-				const T hi = (T)pv[i / 4][i % 4];
-				ph[i] = hi;
-				pl[i] = (T)(pv[i / 4][i % 4] - (float)hi);
-			}
+				for (int c = 0; c < NC; c++) {
+					const unsigned char *col = s_c + (b * TR::KF + lg * TR::KV) * pitch + (min(ct0 + 16 * c, nct - 1) * 16 + lr) * (int)sizeof(T);
+					Frag cf;
 #pragma unroll
-			for (int c = 0; c < NC; c++) {
-				const int ct = min(ct0 + 4 * c, nct - 1);
-				const T *col = reinterpret_cast<const T *>(s_c + (size_t)(b * TR::KF + lg * TR::KV) * pitch) + ct * 16 + lr;
-				Frag cf;
+					for (int i = 0; i < TR::KV; i++) cf[i] = *reinterpret_cast<const T *>(col + i * pitch);
 #pragma unroll
-				for (int i = 0; i < TR::KV; i++) cf[i] = *reinterpret_cast<const T *>(reinterpret_cast<const unsigned char *>(col) + i * pitch);
-				acc[c] = TR::mma(ph, cf, acc[c]);
-				if constexpr (TR::DT == TG_DT_BF16) acc[c] = TR::mma(pl, cf, acc[c]);
+					for (int i = 0; i < PLANES; i++) acc[c] = TR::mma(pf[i], cf, acc[c]);
+				}
 			}
 		}
-		__syncthreads();
+		if (k0 + ST < ke) tg_lds_barrier();
 	}
-	const int hp = (int)blockIdx.y * 16;  // this block's padded heads
-	float *o = a.part_acc + ((size_t)part * heads16 + hp) * a.rankp;
+	const int heads16 = a.groups * blocks * 16, hp = (int)blockIdx.y * 16;  // hp: this block's padded heads
+	float *o = a.part_acc + ((size_t)part * heads16 + hp) * rankp;
 #pragma unroll
 	for (int c = 0; c < NC; c++) {
-		const int ct = ct0 + 4 * c;
+		const int ct = ct0 + 16 * c;
 		if (ct < nct) {
 #pragma unroll
-			for (int e = 0; e < 4; e++) o[(size_t)(4 * lg + e) * a.rankp + ct * 16 + lr] = acc[c][e];
+			for (int e = 0; e < 4; e++) o[(size_t)(4 * lg + e) * rankp + ct * 16 + lr] = acc[c][e];
 		}
 	}
-	if (blockIdx.z == 0 && (lane & 31) == 0) {
-#pragma unroll
-		for (int i = 0; i < 2; i++) {
-			float *ml = a.part_ml + ((size_t)part * heads16 + hp + 4 * w + 2 * i + (lane >> 5)) * 2;
-			ml[0] = m[i];
-			ml[1] = l[i];
-		}
-	}
+	if (blockIdx.z == 0 && w < 4 && lr == 0) *reinterpret_cast<float2 *>(a.part_ml + ((size_t)part * heads16 + hp + 4 * w + lg) * 2) = float2{m, l};
 }
 
 // groups > 0: the normalised sum of real head (group, head) instead, [groups * heads][out_stride]
@@ -622,16 +622,24 @@ template <class TR>
 void launch_step(const TgLatentStep &a, hipStream_t s) {
 	TgLatentStep t = a;
 	const dim3 grid = tg_touch_grid(dim3((unsigned)a.nb, (unsigned)(a.groups * ((a.heads + 15) / 16)), (unsigned)((a.rankp + 511) / 512)), &t.touch, a.touch_blocks);
-	const size_t lds = latent_step_lds<TR>(a.rowp());
-	auto go = [&](auto *kernel) {
-		if (lds > 48 * 1024) (void)hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-		hipLaunchKernelGGL(kernel, grid, dim3(256), lds, s, t);
+	auto go = [&](auto *kernel, size_t lds) {
+		if (lds > 40 * 1024) (void)hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+		hipLaunchKernelGGL(kernel, grid, dim3(1024), lds, s, a.q, a.cache, a.ctr, a.kv, a.host_pos, a.chunk, a.window, a.heads, a.rankp | a.rotp << 16,
+		                   a.groups * a.rowp() * (int)sizeof(typename TR::T), t);
 	};
-	if (a.rotp && a.rankp <= 128) go(latent_step_kernel<TR, true, 2>);
-	else if (a.rotp && a.rankp <= 256) go(latent_step_kernel<TR, true, 4>);
-	else if (a.rotp) go(latent_step_kernel<TR, true, 8>);
-	else if (a.rankp <= 256) go(latent_step_kernel<TR, false, 4>);
-	else go(latent_step_kernel<TR, false, 8>);
+	// tiles of 64 keys wherever they fit, 32 for wider rows; rows of more than 768 bytes take more pieces per wave
+	const size_t wide = latent_step_lds<TR>(a.rankp, a.rotp, 64), narrow = latent_step_lds<TR>(a.rankp, a.rotp, 32);
+	const size_t row = (size_t)a.rowp() * sizeof(typename TR::T);
+	if (row > 2048 || wide > ST_WIDE_LDS) {
+		if (a.rotp) go(latent_step_kernel<TR, true, 32, 7, 2>, narrow);
+		else go(latent_step_kernel<TR, false, 32, 7, 2>, narrow);
+	} else if (row <= 768 && a.rankp <= 256) {
+		if (a.rotp) go(latent_step_kernel<TR, true, 64, 3, 1>, wide);
+		else go(latent_step_kernel<TR, false, 64, 3, 1>, wide);
+	} else {
+		if (a.rotp) go(latent_step_kernel<TR, true, 64, 8, 2>, wide);
+		else go(latent_step_kernel<TR, false, 64, 8, 2>, wide);
+	}
 }
 }  // namespace
 
@@ -639,8 +647,6 @@ void tg_launch_latent_step(const TgLatentStep &a, int dt, hipStream_t s) {
 	if (dt == TG_DT_BF16) launch_step<TgB16>(a, s);
 	else launch_step<TgF32>(a, s);
 }
-
-size_t tg_latent_step_lds(int rowp, int dt) { return dt == TG_DT_BF16 ? latent_step_lds<TgB16>(rowp) : latent_step_lds<TgF32>(rowp); }
 
 void tg_launch_latent_fold(const float *acc, const float *ml, int nb, int heads_padded, int rankp, float *out_acc, float *out_ml, hipStream_t s) {
 	hipLaunchKernelGGL(latent_fold_kernel, dim3((unsigned)heads_padded, (unsigned)((rankp + 63) / 64)), dim3(256), 0, s, acc, ml, nb, heads_padded, rankp,

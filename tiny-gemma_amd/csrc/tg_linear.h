@@ -75,7 +75,8 @@ struct TgTouch {
 	int first = 0;                       // rows of workgroups (blockIdx.y) in front of the touching ones
 };
 #if defined(__HIPCC__)
-// workgroups of 256 threads, appended to a grid along y; one dword per line of 128 bytes, four in flight per lane
+// workgroups of NT threads, appended to a grid along y; one dword per line of 128 bytes, four in flight per lane
+template <int NT>
 __device__ __forceinline__ bool tg_touch(const TgTouch &t) {
 	if (t.ptr == nullptr || (int)blockIdx.y < t.first) return false;
 	if (blockIdx.z != 0) return true;
@@ -83,11 +84,11 @@ __device__ __forceinline__ bool tg_touch(const TgTouch &t) {
 	const unsigned x = (unsigned)(t.first * (int)gridDim.x + pb) & 7u, q = (unsigned)pb >> 3, Q = (unsigned)nb >> 3;
 	if ((int)x >= t.tiles || q >= Q) return true;
 	const unsigned lps = t.slab >> 7, total = (((unsigned)t.tiles - x + 7u) >> 3) * lps, per = (total + Q - 1) / Q, lo = q * per, hi = min(lo + per, total);
-	for (unsigned i0 = lo + threadIdx.x; i0 < hi; i0 += 4u * 256u) {
+	for (unsigned i0 = lo + threadIdx.x; i0 < hi; i0 += 4u * NT) {
 		int sink = 0;
 #pragma unroll
 		for (unsigned k = 0; k < 4; k++) {
-			unsigned i = i0 + k * 256u;
+			unsigned i = i0 + k * NT;
 			i = i < hi ? i : i0;
 			const unsigned j = i / lps, line = i - j * lps;
 			sink += *(const int *)(t.ptr + (size_t)(x + 8 * j) * t.slab + (size_t)line * 128u);

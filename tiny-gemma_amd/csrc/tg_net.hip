@@ -731,19 +731,18 @@ int norm_kind(const TgNet *n) { return n->cfg.norm == TG_NORM_RMS ? TG_VP_RMS : 
 
 // Latent attention of one token: keys per workgroup and the number of parts for a context of ctx keys.
 void latent_parts(int ctx, int *chunk, int *nb) {
-	// As many parts of one tile as a prologue merges; longer contexts need a fold, whose bytes (a partial sum is as large as
-	// 32 keys with 16 heads) bound the number of parts from above.
-	*chunk = TG_LATENT_TILE;
-	if (ctx > TG_LATENT_TILE * TG_LATENT_MAX_PARTS) {
-		const int want = (ctx + TG_LATENT_MAX_BLOCKS - 1) / TG_LATENT_MAX_BLOCKS;
-		*chunk = std::max(2 * TG_LATENT_TILE, tg_up(want, TG_LATENT_TILE));
-	}
+	// As many parts of one tile as a prologue merges, of up to three tiles for more keys: a tile is 1.4 us, a fold behind the launch
+	// 3.3.  Contexts beyond that need the fold, whose bytes (a partial sum is as large as 32 keys with 16 heads) bound the number
+	// of parts from above.
+	const bool merge = ctx <= 3 * TG_LATENT_TILE * TG_LATENT_MAX_PARTS;
+	const int parts = merge ? TG_LATENT_MAX_PARTS : TG_LATENT_MAX_BLOCKS;
+	*chunk = tg_up(std::max((ctx + parts - 1) / parts, 1), TG_LATENT_TILE);
 	*nb = (ctx + *chunk - 1) / *chunk;
 }
-// Grouped rows: as many parts as the output product merges in its prologue, of two tiles at most; more keys go to more parts that
+// Grouped rows: as many parts as the output product merges in its prologue, of one tile at most; more keys go to more parts that
 // meet in a launch of their own.
 void group_parts(int ctx, int heads, int *chunk, int *nb) {
-	const bool merge = ctx <= 2 * TG_LATENT_TILE * TG_VEC_MERGE_MAX && heads <= TG_VEC_MERGE_HEADS_MAX;
+	const bool merge = ctx <= TG_LATENT_TILE * TG_VEC_MERGE_MAX && heads <= TG_VEC_MERGE_HEADS_MAX;
 	const int parts = merge ? TG_VEC_MERGE_MAX : 64;
 	*chunk = tg_up(std::max((ctx + parts - 1) / parts, 1), TG_LATENT_TILE);
 	*nb = (ctx + *chunk - 1) / *chunk;
@@ -774,7 +773,7 @@ int tg_net_open(const char *dir, int dt, int n_cu, hipStream_t s, TgNet **out) {
 	for (const Arch &k : ARCHS)
 		if (a->str == k.name) rc = k.parse(j, &n->cfg);
 	for (const TgNetLayerCfg &l : n->cfg.layers)
-		if (!rc && l.mix.kind == TG_MIX_LATENT && tg_latent_step_lds(tg_up(l.mix.rank, 64) + l.mix.rotp(), dt) > TG_LATENT_LDS_MAX)
+		if (!rc && l.mix.kind == TG_MIX_LATENT && (size_t)(tg_up(l.mix.rank, 64) + l.mix.rotp()) * tg_dt_bytes(dt) > TG_LATENT_ROW_MAX)
 			rc = tg_fail(TG_ERR_UNSUPPORTED_SHAPE, "kv_rank " + std::to_string(l.mix.rank) + " does not fit the LDS in this number format");
 	if (!rc) rc = load_weights(n, std::string(dir) + "/model.safetensors");
 	if (rc) {
@@ -948,6 +947,7 @@ namespace {
 
 constexpr size_t TOUCH_MIN_BYTES = (size_t)12 << 20, TOUCH_MAX_BYTES = (size_t)14 << 20;
 constexpr int TOUCH_BLOCKS = 128;
+constexpr int TOUCH_BLOCKS_WIDE = 240;  // of 1024 threads, behind an attention launch
 
 // One decode step: the launches of a mixer and of a feed-forward, and the residual stream between them (x, and parts that the next
 // norm adds to it).
@@ -1018,7 +1018,7 @@ struct Step {
 		const TgMixerCfg &m = c.layers[(size_t)l].mix;
 		TgLatentStep t = {};
 		t.touch = touch;
-		t.touch_blocks = touch_blocks;
+		t.touch_blocks = touch_blocks ? TOUCH_BLOCKS_WIDE : 0;
 		t.rot = q->rot[(size_t)r];
 		t.rotp = m.rotp();
 		t.eps = c.eps;
@@ -1192,12 +1192,15 @@ struct Step {
 			o.part_stride = Dp;
 			o.y = q->pend_a;
 			o.x = q->mix;
-			// The state or attention launch of a layer leaves most of the chip and the memory idle for 7 to 12 us: workgroups behind its
+			// The state or attention launch of a layer leaves most of the chip and the memory idle for 6 to 7 us: workgroups behind its
 			// own touch the first part of a wide feed-forward's matrix for the launch after next.  24 MB (width 1152, ff 10368): that
 			// launch 8.2 -> 6.0 us, the state launch 6.9 -> 7.4; 600 tokens and 24 steps 42.7 -> 41.8 ms with 60 % of the matrix, 42.9
 			// with all of it.  6 MB (width 640 in fp32, of which the memory-side cache keeps some): no difference.  At most 14 MB, what the
 			// idle time fetches: steps of 8 layer runs with matrices of 48, 111 and 198 MB 334, 571 and 801 us, with 60 % of the matrix
 			// 333, 600 and 895, without 383, 618 and 869 us.
+			// Behind an attention launch 240 workgroups of 1024 threads: a step of 26 layer runs (width 1152) takes 875 us, with 192 of
+			// them 876, with 32, which outlast the launch, 918, with none 889.  More than 128 of 256 threads behind a state launch, or
+			// more of the matrix: 890 to 915.
 			touch = TgTouch();
 			touch_blocks = 0;
 			if (lc.mlp == TG_FF_DENSE && (size_t)w.gate_up.n * w.gate_up.k * tg_dt_bytes(dt) >= TOUCH_MIN_BYTES) {
