@@ -135,6 +135,26 @@ def test_products_in_parts_of_k(tg, folder, ff, n, dtype):
 
 
 # ---- whole models ------------------------------------------------------------------------------------------------------------
+# rows at the edges of tiles of 16, 32 and 48, more than one of them; feed-forwards that give every tile, with and without parts of K,
+# the last part shorter, waves without a step (few steps a part), columns that fill no tile
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("ff", [600, 4100, 9000])
+def test_products_of_few_rows(tg, folder, ff, dtype):
+    """Feed-forwards of portions of few rows, against the same tokens' rows in the oracle; the tolerance is that of the sums' order (fp32)
+    and of the products' rounding (bf16), as for any number of rows."""
+    cfg = one_layer(nm.delta(1, 1, 8, 8, 2), nm.dense(ff), width=300)
+    path, om = folder(("t_few", ff), cfg, seed=18, edit=zero_mixer)
+    ids, taps = ids_of(cfg, 333), []
+    om.step(om.state(), ids, taps)
+    x0 = om.embed(ids)
+    want = taps[0] - x0
+    s = tg.Transformer.from_dir(path, dtype).open_session(333)
+    for n in (2, 15, 16, 17, 32, 33, 48, 49, 96, 97, 130, 161, 333):
+        s.reset()
+        s.forward(ids[:n])
+        rows_close(s.tap(2, rows=n) - x0[:n], want[:n], TOL[dtype], f"{n} rows")
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("name", nm.TUTELIX)
 def test_prompts_and_decoding(tg, folder, name, dtype):

@@ -1092,8 +1092,177 @@ __global__ __launch_bounds__(256) void linear_thin_kernel(TgGemm g) {
 	if (m0 + lr < g.M && n0 + w < nfr) tg_store4(g.C2 + (size_t)(m0 + lr) * g.ldc2 + (n0 + w) * 16 + 4 * lg, r);
 }
 
+// Few rows: a workgroup takes 16 MT rows x 16 NC columns of a part of K, its four waves a quarter of that each, and their sums meet
+// in LDS.  The waves share no operand, so the loop has no barrier: a wave's weights come from memory in operand order, its rows as
+// whole 128-byte lines that it turns in an LDS area of its own (as operands straight from memory, 16 rows of 64 bytes a load, they
+// cost a unit four times as long: 130 rows x 10368 columns x K 1152 18.6 us).  FEW_AHEAD steps of 128 bytes of K are in flight;
+// steps behind a wave's last are loads past the end of the buffers: zeros.
+constexpr int FEW_AHEAD = 2, FEW_PITCH = 9;  // 16-byte pieces from row to row in LDS: operand reads meet every bank once
+template <class TR, int EPI, int MT, int NC>
+__global__ __launch_bounds__(256, 1) void linear_few_kernel(TgGemm g) {
+	static_assert(EPI == TG_GE_F32 || EPI == TG_GE_GELU, "");
+	typedef typename TR::T T;
+	typedef typename TR::Frag Frag;
+	constexpr int AREA = 16 * MT * FEW_PITCH;  // of a wave
+	constexpr int SIZE = 4 * (AREA > MT * NC * 64 ? AREA : MT * NC * 64);
+	__shared__ f32x4_t smem[SIZE];
+	const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lr = lane & 15, lg = lane >> 4;
+	const int nfr = g.N / 16, kfr = g.K / TR::KF, ntn = (nfr + NC - 1) / NC, ntm = (g.M + 16 * MT - 1) / (16 * MT);
+	int b;
+	{  // as in linear_kernel: a run of the tile order per XCD, so that a weight tile goes into one L2
+		const int total = ntm * ntn * g.kparts, q = total >> 3, r = total & 7, x = (int)blockIdx.x & 7, i = (int)blockIdx.x >> 3;
+		if (i >= q + (x < r ? 1 : 0)) return;
+		b = x * q + min(x, r) + i;
+	}
+	const int part = b / (ntm * ntn);
+	b -= part * ntm * ntn;
+	const int tn = b / ntm, m0 = (b - tn * ntm) * 16 * MT;
+	const int nst = kfr / 2, per = (nst + g.kparts - 1) / g.kparts, p0 = min(part * per, nst), n_part = min(per, nst - p0);
+	const int k0 = p0 + n_part * w / 4, n = p0 + n_part * (w + 1) / 4 - k0;  // this wave's steps
+
+	// views of this workgroup's rows and columns: offsets in them are below 4 GiB whatever the product's size
+	const int rows_here = min(16 * MT, g.M - m0), cols_here = min(NC, nfr - tn * NC);
+	const unsigned lda = (unsigned)(g.lda * (int)sizeof(T)), a_bytes = (unsigned)rows_here * lda, w_bytes = (unsigned)cols_here * (unsigned)kfr * 1024u;
+	const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((unsigned char *)g.A + (size_t)m0 * lda, 0, a_bytes, 0x00020000);
+	const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((unsigned char *)g.W + (size_t)tn * NC * kfr * 1024, 0, w_bytes, 0x00020000);
+	unsigned ao[2 * MT], wo[NC];
+#pragma unroll
+	for (int i = 0; i < 2 * MT; i++) ao[i] = (unsigned)min(8 * i + (lane >> 3), rows_here - 1) * lda + (unsigned)(lane & 7) * 16u;
+#pragma unroll
+	for (int j = 0; j < NC; j++) wo[j] = (unsigned)min(j, cols_here - 1) * (unsigned)kfr * 1024u + (unsigned)lane * 16u;
+	Frag fa[FEW_AHEAD][2 * MT], fb[FEW_AHEAD][2][NC];
+	auto fetch = [&](int set, int s) {
+		const unsigned sa = s < n ? (unsigned)(k0 + s) * 128u : a_bytes;
+#pragma unroll
+		for (int h = 0; h < 2; h++)
+#pragma unroll
+			for (int j = 0; j < NC; j++)
+				fb[set][h][j] = __builtin_bit_cast(Frag, __builtin_amdgcn_raw_buffer_load_b128(rw, wo[j], s < n ? (unsigned)(2 * (k0 + s) + h) * 1024u : w_bytes, 0));
+#pragma unroll
+		for (int i = 0; i < 2 * MT; i++) fa[set][i] = __builtin_bit_cast(Frag, __builtin_amdgcn_raw_buffer_load_b128(ra, ao[i], sa, 0));
+	};
+	Frag *rows = reinterpret_cast<Frag *>(smem) + w * AREA;
+	Frag *put = rows + (lane >> 3) * FEW_PITCH + (lane & 7), *get = rows + lr * FEW_PITCH + lg;
+	f32x4_t acc[MT][NC];
+#pragma unroll
+	for (int i = 0; i < MT; i++)
+#pragma unroll
+		for (int j = 0; j < NC; j++) acc[i][j] = f32x4_t{0, 0, 0, 0};
+#pragma unroll
+	for (int d = 0; d < FEW_AHEAD; d++) fetch(d, d);
+	for (int s = 0; s < n; s += FEW_AHEAD) {
+#pragma unroll
+		for (int d = 0; d < FEW_AHEAD; d++) {
+			__builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+			for (int i = 0; i < 2 * MT; i++) put[8 * i * FEW_PITCH] = fa[d][i];
+#pragma unroll
+			for (int h = 0; h < 2; h++)
+#pragma unroll
+				for (int i = 0; i < MT; i++) {
+					const Frag a = get[16 * i * FEW_PITCH + 4 * h];
+#pragma unroll
+					for (int j = 0; j < NC; j++) acc[i][j] = TR::mma(fb[d][h][j], a, acc[i][j]);
+				}
+			__builtin_amdgcn_sched_barrier(0);
+			fetch(d, s + d + FEW_AHEAD);
+		}
+	}
+	__syncthreads();
+	f32x4_t(*s_acc)[MT * NC][64] = reinterpret_cast<f32x4_t(*)[MT * NC][64]>(smem);
+#pragma unroll
+	for (int i = 0; i < MT; i++)
+#pragma unroll
+		for (int j = 0; j < NC; j++) s_acc[w][i * NC + j][lane] = acc[i][j];
+	__syncthreads();
+	// lane: row lr, columns 4 lg ... of tile (i, j)
+	for (int t = w; t < MT * NC; t += 4) {
+		const int i = t / NC, m = m0 + 16 * i + lr, at = (tn * NC + t - i * NC) * 16 + 4 * lg;
+		f32x4_t r;
+#pragma unroll
+		for (int e = 0; e < 4; e++) r[e] = (s_acc[0][t][lane][e] + s_acc[1][t][lane][e]) + (s_acc[2][t][lane][e] + s_acc[3][t][lane][e]);
+		if (m >= g.M || at >= g.N) continue;
+		if (EPI == TG_GE_GELU) {
+#pragma unroll
+			for (int e = 0; e < 4; e++) r[e] = tg_gelu(r[e]);
+			tg_store4((T *)g.C + (size_t)m * g.ldc + at, r);
+		} else {
+			tg_store4(g.C2 + (size_t)part * g.part_stride + (size_t)m * g.ldc2 + at, r);
+		}
+	}
+}
+
 // 128-row tiles where they fill the device's 512 places (two workgroups per compute unit), then 64 rows, then 32
 bool linear_rows32(int rows, int ntn) { return (rows + 127) / 128 * ntn < 448 && (rows + 63) / 64 * ntn < 256; }
+
+// A product of few rows has few tiles, and each walks all of K at the pace of one workgroup on an otherwise idle compute unit
+// (0.33 us a stage of 128 bytes of K: 53 us for 130 rows x 1152 columns x K 10368 in 45 workgroups).  Its K is cut until the parts
+// fill the 512 places or are down to TG_LINEAR_PART_STAGES stages, whose start-up and sums would cost more than they save.  A
+// Tutelix prompt of 600 tokens in portions of 130 (width 1152, 26 layer runs) with 24 steps behind it: 51.0 -> 45.8 ms.
+constexpr int TG_LINEAR_PART_STAGES = 12;
+int linear_tile_parts(int rows, int N, int K, int dt) {
+	const int ntn = (N + 127) / 128, stages = K * (int)tg_dt_bytes(dt) / 128;
+	if (!linear_rows32(rows, ntn)) return 1;
+	const int tiles = (rows + 31) / 32 * ntn;
+	int p = 1;
+	while (p < 8 && 2 * p * tiles <= 512 && stages / (2 * p) >= TG_LINEAR_PART_STAGES) p *= 2;
+	return p;
+}
+
+// Whether a product that the tiles above would cut into 32 rows runs in linear_few_kernel instead, in which of its instances and, where
+// the consumer can add parts of K, in how many.  Times follow a count of steps of K times rounds of 256 workgroups (0.045 us a unit
+// and 2.5 us for the launch, the first loads and the sums): MT + NC units a step in bf16 (a unit's path to its L1), 1.1 MT NC in fp32
+// (the matrix instructions), 8 and 14 of a 32-row tile; a part costs its way through memory once more.  Measured, us, tiles against
+// the choice here: 130 rows, width 1152, feed-forward 10368: up 17.1 and 13.8 (3 x 4), down 17.8 in 8 parts and 13.7 in 4, mixer
+// output 7.1 and 4.1 (3 x 2 in 2); 9 rows: 10.3 and 8.0, 10.8 and 7.2 (1 x 4); 333 rows, width 640: mixer output in fp32 11.9 and
+// 5.3 (1 x 2), down in bf16 7.9 and 6.4 (2 x 4 in 2); 20 rows, fp32: 14.4 and 5.5, 12.9 and 4.8.
+// Only for sums that depend on the number of rows already: products in parts of K, and, in models whose down projections are
+// (width above 256), the one in front of those.  The others keep one order of sums, so that a prompt's rows are the same bits
+// however long it goes on.
+bool linear_split_sums(int width) { return width > 256; }
+struct LinearFew {
+	int mt, nc, parts;  // mt 0: the tiles
+};
+LinearFew linear_few(int rows, int N, int K, int dt, bool can_part) {
+	const int ntn = (N + 127) / 128, stages = K * (int)tg_dt_bytes(dt) / 128;
+	LinearFew best = {0, 0, 1};
+	if (!linear_rows32(rows, ntn)) return best;
+	auto rounds = [](long long wgs) { return (wgs + 255) / 256; };
+	// costs in 1/32 units; a part's 8 bytes an element at 4 TB/s
+	auto cost_of = [&](long long wgs, int parts, int step) {
+		return rounds(wgs * parts) * ((stages + parts - 1) / parts) * step + (parts > 1 ? (long long)parts * rows * N / 710 : 0);
+	};
+	const int tile_parts = can_part ? linear_tile_parts(rows, N, K, dt) : 1;
+	long long least = cost_of((long long)((rows + 31) / 32) * ntn, tile_parts, 32 * (dt == TG_DT_BF16 ? 8 : 14));
+	static const int shapes[][2] = {{1, 2}, {1, 4}, {2, 4}, {3, 2}, {3, 4}};
+	for (const auto &t : shapes)
+		for (int parts = 1; parts <= (can_part ? 8 : 1) && (parts == 1 || stages / parts >= 4); parts *= 2) {
+			const long long wgs = (long long)((rows + 16 * t[0] - 1) / (16 * t[0])) * ((N / 16 + t[1] - 1) / t[1]);
+			const long long c = cost_of(wgs, parts, dt == TG_DT_BF16 ? 32 * (t[0] + t[1]) : 36 * t[0] * t[1]);
+			if (c < least) {
+				least = c;
+				best = {t[0], t[1], parts};
+			}
+		}
+	return best;
+}
+
+template <class TR, int EPI>
+bool launch_few(const TgGemm &g, hipStream_t s) {
+	if (EPI == TG_GE_GELU ? !linear_split_sums(g.K) : g.kparts < 1) return false;
+	const LinearFew f = linear_few(g.M, g.N, g.K, TR::DT, EPI == TG_GE_F32);
+	if (f.mt == 0) return false;
+	TgGemm p = g;
+	p.kparts = f.parts;
+	const dim3 grid((unsigned)((g.N / 16 + f.nc - 1) / f.nc * ((g.M + 16 * f.mt - 1) / (16 * f.mt)) * f.parts + 7));  // (a run per XCD)
+	auto go = [&](auto *kernel) { hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, p); };
+	if (f.mt == 1 && f.nc == 2) go(linear_few_kernel<TR, EPI, 1, 2>);
+	else if (f.mt == 1) go(linear_few_kernel<TR, EPI, 1, 4>);
+	else if (f.mt == 2) go(linear_few_kernel<TR, EPI, 2, 4>);
+	else if (f.nc == 2) go(linear_few_kernel<TR, EPI, 3, 2>);
+	else go(linear_few_kernel<TR, EPI, 3, 4>);
+	return true;
+}
 
 template <class TR, int EPI>
 void launch_linear_t(const TgGemm &g, hipStream_t s) {
@@ -1114,6 +1283,9 @@ void launch_linear_t(const TgGemm &g, hipStream_t s) {
 				hipLaunchKernelGGL((linear_kernel<TR, EPI, 1, 4, 2, 2, true>), dim3(grid), dim3(256), 0, s, g);
 		}
 		return;
+	}
+	if constexpr (EPI == TG_GE_F32 || EPI == TG_GE_GELU) {
+		if (launch_few<TR, EPI>(g, s)) return;
 	}
 	const int ntn = (g.N + 127) / 128, rows = EPI == TG_GE_TRANS ? g.rows_out : g.M;
 	if constexpr (EPI == TG_GE_F32) {
@@ -1180,18 +1352,10 @@ void tg_launch_vec(const TgVec &v, int dt, int pro, int epi, hipStream_t s) {
 	else launch_vec_dt<TgF32>(v, pro, epi, s);
 }
 
-// A product of few rows has few tiles, and each walks all of K at the pace of one workgroup on an otherwise idle compute unit
-// (0.33 us a stage of 128 bytes of K: 53 us for 130 rows x 1152 columns x K 10368 in 45 workgroups).  Its K is cut until the parts
-// fill the 512 places or are down to TG_LINEAR_PART_STAGES stages, whose start-up and sums would cost more than they save.  A
-// Tutelix prompt of 600 tokens in portions of 130 (width 1152, 26 layer runs) with 24 steps behind it: 51.0 -> 45.8 ms.
-constexpr int TG_LINEAR_PART_STAGES = 12;
 int tg_linear_kparts(int rows, int N, int K, int dt) {
-	const int ntn = (N + 127) / 128, stages = K * (int)tg_dt_bytes(dt) / 128;
-	if (N <= 256 || !linear_rows32(rows, ntn)) return 1;
-	const int tiles = (rows + 31) / 32 * ntn;
-	int p = 1;
-	while (p < 8 && 2 * p * tiles <= 512 && stages / (2 * p) >= TG_LINEAR_PART_STAGES) p *= 2;
-	return p;
+	if (!linear_split_sums(N)) return 1;
+	const LinearFew f = linear_few(rows, N, K, dt, true);
+	return f.mt ? f.parts : linear_tile_parts(rows, N, K, dt);
 }
 
 void tg_launch_linear(const TgGemm &g, int dt, int epi, hipStream_t s) {
