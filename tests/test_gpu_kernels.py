@@ -207,6 +207,19 @@ def test_qgemm_two_workgroups_per_unit_equal_the_other_kernels_and_the_closed_fo
     assert np.array_equal(out[0], _digit_plane_closed_form(A, W, s))
 
 
+@pytest.mark.parametrize("m, i, n", [(777, 1152, 6912), (600, 256, 6912), (640, 640, 6912), (641, 256, 6912), (2100, 1024, 2048), (2303, 2048, 2048)])
+def test_qgemm_in_workgroups_of_half_the_rows(tg, m, i, n):
+    """One or two tiles of 128 rows to a compute unit, which run in workgroups of 64 rows: last blocks that are full, have one row and end
+    inside a wave, K of two groups of four k steps to sixteen.  Integer sums and one rounding: equal to the closed form bit for bit."""
+    A, W, s = gi.gemm_inputs(m, i, n, 43)
+    A[m - 1] *= np.float32(3e3)
+    C = np.full((m, n), np.nan, np.float32)
+    before = tg.gemm_launches()
+    tg.launch_qgemm(C, A, W, s, m, i, n)
+    assert tuple(b - a for a, b in zip(before, tg.gemm_launches())) == (0, 0, 1)
+    assert np.array_equal(C, _digit_plane_closed_form(A, W, s))
+
+
 @pytest.mark.parametrize("m, i, n, few", [(449, 6912, 1152, True), (777, 6912, 1152, True), (896, 256, 1152, True), (897, 256, 1152, False),
                                           (1632, 640, 640, True), (1633, 640, 640, False), (1009, 2048, 256, True), (4096, 256, 256, True),
                                           (4097, 256, 256, False)])

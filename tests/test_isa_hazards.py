@@ -205,3 +205,9 @@ def test_no_register_with_a_result_in_flight_is_touched(tmp_path, source, kernel
         assert len(sizes) == 3, sizes
         for name, size in sizes.items():
             assert size <= (16 if "ILb1ELb0EE" in name else 0), (name, size)
+
+
+def test_the_half_height_kernel_touches_no_register_in_flight(tmp_path):
+    text = _compile(tmp_path, "tg_gemm_mfma.hip")
+    assert "gemm_i8_lds_half_kernel" in text
+    assert violations(text, ["gemm_i8_lds_half_kernel"], check_mfma=True) == []

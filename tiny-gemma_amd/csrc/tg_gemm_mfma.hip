@@ -363,7 +363,8 @@ __global__ __launch_bounds__(GNT) void gemm_i8_kernel(float *C, const int8_t *Ap
 //     and a burst of copies or LDS reads from eight waves fills the queue it goes into and holds the matrix
 //     instructions behind it back.
 // Same integer sums, same epilogue arithmetic: the result equals the other kernels' bit for bit.
-constexpr int LDS_NSLOT = 4, LDS_AW = 3072, LDS_BOFF = 4 * LDS_AW, LDS_SLOT = LDS_BOFF + 4096;
+constexpr int LDS_NSLOT = 4, LDS_AW = 3072;
+constexpr int lds_ring_bytes(int waves) { return LDS_NSLOT * (waves * LDS_AW + 4096); }
 
 template <int OFF>
 __device__ __forceinline__ i32x4 lds_read_frag(unsigned addr) {
@@ -401,12 +402,12 @@ __device__ __forceinline__ void gemm_static_for(F &&f) {
 // while the kernel ran (it lowers the clock under the power limit, by an amount that depends on the operand values).
 __device__ unsigned long long *tg_gemm_clk = nullptr;
 
-template <bool GEGLU, bool LUTLDS>
-__global__ __launch_bounds__(GNT, 2) void gemm_i8_lds_kernel(float *C, const int8_t *Apack, const float *rowinv, const int8_t *Wg,
-                                                             const float *scales, int M, int K, int ldc, const float *lut, float gmin,
-                                                             float geps, float ginv, int lut_size, float *rowmax_part, int ntiles,
-                                                             int mblocks, int ksplit, size_t csplit) {
+// NW waves of 32 rows each
+template <bool GEGLU, bool LUTLDS, int NW>
+__device__ __forceinline__ void gemm_i8_lds(float *C, const int8_t *Apack, const float *rowinv, const int8_t *Wg, const float *scales, int M, int K, int ldc, const float *lut, float gmin,
+                                            float geps, float ginv, int lut_size, float *rowmax_part, int ntiles, int mblocks, int ksplit, size_t csplit) {
 	extern __shared__ __attribute__((aligned(1024))) unsigned char ring[];  // LDS_NSLOT slots; the GeLU table afterwards
+	constexpr int BOFF = NW * LDS_AW, SLOT = BOFF + 4096, BP = 4 / NW, Q = 3 + BP;  // pieces of B, and of both operands, a wave copies per k step
 	const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, hb = lane >> 5;
 	const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
 	unsigned long long *const clkp = tg_gemm_clk;
@@ -439,28 +440,28 @@ __global__ __launch_bounds__(GNT, 2) void gemm_i8_lds_kernel(float *C, const int
 	// compute units with a single workgroup and a few with two, which then set the pace.
 	const int mreal = mblocks / ksplit, z = mblock / mreal;
 	mblock -= z * mreal;
-	const int mtile = mblock * 4 + w;
+	const int mtile = mblock * NW + w;
 	const int nstage = (K >> 5) / ksplit, last = nstage - 1;  // one k step (32 rows of K) per stage; a multiple of 4
 	const unsigned char *bsrc = reinterpret_cast<const unsigned char *>(Wg) + (size_t)tile * (size_t)K * TG_CT + (size_t)z * nstage * 4096 +
-	                            (size_t)w * 1024 + 16 * lane;
+	                            (size_t)w * BP * 1024 + 16 * lane;
 	const unsigned char *asrc = reinterpret_cast<const unsigned char *>(Apack) + (size_t)mtile * (size_t)(K >> 5) * 3 * 1024 +
 	                            (size_t)z * nstage * LDS_AW + 16 * lane;
 	C += (size_t)z * csplit;
-	// piece q of the copy of stage st into a slot: q = 0..2 the planes of this wave's 32 rows, q = 3 its quarter of B.
+	// piece q of the copy of stage st into a slot: q = 0..2 the planes of this wave's 32 rows, from 3 on its share of B.
 	// Stages past the end copy the last stage again, into slots nobody reads any more.
 	auto issue = [&](int st, int slot, int q) __attribute__((always_inline)) {
 		st = st < last ? st : last;
 		if (q < 3)
 			__builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(asrc + (size_t)st * LDS_AW + q * 1024),
-			                                 (__attribute__((address_space(3))) void *)(ring + slot * LDS_SLOT + w * LDS_AW + q * 1024), 16, 0, 0);
+			                                 (__attribute__((address_space(3))) void *)(ring + slot * SLOT + w * LDS_AW + q * 1024), 16, 0, 0);
 		else
-			__builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(bsrc + (size_t)st * 4096),
-			                                 (__attribute__((address_space(3))) void *)(ring + slot * LDS_SLOT + LDS_BOFF + w * 1024), 16, 0, 0);
+			__builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(bsrc + (size_t)st * 4096 + (q - 3) * 1024),
+			                                 (__attribute__((address_space(3))) void *)(ring + slot * SLOT + BOFF + (w * BP + q - 3) * 1024), 16, 0, 0);
 	};
 #pragma unroll
 	for (int st = 0; st < LDS_NSLOT - 1; st++)
 #pragma unroll
-		for (int q = 0; q < 4; q++) issue(st, st, q);
+		for (int q = 0; q < Q; q++) issue(st, st, q);
 
 	i32x16 acc[3][4];
 #pragma unroll
@@ -471,11 +472,11 @@ __global__ __launch_bounds__(GNT, 2) void gemm_i8_lds_kernel(float *C, const int
 			for (int i = 0; i < 16; i++) acc[p][j][i] = 0;
 
 	const unsigned lbase = (unsigned)(size_t)ring;
-	const unsigned aaddr = lbase + w * LDS_AW + 16 * lane, baddr = lbase + LDS_BOFF + (hb * TG_CT + c) * 16;
+	const unsigned aaddr = lbase + w * LDS_AW + 16 * lane, baddr = lbase + BOFF + (hb * TG_CT + c) * 16;
 	LdsFrags f;
 	auto stage = [&](int st, auto uc) __attribute__((always_inline)) {
-		constexpr int U = decltype(uc)::value, O = U * LDS_SLOT;
-		wait_copies_in_flight<4 * (LDS_NSLOT - 2)>();  // this wave's copies of stage st have landed
+		constexpr int U = decltype(uc)::value, O = U * SLOT;
+		wait_copies_in_flight<Q * (LDS_NSLOT - 2)>();  // this wave's copies of stage st have landed
 		tg_lds_barrier();                              // everyone's have; everyone has read stage st - 1
 		f.a[0] = lds_read_frag<O>(aaddr);
 		f.a[1] = lds_read_frag<O + 1024>(aaddr);
@@ -488,7 +489,7 @@ __global__ __launch_bounds__(GNT, 2) void gemm_i8_lds_kernel(float *C, const int
 		gemm_static_for<12>([&](auto ic) {
 			constexpr int i = decltype(ic)::value, p = i >> 2, j = i & 3;
 			mfma_i8_asm<(p < 2)>(acc[p][j], f.b[j], f.a[p]);
-			if constexpr (i % 3 == 2) issue(st + LDS_NSLOT - 1, (U + LDS_NSLOT - 1) % LDS_NSLOT, i / 3);  // into the slot of stage st - 1
+			if constexpr (NW == 4 ? i % 3 == 2 : i >= 2 && i % 2 == 0) issue(st + LDS_NSLOT - 1, (U + LDS_NSLOT - 1) % LDS_NSLOT, NW == 4 ? i / 3 : i / 2 - 1);  // into the slot of stage st - 1
 		});
 	};
 	for (int st0 = 0; st0 < nstage; st0 += 4) {
@@ -511,7 +512,7 @@ __global__ __launch_bounds__(GNT, 2) void gemm_i8_lds_kernel(float *C, const int
 	float *lut_lds = reinterpret_cast<float *>(ring);
 	if (GEGLU && LUTLDS) {
 		__syncthreads();  // every wave is done with the ring
-		for (int i = tid; i < lut_size; i += GNT) lut_lds[i] = lut[i];
+		for (int i = tid; i < lut_size; i += 64 * NW) lut_lds[i] = lut[i];
 		__syncthreads();
 	}
 
@@ -558,6 +559,17 @@ __global__ __launch_bounds__(GNT, 2) void gemm_i8_lds_kernel(float *C, const int
 		clkp[2 * (size_t)blockIdx.x] = __builtin_readcyclecounter() - clk_c0;
 		clkp[2 * (size_t)blockIdx.x + 1] = __builtin_amdgcn_s_memrealtime() - clk_r0;
 	}
+}
+template <bool GEGLU, bool LUTLDS>
+__global__ __launch_bounds__(GNT, 2) void gemm_i8_lds_kernel(float *C, const int8_t *Apack, const float *rowinv, const int8_t *Wg, const float *scales, int M, int K, int ldc, const float *lut, float gmin,
+                                                             float geps, float ginv, int lut_size, float *rowmax_part, int ntiles, int mblocks, int ksplit, size_t csplit) {
+	gemm_i8_lds<GEGLU, LUTLDS, 4>(C, Apack, rowinv, Wg, scales, M, K, ldc, lut, gmin, geps, ginv, lut_size, rowmax_part, ntiles, mblocks, ksplit, csplit);
+}
+// half the rows: where they even out the units' shares (tg_gemm_lds_halves)
+template <bool GEGLU, bool LUTLDS>
+__global__ __launch_bounds__(GNT / 2, 2) void gemm_i8_lds_half_kernel(float *C, const int8_t *Apack, const float *rowinv, const int8_t *Wg, const float *scales, int M, int K, int ldc, const float *lut, float gmin,
+                                                                      float geps, float ginv, int lut_size, float *rowmax_part, int ntiles, int mblocks, int ksplit, size_t csplit) {
+	gemm_i8_lds<GEGLU, LUTLDS, 2>(C, Apack, rowinv, Wg, scales, M, K, ldc, lut, gmin, geps, ginv, lut_size, rowmax_part, ntiles, mblocks, ksplit, csplit);
 }
 
 // ---- few rows (a short prompt): the same product with the reduction split over the four waves ----------------
@@ -784,6 +796,15 @@ static bool tg_gemm_lds_taken(int M, int K, int ntiles) {
 	return g_gemm_lds > 0 && (K & 127) == 0 && 2 * tiles >= g_gemm_lds * g_gemm_lds_cus;
 }
 
+// Whether gemm_i8_lds_kernel's product runs in workgroups of half as many rows.  A unit's share is in whole workgroups: where it is one or two tiles of 128
+// rows, half tiles make the largest share smaller (777 rows of the 1B shape, 378 tiles on 256 units: up 34.6 -> 32.0 us with its
+// quantising, the three products of a feed-forward block 100.5 -> 96.6 us; 600 rows 94.4 -> 87.4).  Above that the shares are
+// even enough and a weight tile is fetched twice as often (2000 rows 209 -> 212 us).
+static bool tg_gemm_lds_halves(int M, int ntiles) {
+	auto share = [&](int waves) { return ((long)ntiles * ((M + 32 * waves - 1) / (32 * waves)) + g_gemm_lds_cus - 1) / g_gemm_lds_cus * waves; };
+	return share(4) <= 8 && share(2) < share(4);
+}
+
 // ntiles tiles of 128 (virtual) columns; epi GEGLU: every tile is 64 up | 64 gate columns and C has ntiles * 64 columns;
 // rowmax_part (GEGLU only, may be null): [tg_gemm_mfma_rows(M)] floats cleared by the caller; max|C[m][:]| is folded into it
 void tg_launch_gemm_mfma(float *C, const int8_t *apack, const float *rowfac, const int8_t *Wg, const float *scales, int M, int K,
@@ -823,24 +844,26 @@ void tg_launch_gemm_mfma(float *C, const int8_t *apack, const float *rowfac, con
 	if (tg_gemm_lds_taken(M, K, ntiles) && (K >> 5) % (4 * ksplit) == 0) {
 		g_gemm_launches[2]++;
 		static bool lds_set = false;
-		constexpr int ring_bytes = LDS_NSLOT * LDS_SLOT;
-		if (!lds_set) {  // 64 KB of dynamic LDS
-			(void)hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_i8_lds_kernel<true, true>), hipFuncAttributeMaxDynamicSharedMemorySize, ring_bytes);
-			(void)hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_i8_lds_kernel<true, false>), hipFuncAttributeMaxDynamicSharedMemorySize, ring_bytes);
-			(void)hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_i8_lds_kernel<false, false>), hipFuncAttributeMaxDynamicSharedMemorySize, ring_bytes);
+		if (!lds_set) {  // up to 64 KB of dynamic LDS
+			(void)hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_i8_lds_kernel<true, true>), hipFuncAttributeMaxDynamicSharedMemorySize, lds_ring_bytes(4));
+			(void)hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_i8_lds_kernel<true, false>), hipFuncAttributeMaxDynamicSharedMemorySize, lds_ring_bytes(4));
+			(void)hipFuncSetAttribute(reinterpret_cast<const void *>(gemm_i8_lds_kernel<false, false>), hipFuncAttributeMaxDynamicSharedMemorySize, lds_ring_bytes(4));
 			lds_set = true;
 		}
-		const int mb = (int)mblocks * ksplit;
-		const dim3 grid((unsigned)(ntiles * mb)), block(GNT);
-		if (geglu && lutlds)
-			hipLaunchKernelGGL((gemm_i8_lds_kernel<true, true>), grid, block, ring_bytes, s, C, apack, rowinv, Wg, scales, M, K, ldc, lut, gmin, geps,
-			                   ginv, lut_size, rmp, ntiles, mb, 1, (size_t)0);
-		else if (geglu)
-			hipLaunchKernelGGL((gemm_i8_lds_kernel<true, false>), grid, block, ring_bytes, s, C, apack, rowinv, Wg, scales, M, K, ldc, lut, gmin, geps,
-			                   ginv, lut_size, rmp, ntiles, mb, 1, (size_t)0);
-		else
-			hipLaunchKernelGGL((gemm_i8_lds_kernel<false, false>), grid, block, ring_bytes, s, C, apack, rowinv, Wg, scales, M, K, ldc, lut, gmin,
-			                   geps, ginv, lut_size, rmp, ntiles, mb, ksplit, csplit);
+		const int waves = tg_gemm_lds_halves(M, ntiles * ksplit) ? 2 : 4, mb = (M + 32 * waves - 1) / (32 * waves) * ksplit;
+		auto go = [&](auto *kernel) {
+			hipLaunchKernelGGL(kernel, dim3((unsigned)(ntiles * mb)), dim3((unsigned)(64 * waves)), lds_ring_bytes(waves), s, C, apack, rowinv, Wg, scales, M, K, ldc, lut,
+			                   gmin, geps, ginv, lut_size, rmp, ntiles, mb, ksplit, csplit);
+		};
+		if (waves == 2) {
+			if (geglu && lutlds) go(gemm_i8_lds_half_kernel<true, true>);
+			else if (geglu) go(gemm_i8_lds_half_kernel<true, false>);
+			else go(gemm_i8_lds_half_kernel<false, false>);
+		} else {
+			if (geglu && lutlds) go(gemm_i8_lds_kernel<true, true>);
+			else if (geglu) go(gemm_i8_lds_kernel<true, false>);
+			else go(gemm_i8_lds_kernel<false, false>);
+		}
 		return;
 	}
 	g_gemm_launches[1]++;
