@@ -184,7 +184,7 @@ __global__ __launch_bounds__(NT) void vec_kernel(const void *a0, const void *a1,
 	int tile0 = 0, tiles_here = 1;
 	const Frag *W = nullptr;
 	const Frag *R = nullptr;  // ROUTE: the router's matrix
-	float late = 0.0f;        // a factor or an addend of the epilogue, requested with the weights
+	float late = 0.0f;        // a factor of the epilogue, requested with the weights (ROUTE: the lane's expert's correction)
 	auto weights = [&] { W = reinterpret_cast<const Frag *>(p.W) + ((size_t)zw * p.zfrags + (size_t)tile0 * p.kfrags) * 64 + lane; };
 	// the rest of the descriptor, in one batch, through the address of the argument block: made opaque here, so that no field can be
 	// fetched earlier (which would end with a wait in front of the first loads)
@@ -262,8 +262,12 @@ __global__ __launch_bounds__(NT) void vec_kernel(const void *a0, const void *a1,
 	};
 	auto load_first = [&] {
 		fetch_rest();
-		if constexpr (PRO == TG_VP_ROUTE) load_router(w);
-		else load(kf0);
+		if constexpr (PRO == TG_VP_ROUTE) {
+			load_router(w);
+			late = p.correction[min(lane & 15, p.experts - 1)];  // (where it is used it was a round trip of its own, 0.4 us of 6.1)
+		} else {
+			load(kf0);
+		}
 	};
 
 	// the vector's prologue: elements [k0, k0 + kn), then zeros that the surplus steps of the last round multiply
@@ -609,7 +613,7 @@ __global__ __launch_bounds__(NT) void vec_kernel(const void *a0, const void *a1,
 		const int e = lane & 15;
 		const float logit = (s_misc[e] + s_misc[16 + e]) + (s_misc[32 + e] + s_misc[48 + e]);
 		const bool is = e < p.experts;
-		const float val = tg_sigmoid(logit), score = is ? tg_choice_score(val, p.correction[is ? e : 0]) : -INFINITY;
+		const float val = tg_sigmoid(logit), score = is ? tg_choice_score(val, late) : -INFINITY;
 		int rank = 0;
 #pragma unroll
 		for (int o = 0; o < 16; o++) {
