@@ -263,6 +263,24 @@ def test_rows_do_not_depend_on_the_workgroups(tg, folder, kind, vdim):
     assert np.array_equal(rows[0], rows[1]) and np.array_equal(rows[0], rows[2])
 
 
+@pytest.mark.parametrize("kind", ["gla", "delta"])
+@pytest.mark.parametrize("dim", [40, 64, 250])
+def test_scores_of_single_row_blocks(tg, folder, kind, dim):
+    """Up to 64 chunks and heads the scores take a workgroup per 16 rows, beyond that one per chunk: the same bits on both sides of the line
+    (16 and 17 chunks of 4 heads), in chunks that end at and inside a row block, for key sizes of slabs that do not exist.  (Prompts of
+    128 tokens and more: below, the decay's low-rank columns are part of another product, with another order of sums.)"""
+    mixer = nm.gla(4, dim, 16) if kind == "gla" else nm.delta(4, 2, dim, 16, 3)
+    cfg = nm.config(40, 97, [nm.layer(mixer)]) if kind == "gla" else nm.tutelix(40, 97, [nm.layer(mixer)])
+    path, _ = folder(("row_blocks", kind, dim), cfg, seed=28)
+    s = tg.Transformer.from_dir(path, "float32").open_session(1100)
+    ids = ids_of(cfg, 1100)
+    want = s.forward(ids, np.arange(1024))[1]
+    for n in (129, 143, 144, 145, 191, 192, 193, 1024, 1025):
+        s.reset()
+        places = np.arange(min(n, 1024))
+        assert np.array_equal(s.forward(ids[:n], places)[1], want[places]), n
+
+
 @pytest.mark.parametrize("design,width,dtype", [(d, w, "float32") for d in ("madevik", "tutelix") for w in (1024, 1025, 1152, 1153, 2048, 2049)] +
                          [(d, w, "bfloat16") for d in ("madevik", "tutelix") for w in (1024, 1025, 2048, 2049, 2304, 2305)])
 def test_norms_of_every_length(tg, folder, design, width, dtype):

@@ -83,11 +83,11 @@ __global__ __launch_bounds__(256) void gla_step_kernel(const float *y, TgGla g, 
 }
 
 // ---- running sums of log alpha inside every chunk: 64 channels per workgroup, a wave per 16 tokens ----------------------------
-__global__ __launch_bounds__(256) void gla_decay_kernel(const float *low, int ld_low, TgGla g, int n, float *b) {
+__device__ __forceinline__ void gla_decay(const float *low, int ld_low, const TgGla &g, int n, float *b, int chunk, int group) {
 	__shared__ __align__(16) float s_low[C][20];
 	__shared__ float s_sum[4][64];
-	const int hd = g.heads * g.dimp, tid = threadIdx.x, lane = tid & 63, w = tid >> 6, t0 = blockIdx.x * C;
-	const int c = blockIdx.y * 64 + lane, cc = min(c, hd - 1);
+	const int hd = g.heads * g.dimp, tid = threadIdx.x, lane = tid & 63, w = tid >> 6, t0 = chunk * C;
+	const int c = group * 64 + lane, cc = min(c, hd - 1);
 	const bool real = c < hd && cc % g.dimp < g.dim;
 	// softplus(z) = -log(sigmoid(-z))
 	const float bias = g.a2b[cc], flip = g.a_log ? -1.0f : 1.0f, rate = g.a_log ? expf(g.a_log[cc / g.dimp]) : g.inv_tau;
@@ -129,12 +129,15 @@ __global__ __launch_bounds__(256) void gla_decay_kernel(const float *low, int ld
 #pragma unroll
 		for (int i = 0; i < 16; i++) b[(size_t)(t0 + 16 * w + i) * hd + c] = before + z[i];
 }
+__global__ __launch_bounds__(256) void gla_decay_kernel(const float *low, int ld_low, TgGla g, int n, float *b) {
+	gla_decay(low, ld_low, g, n, b, (int)blockIdx.x, (int)blockIdx.y);
+}
 
 // ---- A: a workgroup per chunk and head, a wave per block of 16 rows ---------------------------------------------------------
 // NS groups of four waves stage a slab of key channels each, and each then takes all of these slabs, in order, for its own
 // share of the sums (block columns of A, columns of the diagonal block).  No sum is split, so its bits do not depend on NS: a
 // router behind these rows picks another expert at a near-tie for one of the last place.  A portion of 130 tokens with four
-// heads has 12 workgroups, each a chain of four slabs: 30 us with one group at key size 128, 16.8 with four.
+// heads has 12 workgroups, each a chain of four slabs: 30 us with one group at key size 128, 16.1 with four, 11.6 with four in SPLIT.
 constexpr int SL = 32, SLP = 36;  // key channels per slab, row pitch
 
 // DELTA: also k . k with the decay between them, T = beta (k . k) below the diagonal, of which it leaves -T outside the 16 x 16
@@ -145,13 +148,15 @@ struct DeltaIntra {
 	float *t;           // [chunks][heads][64][64]
 };
 
-template <class TR, bool DELTA, int NS>
-__global__ __launch_bounds__(256 * NS) void gla_intra_kernel(const typename TR::T *qkv, int ld, int k_off, TgGla g, int n, const float *b, float *A,
-                                                             DeltaIntra x) {
+// SPLIT: a workgroup per block of 16 rows (NS waves, one to a slab and its share), which stages the rows up to its own.
+template <class TR, bool DELTA, int NS, bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? 64 * NS : 256 * NS) void gla_intra_kernel(const typename TR::T *qkv, int ld, int k_off, TgGla g, int n, const float *b, float *A,
+                                                                               DeltaIntra x) {
 	typedef float Slab[C][SLP];
-	constexpr int OWN = 4 / NS;
+	constexpr int OWN = 4 / NS, GROUP = SPLIT ? 64 : 256;  // threads that stage a slab
 	__shared__ __align__(16) float s_all[NS][3][C][SLP];
-	const int ch = blockIdx.x, h = blockIdx.y, kh = DELTA ? h / g.group : h, sg = threadIdx.x >> 8, tid = threadIdx.x & 255, lane = tid & 63, w = tid >> 6;
+	const int ch = blockIdx.x, h = blockIdx.y, kh = DELTA ? h / g.group : h, sg = threadIdx.x / GROUP, tid = threadIdx.x % GROUP, lane = tid & 63;
+	const int w = SPLIT ? (int)blockIdx.z : tid >> 6, rows = SPLIT ? 16 * (w + 1) : C;
 	const int lr = lane & 15, lg = lane >> 4, hd = g.heads * g.dimp, t0 = ch * C, qi = 16 * w + lr, j0 = sg * OWN;
 	f32x4_t off[OWN], koff[OWN];
 	float dia[OWN], kdia[OWN];
@@ -163,18 +168,29 @@ __global__ __launch_bounds__(256 * NS) void gla_intra_kernel(const typename TR::
 	for (int base = 0; base < g.dimp; base += SL * NS) {
 		const int d0 = base + SL * sg;
 		__syncthreads();
-		for (int e = tid; d0 < g.dimp && e < C * SL / 4; e += 256) {
-			const int r = e / (SL / 4), c4 = (e % (SL / 4)) * 4, t = t0 + r;
-			const size_t col = (size_t)h * g.dimp + d0 + c4, kcol = (size_t)kh * g.dimp + d0 + c4;
-			f32x4_t q = tg_load4(qkv + (size_t)min(t, n - 1) * ld + kcol), k = tg_load4(qkv + (size_t)min(t, n - 1) * ld + k_off + kcol);
+		// two pieces of each array at a time
+		for (int e0 = tid; d0 < g.dimp && e0 < rows * SL / 4; e0 += 2 * GROUP) {
+			f32x4_t q[2], k[2], bb[2];
 #pragma unroll
-			for (int i = 0; i < 4; i++) {
-				q[i] = t < n ? q[i] * g.qscale : 0.0f;
-				k[i] = t < n ? k[i] : 0.0f;
+			for (int u = 0; u < 2; u++) {
+				const int e = e0 + u * GROUP, r = e / (SL / 4), c4 = (e % (SL / 4)) * 4, t = t0 + r;  // (rows is a multiple of 16: both pieces exist)
+				const size_t col = (size_t)h * g.dimp + d0 + c4, kcol = (size_t)kh * g.dimp + d0 + c4;
+				q[u] = tg_load4(qkv + (size_t)min(t, n - 1) * ld + kcol);
+				k[u] = tg_load4(qkv + (size_t)min(t, n - 1) * ld + k_off + kcol);
+				bb[u] = tg_load4(b + (size_t)t * hd + col);
 			}
-			tg_store4(&s_all[sg][0][r][c4], q);
-			tg_store4(&s_all[sg][1][r][c4], k);
-			tg_store4(&s_all[sg][2][r][c4], tg_load4(b + (size_t)t * hd + col));
+#pragma unroll
+			for (int u = 0; u < 2; u++) {
+				const int e = e0 + u * GROUP, r = e / (SL / 4), c4 = (e % (SL / 4)) * 4, t = t0 + r;
+#pragma unroll
+				for (int i = 0; i < 4; i++) {
+					q[u][i] = t < n ? q[u][i] * g.qscale : 0.0f;
+					k[u][i] = t < n ? k[u][i] : 0.0f;
+				}
+				tg_store4(&s_all[sg][0][r][c4], q[u]);
+				tg_store4(&s_all[sg][1][r][c4], k[u]);
+				tg_store4(&s_all[sg][2][r][c4], bb[u]);
+			}
 		}
 		__syncthreads();
 		for (int sl = 0; sl < NS && base + SL * sl < g.dimp; sl++) {
@@ -575,12 +591,19 @@ template <class TR, bool DELTA>
 void launch_intra(const typename TR::T *qkv, int ld, int k_off, const TgGla &g, int n, const float *b, float *A, const DeltaIntra &x, hipStream_t s) {
 	const dim3 grid((unsigned)((n + C - 1) / C), (unsigned)g.heads);
 	auto go = [&](auto *kernel, int groups) { hipLaunchKernelGGL(kernel, grid, dim3(256 * groups), 0, s, qkv, ld, k_off, g, n, b, A, x); };
+	// Up to a quarter of the units a workgroup per 16 rows, which then has a unit's vector instructions to itself: the exponentials of
+	// four row blocks on one unit set the time (delta rule, 12 workgroups, key size 128: 16.1 -> 11.6 us; 24, key size 64, fp32 12.2 -> 9.2;
+	// gated linear attention, 64, key size 64: 7.2 -> 6.9)
+	if (g.dimp > 32 && grid.x * grid.y <= 64) {
+		hipLaunchKernelGGL((gla_intra_kernel<TR, DELTA, 4, true>), dim3(grid.x, grid.y, 4), dim3(256), 0, s, qkv, ld, k_off, g, n, b, A, x);
+		return;
+	}
 	// Four groups fill a compute unit; with more workgroups than units two share one (delta rule, key size 128: 256 workgroups 19.4
 	// us with four groups, 21.2 with two, 31.1 with one; 512: 36.0, 31.7 and 37.0; 1024: 71.3, 56.5 and 55.6; key size 64,
 	// 256: 13.4, 13.8 and 18.7)
-	if (g.dimp <= 32) go(gla_intra_kernel<TR, DELTA, 1>, 1);
-	else if (grid.x * grid.y <= 256) go(gla_intra_kernel<TR, DELTA, 4>, 4);
-	else go(gla_intra_kernel<TR, DELTA, 2>, 2);
+	if (g.dimp <= 32) go(gla_intra_kernel<TR, DELTA, 1, false>, 1);
+	else if (grid.x * grid.y <= 256) go(gla_intra_kernel<TR, DELTA, 4, false>, 4);
+	else go(gla_intra_kernel<TR, DELTA, 2, false>, 2);
 }
 
 template <class TI, class TR, int VB, bool DELTA>
@@ -626,19 +649,28 @@ void launch_rows(const TgGla &g, const void *qkv, int ld, int k_off, int v_off, 
 // Chunked form: with the notation above and T_ij = beta_i sum_d k_id k_jd e^{b_id - b_jd} (j < i),
 //     (1 + T) u = beta (v - (k e^b)^T S),   o_i = (q_i e^{b_i})^T S + sum_{j <= i} A_ij u_j,
 //     S' = diag(e^{b_end}) S + sum_j (k_j e^{b_end - b_j}) u_j^T.
-// Launches: convolution and unit norms; b; A, T and the solved keys and values, all chunks at once; the pass over the chunks
+// Launches: convolution, unit norms and b; A, T and the solved keys and values, all chunks at once; the pass over the chunks
 // (u and the state in front of each), 16 value columns per workgroup; the outputs, all chunks at once.
 
 // ---- convolution, silu, unit norm: 8 tokens per wave; y: q heads, k heads, blocks of 256 value channels ------------------------------
 // Inputs before the portion come from the ring.
 // TAPS: the number of taps where it is one of the usual ones (every input row is then read once), else 0.
+// The workgroups behind these take the running sums of the decay, which need neither's results (130 tokens, 4 heads, 128 x 256:
+// 12.2 us together, 10.6 and 6.6 as two launches).
 constexpr int PT = 8;
 template <class TR, int TAPS>
-__global__ __launch_bounds__(256) void delta_prep_kernel(TgDelta d, const typename TR::T *x, int ld, int n, int past, float *qk, float *v_out) {
-	const int t0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * PT, lane = threadIdx.x & 63, kvh = d.g.heads / d.g.group, qc = d.q_channels();
+__global__ __launch_bounds__(256) void delta_prep_kernel(TgDelta d, const typename TR::T *x, int ld, int n, int past, float *qk, float *v_out, const float *low,
+                                                         int ld_low, float *b, int bx, int own) {
+	if ((int)blockIdx.x >= own) {
+		const int i = (int)blockIdx.x - own, chunks = (n + C - 1) / C;
+		gla_decay(low, ld_low, d.g, n, b, i % chunks, i / chunks);
+		return;
+	}
+	const int by = (int)blockIdx.x / bx, t0 = (((int)blockIdx.x - by * bx) * 4 + (threadIdx.x >> 6)) * PT, lane = threadIdx.x & 63;
+	const int kvh = d.g.heads / d.g.group, qc = d.q_channels();
 	if (t0 >= n) return;
-	const bool head = (int)blockIdx.y < 2 * kvh;
-	const int base = head ? (int)blockIdx.y * d.g.dimp : 2 * qc + ((int)blockIdx.y - 2 * kvh) * 256;
+	const bool head = by < 2 * kvh;
+	const int base = head ? by * d.g.dimp : 2 * qc + (by - 2 * kvh) * 256;
 	const int len = head ? d.g.dimp : min(256, d.channels - base);  // (at most 256)
 	const int c = base + min(4 * lane, len - 4);
 	const bool in = 4 * lane < len;
@@ -1018,13 +1050,13 @@ void launch_delta_rows(const TgDelta &d, const void *xv, int ld, const float *lo
 	const int qc = d.q_channels(), hv = g.heads * g.vdimp, hd = g.heads * g.dimp, kvh = g.heads / g.group;
 	const unsigned chunks = (unsigned)((n + C - 1) / C);
 	auto prep = [&](auto *kernel) {
-		hipLaunchKernelGGL(kernel, dim3((unsigned)((n + 4 * PT - 1) / (4 * PT)), (unsigned)(2 * kvh + (hv + 255) / 256)), dim3(256), 0, s, d, x, ld, n, past,
-		                   t.qk, t.v);
+		const int bx = (n + 4 * PT - 1) / (4 * PT), own = bx * (2 * kvh + (hv + 255) / 256);
+		hipLaunchKernelGGL(kernel, dim3((unsigned)own + chunks * (unsigned)((hd + 63) / 64)), dim3(256), 0, s, d, x, ld, n, past, t.qk, t.v, low + a_off, ld_low,
+		                   t.b, bx, own);
 	};
 	if (d.taps == 4) prep(delta_prep_kernel<TR, 4>);
 	else if (d.taps == 3) prep(delta_prep_kernel<TR, 3>);
 	else prep(delta_prep_kernel<TR, 0>);
-	hipLaunchKernelGGL(gla_decay_kernel, dim3(chunks, (unsigned)((hd + 63) / 64)), dim3(256), 0, s, low + a_off, ld_low, g, n, t.b);
 	launch_intra<TgF32, true>(t.qk, 2 * qc, qc, g, n, t.b, t.a, DeltaIntra{low + b_off, ld_low, t.t}, s);
 	const DeltaSolve solve = {t.qk, t.b, t.t, low + b_off, 2 * qc, qc, ld_low, t.v, t.u, t.wk, t.kt};
 	hipLaunchKernelGGL(delta_solve_kernel, dim3(chunks, (unsigned)g.heads, (unsigned)((g.dimp + g.vdimp + 127) / 128)), dim3(256), 0, s, solve, g, n);
