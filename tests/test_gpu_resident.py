@@ -1,5 +1,5 @@
 """GPU: the resident decode step (tg_set_resident_decode; tiny-gemma_amd/csrc/tg_decode_resident.hip), which decode steps take
-unless a knob names another path, against the launch path, which the other tests hold to the CPU checker.
+unless a knob names another path, against the launch path, which the other tests hold to the oracle.
 
 Both compute the same sums in another order and both round at 2^-24 or finer, so with a near-continuous GeLU table a block's
 output differs by a few 1e-7 norm-relative (measured 2e-7 .. 6e-7) and nothing amplifies that within two layers: BOUND leaves
